@@ -53,8 +53,8 @@ FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 vector (and matrix) dense peak
 FP32_PEAK_TFLOPS = 157.3
 LANE_MAX_COMP = 162       # classes up to this many components run one quartet per lane
 PROF_SLOTS = 432          # profiling slots: 72 kind + 36 precision + 6 X + Y
-ROW_KINDS = {1: "true, true", 2: "false, true", 3: "false, false"}   # k_eri_rows <TL, FB>
-GROUP_KINDS = {4: 2, 5: 4}                                            # k_eri_rows_mb <NBR>
+LDS_TAB_MAX_ROOTS = 3     # roots whose table the kernels without LDS rows stage
+ROW_KINDS = {1: "1, true", 2: "1, false", 3: "2, false"}   # k_fock <ROWS, TL>
 MODEL = os.path.join(ROOT, "unomol_amd", "models", "guess_631gs.bin")
 
 
@@ -200,21 +200,17 @@ def class_table(ms, launches, prim, shell):
 
 def kernel_name(cls):
     """Demangled name of the Fock-build kernel of a class entry (as rocprofv3 prints it):
-    kind 0 the wave-task (lane classes) or per-quartet wave kernel, kinds 1-3 the
-    row-merged kernel variants."""
+    kinds 1-3 the row-merged variants of the lane kernel, kind 0 the one without LDS rows or
+    (larger classes) the one-quartet-per-wave kernel."""
     X, Y = PAIR_NAME.index(cls["class"][1:3]), PAIR_NAME.index(cls["class"][4:6])
     la, lb = PAIR_L[X]
     lc, ld = PAIR_L[Y]
     t = "float" if cls["precision"] == "f32" else "double"
-    if cls.get("kind", 0) in GROUP_KINDS:
-        return "void uno::k_eri_rows_mb<%d, %d, %d, %d, 0, %s, %d>(uno::EriArgs)" % (la, lb, lc, ld, t,
-                                                                                     GROUP_KINDS[cls["kind"]])
-    if cls.get("kind", 0):
-        return "void uno::k_eri_rows<%d, %d, %d, %d, 0, %s, %s>(uno::EriArgs)" % (la, lb, lc, ld, t,
-                                                                                  ROW_KINDS[cls["kind"]])
-    lane = ncart(la) * ncart(lb) * ncart(lc) * ncart(ld) <= LANE_MAX_COMP
-    return "void uno::%s<%d, %d, %d, %d, 0, %s>(uno::EriArgs)" % ("k_eri_bra" if lane else "k_eri_wave", la, lb, lc,
-                                                                  ld, t)
+    if ncart(la) * ncart(lb) * ncart(lc) * ncart(ld) > LANE_MAX_COMP:
+        return "void uno::k_fock_wave<%d, %d, %d, %d, 0, %s>(uno::FockArgs)" % (la, lb, lc, ld, t)
+    table = "true" if (la + lb + lc + ld) // 2 + 1 <= LDS_TAB_MAX_ROOTS else "false"
+    return "void uno::k_fock<%d, %d, %d, %d, 0, %s, %s>(uno::FockArgs)" % (
+        la, lb, lc, ld, t, ROW_KINDS.get(cls.get("kind", 0), "0, " + table))
 
 
 def traffic_of(kernel):

@@ -70,7 +70,7 @@ int uno_ctx_destroy(uno_ctx* ctx);
  * takes over when the iteration does not converge; uno_ctx_get "x_newton_steps" reads the
  * last SCF's step count, -1 for the canonical X), "rebuild_every" (incremental builds
  * between full rebuilds; default 10), "deterministic" (1: Fock builds accumulate J and K
- * in 128-bit fixed point with integer atomics, every bra as wave tasks, and uno_scf_run's
+ * in 128-bit fixed point with integer atomics, without LDS rows, and uno_scf_run's
  * dense products run without split K, so the same input gives bitwise the same G, energy,
  * orbital energies and density in every run; default 0, FP64 atomics),
  * "launch_streams" (1-4: the streams a Fock build's ERI launches are spread over, the
@@ -81,13 +81,13 @@ int uno_ctx_destroy(uno_ctx* ctx);
  * builds of uno_fock_rhf/uno_fock_uhf; uno_scf_run takes its own option),
  * "prim_cut" (bare primitive prefactor cut, default 1e-12 as TwoElectronInts.cpp:428),
  * "skip_center" (a centre left out of the nuclear attraction, as the reference leaves out
- * the DPM positron, OneElectronInts.cpp:43; default -1, none), "row_merge" (1: bras with
- * many kets run as blocks that merge their exchange contributions in LDS; 0: every bra
- * as per-wave tasks; default 1), "row_min_kets" (the ket count from which a bra is
- * row-merged; default 192), "row_variant" (LDS layout of the row-merged blocks: 1 every
+ * the DPM positron, OneElectronInts.cpp:43; default -1, none), "row_merge" (1: a block's
+ * exchange contributions are merged in LDS rows of its bra; 0: every output goes straight to
+ * the accumulators; default 1), "row_min_kets" (the ket-run length from which a launch merges
+ * its rows; default 192), "row_variant" (LDS layout of the row-merged blocks: 1 every
  * bra row and the Rys table, 2 every bra row, 3 the first bra shell's rows; 0, the
- * default, takes the first that fits the LDS budget; a forced one that does not fit
- * falls back to that choice), "row_density_lds" (the bra's exchange density rows staged
+ * default, takes the first that fits the LDS budget; another value, or a layout that does not
+ * fit, falls back to that choice), "row_density_lds" (the bra's exchange density rows staged
  * in LDS beside the merged rows: -1, the default, wherever they fit the budget and the
  * autotuner does not prefer otherwise; 0 never; 1 wherever they fit), "rys2_exact" (0, the
  * default: the two-root classes use the reference's own two-root quadrature,
@@ -101,7 +101,8 @@ int uno_ctx_set(uno_ctx* ctx, const char* key, double value);
 /* Reads the knobs above and, read-only: "last_quartets" (shell quartets evaluated by the
  * last Fock build), "last_quartets32" (of which in FP32), "pairs" (significant shell
  * pairs), "pair_runs" (runs of the pair array: one per angular pair class and
- * primitive-count bucket, at most 36), "quartet_launches" (ERI launches per Fock build),
+ * primitive-count bucket, at most 36), "quartet_launches" (quartet spaces of a Fock build, the
+ * pairs of those runs; one launch per class pair and precision walks them),
  * and the context build's host milliseconds: "ctx_ms_pairs" (pair and primitive records
  * and their upload), "ctx_ms_schwarz" (Schwarz bounds on the device), "ctx_ms_runs"
  * (sorted runs, applied on the device) and "ctx_ms_rest". */
@@ -203,12 +204,12 @@ int uno_rys_eval_ref2(int fp32, int npts, const double* x, double* u, double* w)
 /* Debug/parity: Schwarz bounds sqrt(max|(ab|ab)|) per shell pair a>=b, packed order. */
 int uno_schwarz(uno_ctx* ctx, double* q);
 
-/* Autotuner (no reference counterpart): times every row-merge configuration (LDS variant,
- * the ket count from which a bra is row-merged, or wave tasks only) of every quartet space
+/* Autotuner (no reference counterpart): times every row-merge configuration (LDS variant or
+ * none, with and without the density rows and shell maxima in LDS) of every ERI launch
  * of one Fock build on the given density (PB null: RHF P; else UHF Pa, Pb; packed, as
- * uno_fock_rhf/uhf) and keeps the fastest per space, for this context and for every later
+ * uno_fock_rhf/uhf) and keeps the fastest per launch, for this context and for every later
  * context of the same basis layout in this process.  mixed = 1 tunes the mixed-precision
- * build's spaces.  best_ms (optional) receives the tuned build's summed kernel time.
+ * build's launches.  best_ms (optional) receives the tuned launches' summed kernel time.
  * G is not produced; the next Fock build starts from scratch. */
 int uno_autotune(uno_ctx* ctx, const double* P, const double* PB, int mixed, double* best_ms);
 
@@ -220,10 +221,10 @@ int uno_autotune(uno_ctx* ctx, const double* P, const double* PB, int mixed, dou
  * enable=0 turns it off (and clears the stats); stats are read with enable=-1, which
  * waits for the context's stream: builds record their events and counters without
  * synchronising, and the read folds them in.  Arrays hold 432 entries,
- * index 72*kind + 36*prec + 6*X + Y: kind 0 the per-wave-task (or per-quartet) kernels,
- * kinds 1-3 the row-merged kernels (1: every bra row and the Rys table in LDS, 2: every
- * bra row, 3: the first bra shell's rows), kinds 4-5 the bra-group row kernels (groups
- * of 2 and 4 bras); prec 0 FP64, 1 the FP32 launches of mixed builds. */
+ * index 72*kind + 36*prec + 6*X + Y: kind 0 the kernels without LDS rows and the
+ * one-quartet-per-wave kernels, kinds 1-3 the row-merged kernels (1: every bra row and the Rys
+ * table in LDS, 2: every bra row, 3: the first bra shell's rows), kinds 4-5 unused; prec 0
+ * FP64, 1 the FP32 launches of mixed builds. */
 int uno_profile(uno_ctx* ctx, int enable, double* ms, double* launches, double* prim_quartets,
                 double* shell_quartets);
 
@@ -312,19 +313,16 @@ int uno_shell_rotation(int l, const double* Q, double* M);
  * device: one ERI launch per class pair across all molecules, grouped GEMMs and a
  * batched Jacobi eigensolver for the dense steps, Pulay DIIS per molecule.  FP64 full
  * builds from the core-Hamiltonian guess; opts->cflag / eps / maxits as for uno_scf_run.
- * The Fock build's quartet lists are built once per run against a density bound (twice each
- * molecule's largest shell-block density; rebuilt if a density outgrows it) with the
- * costliest bras first, the launches skip converged molecules by a device flag (the wave
- * classes take their work from a device queue), and the whole build is captured once as a
+ * The Fock build's launches (one per class pair and shell kind over all molecules) skip
+ * converged molecules by a device flag, and the whole build is captured once per run as a
  * HIP graph and replayed every iteration. */
 typedef struct uno_batch uno_batch;
 int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_batch** out);
 int uno_batch_destroy(uno_batch* batch);
 int uno_batch_nmol(const uno_batch* batch);
 /* Options of the batched Fock build: "graph" (1: capture and replay, 0: plain launches),
- * "queue" (0: one block per task; 1: the one-quartet-per-wave classes take their quartet
- * blocks from a device work queue; 2: the lane classes' 64-ket tasks as well),
- * "launch_streams" (1-4: streams the list launches are spread over, forked and joined
+ * "queue" (0-2: kept for callers that set it; the launches no longer take work from a queue),
+ * "launch_streams" (1-4: streams the launches are spread over, forked and joined
  * inside the build, parallel branches of the captured graph; default 3).  uno_batch_get
  * also reads the last run's "space_builds", "graph_builds", "graph_replays" and
  * "launches_per_build". */

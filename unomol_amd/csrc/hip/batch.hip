@@ -235,28 +235,36 @@ __global__ __launch_bounds__(256) void k_batch_sym(const MatSlot* __restrict__ s
     }
 }
 
-// Dsh_k[s][t] = max |D| over the function block of shells s, t of slot k's molecule (D1, D2
-// optional further densities of the same layout)
-__global__ __launch_bounds__(256) void k_batch_shell_max(const MatSlot* __restrict__ slots, const int* __restrict__ sh_off,
+// Dsh_m[s][t] = max |D| over the function block of shells s, t of every active molecule m (D1,
+// D2 optional further densities of the same layout), dmax[m] (zeroed) the largest of them
+__global__ __launch_bounds__(256) void k_batch_shell_max(const MolDesc* __restrict__ mols, const int* __restrict__ shoff,
+                                                         const int* __restrict__ active, const int* __restrict__ sh_off,
                                                          const int* __restrict__ sh_n, const double* __restrict__ D,
                                                          const double* __restrict__ D1, const double* __restrict__ D2,
-                                                         double* __restrict__ Dsh) {
-    const MatSlot m = slots[blockIdx.x];
+                                                         double* __restrict__ Dsh, unsigned long long* __restrict__ dmax) {
+    const int mol = blockIdx.y;
+    if (!active[mol]) return;
+    const MolDesc m = mols[mol];
     const int ns = m.nsh;
-    for (int st = threadIdx.x; st < ns * ns; st += blockDim.x) {
+    double big = 0.0;
+    const int st = blockIdx.x * 256 + threadIdx.x;
+    if (st < ns * ns) {
         const int s = st / ns, t = st % ns;
-        const int o1 = sh_off[m.shoff + s], n1 = sh_n[m.shoff + s];
-        const int o2 = sh_off[m.shoff + t], n2 = sh_n[m.shoff + t];
+        const int o1 = sh_off[shoff[mol] + s], n1 = sh_n[shoff[mol] + s];
+        const int o2 = sh_off[shoff[mol] + t], n2 = sh_n[shoff[mol] + t];
         double v = 0.0;
         for (int a = 0; a < n1; ++a)
             for (int b = 0; b < n2; ++b) {
-                const long ij = m.off + (long)(o1 + a) * m.n + o2 + b;
+                const long ij = m.moff + (long)(o1 + a) * m.n + o2 + b;
                 v = fmax(v, fabs(D[ij]));
                 if (D1) v = fmax(v, fabs(D1[ij]));
                 if (D2) v = fmax(v, fabs(D2[ij]));
             }
         Dsh[m.dshoff + st] = v;
+        big = v;
     }
+    for (int o = 32; o > 0; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+    if ((threadIdx.x & 63) == 0 && big > 0.0) atomicMax(dmax + mol, (unsigned long long)__double_as_longlong(big));
 }
 
 // F_k = sum_j c[k * ncoef + j] H_j,k: a linear combination of ncoef stores per slot
@@ -291,10 +299,12 @@ hipError_t batch_sym(int nslot, const MatSlot* slots, const double* W, double* G
     hipLaunchKernelGGL(k_batch_sym, dim3(nslot), dim3(256), 0, st, slots, W, G, acc ? 1 : 0);
     return hipGetLastError();
 }
-hipError_t batch_shell_max(int nslot, const MatSlot* slots, const int* sh_off, const int* sh_n, const double* D,
-                           const double* D1, const double* D2, double* Dsh, hipStream_t st) {
-    if (nslot <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_batch_shell_max, dim3(nslot), dim3(256), 0, st, slots, sh_off, sh_n, D, D1, D2, Dsh);
+hipError_t batch_shell_max(int nmol, int maxsh, const MolDesc* mols, const int* shoff, const int* active,
+                           const int* sh_off, const int* sh_n, const double* D, const double* D1, const double* D2,
+                           double* Dsh, double* dmax, hipStream_t st) {
+    if (nmol <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_batch_shell_max, dim3((maxsh * maxsh + 255) / 256, nmol), dim3(256), 0, st, mols, shoff, active,
+                       sh_off, sh_n, D, D1, D2, Dsh, reinterpret_cast<unsigned long long*>(dmax));
     return hipGetLastError();
 }
 hipError_t batch_lincomb(int nslot, const MatSlot* slots, int ncoef, const double* coef, const double* const* src,

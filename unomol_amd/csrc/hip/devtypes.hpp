@@ -53,80 +53,94 @@ struct MolDesc {
     int n, nsh;
 };
 
+// explicit quartet lists (block and Schwarz modes)
 struct EriArgs {
     const PairHdr* pairs;
     const PrimPair* prims;
-    // implicit quartet space of one launch: bra pairs [bra_off, bra_off+nbra) and ket pairs
-    // from ket_off, both runs of the pair array sorted by Schwarz bound (descending);
-    // prefix[i] = first quartet of bra i, blk[b] = bra holding quartet b*qpb
-    int bra_off, ket_off;
-    const double* pairQ;      // Schwarz bound of every pair, in pair-array order
-    const long long* prefix;
-    const int* blk;
-    const int* kstart;        // first ket of every bra's range (null: 0), FP32 ranges
-                              // start after the bra's FP64 kets
-    // bra-major launches: one wave per (bra, chunk of 64 kets); wpre[i] = first wave
-    // task of bra i, tblk[b] = bra of task 64 b
-    const long long* wpre;
-    const int* tblk;
-    long long ntask;
-    // row-merged launches (bras with many kets): block task b belongs to the r-th listed
-    // bra, rpre[r] <= b < rpre[r+1]; rbra[r] is its entry; a block covers rseg kets of it
-    // and merges its exchange contributions to the bra's rows in LDS before adding them
-    const int* rbra;
-    const long long* rpre;
-    int nrbra;
-    long long nrtask;
-    int rseg;
-    // columns of those LDS rows: the functions the launch's ket run touches, in function
-    // order (whole shells, so a shell's functions stay consecutive); colmap[f] = column of
-    // function f (-1: untouched), colinv[c] = function of column c, ncols columns
-    const int* colmap;
-    const int* colinv;
-    int ncols;
-    // 1: the bra's exchange density rows (every bra function, each spin density, the same
-    // columns) are staged in LDS after the accumulator rows
-    int dlds;
-    // batched launches: entry i (a bra with one ket range) names its bra pair, its first
-    // ket pair and its molecule (null: the run offsets above and molecule view n/D/W)
-    const int* e_bra;
-    const int* e_ket;
-    const int* e_mol;
-    const MolDesc* mols;
+    const int2* explicit_q;   // (bra, ket) pairs
+    long long nquart;
     int qpb;                  // quartets per block of the launch
     int rys2_exact;           // 1: exact two-root Rys quadrature; 0: the reference's
                               // two-root quadrature (Rys.cpp:413-631), the default
-    int nbra;
-    long long nquart;
-    const int2* explicit_q;   // explicit (bra, ket) list (block / Schwarz modes) or null
-    int same_class;           // bra and ket lists are the same list
-    double tau;               // quartet screening threshold on Qab Qcd Dmax
     double primcut;           // bare primitive prefactor cut (reference 1e-12)
-    const double* dsh;        // [nsh*nsh] max |D| over each shell block (null = global bound only)
-    int nsh;
-    double dmax_global;
-    int n;                    // basis functions
+    double* out;              // block / Schwarz output
+};
+
+// ---- Fock builds --------------------------------------------------------------------
+// primitive pair as a bra: read whole, through the scalar cache.  K and s carry the bra's
+// share of the quartet prefactor, 2 pi^(5/2) / p (the ket's is 1 / q)
+struct alignas(16) BraPrim {
+    double p, ip, K, s;
+    double P[3], PA[3];   // product centre, and relative to the first shell's centre
+};
+// fields of a primitive pair as a ket, stored field by field: q, 1/q, K/q, s/q, P
+constexpr int kKetFields = 7;
+
+// One space of a Fock-build launch: the bra run [bra_off, bra_off + nbra) against the ket run
+// [ket_off, ket_off + nket) of the pair array, both sorted by Schwarz bound (descending).  Its
+// blocks are first + bra * nseg + segment; same: both are the same run (kets up to the bra).
+struct FockSpace {
+    int first;
+    int bra_off, nbra, ket_off, nket;
+    int nseg, seg;        // segments per bra, kets per segment
+    int lg;               // 2^lg lanes share a ket (and split its primitives)
+    int same, mol;
+    int col0, ncols;      // LDS row columns: function of column c at colinv[col0 + c]
+    int kstride;          // the ket run's length: primitive j of ket i at kp0 + j kstride + i
+    int pad;
+    long long kp0;
+    long long jo0;        // first ket's Coulomb block in the pair-major arrays
+};
+
+// a run of the pair array, as the kernel that lays the ket records out needs it
+struct PairRun {
+    int off, count;
+    int col0;             // column of function f at colmap[col0 + f]
+    int pad;
+    long long kp0;
+};
+
+constexpr int kQuartSlots = 256;
+
+struct FockArgs {
+    const FockSpace* sp;
+    const int* blk;           // space of every 64th block
+    const PairHdr* pairs;
+    const PrimPair* prims;
+    const BraPrim* bprim;
+    const double* kprim;      // ket primitive fields, kps apart
+    long long kps;
+    const double* kgeo;       // kets' A and AB: six fields, npair apart
+    long long npair;
+    const int4* kidx;         // first functions and shells of the pair
+    const int* knp;           // 2 x primitives + (same shell)
+    const int2* kcol;         // LDS row columns of the pair's first functions
+    const int* colinv;
+    const double* pairQ;      // Schwarz bounds
+    const double* dpair;      // max |D| of the pair's own shell block
+    const double* dp;         // D0 in pair-major blocks
+    double* jp;               // pair-major accumulator of the kets' Coulomb outputs
+    const double* dsh;        // [nsh x nsh] max |D| of every shell block
+    const double* dmax;       // largest of them, per molecule
+    double tau, primcut;
+    double fp32_thr;          // > 0: mixed build, quartets with a bound below it are FP32's
+    int rys2_exact;
+    int n, nsh;
+    int dlds, mlds;           // density rows / shell maxima of the bra staged in LDS
     const double* D0;         // RHF: P (half density); UHF: Pa + Pb (dense n x n)
     const double* D1;         // UHF: Pa
     const double* D2;         // UHF: Pb
     double* W0;               // RHF: W; UHF: Wa
     double* W1;               // UHF: Wb
-    double* out;              // block / Schwarz output
-    double* jp;               // pair-major accumulator of the ket Coulomb outputs (pair.jo)
-                              // of the per-lane kernels; null: they go straight to W
+    const MolDesc* mols;      // batched launches: the molecules' slices of the stores
+    const int* mol_active;    // per molecule: 0 skips its blocks
+    unsigned long long* nquart;   // kQuartSlots counters: quartets within the bounds
     unsigned long long* counter;  // evaluated-quartet counters (may be null): kCounterSlots
                                   // (primitive, shell) pairs, summed by the host
-    // work-queue launches (batched builds): a fixed grid whose waves (or one-wave blocks)
-    // take the next work item from *queue (zeroed before the launch) until it passes the
-    // item count (ntask wave tasks, or nqblk quartet blocks of the wave kernel); null: one
-    // item per wave / block as launched
-    unsigned long long* queue;
-    long long nqblk;
-    const int* mol_active;    // per molecule: 0 skips its items (null: every molecule)
     // deterministic accumulation (0: FP64 atomics): every W entry is two int64 words, the
     // word at the entry's own address and one fix_lo entries further on, holding the sum in
-    // fixed point (integer additions give the same sum in any order); wave-task and
-    // wave kernels only
+    // fixed point (integer additions give the same sum in any order); launches without LDS
+    // rows only
     long long fix_lo;
 };
 

@@ -163,9 +163,9 @@ __device__ __forceinline__ void rys_root_one(T x, int r, T& u, T& w, const T* ta
 // the table of NR roots a launch evaluates: the exact tables, except for two roots, where
 // the reference-compatible table is the default (same layout and size)
 template <int NR, typename T>
-__device__ __forceinline__ const T* rys_table_of(const EriArgs& a) {
+__device__ __forceinline__ const T* rys_table_of(int rys2_exact) {
     if constexpr (NR == 2) {
-        if (!a.rys2_exact) {
+        if (!rys2_exact) {
             if constexpr (sizeof(T) == 4) return uno_rys_ref2_mono_f;
             else return uno_rys_ref2_mono;
         }
@@ -241,8 +241,8 @@ struct ClassInfo {
     }
 };
 
-// The matrices one entry's quartets read and write: the launch's own, or for batched
-// launches the entry's molecule's slice of every store
+// The matrices a block's quartets read and write: the launch's own, or for batched
+// launches its molecule's slice of every store
 struct MolView {
     const double* D0;
     const double* D1;
@@ -252,56 +252,6 @@ struct MolView {
     const double* dsh;
     int n, nsh;
 };
-
-__device__ __forceinline__ MolView mol_view(const EriArgs& a, int entry) {
-    MolView v{a.D0, a.D1, a.D2, a.W0, a.W1, a.dsh, a.n, a.nsh};
-    if (a.mols) {
-        const MolDesc m = a.mols[a.e_mol[entry]];
-        v.D0 = a.D0 + m.moff;
-        v.D1 = a.D1 ? a.D1 + m.moff : nullptr;
-        v.D2 = a.D2 ? a.D2 + m.moff : nullptr;
-        v.W0 = a.W0 + m.moff;
-        v.W1 = a.W1 ? a.W1 + m.moff : nullptr;
-        v.dsh = a.dsh ? a.dsh + m.dshoff : nullptr;
-        v.n = m.n;
-        v.nsh = m.nsh;
-    }
-    return v;
-}
-
-// bra pair and first ket pair of entry i
-__device__ __forceinline__ int entry_bra(const EriArgs& a, int i) { return a.e_bra ? a.e_bra[i] : a.bra_off + i; }
-__device__ __forceinline__ int entry_ket(const EriArgs& a, int i) {
-    return a.e_ket ? a.e_ket[i] : a.ket_off + (a.kstart ? a.kstart[i] : 0);
-}
-
-// Resolve the quartet handled by linear index g: (bra pair, ket pair), the entry, and the
-// product of their Schwarz bounds (negative for explicit lists: no screening)
-__device__ __forceinline__ bool quartet_of(const EriArgs& a, long long g, int& pab, int& pcd, double& q12,
-                                           int& entry) {
-    if (g >= a.nquart) return false;
-    if (a.explicit_q) {
-        const int2 e = a.explicit_q[g];
-        pab = e.x;
-        pcd = e.y;
-        q12 = -1.0;
-        entry = 0;
-        return true;
-    }
-    // the block table brackets the bra of every quartet of this block
-    const long long b = g / a.qpb;
-    int lo = a.blk[b], hi = a.blk[b + 1];
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.prefix[mid] <= g) lo = mid; else hi = mid - 1;
-    }
-    const int jk = (int)(g - a.prefix[lo]);
-    entry = lo;
-    pab = entry_bra(a, lo);
-    pcd = entry_ket(a, lo) + jk;
-    q12 = a.pairQ[pab] * a.pairQ[pcd];
-    return true;
-}
 
 __device__ __forceinline__ void atomic_add_f64(double* p, double v) { unsafeAtomicAdd(p, v); }
 
@@ -320,22 +270,20 @@ __device__ __forceinline__ void fixed_add(double* p, long long lo_off, double v)
     if (hi) atomicAdd(w, (unsigned long long)hi);
     if (lo) atomicAdd(w + lo_off, (unsigned long long)lo);
 }
-// a Fock-matrix contribution of the wave-task and wave kernels
-__device__ __forceinline__ void fock_add(const EriArgs& a, double* p, double v) {
-    if (a.fix_lo) fixed_add(p, a.fix_lo, v);
+// a Fock-matrix contribution straight into W
+__device__ __forceinline__ void fock_add(long long fix_lo, double* p, double v) {
+    if (fix_lo) fixed_add(p, fix_lo, v);
     else unsafeAtomicAdd(p, v);
 }
 
-// density screen: Qab Qcd max(4|D_ab|, 4|D_cd|, |D_ac|, |D_ad|, |D_bc|, |D_bd|) < tau
-__device__ __forceinline__ bool screened(const EriArgs& a, const MolView& v, const PairHdr& P1, const PairHdr& P2,
-                                         double q12) {
-    if (!v.dsh) return q12 * a.dmax_global < a.tau;
+// density screen of a quartet with bounds' product q12:
+// Qab Qcd max(4|D_ab|, 4|D_cd|, |D_ac|, |D_ad|, |D_bc|, |D_bd|) < tau
+__device__ __forceinline__ bool screened(double tau, const MolView& v, int s1, int s2, int s3, int s4, double q12) {
     const int ns = v.nsh;
     const double* m = v.dsh;
-    const int s1 = P1.sh1, s2 = P1.sh2, s3 = P2.sh1, s4 = P2.sh2;
     double d = 4.0 * fmax(m[s1 * ns + s2], m[s3 * ns + s4]);
     d = fmax(d, fmax(fmax(m[s1 * ns + s3], m[s1 * ns + s4]), fmax(m[s2 * ns + s3], m[s2 * ns + s4])));
-    return q12 * d < a.tau;
+    return q12 * d < tau;
 }
 
 }  // namespace uno

@@ -5,34 +5,52 @@
 
 namespace uno {
 
-// ERIs (eri.hip)
-// fp32: evaluate the quartets in single precision (RHF/UHF digestion only), accumulating in FP64
-hipError_t eri_launch(int mode, int bra_class, int ket_class, const EriArgs& a, hipStream_t st, bool fp32 = false);
+// ERIs of explicit quartet lists, block and Schwarz modes, FP64 (eri.hip)
+hipError_t eri_launch(int mode, int bra_class, int ket_class, const EriArgs& a, hipStream_t st);
 int eri_class_ncomp(int bra_class, int ket_class);
-// quartets one block of the class kernel walks (the block table granularity)
-int eri_quartets_per_block(int bra_class, int ket_class);
-// Fock-build launches of this class run as wave tasks (bra, up to 64 kets): the space needs
-// wpre / tblk / ntask instead of the quartet block table
-bool eri_uses_wave_tasks(int bra_class, int ket_class);
-// row-merged Fock-build launch (bras with many kets) of a wave-task class: a.rbra / a.rpre /
-// a.nrtask / a.rseg describe the block tasks, a.colmap / a.colinv / a.ncols the LDS row
-// columns; variant from eri_rows_variant: 1 every bra row and the Rys table in LDS, 2 every
-// bra row, 3 the first bra shell's rows only, 0 none fits the LDS budget at ncols columns
-// (the class then runs as wave tasks only); force 1-3 picks that variant when it fits,
-// force 4 or 5 the bra-group kernel (groups of 2 or 4 bras, every bra row and the table in
-// LDS; FP64 spaces of the classes of at most 9 or 3 components)
-hipError_t eri_launch_rows(int mode, int bra_class, int ket_class, const EriArgs& a, int variant, hipStream_t st,
-                           bool fp32);
-int eri_rows_variant(int bra_class, int ket_class, int mode, int ncols, bool fp32, int force);
-// whether that variant still fits the LDS budget with the bra's exchange density rows
-// staged as well (a.dlds = 1)
-bool eri_rows_dlds_fits(int bra_class, int ket_class, int mode, int ncols, bool fp32, int variant);
-// bras per row task of a variant (2 or 4 for the bra-group variants, else 1)
-int eri_rows_group(int variant);
-// W[f1 + k][f2 + l] += jp[jo + k nd + l] (and W1) for every pair of the array (pair blocks
-// are disjoint, no atomics); the block size of a pair follows from the next pair's jo
+
+// Fock-build launches (fock_core.hpp).  Classes above kLaneMaxComp components run one quartet per
+// wave (fock_is_wave); the others one ket per lane with the exchange rows of the bra merged in
+// LDS (variant 1 every bra row and the Rys table in LDS, 2 every bra row, 3 the first bra
+// shell's rows, 0 none: every output straight to W), the bra's exchange density rows (dlds) and
+// shell maxima (mlds) staged there where they fit.
+struct FockConfig {
+    int variant = 0, dlds = 0, mlds = 0;
+};
+constexpr int kLaneBlock = 256;   // lanes of a block of the lane kernels
+constexpr int kWaveSeg = 8;       // kets of a block of the wave kernels
+bool fock_is_wave(int bra_class, int ket_class);
+// the first of (force, 1, 2, 3) that fits the LDS budget at ncols columns (rows false: 0), with
+// what else fits; dens 0: no density rows
+FockConfig fock_default(int bra_class, int ket_class, int mode, int ncols, int nsh, bool fp32, bool rows, int force,
+                        int dens);
+bool fock_config_fits(int bra_class, int ket_class, const FockConfig& f, int mode, int ncols, int nsh, bool fp32);
+hipError_t fock_launch(int mode, bool fp32, int bra_class, int ket_class, FockArgs a, int nblocks, const FockConfig& f,
+                       int ncols, hipStream_t st);
+// the Fock kernels' copies of the pair data (device arrays), runs sorted by off
+hipError_t pair_store(int np, int nrun, const PairRun* runs, const PairHdr* pairs, const PrimPair* prims,
+                      const int* colmap, BraPrim* bprim, double* kprim, long long kps, double* kgeo, int4* kidx, int* knp,
+                      int2* kcol, hipStream_t st);
+// up to six buffers of 64-bit words zeroed in one launch
+struct ClearList {
+    unsigned long long* p[6];
+    long long len[6];
+    int n = 0;
+    template <class T>
+    void add(T* q, long long count) {
+        static_assert(sizeof(T) == 8, "64-bit words");
+        p[n] = reinterpret_cast<unsigned long long*>(q);
+        len[n++] = count;
+    }
+};
+hipError_t fock_clear(const ClearList& c, hipStream_t st);
+// dp = D0 in pair-major blocks, dpair = every pair's own entry of dsh (mols / pmol: batched
+// stores and every pair's molecule, or null)
+hipError_t pair_density(int npairs, const PairHdr* pairs, long long njp, const double* D0, const double* dsh, int n,
+                        int nsh, const MolDesc* mols, const int* pmol, double* dp, double* dpair, hipStream_t st);
+// W[f1 + k][f2 + l] += jp[jo + k nd + l] (and W1) for every pair of the array
 hipError_t jp_scatter(int npairs, const PairHdr* pairs, long long njp, const double* jp, double* W0, double* W1, int n,
-                      hipStream_t st);
+                      const MolDesc* mols, const int* pmol, hipStream_t st);
 // new pair k = old pair order[k], its primitives at prim0[k], Coulomb block at jo[k]
 // (device arrays; new ones must not overlap the old)
 hipError_t permute_pairs(int np, const int* order, const int* prim0, const int* jo, const PairHdr* oldp,
@@ -59,9 +77,10 @@ constexpr int kRedBlocks = 240;
 hipError_t k_dot(long len, const double* A, const double* B, double* out, double* ws, hipStream_t st);
 // out[0] = sqrt(sum (A-B)^2) / n
 hipError_t k_diffnorm(long len, int n, const double* A, const double* B, double* out, double* ws, hipStream_t st);
-// Dsh[s][t] = max |D_ij| over the function block of shells s, t
+// Dsh[s][t] = max |D_ij| over the function block of shells s, t of up to three matrices;
+// dmax (zeroed by the caller) = the largest of them
 hipError_t k_shell_max(int n, int nsh, const int* sh_off, const int* sh_n, const double* D, const double* D1,
-                       const double* D2, double* Dsh, hipStream_t st);
+                       const double* D2, double* Dsh, double* dmax, hipStream_t st);
 // out[0] = max |x|
 hipError_t k_absmax(long len, const double* x, double* out, hipStream_t st);
 // A_ii += alpha (n x n)

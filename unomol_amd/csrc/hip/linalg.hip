@@ -221,25 +221,35 @@ hipError_t k_trace(int n, const double* A, double* out, hipStream_t st) {
     return hipGetLastError();
 }
 
-// one block per shell pair (s, t): max |D| over its function block of up to three matrices
-__global__ void k_shell_max_(int n, int nsh, const int* off, const int* nf, const double* D, const double* D1,
-                             const double* D2, double* Dsh) {
-    const int s = blockIdx.x / nsh, t = blockIdx.x % nsh;
+// one thread per shell pair (s, t): max |D| over its function block of up to three matrices,
+// and the largest of all (|x| orders as its bit pattern)
+__global__ __launch_bounds__(256) void k_shell_max_(int n, int nsh, const int* __restrict__ off, const int* __restrict__ nf,
+                                                    const double* __restrict__ D, const double* __restrict__ D1,
+                                                    const double* __restrict__ D2, double* __restrict__ Dsh,
+                                                    unsigned long long* dmax) {
+    const long st = (long)blockIdx.x * 256 + threadIdx.x;
     double m = 0.0;
-    const int ns = nf[s], nt = nf[t];
-    for (int q = threadIdx.x; q < ns * nt; q += 64) {
-        const long ij = (long)(off[s] + q / nt) * n + off[t] + q % nt;
-        m = fmax(m, fabs(D[ij]));
-        if (D1) m = fmax(m, fabs(D1[ij]));
-        if (D2) m = fmax(m, fabs(D2[ij]));
+    if (st < (long)nsh * nsh) {
+        const int s = (int)(st / nsh), t = (int)(st - (long)s * nsh);
+        const int ns = nf[s], nt = nf[t];
+        const long o = (long)off[s] * n + off[t];
+        for (int a = 0; a < ns; ++a)
+            for (int b = 0; b < nt; ++b) {
+                const long ij = o + (long)a * n + b;
+                m = fmax(m, fabs(D[ij]));
+                if (D1) m = fmax(m, fabs(D1[ij]));
+                if (D2) m = fmax(m, fabs(D2[ij]));
+            }
+        Dsh[st] = m;
     }
-    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_down(m, o, 64));
-    if (threadIdx.x == 0) Dsh[blockIdx.x] = m;
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0 && m > 0.0) atomicMax(dmax, (unsigned long long)__double_as_longlong(m));
 }
 hipError_t k_shell_max(int n, int nsh, const int* sh_off, const int* sh_n, const double* D, const double* D1,
-                       const double* D2, double* Dsh, hipStream_t st) {
-    hipLaunchKernelGGL(k_shell_max_, dim3((unsigned)(nsh * nsh)), dim3(64), 0, st, n, nsh, sh_off, sh_n, D, D1, D2,
-                       Dsh);
+                       const double* D2, double* Dsh, double* dmax, hipStream_t st) {
+    const long len = (long)nsh * nsh;
+    hipLaunchKernelGGL(k_shell_max_, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, st, n, nsh, sh_off, sh_n, D, D1,
+                       D2, Dsh, reinterpret_cast<unsigned long long*>(dmax));
     return hipGetLastError();
 }
 

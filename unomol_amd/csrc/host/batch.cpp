@@ -4,10 +4,9 @@
 //
 // Every molecule keeps its own context for the pair data (shell pairs, Schwarz bounds,
 // runs sorted by bound); their pair and primitive arrays are concatenated into one device
-// array.  A Fock build is one launch per (bra class, ket class, RHF/UHF) over all
-// molecules: the quartet space is a list of entries (bra pair, first ket pair, ket count,
-// molecule) built from the same screened prefixes as a single-molecule build, and the
-// kernels read and accumulate each molecule's slice of the density / accumulator stores.
+// array.  A Fock build is one launch per (bra class, ket class, RHF/UHF) over all molecules'
+// quartet spaces (FockStore), each of which names its molecule's slice of the density and
+// accumulator stores.
 // Dense steps run as grouped GEMMs over every (molecule, spin) slot and a batched Jacobi
 // eigensolver (one block per matrix).  The iteration is the single-molecule one with Pulay
 // DIIS (8 vectors, error X^T(FPS - SPF)X); molecules stop updating once converged.
@@ -17,8 +16,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <map>
-#include <tuple>
 #include "engine.hpp"
 #include "../hip/batch_kernels.hpp"
 #include "../hip/kernels.hpp"
@@ -75,6 +72,7 @@ struct uno_batch {
     DBuf<double> pairQ;
     DBuf<int> sh_off, sh_n;
     DBuf<MolDesc> mdesc;
+    DBuf<int> mshoff;           // per molecule: its first shell in the shell tables
     // stores (each sum_m N_m^2 doubles); index 0 alpha / closed shell, 1 beta
     DBuf<double> H, S, X, P[2], Pold[2], F[2], G[2], C[2], Fp, Tm, Tm2, V, Z, D0, D1, D2, W0, W1, Dsh, ev[2];
     // per spin: the last eigenvectors of X^T F X (orthogonal basis), the next eigensolve's
@@ -84,30 +82,20 @@ struct uno_batch {
     DBuf<double> dF[kBatchDiis][2], dE[kBatchDiis][2];
     DBuf<double> red;
     Scratch scratch;
-    // the Fock build's static quartet spaces (one per bra class, ket class, open shell),
-    // their work-queue counters, the per-molecule active flags, and the build captured as
-    // a HIP graph (replayed every iteration while the spaces stay)
-    struct Group {
-        int cx, cy, uhf, tasks, qpb, ne;
-        long long nq, ntask;
-        int *bra, *ket, *mol, *tblk, *blk;
-        long long *prefix, *wpre;
-    };
-    std::vector<Group> groups;
-    DBuf<char> gstore;
-    DBuf<unsigned long long> queues;
-    DBuf<int> active_d;
-    std::vector<double> dbound;     // per molecule: the density bound the spaces were built with
-    std::vector<double> mol_quartets;   // per molecule: quartets in the static spaces
+    // the Fock kernels' pair data and launches over all molecules, every pair's molecule, the
+    // per-molecule active flags, and the build captured as a HIP graph (replayed every
+    // iteration of a run)
+    FockStore fs;
+    DBuf<int> pmol, active_d;
+    int maxn = 0, maxsh = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    int use_graph = 1, use_queue = 1;
-    // the groups' launches go round-robin over st and launch_streams - 1 worker streams
-    // (forked from st after the fills and joined back; under capture the graph then holds
-    // parallel branches)
+    int use_graph = 1;
+    int use_queue = 1;   // accepted and read back; the launches take no work from a queue
+    // the launches go round-robin over st and launch_streams - 1 worker streams (forked from st
+    // and joined back; under capture the graph then holds parallel branches)
     int launch_streams = 3;
-    hipStream_t wst[kMaxLaunchStreams - 1] = {};
-    hipEvent_t wfork = nullptr, wjoin[kMaxLaunchStreams - 1] = {};
+    LaunchStreams ls;
     int graph_builds = 0, graph_replays = 0, space_builds = 0;
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -120,11 +108,6 @@ struct uno_batch {
         for (BatchMol& m : mol)
             if (m.ctx) uno_ctx_destroy(m.ctx);
         if (st) (void)hipStreamSynchronize(st);
-        for (int w = 0; w + 1 < kMaxLaunchStreams; ++w) {
-            if (wst[w]) (void)hipStreamDestroy(wst[w]);
-            if (wjoin[w]) (void)hipEventDestroy(wjoin[w]);
-        }
-        if (wfork) (void)hipEventDestroy(wfork);
         if (st) (void)hipStreamDestroy(st);
     }
 };
@@ -139,7 +122,7 @@ void make_slots(const uno_batch* b, bool only_active, int spin, std::vector<MatS
         const BatchMol& x = b->mol[m];
         if (only_active && !x.active) continue;
         if (spin == 1 && !x.uhf) continue;
-        out.push_back(MatSlot{x.moff, x.n, x.nsh, x.shoff, x.dshoff});
+        out.push_back(MatSlot{x.moff, x.n});
         who.push_back(m);
     }
 }
@@ -187,203 +170,63 @@ int batch_eigh(uno_batch* b, const std::vector<MatSlot>& sl, double* A, double* 
 
 namespace uno {
 
-// Static quartet spaces of the batched Fock build: every molecule's screened prefixes built
-// with a density bound (twice the largest |D| block maximum seen so far, per molecule)
-// instead of the current density, so that the launches -- their index arrays, counts and
-// pointers -- stay the same from build to build.  The kernels apply the exact per-shell-block
-// density screen, which selects the same quartets prefixes built at the current density
-// would; a density that exceeds its bound rebuilds the spaces.  Entries are sorted by
-// their ket count (largest first) so that the work queue hands out the costly bras first.
-static int build_static(uno_batch* b, const std::vector<double>& dmax) {
-    b->drop_graph();
-    const int nm = (int)b->mol.size();
-    if ((int)b->dbound.size() != nm) b->dbound.assign(nm, 0.0);
-    for (int m = 0; m < nm; ++m) b->dbound[m] = std::max(2.0 * dmax[m], b->dbound[m]);
-    struct Ent { std::vector<int> bra, ket, mol; std::vector<long long> cnt; };
-    std::map<std::tuple<int, int, int>, Ent> groups;
-    b->mol_quartets.assign(nm, 0.0);
-    for (int m = 0; m < nm; ++m) {
-        BatchMol& x = b->mol[m];
-        uno_ctx* c = x.ctx;
-        for (QuartetClass& q : c->qcls) {
-            build_prefix(c, q, 4.0 * b->dbound[m], 0.0, c->tau);
-            if (q.s64.nq == 0) continue;
-            b->mol_quartets[m] += (double)q.s64.nq;
-            const PairClassList& LX = c->cls[q.X];
-            const PairClassList& LY = c->cls[q.Y];
-            Ent& e = groups[std::make_tuple(LX.lcls, LY.lcls, x.uhf ? 1 : 0)];
-            for (int i = 0; i + 1 < (int)q.s64.prefix.size(); ++i) {
-                const long long cnt = q.s64.prefix[i + 1] - q.s64.prefix[i];
-                if (cnt == 0) continue;
-                e.bra.push_back(x.pair_off + LX.off + q.s64.b0 + i);
-                e.ket.push_back(x.pair_off + LY.off);
-                e.mol.push_back(m);
-                e.cnt.push_back(cnt);
-            }
-        }
-    }
-    // host layout of every group's arrays in one buffer (16-byte aligned pieces)
-    std::vector<char> hs;
-    auto put = [&](const auto& v) -> size_t {
-        const size_t off = (hs.size() + 15) / 16 * 16;
-        const size_t bytes = v.size() * sizeof(v[0]);
-        hs.resize(off + std::max<size_t>(bytes, 16));
-        if (bytes) std::memcpy(hs.data() + off, v.data(), bytes);
-        return off;
-    };
-    struct Offs { size_t bra, ket, mol, prefix, wpre, tblk, blk; };
-    std::vector<Offs> offs;
-    b->groups.clear();
-    for (auto& kv : groups) {
-        Ent& e = kv.second;
-        const int ne = (int)e.bra.size();
-        std::vector<int> order(ne);
-        for (int i = 0; i < ne; ++i) order[i] = i;
-        std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return e.cnt[u] > e.cnt[v]; });
-        std::vector<int> bra(ne), ket(ne), mol(ne);
-        QuartetSpace sp;
-        sp.prefix.assign(ne + 1, 0);
-        for (int i = 0; i < ne; ++i) {
-            bra[i] = e.bra[order[i]];
-            ket[i] = e.ket[order[i]];
-            mol[i] = e.mol[order[i]];
-            sp.prefix[i + 1] = sp.prefix[i] + e.cnt[order[i]];
-        }
-        sp.nq = sp.prefix[ne];
-        uno_batch::Group g{};
-        g.cx = std::get<0>(kv.first);
-        g.cy = std::get<1>(kv.first);
-        g.uhf = std::get<2>(kv.first);
-        g.tasks = eri_uses_wave_tasks(g.cx, g.cy) ? 1 : 0;
-        g.qpb = eri_quartets_per_block(g.cx, g.cy);
-        g.ne = ne;
-        g.nq = sp.nq;
-        Offs o{};
-        o.bra = put(bra);
-        o.ket = put(ket);
-        o.mol = put(mol);
-        o.prefix = put(sp.prefix);
-        if (g.tasks) {
-            build_tasks(sp);
-            g.ntask = sp.ntask;
-            o.wpre = put(sp.wpre);
-            o.tblk = put(sp.tblk);
-        } else {
-            build_blocks(sp, g.qpb);
-            o.blk = put(sp.blk);
-        }
-        b->groups.push_back(g);
-        offs.push_back(o);
-    }
-    UNO_HIP(b->gstore.alloc(std::max<size_t>(hs.size(), 16)));
-    UNO_HIP(hipMemcpyAsync(b->gstore.p, hs.data(), hs.size(), hipMemcpyHostToDevice, b->st));
-    UNO_HIP(b->queues.alloc(std::max<size_t>(b->groups.size(), 1)));
-    UNO_HIP(b->active_d.alloc(std::max(nm, 1)));
-    for (size_t k = 0; k < b->groups.size(); ++k) {
-        uno_batch::Group& g = b->groups[k];
-        const Offs& o = offs[k];
-        char* base = b->gstore.p;
-        g.bra = reinterpret_cast<int*>(base + o.bra);
-        g.ket = reinterpret_cast<int*>(base + o.ket);
-        g.mol = reinterpret_cast<int*>(base + o.mol);
-        g.prefix = reinterpret_cast<long long*>(base + o.prefix);
-        g.wpre = g.tasks ? reinterpret_cast<long long*>(base + o.wpre) : nullptr;
-        g.tblk = g.tasks ? reinterpret_cast<int*>(base + o.tblk) : nullptr;
-        g.blk = g.tasks ? nullptr : reinterpret_cast<int*>(base + o.blk);
-    }
-    UNO_HIP(hipStreamSynchronize(b->st));   // hs is freed on return
-    ++b->space_builds;
-    return UNO_OK;
-}
-
-// the launches of one build: accumulators and queue counters cleared by fill kernels (no
-// memset nodes when captured), then one launch per static space
-// the worker streams and events, made before any capture
-static int ensure_workers(uno_batch* b) {
-    const int nls = std::max(1, std::min(kMaxLaunchStreams, b->launch_streams));
-    for (int w = 0; w + 1 < nls; ++w)
-        if (!b->wst[w]) {
-            UNO_HIP(hipStreamCreate(&b->wst[w]));
-            UNO_HIP(hipEventCreateWithFlags(&b->wjoin[w], hipEventDisableTiming));
-        }
-    if (nls > 1 && !b->wfork) UNO_HIP(hipEventCreateWithFlags(&b->wfork, hipEventDisableTiming));
-    return UNO_OK;
-}
-
+// the launches of one build: accumulators and density maxima cleared by a fill kernel (no memset
+// nodes when captured), the densities in the pairs' order, one launch per class pair and shell
+// kind, and the Coulomb accumulator into W
 static int enqueue_fock(uno_batch* b) {
     hipStream_t st = b->st;
-    UNO_HIP(k_fill(b->store, 0.0, b->W0.p, st));
-    UNO_HIP(k_fill(b->store, 0.0, b->W1.p, st));
-    if (b->use_queue && !b->groups.empty())
-        UNO_HIP(k_fill((long)b->groups.size(), 0.0, reinterpret_cast<double*>(b->queues.p), st));
+    FockStore& fs = b->fs;
+    const int np = fs.npair, nm = (int)b->mol.size();
+    ClearList cl;
+    cl.add(b->W0.p, b->store);
+    cl.add(b->W1.p, b->store);
+    cl.add(fs.jp.p, fs.njp);
+    cl.add(fs.dmax.p, nm);
+    UNO_HIP(fock_clear(cl, st));
+    UNO_HIP(batch_shell_max(nm, b->maxsh, b->mdesc.p, b->mshoff.p, b->active_d.p, b->sh_off.p, b->sh_n.p, b->D0.p, b->D1.p, b->D2.p,
+                            b->Dsh.p, fs.dmax.p, st));
+    UNO_HIP(pair_density(np, b->pairs.p, fs.njp, b->D0.p, b->Dsh.p, 0, 0, b->mdesc.p, b->pmol.p, fs.dp.p, fs.dpair.p, st));
     const int nls = std::max(1, std::min(kMaxLaunchStreams, b->launch_streams));
-    if (nls > 1) {
-        UNO_HIP(hipEventRecord(b->wfork, st));
-        for (int w = 0; w + 1 < nls; ++w) UNO_HIP(hipStreamWaitEvent(b->wst[w], b->wfork, 0));
-    }
-    for (size_t k = 0; k < b->groups.size(); ++k) {
-        const int li = (int)(k % (size_t)nls);
-        const hipStream_t ls = li == 0 ? st : b->wst[li - 1];
-        const uno_batch::Group& g = b->groups[k];
-        EriArgs a{};
-        a.pairs = b->pairs.p;
-        a.prims = b->prims.p;
-        a.pairQ = b->pairQ.p;
-        a.tau = b->mol[0].ctx->tau;
-        a.primcut = b->mol[0].ctx->primcut;
-        a.rys2_exact = b->mol[0].ctx->rys2_exact;
-        a.prefix = g.prefix;
-        a.blk = g.blk;
-        a.wpre = g.wpre;
-        a.tblk = g.tblk;
-        a.ntask = g.tasks ? g.ntask : 0;
-        a.qpb = g.qpb;
-        a.nquart = g.nq;
-        a.e_bra = g.bra;
-        a.e_ket = g.ket;
-        a.e_mol = g.mol;
-        a.mols = b->mdesc.p;
+    if (int rc = b->ls.begin(nls, st)) return rc;
+    for (size_t k = 0; k < fs.launches.size(); ++k) {
+        const FockLaunch& l = fs.launches[k];
+        const bool uhf = l.group != 0;
+        FockArgs a = fs.args(l, b->pairs.p, b->prims.p, b->pairQ.p);
+        const uno_ctx* c0 = b->mol[0].ctx;
+        a.tau = c0->tau;
+        a.primcut = c0->primcut;
+        a.rys2_exact = c0->rys2_exact;
+        a.n = b->maxn;
+        a.nsh = b->maxsh;
         a.dsh = b->Dsh.p;
-        a.dmax_global = 0.0;
+        a.jp = fs.jp.p;
+        a.nquart = fs.nquart.p;
         a.D0 = b->D0.p;
         a.W0 = b->W0.p;
-        if (g.uhf) {
+        if (uhf) {
             a.D1 = b->D1.p;
             a.D2 = b->D2.p;
             a.W1 = b->W1.p;
         }
-        // queue 1: the wave-per-quartet classes take their blocks from the queue; queue 2:
-        // the lane classes' 64-ket tasks too (one atomic per task)
-        const bool q = b->use_queue >= 2 || (b->use_queue == 1 && !g.tasks);
-        a.queue = q ? b->queues.p + k : nullptr;
+        a.mols = b->mdesc.p;
         a.mol_active = b->active_d.p;
-        UNO_HIP(eri_launch(g.uhf ? kDigestUHF : kDigestRHF, g.cx, g.cy, a, ls));
+        const int mode = uhf ? kDigestUHF : kDigestRHF;
+        const FockConfig f = fock_default(l.cx, l.cy, mode, l.ncols, b->maxsh, false, true, 0, -1);
+        UNO_HIP(fock_launch(mode, false, l.cx, l.cy, a, l.nblocks, f, l.ncols, b->ls.of((int)(k % (size_t)nls), st)));
     }
-    for (int w = 0; w + 1 < nls; ++w) {
-        UNO_HIP(hipEventRecord(b->wjoin[w], b->wst[w]));
-        UNO_HIP(hipStreamWaitEvent(st, b->wjoin[w], 0));
-    }
+    if (int rc = b->ls.end(nls, st)) return rc;
+    UNO_HIP(jp_scatter(np, b->pairs.p, fs.njp, fs.jp.p, b->W0.p, b->W1.p, 0, b->mdesc.p, b->pmol.p, st));
     return UNO_OK;
 }
 
-
-// batched Fock build on the densities in D0 (D1, D2): W0 (W1) accumulators.  dmax: each
-// molecule's largest shell-block density maximum.
-static int batch_fock(uno_batch* b, const std::vector<double>& dmax, double& quartets) {
+// batched Fock build on the densities in D0 (D1, D2): W0 (W1) accumulators
+static int batch_fock(uno_batch* b) {
     hipStream_t st = b->st;
     const int nm = (int)b->mol.size();
-    bool rebuild = b->groups.empty() && b->space_builds == 0;
-    for (int m = 0; m < nm && !rebuild; ++m)
-        if (b->mol[m].active && dmax[m] > b->dbound[m]) rebuild = true;
-    if (rebuild)
-        if (int rc = build_static(b, dmax)) return rc;
     std::vector<int> act(nm);
-    for (int m = 0; m < nm; ++m) {
-        act[m] = b->mol[m].active ? 1 : 0;
-        if (act[m]) quartets += b->mol_quartets[m];   // before the kernels' density screen
-    }
+    for (int m = 0; m < nm; ++m) act[m] = b->mol[m].active ? 1 : 0;
     UNO_HIP(hipMemcpyAsync(b->active_d.p, act.data(), nm * sizeof(int), hipMemcpyHostToDevice, st));
-    if (int rc = ensure_workers(b)) return rc;
+    if (int rc = b->ls.prepare(std::max(1, std::min(kMaxLaunchStreams, b->launch_streams)))) return rc;
     if (b->use_graph) {
         if (!b->gexec) {
             UNO_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
@@ -421,6 +264,8 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
     std::vector<double> q;
     std::vector<int> shoff, shn;
     std::vector<MolDesc> md;
+    std::vector<int> pmol, mshoff;
+    long long njp = 0;
     for (int m = 0; m < nmol; ++m) {
         BatchMol& x = b->mol[m];
         if (int rc = uno_ctx_create(&bases[m], 0, &x.ctx)) { delete b; return rc; }
@@ -450,8 +295,14 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
         const int p0 = (int)prims.size();
         for (PairHdr h : c->pairs) {
             h.prim0 += p0;
+            h.jo += (int)njp;
             pairs.push_back(h);
+            pmol.push_back(m);
         }
+        njp += c->fs.njp;
+        mshoff.push_back(x.shoff);
+        b->maxn = std::max(b->maxn, x.n);
+        b->maxsh = std::max(b->maxsh, x.nsh);
         prims.insert(prims.end(), c->prims.begin(), c->prims.end());
         q.insert(q.end(), c->pairQ.begin(), c->pairQ.end());
         md.push_back(MolDesc{x.moff, x.dshoff, x.n, x.nsh});
@@ -470,10 +321,22 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
     hipStream_t st = b->st;
     auto up = [&](auto& buf, const auto& v) { return buf.upload(v.data(), v.size(), st); };
     if (up(b->pairs, pairs) != hipSuccess || up(b->prims, prims) != hipSuccess || up(b->pairQ, q) != hipSuccess ||
-        up(b->sh_off, shoff) != hipSuccess || up(b->sh_n, shn) != hipSuccess || up(b->mdesc, md) != hipSuccess) {
+        up(b->sh_off, shoff) != hipSuccess || up(b->sh_n, shn) != hipSuccess || up(b->mdesc, md) != hipSuccess || up(b->pmol, pmol) != hipSuccess ||
+        up(b->mshoff, mshoff) != hipSuccess || b->active_d.alloc(nmol) != hipSuccess) {
         set_error("batched SCF: device upload failed");
         delete b;
         return UNO_ENOMEM;
+    }
+    {
+        std::vector<FockMol> fm(nmol);
+        for (int m = 0; m < nmol; ++m) {
+            const BatchMol& x = b->mol[m];
+            fm[m] = FockMol{x.n, m, x.uhf ? 1 : 0, &x.ctx->cls, x.pair_off, pairs.data() + x.pair_off};
+        }
+        if (int rc = b->fs.build(fm, b->pairs.p, b->prims.p, (int)pairs.size(), (long long)prims.size(), njp, st)) {
+            delete b;
+            return rc;
+        }
     }
     const size_t S = (size_t)b->store;
     DBuf<double>* stores[] = {&b->H, &b->S, &b->X, &b->P[0], &b->P[1], &b->Pold[0], &b->Pold[1], &b->F[0], &b->F[1],
@@ -528,7 +391,7 @@ int uno_batch_get(const uno_batch* b, const char* key, double* v) {
     else if (k == "space_builds") *v = b->space_builds;
     else if (k == "graph_builds") *v = b->graph_builds;
     else if (k == "graph_replays") *v = b->graph_replays;
-    else if (k == "launches_per_build") *v = (double)b->groups.size();
+    else if (k == "launches_per_build") *v = (double)b->fs.launches.size();
     else { set_error("unknown batch option " + k); return UNO_EINVAL; }
     return UNO_OK;
 }
@@ -556,11 +419,15 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
     hipStream_t st = b->st;
     b->scratch.reset();
     b->warm[0] = b->warm[1] = false;
-    // static spaces and the captured build belong to one run (its density bounds)
+    // the captured build belongs to one run
     b->drop_graph();
-    b->groups.clear();
-    b->dbound.clear();
-    b->space_builds = b->graph_builds = b->graph_replays = 0;
+    b->space_builds = 1;
+    b->graph_builds = b->graph_replays = 0;
+    {
+        ClearList cl;
+        cl.add(b->fs.nquart.p, 2 * kQuartSlots);
+        UNO_HIP(fock_clear(cl, st));
+    }
     const int nm = (int)b->mol.size();
     const long long S = b->store;
     // per-molecule eigenvalue offsets into ev stores: reuse the matrix offsets (n <= n^2)
@@ -696,7 +563,6 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
     std::vector<double> Bm((size_t)nm * kBatchDiis * kBatchDiis, 0.0);
     int iteration = 0;
     double fock_s = 0.0;
-    double quartets = 0.0;
     int nstopped = 0;
     double wall99 = -1.0;
     while (true) {
@@ -706,17 +572,7 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
         UNO_HIP(hipMemcpyAsync(b->D1.p, b->P[0].p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
         UNO_HIP(hipMemcpyAsync(b->D2.p, b->P[1].p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
         UNO_HIP(k_axpby(S, 1.0, b->D1.p, 1.0, b->D2.p, b->D0.p, st));
-        UNO_HIP(batch_shell_max((int)sl[0].size(), dsl[0].p, b->sh_off.p, b->sh_n.p, b->D0.p, b->D1.p, b->D2.p,
-                                b->Dsh.p, st));
-        std::vector<double> dsh(b->dsh_total);
-        UNO_HIP(hipMemcpyAsync(dsh.data(), b->Dsh.p, dsh.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-        UNO_HIP(hipStreamSynchronize(st));
-        std::vector<double> dmax(nm, 0.0);
-        for (int m = 0; m < nm; ++m)
-            if (b->mol[m].active)
-                for (long long k = 0; k < (long long)b->mol[m].nsh * b->mol[m].nsh; ++k)
-                    dmax[m] = std::max(dmax[m], dsh[b->mol[m].dshoff + k]);
-        if (int rc = batch_fock(b, dmax, quartets)) return rc;
+        if (int rc = batch_fock(b)) return rc;
         UNO_HIP(batch_sym((int)sl[0].size(), dsl[0].p, b->W0.p, b->G[0].p, false, st));
         if (!sl[1].empty()) UNO_HIP(batch_sym((int)sl[1].size(), dsl[1].p, b->W1.p, b->G[1].p, false, st));
         fock_s += secs(tf, clk::now());
@@ -850,6 +706,13 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
         }
     }
     const double wall = secs(t0, clk::now());
+    double quartets = 0.0;
+    {
+        std::vector<unsigned long long> h(2 * kQuartSlots);
+        UNO_HIP(hipMemcpyAsync(h.data(), b->fs.nquart.p, h.size() * sizeof(h[0]), hipMemcpyDeviceToHost, st));
+        UNO_HIP(hipStreamSynchronize(st));
+        for (unsigned long long v : h) quartets += (double)v;
+    }
     int rc = UNO_OK;
     for (int m = 0; m < nm; ++m) {
         const BatchMol& x = b->mol[m];

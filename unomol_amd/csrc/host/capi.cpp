@@ -341,10 +341,12 @@ int uno_ctx_get(uno_ctx* c, const char* key, double* v) {
     else if (k == "ctx_ms_schwarz") *v = c->ctx_ms[1];
     else if (k == "ctx_ms_runs") *v = c->ctx_ms[2];
     else if (k == "ctx_ms_rest") *v = c->ctx_ms[3];
-    else if (k == "last_quartets") *v = c->last_quartets;
-    else if (k == "last_quartets32") *v = c->last_quartets32;
+    else if (k == "last_quartets" || k == "last_quartets32") {
+        if (int rc = fock_quartets(c)) return rc;
+        *v = k == "last_quartets" ? c->last_quartets : c->last_quartets32;
+    }
     else if (k == "pair_runs") *v = (double)c->cls.size();
-    else if (k == "quartet_launches") *v = (double)c->qcls.size();
+    else if (k == "quartet_launches") *v = (double)(c->cls.size() * (c->cls.size() + 1) / 2);
     else if (k == "pairs") *v = (double)c->pairs.size();
     else { set_error("unknown option " + k); return UNO_EINVAL; }
     return UNO_OK;
@@ -357,7 +359,7 @@ int uno_fock_rhf(uno_ctx* c, const double* P, double* G) {
     hipStream_t st = c->st;
     UNO_HIP(c->pk.upload(P, n2, st));
     UNO_HIP(k_unpack(n, c->pk.p, c->D0.p, st));
-    if (int rc = fock_build(c, false, -1.0, c->precision == 1)) return rc;
+    if (int rc = fock_build(c, false, c->precision == 1)) return rc;
     UNO_HIP(c->pk.upload(G, n2, st));
     UNO_HIP(k_pack_sym_add(n, c->W0.p, c->pk.p, st));
     UNO_HIP(hipMemcpyAsync(G, c->pk.p, n2 * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -375,7 +377,7 @@ int uno_fock_uhf(uno_ctx* c, const double* PA, const double* PB, double* GA, dou
     UNO_HIP(c->pk.upload(PB, n2, st));
     UNO_HIP(k_unpack(n, c->pk.p, c->D2.p, st));
     UNO_HIP(k_axpby(nn, 1.0, c->D1.p, 1.0, c->D2.p, c->D0.p, st));
-    if (int rc = fock_build(c, true, -1.0, c->precision == 1)) return rc;
+    if (int rc = fock_build(c, true, c->precision == 1)) return rc;
     double* Gs[2] = {GA, GB};
     double* Ws[2] = {c->W0.p, c->W1.p};
     for (int s = 0; s < 2; ++s) {
@@ -402,7 +404,7 @@ int uno_autotune(uno_ctx* c, const double* PA, const double* PB, int mixed, doub
     }
     c->tuning = 1;
     c->tune_ms = 0.0;
-    const int rc = fock_build(c, uhf, -1.0, mixed != 0);
+    const int rc = fock_build(c, uhf, mixed != 0);
     c->tuning = 0;
     if (rc) return rc;
     UNO_HIP(hipStreamSynchronize(st));

@@ -161,18 +161,7 @@ void delete_eigen(EigenWS* w) { delete w; }
 
 uno_ctx::~uno_ctx() {
     uno::delete_eigen(eig);
-    if (stage_ev) (void)hipEventSynchronize(stage_ev);
-    if (stage_pin) (void)hipHostFree(stage_pin);
-    if (stage_ev) (void)hipEventDestroy(stage_ev);
     if (st) (void)hipStreamSynchronize(st);
     for (hipEvent_t e : prof_ev) (void)hipEventDestroy(e);
-    for (int w = 0; w + 1 < uno::kMaxLaunchStreams; ++w) {
-        if (wst[w]) {
-            (void)hipStreamSynchronize(wst[w]);
-            (void)hipStreamDestroy(wst[w]);
-        }
-        if (wjoin[w]) (void)hipEventDestroy(wjoin[w]);
-    }
-    if (wfork) (void)hipEventDestroy(wfork);
     if (st) (void)hipStreamDestroy(st);
 }

@@ -7,6 +7,7 @@
 #include <vector>
 #include "../../../include/unomol.h"
 #include "../hip/devtypes.hpp"
+#include "../hip/kernels.hpp"
 #include "../hip/oneint_kernels.hpp"
 #include "basis.hpp"
 
@@ -66,43 +67,14 @@ struct PairClassList {
     std::vector<double> Q;      // host copy of the bounds of the run
 };
 
-// One quartet space of a launch: per bra, a contiguous range of kets (prefix counts, the
-// first ket of each range when it does not start at 0) and the block table.
-struct QuartetSpace {
-    // bras b0 .. b0 + prefix.size() - 2 of the bra run (the empty bras at either end are
-    // trimmed); prefix[i] = first quartet of bra b0 + i
-    int b0 = 0;
-    std::vector<long long> prefix, wpre, rpre;
-    std::vector<int> kstart, blk, tblk, rbra;
-    DBuf<long long> d_prefix, d_wpre, d_rpre;
-    DBuf<int> d_kstart, d_blk, d_tblk, d_rbra;
-    long long nq = 0, ntask = 0, nrtask = 0;
-};
-
-// row-merged Fock-build tasks: bras with at least row_min_kets (default kRowMinKets) kets
-// in a space run as blocks of kRowSeg kets whose exchange contributions are merged in LDS
-// (the LDS variant per class and n from eri_rows_variant)
-constexpr long long kRowMinKets = 192;
-constexpr int kRowSeg = 1024;
-
-struct TuneChoice {
-    int variant;
-    long long min_kets;
-    int dlds = 0;   // the bra's exchange density rows staged in LDS as well
-};
-
-struct QuartetClass {
-    int X, Y;                   // indices into the runs, X >= Y (bra run, ket run)
-    QuartetSpace s64;           // FP64 quartets (all of them unless the build is mixed)
-    QuartetSpace s32;           // mixed builds: quartets whose Schwarz bound is below fp32_thr
-};
-
-// profiling slots: kernel kind (0 the wave-task / per-quartet kernels, 1-3 the row-merged
-// variants, 4-5 the bra-group row kernels), then precision (FP64, FP32), then the class
-// pair (6 X + Y): slot = 72 kind + 36 prec + 6 X + Y
+// profiling slots: kernel kind (0 the kernels without LDS rows and the wave kernels, 1-3 the
+// row-merged variants), then precision (FP64, FP32), then the class pair (6 X + Y): slot =
+// 72 kind + 36 prec + 6 X + Y
 constexpr int kProfKinds = 6;
 constexpr int kProfSlots = kProfKinds * 2 * kNumPairClasses * kNumPairClasses;
 
+// ket count from which a launch merges the bra's exchange rows in LDS
+constexpr long long kRowMinKets = 192;
 constexpr int kNumBuckets = 6;
 // streams a Fock build's ERI launches may be spread over (HIP's default is four hardware
 // queues per process)
@@ -112,6 +84,48 @@ inline int prim_bucket(int nprim) {
 }
 
 struct EigenWS;
+
+// What the Fock kernels read (fock.cpp, fock_core.hpp): the pair data in their layouts and the
+// quartet spaces of every launch, fixed when the pair data is.  One for a context, or one for
+// all molecules of a batch (their pair arrays concatenated).
+struct FockMol {
+    int n = 0, mol = 0, group = 0;         // functions; molecule; launch group (open shell)
+    const std::vector<PairClassList>* runs = nullptr;
+    int pair_off = 0;                      // of the molecule's pairs in the whole array
+    const PairHdr* pairs = nullptr;        // host records of its pairs
+};
+struct FockLaunch {
+    int cx, cy, group;      // class pair, launch group
+    int nblocks, ncols;     // grid, largest column count
+    int nket;               // longest ket run
+    size_t sp, blk;         // offsets of its tables
+};
+struct FockStore {
+    int npair = 0;
+    long long njp = 0, kps = 0;
+    std::vector<FockLaunch> launches;
+    DBuf<char> tables;
+    DBuf<BraPrim> bprim;
+    DBuf<double> kprim, kgeo, dp, jp, dpair, dmax;
+    DBuf<int4> kidx;
+    DBuf<int> knp, colinv;
+    DBuf<int2> kcol;
+    DBuf<unsigned long long> nquart;       // FP64 launches' counters, then FP32's
+    int build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, const PrimPair* d_prims, int np, long long nprims,
+              long long njp, hipStream_t st);
+    FockArgs args(const FockLaunch& l, const PairHdr* d_pairs, const PrimPair* d_prims, const double* pairQ) const;
+};
+// streams that launches are spread over: the caller's and up to kMaxLaunchStreams - 1 workers at
+// the default priority, forked from and joined back to the caller's
+struct LaunchStreams {
+    hipStream_t w[kMaxLaunchStreams - 1] = {};
+    hipEvent_t fork = nullptr, join[kMaxLaunchStreams - 1] = {};
+    int prepare(int n);                    // makes what n streams need
+    int begin(int n, hipStream_t st);
+    int end(int n, hipStream_t st);
+    hipStream_t of(int i, hipStream_t st) const { return i == 0 ? st : w[i - 1]; }
+    ~LaunchStreams();
+};
 
 }  // namespace uno
 
@@ -137,59 +151,45 @@ struct uno_ctx {
     uno::DBuf<uno::PairHdr> d_pairs;
     uno::DBuf<uno::PrimPair> d_prims;
     std::vector<uno::PairClassList> cls;   // runs ordered by (angular class, bucket)
-    std::vector<uno::QuartetClass> qcls;
+    uno::FockStore fs;
     uno::DBuf<double> d_pairQ;
     // per-shell function layout for the density screen
     uno::DBuf<int> d_shoff, d_shn;
     // device work matrices (n x n)
     uno::DBuf<double> D0, D1, D2, W0, W1, Dsh, pk, scal;
-    uno::DBuf<double> JP;        // pair-major accumulator of the kets' Coulomb outputs
     uno::DBuf<double> red;       // partial sums of the two-pass reductions
-    // LDS row columns of the row-merged launches, per pair run (ket side): run_ncols[r]
-    // columns, d_colmap[r n + f] = column of function f or -1, d_colinv[r n + c] = function
-    std::vector<int> run_ncols;
-    uno::DBuf<int> d_colmap, d_colinv;
-    std::vector<char> stage_h;   // a Fock build's index arrays, uploaded once per build
-    char* stage_pin = nullptr;   // pinned copy of stage_h that the (asynchronous) upload reads
-    size_t stage_pin_cap = 0;
-    hipEvent_t stage_ev = nullptr;   // recorded after the upload: stage_pin is free again
-    uno::DBuf<char> stage_d;
-    long long njp = 0;
     uno::EigenWS* eig = nullptr;
+    // quartets of the last build (read back from fs.nquart when asked for)
     double last_quartets = 0.0, last_quartets32 = 0.0;
-    // host milliseconds of the last build: density bound read-back, quartet spaces and
-    // index arrays, staging upload, launch enqueue (the kernels run asynchronously)
-    double last_ms[4] = {0.0, 0.0, 0.0, 0.0};
+    bool quartets_known = true;
     // host milliseconds of the context build: pair records, Schwarz bounds (device),
     // sorted runs and their upload, the rest (columns, one-electron data, buffers)
     double ctx_ms[4] = {0.0, 0.0, 0.0, 0.0};
     // profiling pass: per quartet class (bra X, ket Y) kernel milliseconds and the
     // primitive / shell quartets the kernels evaluated
     int profile = 0;
-    // Fock builds run bras with many kets as row-merged blocks (1) or all as wave tasks (0)
+    // exchange rows of the bra merged in LDS (1) or every output straight to W (0), for launches
+    // whose ket runs reach row_min_kets
     int row_merge = 1;
     long long row_min_kets = uno::kRowMinKets;
-    int row_variant = 0;     // row-merged LDS variant: 0 the best that fits, 1-3 forced
+    int row_variant = 0;     // LDS layout: 0 the best that fits, 1-3 forced where they fit
     int rys2_exact = 0;      // 1: exact two-root Rys quadrature; 0: the reference's (default)
     int purify = -1;         // SCF densities by purification: -1 from 256 functions, 0 never, 1 always
     int x_newton = -1;       // X = S^-1/2 by Newton-Schulz: -1 from kSp2MinN functions on, 0 never, 1 always
     int last_x_steps = -1;   // the last SCF's Newton-Schulz steps (-1: the canonical X)
     // 1: Fock builds accumulate in fixed point (bitwise the same G for the same input, in
-    // any launch order) and run every bra as wave tasks (the row kernels merge with FP64
-    // atomics); the SCF's dense products run without split K
+    // any launch order) without LDS rows (those merge with FP64 atomics); the SCF's dense
+    // products run without split K
     int deterministic = 0;
     // the ERI launches of a Fock build go round-robin over the context's stream and
     // launch_streams - 1 worker streams (default priority), joined back before the build's
-    // last steps: the many small launches (FP32 tails, small quartet spaces) then run side
-    // by side instead of each leaving most of the GPU idle
+    // last steps: the small launches then run side by side
     int launch_streams = 3;
-    hipStream_t wst[uno::kMaxLaunchStreams - 1] = {};
-    hipEvent_t wfork = nullptr, wjoin[uno::kMaxLaunchStreams - 1] = {};
+    uno::LaunchStreams ls;
     int row_dens = -1;       // exchange density rows in LDS: -1 when they fit, 0 never, 1 forced where they fit
-    // autotuned row-merge configuration per quartet space (run-pair index, precision, UHF,
-    // mixed build): LDS variant (0 = wave tasks only) and the ket count from which a bra is
-    // row-merged.  tuning = 1 while uno_autotune times the candidates.
-    std::map<std::tuple<int, int, int, int>, uno::TuneChoice> tune;
+    // autotuned configuration per launch (class pair, precision, UHF, mixed build); tuning = 1
+    // while uno_autotune times the candidates
+    std::map<std::tuple<int, int, int, int>, uno::FockConfig> tune;
     int tuning = 0;
     double tune_ms = 0.0;
     double prof_ms[uno::kProfSlots] = {};
@@ -218,14 +218,10 @@ struct uno_ctx {
 namespace uno {
 
 int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell);
-// quartet-space helpers of the Fock build (ctx.cpp)
-void build_prefix(uno_ctx* c, QuartetClass& q, double dmax, double fp32_thr, double tau);
-void build_tasks(QuartetSpace& s, long long row_min_kets = 0);
-void build_rows(QuartetSpace& s, long long min_kets, int seg, int group = 1);
-void build_blocks(QuartetSpace& s, int qpb);
 EriArgs base_args(uno_ctx* c);
-// keeps c's tuned configurations for later contexts of the same layout
+// tuned configurations, kept for later contexts of the same layout
 void remember_tuning(uno_ctx* c);
+void recall_tuning(uno_ctx* c);
 // profiling: reset (and, when enabling, zero the device counters), or fold the pending
 // event pairs and the counters into the context's per-slot totals
 int profile_reset(uno_ctx* c, bool enable);
@@ -235,7 +231,9 @@ int oneint_device(uno_ctx* c, double* S, double* T, double* H);
 // Fock build from dense device densities already in c->D0 (and D1, D2 for UHF).
 // Leaves W0 (and W1) = unsymmetrised accumulators; G = W + W^T.  mixed: quartets whose
 // Schwarz bound Qab Qcd is below c->fp32_thr are evaluated in FP32.
-int fock_build(uno_ctx* c, bool uhf, double dmax_hint, bool mixed = false);
+int fock_build(uno_ctx* c, bool uhf, bool mixed = false);
+// c->last_quartets / last_quartets32 of the last build (waits for it)
+int fock_quartets(uno_ctx* c);
 int eri_emit(uno_ctx* c, long cap, double* val, int* ijkl, long* count);
 
 // dense symmetric eigensolver on device data: A (destroyed) -> Z (eigenvectors in

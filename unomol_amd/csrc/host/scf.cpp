@@ -335,7 +335,7 @@ int scf_run(uno_ctx* c, int nelec, const uno_scf_opts& o, uno_scf_result& r, dou
         const bool mixed = o.precision == 1;
         const double tau0 = c->tau;
         if (mixed) c->tau = std::max(tau0, c->tau_mixed);
-        const int rc = fock_build(c, uhf, -1.0, mixed);
+        const int rc = fock_build(c, uhf, mixed);
         c->tau = tau0;
         if (rc) return rc;
         double h[2];
@@ -468,7 +468,7 @@ int scf_run(uno_ctx* c, int nelec, const uno_scf_opts& o, uno_scf_result& r, dou
             // iterations; the FP64 phase starts with a full rebuild at the context's tau)
             const double tau0 = c->tau;
             if (mixed) c->tau = std::max(tau0, c->tau_mixed);
-            const int rc = fock_build(c, uhf, -1.0, mixed);
+            const int rc = fock_build(c, uhf, mixed);
             c->tau = tau0;
             if (rc) return rc;
         }
@@ -479,7 +479,6 @@ int scf_run(uno_ctx* c, int nelec, const uno_scf_opts& o, uno_scf_result& r, dou
         }
         if (full) { need_full = false; nincr = 0; ++r.nfull; } else ++nincr;
         if (!mixed) ++fp64_updates;
-        r.quartets32 += c->last_quartets32;
         UNO_HIP(k_fill(4, 0.0, c->scal.p, st));
         for (int s = 0; s < ns; ++s) {
             UNO_HIP(k_dot(nn, P[s], b.H.p, c->scal.p, c->red.p, st));
@@ -489,12 +488,13 @@ int scf_run(uno_ctx* c, int nelec, const uno_scf_opts& o, uno_scf_result& r, dou
         UNO_HIP(hipStreamSynchronize(st));
         const double build_s = secs(t0, clk::now());
         fock_s += build_s;
+        if (int rc = fock_quartets(c)) return rc;
+        r.quartets32 += c->last_quartets32;
         if (o.verbose > 1)
             std::fprintf(stderr,
-                         "[scf] build %d: %s %s, %.2f ms (host: bound %.2f, spaces %.2f, staging %.2f, enqueue %.2f), "
-                         "%.3e shell quartets (%.3e FP32)\n",
-                         r.nfock + 1, full ? "full" : "incremental", mixed ? "mixed" : "FP64", 1e3 * build_s, c->last_ms[0],
-                         c->last_ms[1], c->last_ms[2], c->last_ms[3], c->last_quartets, c->last_quartets32);
+                         "[scf] build %d: %s %s, %.2f ms, %.3e shell quartets (%.3e FP32)\n", r.nfock + 1,
+                         full ? "full" : "incremental", mixed ? "mixed" : "FP64", 1e3 * build_s, c->last_quartets,
+                         c->last_quartets32);
         r.quartets += c->last_quartets;
         ++r.nfock;
         energy = uhf ? hs[0] + 0.5 * hs[1] : 2.0 * hs[0] + hs[1];

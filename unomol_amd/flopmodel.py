@@ -2,7 +2,7 @@
 
 The count replays the arithmetic of one primitive quartet of the lane kernel
 (``eri_block`` in csrc/hip/eri.hip with ``rys_roots``/``axis_table`` from eri_core.hpp)
-and of one shell quartet's normalisation and RHF J/K digestion (``k_eri_bra``) on
+and of one shell quartet's normalisation and RHF J/K digestion (``k_fock``) on
 symbolic values, the way the compiler sees the fully unrolled code:
 
 * constants fold (products with 1 or 0, sums with 0, constant-only arithmetic);
