@@ -148,8 +148,11 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                 std::stable_sort(cs.begin(), cs.end(), [](const Cand& u, const Cand& v) { return u.work > v.work; });
                 std::vector<FockSpace> sp;
                 long long nb = 0;
-                // segments as long as leaves enough blocks to balance the launch (and their
-                // number within a grid)
+                // segments as long as leaves about 8192 passes' worth of blocks to balance the
+                // launch (and their number within a grid): each block ends by adding its rows to
+                // W, an atomic per row and column, which at 1024 kets a block was as many as the
+                // kets' own (64 waters, one stream: 93.5 ms at up to 4 passes, 75.0 at up to 32;
+                // (ds|ss) 11.2 -> 6.6, (ss|ss) 10.1 -> 6.1)
                 for (int longer = 1;; longer *= 2) {
                     sp.clear();
                     nb = 0;
@@ -160,7 +163,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                         } else {
                             while ((1 << s.lg) < c.maxprim && s.lg < 6 && total * (2 << s.lg) <= kFillLanes) ++s.lg;
                             const int pass = kLaneBlock >> s.lg;
-                            s.seg = longer * pass * (int)std::max(1.0, std::min(4.0, total / (pass * 8192.0)));
+                            s.seg = longer * pass * (int)std::max(1.0, std::min(32.0, total / (pass * 8192.0)));
                         }
                         s.nseg = (s.nket + s.seg - 1) / s.seg;
                         s.first = (int)std::min<long long>(nb, INT32_MAX);
