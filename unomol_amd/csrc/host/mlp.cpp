@@ -29,8 +29,9 @@ struct uno_mlp {
     DBuf<__bf16> xb, dzb[2];
     std::vector<DBuf<float>> z;
     std::vector<DBuf<__bf16>> h;
-    DBuf<float> y, dy, dz[2], part, tb, mb;
-    DBuf<float> xin;   // inference inputs, kept between calls (no allocation per call)
+    DBuf<float> y, dz[2], part, tb, mb, wpart;
+    DBuf<double> norm;
+    DBuf<float> xin;   // host inputs as uploaded, kept between calls (no allocation per call)
     DBuf<int> idx;
     ~uno_mlp() {
         if (st) (void)hipStreamDestroy(st);
@@ -91,7 +92,10 @@ int ensure_batch(uno_mlp* m, int B) {
     }
     const int out = m->dims[L];
     UNO_HIP(m->y.alloc((size_t)B * out));
-    UNO_HIP(m->dy.alloc((size_t)B * out));
+    size_t wp = 0;
+    for (int l = 0; l < L; ++l) wp = std::max(wp, wgrad_part(m->dims[l], m->dims[l + 1]));
+    UNO_HIP(m->wpart.alloc(wp));
+    UNO_HIP(m->norm.alloc(1 + kMaskBlocks));
     UNO_HIP(m->tb.alloc((size_t)B * out));
     UNO_HIP(m->mb.alloc((size_t)B * out));
     UNO_HIP(m->part.alloc(((size_t)B * out + 255) / 256));
@@ -115,48 +119,38 @@ int forward(uno_mlp* m, int B) {
         } else {
             ep.out_f32 = m->y.p;
         }
-        UNO_HIP(gemm_bf16(false, false, last ? kEpiStore : kEpiBiasSilu, B, m->dims[l + 1], m->dims[l], in, m->dims[l],
+        UNO_HIP(gemm_bf16(false, last ? kEpiStore : kEpiBiasSilu, B, m->dims[l + 1], m->dims[l], in, m->dims[l],
                           m->pb.p + m->woff[l], m->dims[l + 1], ep, m->st));
         in = m->h[l].p;
     }
     return UNO_OK;
 }
 
-// loss on the staged batch (targets tb, mask mb, norm = sum of the mask) and gradients in g
-int backward(uno_mlp* m, int B, float inv_norm, int* nblk) {
+// loss on the staged batch (targets tb, mask mb, norm = sum of the mask, by its reciprocal or on the
+// device) and gradients in g
+int backward(uno_mlp* m, int B, float inv_norm, const double* norm, int* nblk) {
     const int L = nlayers(m);
     const int out = m->dims[L];
-    UNO_HIP(mse_loss((long)B * out, m->y.p, m->tb.p, m->mb.p, inv_norm, m->dz[0].p, m->dzb[0].p, m->part.p, nblk,
-                     m->st));
+    UNO_HIP(mse_loss((long)B * out, m->y.p, m->tb.p, m->mb.p, inv_norm, norm, m->dz[0].p, m->dzb[0].p, m->part.p,
+                     nblk, m->st));
     int cur = 0;
     for (int l = L - 1; l >= 0; --l) {
         const __bf16* a_in = l == 0 ? m->xb.p : m->h[l - 1].p;
-        MlpEpilogue ew{};
-        ew.ldc = m->dims[l + 1];
-        ew.out_f32 = m->g.p + m->woff[l];
-        UNO_HIP(gemm_bf16(true, false, kEpiStore, m->dims[l], m->dims[l + 1], B, a_in, m->dims[l], m->dzb[cur].p,
-                          m->dims[l + 1], ew, m->st));
-        UNO_HIP(col_sum(B, m->dims[l + 1], m->dz[cur].p, m->g.p + m->boff[l], m->st));
+        // dW and, behind it, db (b_l follows W_l in the parameters)
+        UNO_HIP(wgrad(m->dims[l], m->dims[l + 1], B, a_in, m->dzb[cur].p, m->dz[cur].p, m->wpart.p, m->g.p + m->woff[l],
+                      m->st));
         if (l > 0) {
             MlpEpilogue eh{};
             eh.ldc = m->dims[l];
             eh.aux_f32 = m->z[l - 1].p;
             eh.out_f32 = m->dz[1 - cur].p;
             eh.out_bf16 = m->dzb[1 - cur].p;
-            UNO_HIP(gemm_bf16(false, true, kEpiSiluGrad, B, m->dims[l], m->dims[l + 1], m->dzb[cur].p, m->dims[l + 1],
+            UNO_HIP(gemm_bf16(true, kEpiSiluGrad, B, m->dims[l], m->dims[l + 1], m->dzb[cur].p, m->dims[l + 1],
                               m->pb.p + m->woff[l], m->dims[l + 1], eh, m->st));
             cur = 1 - cur;
         }
     }
     return UNO_OK;
-}
-
-float mask_sum(const float* M, const std::vector<int>& rows, int out) {
-    double s = 0.0;
-    for (int r : rows)
-        if (r >= 0)
-            for (int c = 0; c < out; ++c) s += M[(long)r * out + c];
-    return (float)s;
 }
 
 // stage rows of host arrays (X as BF16; T, M as f32) through a device copy of the rows
@@ -241,14 +235,14 @@ int uno_mlp_forward(uno_mlp* m, long n, const float* X, float* Y) {
     const int in = m->dims[0], out = m->dims.back();
     const int chunk = 4096;
     if (int rc = ensure_batch(m, chunk)) return rc;
-    DBuf<float>& dX = m->xin;
-    UNO_HIP(dX.upload(X, (size_t)n * in, m->st));
+    const size_t rows = (size_t)((n + 63) / 64) * 64;
+    UNO_HIP(m->xin.alloc(rows * in));
+    UNO_HIP(hipMemcpyAsync(m->xin.p, X, (size_t)n * in * sizeof(float), hipMemcpyHostToDevice, m->st));
+    if (rows > (size_t)n) UNO_HIP(hipMemsetAsync(m->xin.p + (size_t)n * in, 0, (rows - n) * in * sizeof(float), m->st));
     for (long r0 = 0; r0 < n; r0 += chunk) {
         const int cnt = (int)std::min<long>(chunk, n - r0);
         const int B = round_up(cnt, 64);
-        std::vector<int> rows(B, -1);
-        for (int r = 0; r < cnt; ++r) rows[r] = (int)(r0 + r);
-        if (int rc = stage_rows(m, rows, dX, nullptr, nullptr)) return rc;
+        UNO_HIP(to_bf16((long)B * in, m->xin.p + r0 * in, m->xb.p, m->st));
         if (int rc = forward(m, B)) return rc;
         UNO_HIP(hipMemcpyAsync(Y + r0 * out, m->y.p, (size_t)cnt * out * sizeof(float), hipMemcpyDeviceToHost, m->st));
         UNO_HIP(hipStreamSynchronize(m->st));
@@ -262,18 +256,27 @@ int uno_mlp_loss_grad(uno_mlp* m, long n, const float* X, const float* T, const 
     const int in = m->dims[0], out = m->dims.back();
     const int B = round_up((int)n, 64);
     if (int rc = ensure_batch(m, B)) return rc;
-    DBuf<float> dX, dT, dM;
-    UNO_HIP(dX.upload(X, (size_t)n * in, m->st));
-    UNO_HIP(dT.upload(T, (size_t)n * out, m->st));
-    UNO_HIP(dM.upload(M, (size_t)n * out, m->st));
-    std::vector<int> rows(B, -1);
-    std::iota(rows.begin(), rows.begin() + n, 0);
-    if (int rc = stage_rows(m, rows, dX, &dT, &dM)) return rc;
-    const float norm = mask_sum(M, rows, out);
-    if (!(norm > 0.0f)) { set_error("mask is empty"); return UNO_EINVAL; }
+    // the rows go up as they are (the padding rows' inputs, targets and mask are zero)
+    const size_t pad = (size_t)(B - n);
+    UNO_HIP(m->xin.alloc((size_t)B * in));
+    UNO_HIP(hipMemcpyAsync(m->xin.p, X, (size_t)n * in * sizeof(float), hipMemcpyHostToDevice, m->st));
+    UNO_HIP(hipMemcpyAsync(m->tb.p, T, (size_t)n * out * sizeof(float), hipMemcpyHostToDevice, m->st));
+    UNO_HIP(hipMemcpyAsync(m->mb.p, M, (size_t)n * out * sizeof(float), hipMemcpyHostToDevice, m->st));
+    if (pad) {
+        UNO_HIP(hipMemsetAsync(m->xin.p + (size_t)n * in, 0, pad * in * sizeof(float), m->st));
+        UNO_HIP(hipMemsetAsync(m->tb.p + (size_t)n * out, 0, pad * out * sizeof(float), m->st));
+        UNO_HIP(hipMemsetAsync(m->mb.p + (size_t)n * out, 0, pad * out * sizeof(float), m->st));
+    }
+    UNO_HIP(to_bf16((long)B * in, m->xin.p, m->xb.p, m->st));
+    UNO_HIP(mask_norm((long)B * out, m->mb.p, m->norm.p, m->st));
     if (int rc = forward(m, B)) return rc;
     int nblk = 0;
-    if (int rc = backward(m, B, 1.0f / norm, &nblk)) return rc;
+    if (int rc = backward(m, B, 0.0f, m->norm.p, &nblk)) return rc;
+    double dnorm = 0.0;
+    UNO_HIP(hipMemcpyAsync(&dnorm, m->norm.p, sizeof(double), hipMemcpyDeviceToHost, m->st));
+    UNO_HIP(hipStreamSynchronize(m->st));
+    const float norm = (float)dnorm;
+    if (!(norm > 0.0f)) { set_error("mask is empty"); return UNO_EINVAL; }
     std::vector<float> part(nblk);
     UNO_HIP(hipMemcpyAsync(part.data(), m->part.p, nblk * sizeof(float), hipMemcpyDeviceToHost, m->st));
     if (grad) UNO_HIP(hipMemcpyAsync(grad, m->g.p, m->np * sizeof(float), hipMemcpyDeviceToHost, m->st));
@@ -320,7 +323,7 @@ int uno_mlp_train(uno_mlp* m, long n, const float* X, const float* T, const floa
         if (int rc = stage_rows(m, rows, dX, &dT, &dM)) return rc;
         if (int rc = forward(m, batch)) return rc;
         int nblk = 0;
-        if (int rc = backward(m, batch, norm > 0.0 ? (float)(1.0 / norm) : 0.0f, &nblk)) return rc;
+        if (int rc = backward(m, batch, norm > 0.0 ? (float)(1.0 / norm) : 0.0f, nullptr, &nblk)) return rc;
         // cosine-decayed learning rate
         const float lr_t = lr * 0.5f * (1.0f + std::cos(3.14159265f * (float)it / (float)steps));
         ++m->step;
@@ -338,8 +341,8 @@ int uno_mlp_train(uno_mlp* m, long n, const float* X, const float* T, const floa
             if (int rc = stage_rows(m, rr, dX, &dT, &dM)) return rc;
             if (int rc = forward(m, chunk)) return rc;
             int nblk = 0;
-            UNO_HIP(mse_loss((long)chunk * out, m->y.p, m->tb.p, m->mb.p, 1.0f, m->dz[0].p, m->dzb[0].p, m->part.p,
-                             &nblk, m->st));
+            UNO_HIP(mse_loss((long)chunk * out, m->y.p, m->tb.p, m->mb.p, 1.0f, nullptr, m->dz[0].p, m->dzb[0].p,
+                             m->part.p, &nblk, m->st));
             std::vector<float> part(nblk);
             UNO_HIP(hipMemcpyAsync(part.data(), m->part.p, nblk * sizeof(float), hipMemcpyDeviceToHost, m->st));
             UNO_HIP(hipStreamSynchronize(m->st));
