@@ -9,6 +9,7 @@
 //    columns, then the eigenvector columns; eigenvalues ascending with their vectors;
 //  * per-molecule reductions (trace products, difference norms) and helpers.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include "batch_kernels.hpp"
 
 namespace uno {
@@ -81,6 +82,7 @@ hipError_t grouped_gemm(int ntiles, const GemmTile* tiles, const GemmGroup* grou
 // relative test alone never settles next to zero diagonal entries, where rounding keeps
 // a_pq above it); sweeps stop when none is applied.
 constexpr int kJacobiThreads = 1024;
+constexpr int kJacobiLdsN = 140;   // largest matrix of the LDS kernel below
 __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMat* __restrict__ mats, int max_sweeps,
                                                                    int* __restrict__ sweeps_out) {
     __shared__ double cs[128], sn[128];
@@ -89,6 +91,7 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMa
     __shared__ double red[kJacobiThreads / 64];
     const BatchMat M = mats[blockIdx.x];
     const int n = M.n;
+    if (n <= kJacobiLdsN) return;   // the LDS kernel's
     double* A = M.A;
     double* V = M.V;
     const int tid = threadIdx.x;
@@ -180,9 +183,182 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMa
     if (tid == 0 && sweeps_out) sweeps_out[blockIdx.x] = sweep;
 }
 
-hipError_t batched_jacobi(int nmat, const BatchMat* mats, int max_sweeps, int* sweeps, hipStream_t st) {
+// The same rotations in the same order with the matrix in LDS, for n <= kJacobiLdsN (157 KB of the
+// 160 at 140 functions): a round is two phases, the rotations and one pass that applies them
+// to both sides of every 2 x 2 block of the pairs (k, l), k <= l, writing the mirrored block too,
+// and to the eigenvectors.  The eigenvectors are kept transposed (the two vectors of a rotation are
+// rows), in LDS as well while both fit, else in V.  With the matrix in global memory every round
+// made three passes over it at L2 latency: 5.7 ms a launch for 32 molecules of up to 95 functions (mean
+// of an SCF, most of them warm), 1.0 ms here.
+__host__ __device__ constexpr int jacobi_ld(int n) { return n | 1; }   // odd: columns fall on different banks
+__host__ __device__ constexpr bool jacobi_v_fits(int n) { return 2 * n * jacobi_ld(n) <= kJacobiLdsN * jacobi_ld(kJacobiLdsN); }
+__global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const BatchMat* __restrict__ mats, int max_sweeps,
+                                                                       int* __restrict__ sweeps_out) {
+    extern __shared__ double lds[];
+    __shared__ double cs[kJacobiLdsN / 2], sn[kJacobiLdsN / 2];
+    __shared__ int pp[kJacobiLdsN / 2], qq[kJacobiLdsN / 2];
+    __shared__ int nrot;
+    __shared__ double red[kJacobiThreads / 64];
+    const BatchMat M = mats[blockIdx.x];
+    const int n = M.n, ld = jacobi_ld(n);
+    if (n > kJacobiLdsN) return;   // the other kernel's
+    double* A = lds;
+    const bool vl = jacobi_v_fits(n);
+    double* V = vl ? lds + n * ld : M.V;   // V[p ldv + i] = component i of vector p
+    const int ldv = vl ? ld : n;
+    const int tid = threadIdx.x;
+    double f2 = 0.0;
+    for (int e = tid; e < n * n; e += kJacobiThreads) {
+        const int i = e / n, j = e - i * n;
+        const double v = M.A[e];
+        A[i * ld + j] = v;
+        V[i * ldv + j] = i == j ? 1.0 : 0.0;
+        f2 = fma(v, v, f2);
+    }
+    for (int o = 32; o >= 1; o >>= 1) f2 += __shfl_xor(f2, o, 64);
+    if ((tid & 63) == 0) red[tid >> 6] = f2;
+    __syncthreads();
+    double fro2 = 0.0;
+    for (int w = 0; w < kJacobiThreads / 64; ++w) fro2 += red[w];
+    const double abs_tol = 1e-15 * sqrt(fro2);
+    const int m = n + (n & 1), mk = m / 2;
+    // this thread's pair blocks (k, l), the same in every round: rows k and mk - 1 - k of the
+    // triangle together are mk + 1 blocks long
+    constexpr int kItems = (kJacobiLdsN / 2 * (kJacobiLdsN / 2 + 1) / 2 + kJacobiLdsN / 2 + kJacobiThreads - 1) / kJacobiThreads;
+    int ik[kItems], il[kItems];
+#pragma unroll
+    for (int x = 0; x < kItems; ++x) {
+        const int t = tid + x * kJacobiThreads, r = t / (mk + 1), c = t - r * (mk + 1);
+        ik[x] = -1;
+        il[x] = 0;
+        if (2 * r < mk) {
+            if (c < mk - r) {
+                ik[x] = r;
+                il[x] = r + c;
+            } else if (mk - 1 - r != r) {
+                ik[x] = mk - 1 - r;
+                il[x] = c - 1;
+            }
+        }
+    }
+    int sweep = 0;
+    while (sweep < max_sweeps && n > 1) {
+        ++sweep;
+        if (tid == 0) nrot = 0;
+        __syncthreads();
+        for (int r = 0; r < m - 1; ++r) {
+            if (tid < mk) {
+                int a, b;
+                if (tid == 0) {
+                    a = m - 1;
+                    b = r;
+                } else {
+                    a = r + tid;
+                    if (a >= m - 1) a -= m - 1;
+                    b = r - tid;
+                    if (b < 0) b += m - 1;
+                }
+                const int p = a < b ? a : b, q = a < b ? b : a;
+                double c = 1.0, s = 0.0;
+                if (q < n) {
+                    const double apq = A[p * ld + q];
+                    const double app = A[p * ld + p], aqq = A[q * ld + q];
+                    if (fabs(apq) > fmax(1.1102230246251565e-16 * sqrt(fabs(app * aqq)), abs_tol)) {
+                        const double theta = (aqq - app) / (2.0 * apq);
+                        const double t = fabs(theta) < 1e150
+                                             ? (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0))
+                                             : 0.5 / theta;
+                        c = 1.0 / sqrt(t * t + 1.0);
+                        s = t * c;
+                        atomicAdd(&nrot, 1);
+                    }
+                }
+                pp[tid] = p;
+                qq[tid] = q;
+                cs[tid] = c;
+                sn[tid] = s;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int x = 0; x < kItems; ++x) {
+                const int k = ik[x], l = il[x];
+                if (k < 0) continue;
+                const double ck = cs[k], sk = sn[k], cl = cs[l], sl = sn[l];
+                if (sk == 0.0 && sl == 0.0) continue;
+                // (the dummy index of an odd n only meets rotations with s = 0: its row and
+                // column are left out)
+                const int pk = pp[k], qk = qq[k], pl = pp[l], ql = qq[l];
+                const bool vk = qk < n, vl2 = ql < n;
+                const double a00 = A[pk * ld + pl], a01 = vl2 ? A[pk * ld + ql] : 0.0;
+                const double a10 = vk ? A[qk * ld + pl] : 0.0, a11 = vk && vl2 ? A[qk * ld + ql] : 0.0;
+                const double r00 = ck * a00 - sk * a10, r01 = ck * a01 - sk * a11;
+                const double r10 = sk * a00 + ck * a10, r11 = sk * a01 + ck * a11;
+                const double b00 = cl * r00 - sl * r01, b01 = sl * r00 + cl * r01;
+                const double b10 = cl * r10 - sl * r11, b11 = sl * r10 + cl * r11;
+                A[pk * ld + pl] = b00;
+                if (vl2) A[pk * ld + ql] = b01;
+                if (vk) A[qk * ld + pl] = b10;
+                if (vk && vl2) A[qk * ld + ql] = b11;
+                if (k != l) {
+                    A[pl * ld + pk] = b00;
+                    if (vl2) A[ql * ld + pk] = b01;
+                    if (vk) A[pl * ld + qk] = b10;
+                    if (vk && vl2) A[ql * ld + qk] = b11;
+                }
+            }
+            for (int e = tid; e < mk * n; e += kJacobiThreads) {
+                const int k = e / n, i = e - k * n;
+                const double s = sn[k];
+                if (s == 0.0) continue;
+                const double c = cs[k];
+                const int p = pp[k] * ldv + i, q = qq[k] * ldv + i;
+                const double vp = V[p], vq = V[q];
+                V[p] = c * vp - s * vq;
+                V[q] = s * vp + c * vq;
+            }
+            __syncthreads();
+        }
+        const int done = nrot == 0;
+        __syncthreads();
+        if (done) break;
+    }
+    __syncthreads();
+    // eigenvalues ascending (ties by index) with their vectors as columns of Z
+    int* rank = reinterpret_cast<int*>(cs);   // n <= 140 ints in 70 doubles
+    for (int i = tid; i < n; i += kJacobiThreads) {
+        const double di = A[i * ld + i];
+        int r = 0;
+        for (int j = 0; j < n; ++j) {
+            const double dj = A[j * ld + j];
+            if (dj < di || (dj == di && j < i)) ++r;
+        }
+        M.evals[r] = di;
+        rank[i] = r;
+    }
+    __syncthreads();
+    for (int e = tid; e < n * n; e += kJacobiThreads) {
+        const int i = e / n, r = e - i * n;
+        M.Z[(long)r * n + rank[i]] = V[i * ldv + r];
+    }
+    if (tid == 0 && sweeps_out) sweeps_out[blockIdx.x] = sweep;
+}
+
+hipError_t batched_jacobi(int nmat, const BatchMat* mats, int maxn, int max_sweeps, int* sweeps, hipStream_t st) {
     if (nmat <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_batched_jacobi, dim3(nmat), dim3(kJacobiThreads), 0, st, mats, max_sweeps, sweeps);
+    const int nl = std::min(maxn, kJacobiLdsN);
+    const size_t lds = sizeof(double) * (size_t)(jacobi_v_fits(nl) ? 2 : 1) * nl * jacobi_ld(nl);
+    // (a smaller matrix of the launch may keep its vectors in LDS where the largest does not)
+    const size_t need = jacobi_v_fits(nl) ? lds : sizeof(double) * (size_t)kJacobiLdsN * jacobi_ld(kJacobiLdsN);
+    static size_t attr = 0;
+    if (need > attr) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_batched_jacobi_lds),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)need);
+        if (e != hipSuccess) return e;
+        attr = need;
+    }
+    hipLaunchKernelGGL(k_batched_jacobi_lds, dim3(nmat), dim3(kJacobiThreads), need, st, mats, max_sweeps, sweeps);
+    if (maxn > kJacobiLdsN)
+        hipLaunchKernelGGL(k_batched_jacobi, dim3(nmat), dim3(kJacobiThreads), 0, st, mats, max_sweeps, sweeps);
     return hipGetLastError();
 }
 

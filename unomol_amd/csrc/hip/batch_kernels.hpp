@@ -29,8 +29,8 @@ struct BatchMat {
     double* evals;
     double* Z;
 };
-// n <= 256 per matrix; sweeps[b] (optional) receives the sweeps taken
-hipError_t batched_jacobi(int nmat, const BatchMat* mats, int max_sweeps, int* sweeps, hipStream_t st);
+// n <= 256 per matrix, maxn the largest; sweeps[b] (optional) receives the sweeps taken
+hipError_t batched_jacobi(int nmat, const BatchMat* mats, int maxn, int max_sweeps, int* sweeps, hipStream_t st);
 
 // one molecule's n x n matrix in a store
 struct MatSlot {

@@ -161,7 +161,7 @@ int batch_eigh(uno_batch* b, const std::vector<MatSlot>& sl, double* A, double* 
         bm[k] = BatchMat{sl[k].n, A + sl[k].off, b->V.p + sl[k].off, evals_base + evoff[k], b->Z.p + sl[k].off};
     BatchMat* d = nullptr;
     UNO_HIP(b->scratch.upload(bm.data(), bm.size(), b->st, &d));
-    UNO_HIP(batched_jacobi((int)bm.size(), d, 50, nullptr, b->st));
+    UNO_HIP(batched_jacobi((int)bm.size(), d, b->maxn, 50, nullptr, b->st));
     UNO_HIP(hipStreamSynchronize(b->st));
     return UNO_OK;
 }
@@ -515,7 +515,7 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
             }
             BatchMat* d = nullptr;
             UNO_HIP(b->scratch.upload(bm.data(), bm.size(), st, &d));
-            UNO_HIP(batched_jacobi((int)bm.size(), d, 50, nullptr, st));
+            UNO_HIP(batched_jacobi((int)bm.size(), d, b->maxn, 50, nullptr, st));
             // bm is pageable host memory: its upload must be done before it goes
             UNO_HIP(hipStreamSynchronize(st));
         }
