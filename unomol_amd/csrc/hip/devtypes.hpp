@@ -17,8 +17,7 @@ struct alignas(16) PairHdr {
     int nprim;      // number of primitive pairs
     int same;       // both shells are the same shell (a == b)
     int sh1, sh2;   // shell indices (first, second)
-    int jo;         // offset of the pair's function block in the pair-major Coulomb
-                    // accumulator (runs of pairs are contiguous there)
+    int pad;
 };
 
 struct alignas(16) PrimPair {
@@ -89,16 +88,19 @@ struct FockSpace {
     int kstride;          // the ket run's length: primitive j of ket i at kp0 + j kstride + i
     int pad;
     long long kp0;
-    long long jo0;        // first ket's Coulomb block in the pair-major arrays
+    long long jo0;        // component c of ket i at jo0 + c kstride + i of the pair-major arrays
 };
 
 // a run of the pair array, as the kernel that lays the ket records out needs it
 struct PairRun {
     int off, count;
     int col0;             // column of function f at colmap[col0 + f]
-    int pad;
-    long long kp0;
+    int lcls;
+    long long kp0, jo0;
 };
+// components of a pair class and of its second shell
+constexpr int pair_comps(int cls) { return cls == 0 ? 1 : cls == 1 ? 3 : cls == 2 ? 9 : cls == 3 ? 6 : cls == 4 ? 18 : 36; }
+constexpr int pair_comps2(int cls) { return cls == 2 || cls == 4 ? 3 : cls == 5 ? 6 : 1; }
 
 constexpr int kQuartSlots = 256;
 

@@ -200,7 +200,8 @@ static size_t fock_lds(int cb, int ck, const FockConfig& f, int mode, int ncols,
     const int nr = (lsum[cb] + lsum[ck]) / 2 + 1;
     const size_t tab = fp32 ? (size_t)kRysAsym[nr] * 2 * nr * UNO_RYS_NCOEF_F * sizeof(float)
                             : (size_t)kRysAsym[nr] * 2 * nr * UNO_RYS_NCOEF * sizeof(double);
-    const size_t sp = mode == kDigestUHF ? 2 : 1, reserve = 1536;
+    // beside it: the waves' ket queues and the reductions of the bra's Coulomb block
+    const size_t sp = mode == kDigestUHF ? 2 : 1, reserve = 8 * (128 * sizeof(int) + na[cb] * nb[cb] * sizeof(double)) + 256;
     const size_t all = (size_t)(na[cb] + nb[cb]) * sp * ncols * sizeof(double);
     size_t dyn = f.mlds ? (size_t)nsh * sizeof(double) : 0;
     if (f.variant == 1 || f.variant == 2) dyn += all;
@@ -279,56 +280,50 @@ hipError_t fock_clear(const ClearList& c, hipStream_t st) {
 __device__ __forceinline__ MolDesc mol_of(const MolDesc* mols, const int* pmol, int p, int n, int nsh) {
     return mols ? mols[pmol[p]] : MolDesc{0, 0, n, nsh};
 }
-// block shape of a pair from its size: 1 ss, 3 ps, 9 pp, 6 ds, 18 dp, 36 dd
-__device__ __forceinline__ int pair_nd(int nc) { return nc == 9 || nc == 18 ? 3 : nc == 36 ? 6 : 1; }
-
 // D0 in pair-major blocks (a wave of kets then reads its density blocks at consecutive
 // addresses) and each pair's own shell-block maximum, for the kernels' screen
-__global__ __launch_bounds__(256) void k_pair_density(int np, const PairHdr* __restrict__ pairs, long long njp,
+__global__ __launch_bounds__(256) void k_pair_density(int np, const int4* __restrict__ kidx, const int4* __restrict__ kjo,
                                                       const double* __restrict__ D0, const double* __restrict__ dsh,
                                                       int n, int nsh, const MolDesc* mols, const int* pmol,
                                                       double* __restrict__ dp, double* __restrict__ dpair) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
-    const PairHdr h = pairs[p];
+    const int4 h = kidx[p], o = kjo[p];
     const MolDesc m = mol_of(mols, pmol, p, n, nsh);
-    const int nc = (int)((p + 1 < np ? (long long)pairs[p + 1].jo : njp) - h.jo), nd = pair_nd(nc);
-    const double* D = D0 + m.moff + (long)h.f1 * m.n + h.f2;
-    for (int kl = 0; kl < nc; ++kl) dp[h.jo + kl] = D[(long)(kl / nd) * m.n + kl % nd];
-    dpair[p] = dsh[m.dshoff + (long)h.sh1 * m.nsh + h.sh2];
+    const double* D = D0 + m.moff + (long)h.x * m.n + h.y;
+    for (int kl = 0; kl < o.z; ++kl) dp[o.x + (long)kl * o.y] = D[(long)(kl / o.w) * m.n + kl % o.w];
+    dpair[p] = dsh[m.dshoff + (long)h.z * m.nsh + h.w];
 }
 
-hipError_t pair_density(int npairs, const PairHdr* pairs, long long njp, const double* D0, const double* dsh, int n,
+hipError_t pair_density(int npairs, const int4* kidx, const int4* kjo, const double* D0, const double* dsh, int n,
                         int nsh, const MolDesc* mols, const int* pmol, double* dp, double* dpair, hipStream_t st) {
     if (npairs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pair_density, dim3((npairs + 255) / 256), dim3(256), 0, st, npairs, pairs, njp, D0, dsh, n, nsh,
-                       mols, pmol, dp, dpair);
+    hipLaunchKernelGGL(k_pair_density, dim3((npairs + 255) / 256), dim3(256), 0, st, npairs, kidx, kjo, D0, dsh, n, nsh, mols,
+                       pmol, dp, dpair);
     return hipGetLastError();
 }
 
 // pair-major Coulomb accumulator into W (pair blocks are disjoint: plain adds)
-__global__ __launch_bounds__(256) void k_jp_scatter(int np, const PairHdr* __restrict__ pairs, long long njp,
+__global__ __launch_bounds__(256) void k_jp_scatter(int np, const int4* __restrict__ kidx, const int4* __restrict__ kjo,
                                                     const double* __restrict__ jp, double* W0, double* W1, int n,
                                                     const MolDesc* mols, const int* pmol) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
-    const PairHdr h = pairs[p];
+    const int4 h = kidx[p], o = kjo[p];
     const MolDesc m = mol_of(mols, pmol, p, n, 0);
-    const int nc = (int)((p + 1 < np ? (long long)pairs[p + 1].jo : njp) - h.jo), nd = pair_nd(nc);
-    for (int kl = 0; kl < nc; ++kl) {
-        const double v = jp[h.jo + kl];
+    for (int kl = 0; kl < o.z; ++kl) {
+        const double v = jp[o.x + (long)kl * o.y];
         if (v == 0.0) continue;
-        const long o = m.moff + (long)(h.f1 + kl / nd) * m.n + h.f2 + kl % nd;
-        W0[o] += v;
-        if (W1) W1[o] += v;
+        const long w = m.moff + (long)(h.x + kl / o.w) * m.n + h.y + kl % o.w;
+        W0[w] += v;
+        if (W1) W1[w] += v;
     }
 }
 
-hipError_t jp_scatter(int npairs, const PairHdr* pairs, long long njp, const double* jp, double* W0, double* W1, int n,
+hipError_t jp_scatter(int npairs, const int4* kidx, const int4* kjo, const double* jp, double* W0, double* W1, int n,
                       const MolDesc* mols, const int* pmol, hipStream_t st) {
     if (npairs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_jp_scatter, dim3((npairs + 255) / 256), dim3(256), 0, st, npairs, pairs, njp, jp, W0, W1, n, mols,
-                       pmol);
+    hipLaunchKernelGGL(k_jp_scatter, dim3((npairs + 255) / 256), dim3(256), 0, st, npairs, kidx, kjo, jp, W0, W1, n, mols, pmol);
     return hipGetLastError();
 }
 
@@ -338,7 +333,7 @@ __global__ __launch_bounds__(256) void k_pair_store(int np, int nrun, const Pair
                                                     const PairHdr* __restrict__ pairs, const PrimPair* __restrict__ prims,
                                                     const int* __restrict__ colmap, BraPrim* __restrict__ bprim,
                                                     double* __restrict__ kprim, long long kps, double* __restrict__ kgeo,
-                                                    int4* __restrict__ kidx, int* __restrict__ knp,
+                                                    int4* __restrict__ kidx, int4* __restrict__ kjo, int* __restrict__ knp,
                                                     int2* __restrict__ kcol) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= np) return;
@@ -354,6 +349,7 @@ __global__ __launch_bounds__(256) void k_pair_store(int np, int nrun, const Pair
         kgeo[(long)(3 + x) * np + p] = h.AB[x];
     }
     kidx[p] = make_int4(h.f1, h.f2, h.sh1, h.sh2);
+    kjo[p] = make_int4((int)(r.jo0 + (p - r.off)), r.count, pair_comps(r.lcls), pair_comps2(r.lcls));
     knp[p] = 2 * h.nprim + (h.same ? 1 : 0);
     kcol[p] = make_int2(colmap[r.col0 + h.f1], colmap[r.col0 + h.f2]);
     for (int j = 0; j < h.nprim; ++j) {
@@ -378,18 +374,18 @@ __global__ __launch_bounds__(256) void k_pair_store(int np, int nrun, const Pair
 }
 
 hipError_t pair_store(int np, int nrun, const PairRun* runs, const PairHdr* pairs, const PrimPair* prims,
-                      const int* colmap, BraPrim* bprim, double* kprim, long long kps, double* kgeo, int4* kidx, int* knp,
-                      int2* kcol, hipStream_t st) {
+                      const int* colmap, BraPrim* bprim, double* kprim, long long kps, double* kgeo, int4* kidx, int4* kjo,
+                      int* knp, int2* kcol, hipStream_t st) {
     if (np <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_pair_store, dim3((np + 255) / 256), dim3(256), 0, st, np, nrun, runs, pairs, prims, colmap, bprim,
-                       kprim, kps, kgeo, kidx, knp, kcol);
+                       kprim, kps, kgeo, kidx, kjo, knp, kcol);
     return hipGetLastError();
 }
 
 // the pair and primitive arrays reordered on the device: new pair k is old pair order[k],
-// its primitive records moved to prim0[k] and its Coulomb block offset set to jo[k]
+// its primitive records moved to prim0[k]
 __global__ __launch_bounds__(256) void k_permute_pairs(int np, const int* __restrict__ order,
-                                                       const int* __restrict__ prim0, const int* __restrict__ jo,
+                                                       const int* __restrict__ prim0,
                                                        const PairHdr* __restrict__ oldp,
                                                        const PrimPair* __restrict__ oldq, PairHdr* __restrict__ newp,
                                                        PrimPair* __restrict__ newq) {
@@ -398,15 +394,14 @@ __global__ __launch_bounds__(256) void k_permute_pairs(int np, const int* __rest
     PairHdr h = oldp[order[k]];
     const int p0 = h.prim0;
     h.prim0 = prim0[k];
-    h.jo = jo[k];
     newp[k] = h;
     for (int q = 0; q < h.nprim; ++q) newq[h.prim0 + q] = oldq[p0 + q];
 }
 
-hipError_t permute_pairs(int np, const int* order, const int* prim0, const int* jo, const PairHdr* oldp,
-                         const PrimPair* oldq, PairHdr* newp, PrimPair* newq, hipStream_t st) {
+hipError_t permute_pairs(int np, const int* order, const int* prim0, const PairHdr* oldp, const PrimPair* oldq,
+                         PairHdr* newp, PrimPair* newq, hipStream_t st) {
     if (np <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_permute_pairs, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, np, order, prim0, jo,
+    hipLaunchKernelGGL(k_permute_pairs, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, np, order, prim0,
                        oldp, oldq, newp, newq);
     return hipGetLastError();
 }

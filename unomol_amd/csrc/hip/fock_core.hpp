@@ -24,6 +24,9 @@ namespace uno {
 // classes up to kLaneMaxComp components run one ket per lane (the component block in registers);
 // larger ones one quartet per wave
 constexpr int kLaneMaxComp = 162;
+#ifndef UNO_NT_COMP
+#define UNO_NT_COMP 0
+#endif
 // Rys tables of up to this many roots are staged in LDS by the kernels without LDS rows
 constexpr int kLdsTabMaxRoots = 3;
 // every quartet class: pair classes (0 ss, 1 ps, 2 pp, 3 ds, 4 dp, 5 dd) and shells
@@ -249,8 +252,12 @@ __host__ __device__ constexpr int dens_row_count() {
     return (ncart_c(LA) + ncart_c(LB)) * (MODE == kDigestUHF ? 2 : 1);
 }
 
-constexpr int kRowThreads = 256;
-constexpr int kRowWaves = kRowThreads / 64;
+// threads of a block: the waves of a block share its LDS rows, so the classes whose registers
+// allow four waves per SIMD run eight waves a block
+template <int LA, int LB, int LC, int LD>
+constexpr int row_threads() {
+    return ClassInfo<LA, LB, LC, LD>::NCOMP <= UNO_NT_COMP ? 512 : 256;
+}
 
 // ---------------------------------------------------------------------------
 // Classes of up to kLaneMaxComp components: one block per (bra, segment of kets), one lane
@@ -264,7 +271,8 @@ constexpr int kRowWaves = kRowThreads / 64;
 // TL the Rys table.
 // ---------------------------------------------------------------------------
 template <int LA, int LB, int LC, int LD, int MODE, typename T, int ROWS, bool TL>
-__global__ __launch_bounds__(kRowThreads) void k_fock(const FockArgs a) {
+__global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void k_fock(const FockArgs a) {
+    constexpr int kRowThreads = row_threads<LA, LB, LC, LD>(), kRowWaves = kRowThreads / 64;
     using CI = ClassInfo<LA, LB, LC, LD>;
     constexpr int NA = CI::NA, NB = CI::NB, NC = CI::NC, ND = CI::ND, NCOMP = CI::NCOMP, NR = CI::NR;
     constexpr bool FB = ROWS == kRowsAll, RW = ROWS != kRowsNone, F32 = sizeof(T) == 4;
@@ -275,6 +283,7 @@ __global__ __launch_bounds__(kRowThreads) void k_fock(const FockArgs a) {
     __shared__ T tab_lds[TL ? rys_table_size<NR, T>() : 1];
     __shared__ double jred[kRowWaves][NA * NB];
     __shared__ unsigned cred[kRowWaves][3];
+    __shared__ int queue[kRowWaves][128];
     FockTask t;
     if (!fock_task<F32>(a, t)) return;   // whole block
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -322,22 +331,46 @@ __global__ __launch_bounds__(kRowThreads) void k_fock(const FockArgs a) {
             dab[i * NB + j] = (T)mv.D0[(long)(fa + i) * n + fb + j];
         }
     unsigned nprim = 0, nshell = 0, nin = 0;
-    const int lg = t.s.lg, sub = threadIdx.x & ((1 << lg) - 1);
-    for (int base = t.k0; base < t.k1; base += kRowThreads >> lg) {
-        const int kk = base + (threadIdx.x >> lg);
-        if (kk >= t.k1) continue;
-        const int pcd = t.s.ket_off + kk;
-        const double qk = a.pairQ[pcd];
-        if (!fock_ket_in<F32>(t, qk)) continue;
-        if (sub == 0) ++nin;
-        const int4 ki = a.kidx[pcd];   // first functions, shells
-        {
-            // the density screen of eri_core.hpp's screened()
-            double d = fmax(dab4, 4.0 * a.dpair[pcd]);
-            if (ml) d = fmax(d, fmax(mrow[ki.z], mrow[ki.w]));
-            else d = fmax(d, fmax(fmax(m1[ki.z], m1[ki.w]), fmax(m2[ki.z], m2[ki.w])));
-            if (t.qi * qk * d < a.tau) continue;
+    // Each wave screens its kets 64 at a time (fewer where the segment is short) into a queue of
+    // survivors and evaluates them a wavefull at a time, so that the lanes it pays for are
+    // busy: of the kets within the bounds two thirds survive the screen of a full build, and a
+    // small part that of an incremental one.
+    const int lg = t.s.lg, sub = lane & ((1 << lg) - 1), per = 64 >> lg;
+    const int step = min(64, max(per, (t.k1 - t.k0 + kRowWaves - 1) / kRowWaves));
+    int next = t.k0 + wave * step, nq = 0;
+    int* q = queue[wave];
+    for (;;) {
+        while (nq < per && next < t.k1) {
+            const int kk = next + lane;
+            bool in = lane < step && kk < t.k1, live = false;
+            if (in) {
+                const int pcd = t.s.ket_off + kk;
+                const double qk = a.pairQ[pcd];
+                in = fock_ket_in<F32>(t, qk);
+                if (in) {
+                    // the density screen of eri_core.hpp's screened()
+                    const int4 ki = a.kidx[pcd];
+                    double d = fmax(dab4, 4.0 * a.dpair[pcd]);
+                    if (ml) d = fmax(d, fmax(mrow[ki.z], mrow[ki.w]));
+                    else d = fmax(d, fmax(fmax(m1[ki.z], m1[ki.w]), fmax(m2[ki.z], m2[ki.w])));
+                    live = !(t.qi * qk * d < a.tau);
+                }
+            }
+            const unsigned long long m = __ballot(live);
+            nin += __popcll(__ballot(in));
+            if (live) q[nq + __popcll(m & ((1ull << lane) - 1))] = kk;
+            nq += __popcll(m);
+            next += kRowWaves * step;
         }
+        if (nq == 0) break;
+        // the queue is the wave's own: its writes above precede its reads below
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int take = min(nq, per);
+        nq -= take;
+        if ((lane >> lg) >= take) continue;
+        const int kk = q[nq + (lane >> lg)];
+        const int pcd = t.s.ket_off + kk;
+        const int4 ki = a.kidx[pcd];   // first functions, shells
         const int kn = a.knp[pcd];     // primitives, twice, plus 1 for a same-shell pair
         T e[NCOMP];
         nprim += fock_eri<LA, LB, LC, LD, T>(a, t, P1.prim0, P1.nprim, ab, kk, kn >> 1, sub, lg, e, tab);
@@ -346,12 +379,14 @@ __global__ __launch_bounds__(kRowThreads) void k_fock(const FockArgs a) {
         const T f = (P1.same ? (T)0.5 : (T)1) * ((kn & 1) ? (T)0.5 : (T)1) * (t.bra == pcd ? (T)0.5 : (T)1);
         normalise_block<LA, LB, LC, LD, T>(e, f);
         const int fc = ki.x, fd = ki.y;
-        const long jo = t.s.jo0 + (long)kk * (NC * ND);
+        // the ket's entries of the pair-major arrays: component by component over the run, so that
+        // a wave's kets meet at consecutive addresses
+        const long jo = t.s.jo0 + kk, js = t.s.kstride;
         // Coulomb, bra outputs: kept per thread
         {
             T dcd[NC * ND];
 #pragma unroll
-            for (int kl = 0; kl < NC * ND; ++kl) dcd[kl] = (T)a.dp[jo + kl];
+            for (int kl = 0; kl < NC * ND; ++kl) dcd[kl] = (T)a.dp[jo + kl * js];
 #pragma unroll
             for (int ij = 0; ij < NA * NB; ++ij) {
                 T s = 0;
@@ -369,7 +404,7 @@ __global__ __launch_bounds__(kRowThreads) void k_fock(const FockArgs a) {
             for (int ij = 0; ij < NA * NB; ++ij) s = fma(e[ij * NC * ND + kl], dab[ij], s);
             const double v = (double)(jf * s);
             if (RW || a.jp) {
-                atomic_add_f64(a.jp + jo + kl, v);
+                atomic_add_f64(a.jp + jo + kl * js, v);
             } else {
                 const long o = (long)(fc + kl / ND) * n + fd + kl % ND;
                 fock_add(a.fix_lo, mv.W0 + o, v);
@@ -476,10 +511,9 @@ __global__ __launch_bounds__(kRowThreads) void k_fock(const FockArgs a) {
         const double v = wave_sum(jacc[ij]);
         if (lane == 0) jred[wave][ij] = v;
     }
+    if (a.counter) {
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        nin += __shfl_xor(nin, m, 64);
-        if (a.counter) {
+        for (int m = 32; m >= 1; m >>= 1) {
             nprim += __shfl_xor(nprim, m, 64);
             nshell += __shfl_xor(nshell, m, 64);
         }

@@ -14,7 +14,7 @@ static hipError_t fock_launch_v(const FockArgs& a, int nblocks, size_t dyn, hipS
         if (e != hipSuccess) return e;
         attr = dyn;
     }
-    hipLaunchKernelGGL((k_fock<LA, LB, LC, LD, MODE, T, ROWS, TL>), dim3((unsigned)nblocks), dim3(kRowThreads), dyn, st,
+    hipLaunchKernelGGL((k_fock<LA, LB, LC, LD, MODE, T, ROWS, TL>), dim3((unsigned)nblocks), dim3((row_threads<LA, LB, LC, LD>())), dyn, st,
                        a);
     return hipGetLastError();
 }

@@ -29,8 +29,8 @@ hipError_t fock_launch(int mode, bool fp32, int bra_class, int ket_class, FockAr
                        int ncols, hipStream_t st);
 // the Fock kernels' copies of the pair data (device arrays), runs sorted by off
 hipError_t pair_store(int np, int nrun, const PairRun* runs, const PairHdr* pairs, const PrimPair* prims,
-                      const int* colmap, BraPrim* bprim, double* kprim, long long kps, double* kgeo, int4* kidx, int* knp,
-                      int2* kcol, hipStream_t st);
+                      const int* colmap, BraPrim* bprim, double* kprim, long long kps, double* kgeo, int4* kidx, int4* kjo,
+                      int* knp, int2* kcol, hipStream_t st);
 // up to six buffers of 64-bit words zeroed in one launch
 struct ClearList {
     unsigned long long* p[6];
@@ -46,15 +46,15 @@ struct ClearList {
 hipError_t fock_clear(const ClearList& c, hipStream_t st);
 // dp = D0 in pair-major blocks, dpair = every pair's own entry of dsh (mols / pmol: batched
 // stores and every pair's molecule, or null)
-hipError_t pair_density(int npairs, const PairHdr* pairs, long long njp, const double* D0, const double* dsh, int n,
+hipError_t pair_density(int npairs, const int4* kidx, const int4* kjo, const double* D0, const double* dsh, int n,
                         int nsh, const MolDesc* mols, const int* pmol, double* dp, double* dpair, hipStream_t st);
-// W[f1 + k][f2 + l] += jp[jo + k nd + l] (and W1) for every pair of the array
-hipError_t jp_scatter(int npairs, const PairHdr* pairs, long long njp, const double* jp, double* W0, double* W1, int n,
+// the pair-major jp added into W (and W1)
+hipError_t jp_scatter(int npairs, const int4* kidx, const int4* kjo, const double* jp, double* W0, double* W1, int n,
                       const MolDesc* mols, const int* pmol, hipStream_t st);
-// new pair k = old pair order[k], its primitives at prim0[k], Coulomb block at jo[k]
-// (device arrays; new ones must not overlap the old)
-hipError_t permute_pairs(int np, const int* order, const int* prim0, const int* jo, const PairHdr* oldp,
-                         const PrimPair* oldq, PairHdr* newp, PrimPair* newq, hipStream_t st);
+// new pair k = old pair order[k], its primitives at prim0[k] (device arrays; new ones must not
+// overlap the old)
+hipError_t permute_pairs(int np, const int* order, const int* prim0, const PairHdr* oldp, const PrimPair* oldq,
+                         PairHdr* newp, PrimPair* newq, hipStream_t st);
 // deterministic builds: W accumulated in fixed point (entry i: int64 words i and i + lo_off)
 // back to FP64 in place, first nn entries
 hipError_t fixed_to_f64(long long nn, double* W, long long lo_off, hipStream_t st);

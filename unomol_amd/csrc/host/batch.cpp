@@ -185,7 +185,7 @@ static int enqueue_fock(uno_batch* b) {
     UNO_HIP(fock_clear(cl, st));
     UNO_HIP(batch_shell_max(nm, b->maxsh, b->mdesc.p, b->mshoff.p, b->active_d.p, b->sh_off.p, b->sh_n.p, b->D0.p, b->D1.p, b->D2.p,
                             b->Dsh.p, fs.dmax.p, st));
-    UNO_HIP(pair_density(np, b->pairs.p, fs.njp, b->D0.p, b->Dsh.p, 0, 0, b->mdesc.p, b->pmol.p, fs.dp.p, fs.dpair.p, st));
+    UNO_HIP(pair_density(np, fs.kidx.p, fs.kjo.p, b->D0.p, b->Dsh.p, 0, 0, b->mdesc.p, b->pmol.p, fs.dp.p, fs.dpair.p, st));
     const int nls = std::max(1, std::min(kMaxLaunchStreams, b->launch_streams));
     if (int rc = b->ls.begin(nls, st)) return rc;
     for (size_t k = 0; k < fs.launches.size(); ++k) {
@@ -215,7 +215,7 @@ static int enqueue_fock(uno_batch* b) {
         UNO_HIP(fock_launch(mode, false, l.cx, l.cy, a, l.nblocks, f, l.ncols, b->ls.of((int)(k % (size_t)nls), st)));
     }
     if (int rc = b->ls.end(nls, st)) return rc;
-    UNO_HIP(jp_scatter(np, b->pairs.p, fs.njp, fs.jp.p, b->W0.p, b->W1.p, 0, b->mdesc.p, b->pmol.p, st));
+    UNO_HIP(jp_scatter(np, fs.kidx.p, fs.kjo.p, fs.jp.p, b->W0.p, b->W1.p, 0, b->mdesc.p, b->pmol.p, st));
     return UNO_OK;
 }
 
@@ -265,7 +265,6 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
     std::vector<int> shoff, shn;
     std::vector<MolDesc> md;
     std::vector<int> pmol, mshoff;
-    long long njp = 0;
     for (int m = 0; m < nmol; ++m) {
         BatchMol& x = b->mol[m];
         if (int rc = uno_ctx_create(&bases[m], 0, &x.ctx)) { delete b; return rc; }
@@ -295,11 +294,9 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
         const int p0 = (int)prims.size();
         for (PairHdr h : c->pairs) {
             h.prim0 += p0;
-            h.jo += (int)njp;
             pairs.push_back(h);
             pmol.push_back(m);
         }
-        njp += c->fs.njp;
         mshoff.push_back(x.shoff);
         b->maxn = std::max(b->maxn, x.n);
         b->maxsh = std::max(b->maxsh, x.nsh);
@@ -333,7 +330,7 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
             const BatchMol& x = b->mol[m];
             fm[m] = FockMol{x.n, m, x.uhf ? 1 : 0, &x.ctx->cls, x.pair_off, pairs.data() + x.pair_off};
         }
-        if (int rc = b->fs.build(fm, b->pairs.p, b->prims.p, (int)pairs.size(), (long long)prims.size(), njp, st)) {
+        if (int rc = b->fs.build(fm, b->pairs.p, b->prims.p, (int)pairs.size(), (long long)prims.size(), st)) {
             delete b;
             return rc;
         }

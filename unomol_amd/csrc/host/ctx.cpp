@@ -192,20 +192,11 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
         if (runkey[x] != runkey[y]) return runkey[x] < runkey[y];
         return c->pairQ[x] > c->pairQ[y];
     });
-    // new primitive offsets and pair-major Coulomb offsets (each pair's function block), in
-    // run order
-    static const int kPairComp[kNumPairClasses] = {1, 3, 9, 6, 18, 36};
-    std::vector<int> nprim0(np), njo(np);
-    long long njp = 0;
-    {
-        long long tp = 0, jo = 0;
-        for (int k = 0; k < np; ++k) {
-            nprim0[k] = (int)tp;
-            tp += c->pairs[order[k]].nprim;
-            njo[k] = (int)jo;
-            jo += kPairComp[runkey[order[k]] / kNumBuckets];
-        }
-        njp = jo;
+    // new primitive offsets, in run order
+    std::vector<int> nprim0(np);
+    for (int k = 0, tp = 0; k < np; ++k) {
+        nprim0[k] = tp;
+        tp += c->pairs[order[k]].nprim;
     }
     std::vector<PairHdr> pairs2(np);
     std::vector<PrimPair> prims2(c->prims.size());
@@ -216,7 +207,6 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
         PairHdr h = c->pairs[order[k]];
         const int p0 = h.prim0;
         h.prim0 = nprim0[k];
-        h.jo = njo[k];
         std::copy(c->prims.begin() + p0, c->prims.begin() + p0 + h.nprim, prims2.begin() + h.prim0);
         pairs2[k] = h;
         q2[k] = c->pairQ[order[k]];
@@ -228,17 +218,16 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     c->prims.swap(prims2);
     c->pairQ.swap(q2);
     // the device copies: the same permutation applied to the arrays uploaded above (the
-    // three index arrays go up instead of the records themselves)
+    // two index arrays go up instead of the records themselves)
     {
-        DBuf<int> dorder, dp0, djo;
+        DBuf<int> dorder, dp0;
         DBuf<PairHdr> np_d;
         DBuf<PrimPair> nq_d;
         UNO_HIP(dorder.upload(order.data(), np, st));
         UNO_HIP(dp0.upload(nprim0.data(), np, st));
-        UNO_HIP(djo.upload(njo.data(), np, st));
         UNO_HIP(np_d.alloc(np));
         UNO_HIP(nq_d.alloc(c->prims.size()));
-        UNO_HIP(permute_pairs(np, dorder.p, dp0.p, djo.p, c->d_pairs.p, c->d_prims.p, np_d.p, nq_d.p, st));
+        UNO_HIP(permute_pairs(np, dorder.p, dp0.p, c->d_pairs.p, c->d_prims.p, np_d.p, nq_d.p, st));
         UNO_HIP(hipStreamSynchronize(st));
         c->d_pairs = std::move(np_d);
         c->d_prims = std::move(nq_d);
@@ -273,7 +262,7 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
         m.n = c->n;
         m.runs = &c->cls;
         m.pairs = c->pairs.data();
-        if (int rc = c->fs.build({m}, c->d_pairs.p, c->d_prims.p, np, (long long)c->prims.size(), njp, st)) return rc;
+        if (int rc = c->fs.build({m}, c->d_pairs.p, c->d_prims.p, np, (long long)c->prims.size(), st)) return rc;
     }
     recall_tuning(c);
     std::vector<int> shoff(nsh), shn(nsh);

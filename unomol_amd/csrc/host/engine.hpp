@@ -107,12 +107,12 @@ struct FockStore {
     DBuf<char> tables;
     DBuf<BraPrim> bprim;
     DBuf<double> kprim, kgeo, dp, jp, dpair, dmax;
-    DBuf<int4> kidx;
+    DBuf<int4> kidx, kjo;
     DBuf<int> knp, colinv;
     DBuf<int2> kcol;
     DBuf<unsigned long long> nquart;       // FP64 launches' counters, then FP32's
     int build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, const PrimPair* d_prims, int np, long long nprims,
-              long long njp, hipStream_t st);
+              hipStream_t st);
     FockArgs args(const FockLaunch& l, const PairHdr* d_pairs, const PrimPair* d_prims, const double* pairQ) const;
 };
 // streams that launches are spread over: the caller's and up to kMaxLaunchStreams - 1 workers at

@@ -48,11 +48,27 @@ LaunchStreams::~LaunchStreams() {
 // kets get several lanes each
 constexpr double kFillLanes = 1 << 20;
 
+// log2 of the lanes that share a ket of kprim primitives against a bra of bprim, in a launch of
+// `quartets` shell quartets: doubled while the launch would leave the chip idle otherwise, or
+// while the split costs next to nothing (the rounds over the ket's primitives stay nearly full, and
+// each lane keeps primitive quartets enough that adding up the group's blocks does not show)
+static int lanes_per_ket(int bprim, int kprim, double quartets) {
+    int lg = 0;
+    while ((1 << lg) < kprim && lg < 6) {
+        const int g = 2 << lg, rounds = (kprim + g - 1) / g;
+        const bool fill = quartets * g <= kFillLanes;
+        const bool cheap = kprim >= 0.85 * rounds * g && bprim * rounds >= 16;
+        if (!fill && !cheap) break;
+        ++lg;
+    }
+    return lg;
+}
+
 int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, const PrimPair* d_prims, int np,
-                     long long nprims, long long njp_, hipStream_t st) {
+                     long long nprims, hipStream_t st) {
     static const int kPairL[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
     npair = np;
-    njp = njp_;
+    njp = 0;
     // runs of the whole array, with their ket layout, and the LDS row columns: per molecule and
     // ket class the functions its pairs touch (whole shells), in function order
     struct Run {
@@ -73,7 +89,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
         cinv.resize(colmap.size(), 0);
         std::vector<char> used((size_t)kNumPairClasses * x.n, 0);
         for (const PairClassList& L : *x.runs) {
-            Run r{x.pair_off + L.off, L.count, 1, L.lcls, kps, 0};
+            Run r{x.pair_off + L.off, L.count, 1, L.lcls, kps, njp};
             const int n1 = ncart(kPairL[L.lcls][0]), n2 = ncart(kPairL[L.lcls][1]);
             char* u = used.data() + (size_t)L.lcls * x.n;
             for (int k = L.off; k < L.off + L.count; ++k) {
@@ -82,10 +98,10 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                 for (int f = 0; f < n1; ++f) u[h.f1 + f] = 1;
                 for (int f = 0; f < n2; ++f) u[h.f2 + f] = 1;
             }
-            r.jo0 = x.pairs[L.off].jo;
+            njp += (long long)pair_comps(L.lcls) * L.count;
             kps += (long long)r.maxprim * L.count;
             runs[m].push_back(r);
-            pr.push_back(PairRun{r.off, r.count, base + L.lcls * x.n, 0, r.kp0});
+            pr.push_back(PairRun{r.off, r.count, base + L.lcls * x.n, L.lcls, r.kp0, r.jo0});
         }
         for (int c = 0; c < kNumPairClasses; ++c) {
             int k = 0;
@@ -97,6 +113,10 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                 }
             ncols[m][c] = k;
         }
+    }
+    if (njp > (long long)INT32_MAX) {
+        set_error("too many shell pairs for 32-bit offsets");
+        return UNO_EINVAL;
     }
     // the launches: per launch group and class pair the spaces of every molecule, the ones with
     // the longest primitive loops first
@@ -113,8 +133,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
             for (int cy = cx; cy >= 0; --cy) {
                 struct Cand {
                     FockSpace s;
-                    long work;
-                    int maxprim;
+                    int bprim, kprim;
                 };
                 std::vector<Cand> cs;
                 double total = 0.0;
@@ -138,14 +157,14 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                             s.kstride = k.count;
                             s.kp0 = k.kp0;
                             s.jo0 = k.jo0;
-                            cs.push_back(Cand{s, (long)b.maxprim * k.maxprim, k.maxprim});
+                            cs.push_back(Cand{s, b.maxprim, k.maxprim});
                             total += (s.same ? 0.5 : 1.0) * s.nbra * (double)s.nket;
                             L.ncols = std::max(L.ncols, s.ncols);
                             L.nket = std::max(L.nket, s.nket);
                         }
                 }
                 if (cs.empty()) continue;
-                std::stable_sort(cs.begin(), cs.end(), [](const Cand& u, const Cand& v) { return u.work > v.work; });
+                std::stable_sort(cs.begin(), cs.end(), [](const Cand& u, const Cand& v) { return (long)u.bprim * u.kprim > (long)v.bprim * v.kprim; });
                 std::vector<FockSpace> sp;
                 long long nb = 0;
                 // segments as long as leaves about 8192 passes' worth of blocks to balance the
@@ -161,7 +180,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                         if (fock_is_wave(cx, cy)) {
                             s.seg = longer * (int)std::max(1.0, std::min<double>(kWaveSeg, total / 4096.0));
                         } else {
-                            while ((1 << s.lg) < c.maxprim && s.lg < 6 && total * (2 << s.lg) <= kFillLanes) ++s.lg;
+                            s.lg = lanes_per_ket(c.bprim, c.kprim, total);
                             const int pass = kLaneBlock >> s.lg;
                             s.seg = longer * pass * (int)std::max(1.0, std::min(32.0, total / (pass * 8192.0)));
                         }
@@ -197,6 +216,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
     UNO_HIP(kprim.alloc((size_t)std::max(kKetFields * kps, 1LL)));
     UNO_HIP(kgeo.alloc(6 * (size_t)std::max(np, 1)));
     UNO_HIP(kidx.alloc(np));
+    UNO_HIP(kjo.alloc(np));
     UNO_HIP(knp.alloc(np));
     UNO_HIP(kcol.alloc(np));
     UNO_HIP(dpair.alloc(np));
@@ -204,8 +224,8 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
     UNO_HIP(jp.alloc((size_t)std::max(njp, 1LL)));
     UNO_HIP(dmax.alloc(mols.size()));
     UNO_HIP(nquart.alloc(2 * kQuartSlots));
-    UNO_HIP(pair_store(np, (int)pr.size(), dr.p, d_pairs, d_prims, dcm.p, bprim.p, kprim.p, kps, kgeo.p, kidx.p, knp.p,
-                       kcol.p, st));
+    UNO_HIP(pair_store(np, (int)pr.size(), dr.p, d_pairs, d_prims, dcm.p, bprim.p, kprim.p, kps, kgeo.p, kidx.p, kjo.p,
+                       knp.p, kcol.p, st));
     UNO_HIP(hipStreamSynchronize(st));   // the host tables and the scratch buffers go
     return UNO_OK;
 }
@@ -275,7 +295,7 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
     // pairs' order
     UNO_HIP(k_shell_max(c->n, c->nsh, c->d_shoff.p, c->d_shn.p, c->D0.p, uhf ? c->D1.p : nullptr,
                         uhf ? c->D2.p : nullptr, c->Dsh.p, fs.dmax.p, st));
-    UNO_HIP(pair_density(fs.npair, c->d_pairs.p, fs.njp, c->D0.p, c->Dsh.p, c->n, c->nsh, nullptr, nullptr, fs.dp.p,
+    UNO_HIP(pair_density(fs.npair, fs.kidx.p, fs.kjo.p, c->D0.p, c->Dsh.p, c->n, c->nsh, nullptr, nullptr, fs.dp.p,
                          fs.dpair.p, st));
     const int mode = uhf ? kDigestUHF : kDigestRHF;
     // (the tuner times each launch on the context's stream)
@@ -379,7 +399,7 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
         if (uhf) UNO_HIP(fixed_to_f64(nn, c->W1.p, nn, st));
     } else {
         // the kets' Coulomb outputs, accumulated per pair, into W
-        UNO_HIP(jp_scatter(fs.npair, c->d_pairs.p, fs.njp, fs.jp.p, c->W0.p, uhf ? c->W1.p : nullptr, c->n, nullptr,
+        UNO_HIP(jp_scatter(fs.npair, fs.kidx.p, fs.kjo.p, fs.jp.p, c->W0.p, uhf ? c->W1.p : nullptr, c->n, nullptr,
                            nullptr, st));
     }
     c->quartets_known = false;
