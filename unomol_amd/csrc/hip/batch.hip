@@ -185,8 +185,9 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMa
 
 // The same rotations in the same order with the matrix in LDS, for n <= kJacobiLdsN (157 KB of the
 // 160 at 140 functions): a round is two phases, the rotations and one pass that applies them
-// to both sides of every 2 x 2 block of the pairs (k, l), k <= l, writing the mirrored block too,
-// and to the eigenvectors.  The eigenvectors are kept transposed (the two vectors of a rotation are
+// to both sides of every 2 x 2 block of the pairs (k, l), rows first, and to the eigenvectors: the
+// other kernel's arithmetic, so that the vectors it picks inside an exactly degenerate level (a
+// linear molecule's pi pairs) are the same.  The eigenvectors are kept transposed (the two vectors of a rotation are
 // rows), in LDS as well while both fit, else in V.  With the matrix in global memory every round
 // made three passes over it at L2 latency: 5.7 ms a launch for 32 molecules of up to 95 functions (mean
 // of an SCF, most of them warm), 1.0 ms here.
@@ -222,25 +223,6 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const Bat
     for (int w = 0; w < kJacobiThreads / 64; ++w) fro2 += red[w];
     const double abs_tol = 1e-15 * sqrt(fro2);
     const int m = n + (n & 1), mk = m / 2;
-    // this thread's pair blocks (k, l), the same in every round: rows k and mk - 1 - k of the
-    // triangle together are mk + 1 blocks long
-    constexpr int kItems = (kJacobiLdsN / 2 * (kJacobiLdsN / 2 + 1) / 2 + kJacobiLdsN / 2 + kJacobiThreads - 1) / kJacobiThreads;
-    int ik[kItems], il[kItems];
-#pragma unroll
-    for (int x = 0; x < kItems; ++x) {
-        const int t = tid + x * kJacobiThreads, r = t / (mk + 1), c = t - r * (mk + 1);
-        ik[x] = -1;
-        il[x] = 0;
-        if (2 * r < mk) {
-            if (c < mk - r) {
-                ik[x] = r;
-                il[x] = r + c;
-            } else if (mk - 1 - r != r) {
-                ik[x] = mk - 1 - r;
-                il[x] = c - 1;
-            }
-        }
-    }
     int sweep = 0;
     while (sweep < max_sweeps && n > 1) {
         ++sweep;
@@ -279,32 +261,22 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const Bat
                 sn[tid] = s;
             }
             __syncthreads();
-#pragma unroll
-            for (int x = 0; x < kItems; ++x) {
-                const int k = ik[x], l = il[x];
-                if (k < 0) continue;
+            for (int x = tid; x < mk * mk; x += kJacobiThreads) {
+                const int k = x / mk, l = x - k * mk;
                 const double ck = cs[k], sk = sn[k], cl = cs[l], sl = sn[l];
                 if (sk == 0.0 && sl == 0.0) continue;
                 // (the dummy index of an odd n only meets rotations with s = 0: its row and
                 // column are left out)
                 const int pk = pp[k], qk = qq[k], pl = pp[l], ql = qq[l];
-                const bool vk = qk < n, vl2 = ql < n;
-                const double a00 = A[pk * ld + pl], a01 = vl2 ? A[pk * ld + ql] : 0.0;
-                const double a10 = vk ? A[qk * ld + pl] : 0.0, a11 = vk && vl2 ? A[qk * ld + ql] : 0.0;
+                const bool vk = qk < n, vq = ql < n;
+                const double a00 = A[pk * ld + pl], a01 = vq ? A[pk * ld + ql] : 0.0;
+                const double a10 = vk ? A[qk * ld + pl] : 0.0, a11 = vk && vq ? A[qk * ld + ql] : 0.0;
                 const double r00 = ck * a00 - sk * a10, r01 = ck * a01 - sk * a11;
                 const double r10 = sk * a00 + ck * a10, r11 = sk * a01 + ck * a11;
-                const double b00 = cl * r00 - sl * r01, b01 = sl * r00 + cl * r01;
-                const double b10 = cl * r10 - sl * r11, b11 = sl * r10 + cl * r11;
-                A[pk * ld + pl] = b00;
-                if (vl2) A[pk * ld + ql] = b01;
-                if (vk) A[qk * ld + pl] = b10;
-                if (vk && vl2) A[qk * ld + ql] = b11;
-                if (k != l) {
-                    A[pl * ld + pk] = b00;
-                    if (vl2) A[ql * ld + pk] = b01;
-                    if (vk) A[pl * ld + qk] = b10;
-                    if (vk && vl2) A[ql * ld + qk] = b11;
-                }
+                A[pk * ld + pl] = cl * r00 - sl * r01;
+                if (vq) A[pk * ld + ql] = sl * r00 + cl * r01;
+                if (vk) A[qk * ld + pl] = cl * r10 - sl * r11;
+                if (vk && vq) A[qk * ld + ql] = sl * r10 + cl * r11;
             }
             for (int e = tid; e < mk * n; e += kJacobiThreads) {
                 const int k = e / n, i = e - k * n;

@@ -77,7 +77,7 @@ constexpr int kKetFields = 7;
 
 // One space of a Fock-build launch: the bra run [bra_off, bra_off + nbra) against the ket run
 // [ket_off, ket_off + nket) of the pair array, both sorted by Schwarz bound (descending).  Its
-// blocks are first + bra * nseg + segment; same: both are the same run (kets up to the bra).
+// candidates are first + bra * nseg + segment; same: both are the same run (kets up to the bra).
 struct FockSpace {
     int first;
     int bra_off, nbra, ket_off, nket;
@@ -104,9 +104,28 @@ constexpr int pair_comps2(int cls) { return cls == 2 || cls == 4 ? 3 : cls == 5 
 
 constexpr int kQuartSlots = 256;
 
+// A launch as the kernel that lists a build's tasks sees it: candidate c of the launch (a bra and
+// a ket segment) is thread (blockIdx - block0) * kTaskThreads + threadIdx
+struct FockTaskSource {
+    long long sp, blk;        // byte offsets of its tables
+    int block0, ncand;
+    int list;                 // its list's offset
+    int f32;                  // the FP32 half of a mixed build
+};
+constexpr int kTaskThreads = 1024;
+struct alignas(128) FockCounter {   // a cache line each
+    int count, head;          // tasks listed, tasks handed out
+    int pad[30];
+};
+
 struct FockArgs {
     const FockSpace* sp;
     const int* blk;           // space of every 64th block
+    // the blocks of a launch take tasks until none is left: the listed ones, or (list null) every
+    // candidate 0 .. ncand - 1
+    const int* list;
+    FockCounter* ctr;
+    int ncand;
     const PairHdr* pairs;
     const PrimPair* prims;
     const BraPrim* bprim;

@@ -182,15 +182,19 @@ int eri_class_ncomp(int cb, int ck) {
 // ---------------------------------------------------------------------------
 // Fock-build launches: the kernels are instantiated per (mode, precision) in fock_*.hip
 // ---------------------------------------------------------------------------
-hipError_t fock_launch_rhf64(int, int, const FockArgs&, int, int, size_t, hipStream_t);
-hipError_t fock_launch_uhf64(int, int, const FockArgs&, int, int, size_t, hipStream_t);
-hipError_t fock_launch_rhf32(int, int, const FockArgs&, int, int, size_t, hipStream_t);
-hipError_t fock_launch_uhf32(int, int, const FockArgs&, int, int, size_t, hipStream_t);
+hipError_t fock_launch_rhf64(int, int, const FockArgs&, int, size_t, hipStream_t);
+hipError_t fock_launch_uhf64(int, int, const FockArgs&, int, size_t, hipStream_t);
+hipError_t fock_launch_rhf32(int, int, const FockArgs&, int, size_t, hipStream_t);
+hipError_t fock_launch_uhf32(int, int, const FockArgs&, int, size_t, hipStream_t);
 
 bool fock_is_wave(int cb, int ck) { return eri_class_ncomp(cb, ck) > kLaneMaxComp; }
 
-// LDS a block may take (rows, then the Rys table if it still fits): two blocks per compute unit
-static constexpr size_t kRowLdsBudget = 80 * 1024;
+// LDS a block may take (rows, then the Rys table if it still fits): two blocks per compute unit,
+// or nearly all of it for the classes whose registers leave one wave per SIMD, so one block per
+// compute unit, anyway
+static size_t row_lds_budget(int cb, int ck) {
+    return (eri_class_ncomp(cb, ck) >= 54 || cb == 5 ? 156 : 80) * 1024;
+}
 
 // the LDS a block of this launch needs: dynamic part, and whether all of it fits the budget
 static size_t fock_lds(int cb, int ck, const FockConfig& f, int mode, int ncols, int nsh, bool fp32, bool& fits) {
@@ -208,7 +212,7 @@ static size_t fock_lds(int cb, int ck, const FockConfig& f, int mode, int ncols,
     if (f.variant == 3) dyn += (size_t)na[cb] * sp * ncols * sizeof(double);
     if (f.variant && f.dlds) dyn += all;
     const bool table = f.variant == 1 || (f.variant == 0 && nr <= kLdsTabMaxRoots);
-    fits = dyn + (table ? tab : 0) + reserve <= kRowLdsBudget;
+    fits = dyn + (table ? tab : 0) + reserve <= row_lds_budget(cb, ck);
     return dyn;
 }
 
@@ -239,21 +243,20 @@ FockConfig fock_default(int cb, int ck, int mode, int ncols, int nsh, bool fp32,
     return f;
 }
 
-hipError_t fock_launch(int mode, bool fp32, int cb, int ck, FockArgs a, int nblocks, const FockConfig& f, int ncols,
-                       hipStream_t st) {
-    if (nblocks <= 0) return hipSuccess;
+hipError_t fock_launch(int mode, bool fp32, int cb, int ck, FockArgs a, const FockConfig& f, int ncols, hipStream_t st) {
+    if (a.ncand <= 0) return hipSuccess;
     // the rows merge in LDS with FP64 atomics: no deterministic form
-    if (!a.sp || !a.blk || !a.nquart || (f.variant && (a.fix_lo || !a.jp || ncols <= 0)) || f.variant < 0 || f.variant > 3)
+    if (!a.sp || !a.blk || !a.ctr || !a.nquart || (f.variant && (a.fix_lo || !a.jp || ncols <= 0)) || f.variant < 0 || f.variant > 3)
         return hipErrorInvalidValue;
     bool fits = false;
     const size_t dyn = fock_lds(cb, ck, f, mode, ncols, a.nsh, fp32, fits);
     if (!fits && !fock_is_wave(cb, ck)) return hipErrorInvalidValue;
     a.mlds = f.mlds;
     a.dlds = f.dlds;
-    if (mode == kDigestRHF) return fp32 ? fock_launch_rhf32(cb, ck, a, nblocks, f.variant, dyn, st)
-                                        : fock_launch_rhf64(cb, ck, a, nblocks, f.variant, dyn, st);
-    if (mode == kDigestUHF) return fp32 ? fock_launch_uhf32(cb, ck, a, nblocks, f.variant, dyn, st)
-                                        : fock_launch_uhf64(cb, ck, a, nblocks, f.variant, dyn, st);
+    if (mode == kDigestRHF) return fp32 ? fock_launch_rhf32(cb, ck, a, f.variant, dyn, st)
+                                        : fock_launch_rhf64(cb, ck, a, f.variant, dyn, st);
+    if (mode == kDigestUHF) return fp32 ? fock_launch_uhf32(cb, ck, a, f.variant, dyn, st)
+                                        : fock_launch_uhf64(cb, ck, a, f.variant, dyn, st);
     return hipErrorInvalidValue;
 }
 
@@ -273,6 +276,71 @@ hipError_t fock_clear(const ClearList& c, hipStream_t st) {
     if (most <= 0) return hipSuccess;
     const long long nb = std::min<long long>((most + 1023) / 1024, 2048);
     hipLaunchKernelGGL(k_clear, dim3((unsigned)nb, (unsigned)c.n), dim3(256), 0, st, c);
+    return hipGetLastError();
+}
+
+// The tasks of every launch that hold a quartet of this build: a candidate segment counts when
+// its first ket (the largest bound) is within the build and, in a mixed build, some of it lies
+// on the launch's side of the FP32 threshold (fock_task's tests).  Half the candidates are
+// above the diagonal or below the threshold in a full 64-water build and nearly all of them in
+// an incremental one; as blocks of their own each cost a launch slot and a chain of
+// scalar loads.
+__global__ __launch_bounds__(kTaskThreads) void k_fock_tasks(int nsrc, const FockTaskSource* __restrict__ src,
+                                                             const char* __restrict__ tables, const FockArgs a,
+                                                             FockCounter* ctr, int* __restrict__ lists) {
+    __shared__ int wtot[kTaskThreads / 64], base;
+    int lo = 0, hi = nsrc - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (src[mid].block0 <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
+    }
+    const FockTaskSource S = src[lo];
+    const int c = ((int)blockIdx.x - S.block0) * kTaskThreads + (int)threadIdx.x;
+    bool live = false;
+    if (c < S.ncand) {
+        const FockSpace* sp = reinterpret_cast<const FockSpace*>(tables + S.sp);
+        const int* blk = reinterpret_cast<const int*>(tables + S.blk);
+        int x = blk[c >> 6], y = blk[(c >> 6) + 1];
+        while (x < y) {
+            const int mid = (x + y + 1) >> 1;
+            if (sp[mid].first <= c) x = mid; else y = mid - 1;
+        }
+        const FockSpace& s = sp[x];
+        const int l = c - s.first, ibra = l / s.nseg, k0 = (l - ibra * s.nseg) * s.seg;
+        int k1 = min(s.nket, k0 + s.seg);
+        if (s.same) k1 = min(k1, ibra + 1);
+        const int mol = a.mols ? s.mol : 0;
+        if (k0 < k1 && !(a.mol_active && !a.mol_active[mol])) {
+            const double qi = a.pairQ[s.bra_off + ibra], qd = qi * (4.0 * a.dmax[mol]);
+            const double q0 = a.pairQ[s.ket_off + k0];
+            live = qd > 0.0 && q0 >= a.tau / qd;
+            if (live && a.fp32_thr > 0.0) {
+                const double t32 = a.fp32_thr / qi;
+                live = S.f32 ? a.pairQ[s.ket_off + k1 - 1] < t32 : q0 >= t32;
+            }
+        }
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned long long m = __ballot(live);
+    if (lane == 0) wtot[wave] = __popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int w = 0; w < kTaskThreads / 64; ++w) {
+            const int v = wtot[w];
+            wtot[w] = t;
+            t += v;
+        }
+        base = t ? atomicAdd(&ctr[lo].count, t) : 0;
+    }
+    __syncthreads();
+    if (live) lists[S.list + base + wtot[wave] + __popcll(m & ((1ull << lane) - 1))] = c;
+}
+
+hipError_t fock_tasks(int nsrc, const FockTaskSource* src, int nblocks, const char* tables, const FockArgs& a,
+                      FockCounter* ctr, int* lists, hipStream_t st) {
+    if (nsrc <= 0 || nblocks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_fock_tasks, dim3((unsigned)nblocks), dim3(kTaskThreads), 0, st, nsrc, src, tables, a, ctr, lists);
     return hipGetLastError();
 }
 

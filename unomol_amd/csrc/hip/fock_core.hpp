@@ -3,12 +3,13 @@
 //
 // The quartet space of a launch is implicit.  A launch walks a short table of spaces
 // (FockSpace): a run of bra pairs against a run of ket pairs, both sorted by Schwarz bound,
-// descending.  A block is one bra of a space and one segment of its kets.  Which kets of a
+// descending.  A task is one bra of a space and one segment of its kets.  Which kets of a
 // segment belong to the build (Q_ab Q_cd 4 max|D| >= tau, and on which side of the FP32
 // threshold they lie) each lane reads off the bounds themselves against the density maximum in
-// device memory, and a block whose segment starts below the threshold returns at once.  So a
-// build needs no index arrays, no count on the host and no wait for the density bound: its
-// grids are fixed when the context is built.  (Before: prefix and task arrays built and
+// device memory.  So a build needs no index arrays from the host, no count there and no wait for
+// the density bound.  In large builds one kernel first lists the tasks of every launch that
+// hold any quartet (k_fock_tasks); a launch's blocks take tasks from a counter until none is
+// left.  (Before: prefix and task arrays built and
 // uploaded by the host per build, one launch per run pair -- 210 to 245 launches, of which a
 // single water's 210 took 8.0 ms one after the other, 38 us each.)
 //
@@ -63,7 +64,7 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// The space and bra of a block, and its segment's kets [k0, k1) (indices in the ket run);
+// The space and bra of a task, and its segment's kets [k0, k1) (indices in the ket run);
 // false: nothing of it belongs to this build
 struct FockTask {
     FockSpace s;
@@ -77,9 +78,8 @@ struct FockTask {
 };
 
 template <bool F32>
-__device__ __forceinline__ bool fock_task(const FockArgs& a, FockTask& t) {
-    const int b = blockIdx.x;
-    // the table brackets the space of every 64th block
+__device__ __forceinline__ bool fock_task(const FockArgs& a, const int b, FockTask& t) {
+    // the table brackets the space of every 64th candidate
     const auto* bt = scalar_ptr(a.blk);
     int lo = bt[b >> 6], hi = bt[(b >> 6) + 1];
     const auto* sp = scalar_ptr(a.sp);
@@ -125,6 +125,23 @@ __device__ __forceinline__ bool fock_task(const FockArgs& a, FockTask& t) {
     }
     return true;
 }
+
+// How a launch's blocks share out its tasks, the costliest first: the first `grid` of them (or, for
+// the many short tasks of the wave kernels, half of all) round robin, the rest to whoever asks
+// next.  (All of them round robin leaves the launch waiting for its unluckiest block: 66 against
+// 55 ms at 64 waters.  Every short task on request keeps thousands of waves on one counter at
+// memory-side atomics' pace.)  A block asks for its next task ahead of the work on the current one.
+struct FockQueue {
+    int total, base;
+    __device__ __forceinline__ FockQueue(const FockArgs& a, bool half) {
+        total = a.list ? scalar_ptr(&a.ctr->count)[0] : a.ncand;
+        const int grid = (int)gridDim.x;
+        base = half ? max(grid, total / 2 / grid * grid) : grid;
+    }
+    __device__ __forceinline__ bool asks(int item) const { return item + (int)gridDim.x >= base && base < total; }
+    __device__ __forceinline__ int ask(const FockArgs& a) const { return base + atomicAdd(&a.ctr->head, 1); }
+    __device__ __forceinline__ int after(int item) const { return item + (int)gridDim.x; }
+};
 
 // whether ket k (bound q) belongs to this launch
 template <bool F32>
@@ -260,7 +277,7 @@ constexpr int row_threads() {
 }
 
 // ---------------------------------------------------------------------------
-// Classes of up to kLaneMaxComp components: one block per (bra, segment of kets), one lane
+// Classes of up to kLaneMaxComp components: one task per block at a time, one lane
 // (or a group of 2^lg lanes, each with a share of the ket's primitives) per ket.  The
 // exchange contributions all land in the bra's rows of W (rows fa.., fb..), so the block merges
 // them in LDS (one row per bra function and spin, a column per function the ket class touches)
@@ -284,9 +301,19 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void k_fock(const 
     __shared__ double jred[kRowWaves][NA * NB];
     __shared__ unsigned cred[kRowWaves][3];
     __shared__ int queue[kRowWaves][128];
-    FockTask t;
-    if (!fock_task<F32>(a, t)) return;   // whole block
+    __shared__ int upcoming;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const T* tab = rys_table_of<NR, T>(a.rys2_exact);
+    if constexpr (TL) {
+        for (int i = threadIdx.x; i < rys_table_size<NR, T>(); i += kRowThreads) tab_lds[i] = tab[i];
+        tab = tab_lds;
+    }
+    const FockQueue fq(a, false);
+    for (int item = blockIdx.x; item < fq.total;) {
+    const bool asks = fq.asks(item);
+    if (asks && threadIdx.x == 0) upcoming = fq.ask(a);
+    FockTask t;
+    if (fock_task<F32>(a, a.list ? scalar_ptr(a.list)[item] : item, t)) {
     const MolView& mv = t.mv;
     const int n = mv.n, ns = mv.nsh, nc = t.s.ncols;
     const PairHdr P1 = scalar_load(a.pairs + t.bra);
@@ -312,11 +339,6 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void k_fock(const 
     const double* m2 = mv.dsh + (long)P1.sh2 * ns;
     if (ml)
         for (int s = threadIdx.x; s < ns; s += kRowThreads) mrow[s] = fmax(m1[s], m2[s]);
-    const T* tab = rys_table_of<NR, T>(a.rys2_exact);
-    if constexpr (TL) {
-        for (int i = threadIdx.x; i < rys_table_size<NR, T>(); i += kRowThreads) tab_lds[i] = tab[i];
-        tab = tab_lds;
-    }
     __syncthreads();
     const double dab4 = 4.0 * m1[P1.sh2];
     const T ab[3] = {(T)P1.AB[0], (T)P1.AB[1], (T)P1.AB[2]};
@@ -540,9 +562,9 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void k_fock(const 
             c1 += cred[w][1];
             c2 += cred[w][2];
         }
-        atomicAdd(a.nquart + (blockIdx.x & (kQuartSlots - 1)), c0);
+        atomicAdd(a.nquart + (item & (kQuartSlots - 1)), c0);
         if (a.counter) {
-            unsigned long long* slot = a.counter + 2 * (blockIdx.x & (kCounterSlots - 1));
+            unsigned long long* slot = a.counter + 2 * (item & (kCounterSlots - 1));
             atomicAdd(slot, c1);
             atomicAdd(slot + 1, c2);
         }
@@ -557,6 +579,15 @@ __global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void k_fock(const 
             const double v = rows[r * nc + col];
             if (v != 0.0) atomic_add_f64(W + (long)grow * n + colinv[col], v);
         }
+    }
+    }
+    __syncthreads();   // every wave is done with this task's LDS
+    if (asks) {
+        item = __builtin_amdgcn_readfirstlane(upcoming);
+        __syncthreads();
+    } else {
+        item = fq.after(item);
+    }
     }
 }
 
@@ -744,7 +775,7 @@ constexpr int wave_min_waves() {
 }
 
 // ---------------------------------------------------------------------------
-// Larger classes: one wave (one block) per (bra, segment of up to 64 kets, the host's choice is
+// Larger classes: one wave (one block) per task (a segment of up to 64 kets, the host's choice is
 // kWaveSeg).  Lane i screens ket i, then the wave evaluates the survivors one after another and
 // adds their outputs to W.  Segments stay short: the blocks are many, so enough waves are in
 // flight to cover each one's serial latency (64 per block was measured 2.5x slower).
@@ -755,9 +786,14 @@ __global__ __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>())) void k_fock
     constexpr int NA = CI::NA, NB = CI::NB, NC = CI::NC, ND = CI::ND, NCOMP = CI::NCOMP;
     constexpr bool F32 = sizeof(T) == 4;
     __shared__ T sE[NCOMP];
-    FockTask t;
-    if (!fock_task<F32>(a, t)) return;   // whole block
     const int lane = threadIdx.x;
+    const FockQueue fq(a, true);
+    for (int item = blockIdx.x; item < fq.total;) {
+    const bool asks = fq.asks(item);
+    int upcoming = 0;
+    if (asks && lane == 0) upcoming = fq.ask(a);
+    FockTask t;
+    if (fock_task<F32>(a, a.list ? scalar_ptr(a.list)[item] : item, t)) {
     const MolView& mv = t.mv;
     const PairHdr P1 = scalar_load(a.pairs + t.bra);
     const int pcd = t.s.ket_off + t.k0 + lane;
@@ -838,12 +874,15 @@ __global__ __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>())) void k_fock
         __syncthreads();
     }
     if (lane == 0) {
-        atomicAdd(a.nquart + (blockIdx.x & (kQuartSlots - 1)), (unsigned long long)nin);
+        atomicAdd(a.nquart + (item & (kQuartSlots - 1)), (unsigned long long)nin);
         if (a.counter && nshell) {
-            unsigned long long* slot = a.counter + 2 * (blockIdx.x & (kCounterSlots - 1));
+            unsigned long long* slot = a.counter + 2 * (item & (kCounterSlots - 1));
             atomicAdd(slot, nprim);
             atomicAdd(slot + 1, nshell);
         }
+    }
+    }
+    item = asks ? __builtin_amdgcn_readfirstlane(upcoming) : fq.after(item);
     }
 }
 

@@ -25,8 +25,12 @@ bool fock_is_wave(int bra_class, int ket_class);
 FockConfig fock_default(int bra_class, int ket_class, int mode, int ncols, int nsh, bool fp32, bool rows, int force,
                         int dens);
 bool fock_config_fits(int bra_class, int ket_class, const FockConfig& f, int mode, int ncols, int nsh, bool fp32);
-hipError_t fock_launch(int mode, bool fp32, int bra_class, int ket_class, FockArgs a, int nblocks, const FockConfig& f,
-                       int ncols, hipStream_t st);
+hipError_t fock_launch(int mode, bool fp32, int bra_class, int ket_class, FockArgs a, const FockConfig& f, int ncols,
+                       hipStream_t st);
+// lists the tasks of nsrc launches that hold a quartet (a: the build's thresholds, bounds and
+// density maxima); nblocks of kTaskThreads candidates in all, the counters zeroed
+hipError_t fock_tasks(int nsrc, const FockTaskSource* src, int nblocks, const char* tables, const FockArgs& a,
+                      FockCounter* ctr, int* lists, hipStream_t st);
 // the Fock kernels' copies of the pair data (device arrays), runs sorted by off
 hipError_t pair_store(int np, int nrun, const PairRun* runs, const PairHdr* pairs, const PrimPair* prims,
                       const int* colmap, BraPrim* bprim, double* kprim, long long kps, double* kgeo, int4* kidx, int4* kjo,
@@ -38,9 +42,9 @@ struct ClearList {
     int n = 0;
     template <class T>
     void add(T* q, long long count) {
-        static_assert(sizeof(T) == 8, "64-bit words");
+        static_assert(sizeof(T) % 8 == 0, "64-bit words");
         p[n] = reinterpret_cast<unsigned long long*>(q);
-        len[n++] = count;
+        len[n++] = count * (long long)(sizeof(T) / 8);
     }
 };
 hipError_t fock_clear(const ClearList& c, hipStream_t st);

@@ -182,17 +182,25 @@ static int enqueue_fock(uno_batch* b) {
     cl.add(b->W1.p, b->store);
     cl.add(fs.jp.p, fs.njp);
     cl.add(fs.dmax.p, nm);
+    cl.add(fs.ctr.p, 2 * (long long)fs.launches.size());
     UNO_HIP(fock_clear(cl, st));
     UNO_HIP(batch_shell_max(nm, b->maxsh, b->mdesc.p, b->mshoff.p, b->active_d.p, b->sh_off.p, b->sh_n.p, b->D0.p, b->D1.p, b->D2.p,
                             b->Dsh.p, fs.dmax.p, st));
     UNO_HIP(pair_density(np, fs.kidx.p, fs.kjo.p, b->D0.p, b->Dsh.p, 0, 0, b->mdesc.p, b->pmol.p, fs.dp.p, fs.dpair.p, st));
+    const uno_ctx* c0 = b->mol[0].ctx;
+    if (!fs.launches.empty()) {
+        FockArgs a = fs.args(0, 0, false, b->pairs.p, b->prims.p, b->pairQ.p);
+        a.tau = c0->tau;
+        a.mols = b->mdesc.p;
+        a.mol_active = b->active_d.p;
+        if (int rc = fs.list_tasks(false, a, st)) return rc;
+    }
     const int nls = std::max(1, std::min(kMaxLaunchStreams, b->launch_streams));
     if (int rc = b->ls.begin(nls, st)) return rc;
     for (size_t k = 0; k < fs.launches.size(); ++k) {
         const FockLaunch& l = fs.launches[k];
         const bool uhf = l.group != 0;
-        FockArgs a = fs.args(l, b->pairs.p, b->prims.p, b->pairQ.p);
-        const uno_ctx* c0 = b->mol[0].ctx;
+        FockArgs a = fs.args((int)k, 0, false, b->pairs.p, b->prims.p, b->pairQ.p);
         a.tau = c0->tau;
         a.primcut = c0->primcut;
         a.rys2_exact = c0->rys2_exact;
@@ -212,7 +220,7 @@ static int enqueue_fock(uno_batch* b) {
         a.mol_active = b->active_d.p;
         const int mode = uhf ? kDigestUHF : kDigestRHF;
         const FockConfig f = fock_default(l.cx, l.cy, mode, l.ncols, b->maxsh, false, true, 0, -1);
-        UNO_HIP(fock_launch(mode, false, l.cx, l.cy, a, l.nblocks, f, l.ncols, b->ls.of((int)(k % (size_t)nls), st)));
+        UNO_HIP(fock_launch(mode, false, l.cx, l.cy, a, f, l.ncols, b->ls.of((int)(k % (size_t)nls), st)));
     }
     if (int rc = b->ls.end(nls, st)) return rc;
     UNO_HIP(jp_scatter(np, fs.kidx.p, fs.kjo.p, fs.jp.p, b->W0.p, b->W1.p, 0, b->mdesc.p, b->pmol.p, st));

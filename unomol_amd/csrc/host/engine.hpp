@@ -96,15 +96,23 @@ struct FockMol {
 };
 struct FockLaunch {
     int cx, cy, group;      // class pair, launch group
-    int nblocks, ncols;     // grid, largest column count
+    int ncand, ncols;       // candidate tasks, largest column count
     int nket;               // longest ket run
     size_t sp, blk;         // offsets of its tables
+    int list[2];            // offsets of its task lists, FP64 and FP32
 };
 struct FockStore {
     int npair = 0;
     long long njp = 0, kps = 0;
     std::vector<FockLaunch> launches;
     DBuf<char> tables;
+    // task lists (builds of more than a few thousand candidates): the launches as sources, FP64
+    // ones alone and with the FP32 ones of a mixed build, and a counter per launch and precision
+    bool listed = false;
+    DBuf<FockTaskSource> src[2];
+    int nsrc[2] = {0, 0}, src_blocks[2] = {0, 0};
+    DBuf<int> lists;
+    DBuf<FockCounter> ctr;
     DBuf<BraPrim> bprim;
     DBuf<double> kprim, kgeo, dp, jp, dpair, dmax;
     DBuf<int4> kidx, kjo;
@@ -113,7 +121,10 @@ struct FockStore {
     DBuf<unsigned long long> nquart;       // FP64 launches' counters, then FP32's
     int build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, const PrimPair* d_prims, int np, long long nprims,
               hipStream_t st);
-    FockArgs args(const FockLaunch& l, const PairHdr* d_pairs, const PrimPair* d_prims, const double* pairQ) const;
+    // arguments of launch k's FP64 (prec 0) or FP32 half, but for the densities and thresholds
+    FockArgs args(int k, int prec, bool mixed, const PairHdr* d_pairs, const PrimPair* d_prims, const double* pairQ) const;
+    // lists the tasks of a build (a: any launch's arguments with the thresholds set)
+    int list_tasks(bool mixed, const FockArgs& a, hipStream_t st) const;
 };
 // streams that launches are spread over: the caller's and up to kMaxLaunchStreams - 1 workers at
 // the default priority, forked from and joined back to the caller's

@@ -47,6 +47,9 @@ LaunchStreams::~LaunchStreams() {
 // lanes that fill the chip several times over (1024 SIMDs x 8 waves x 64): below it a launch's
 // kets get several lanes each
 constexpr double kFillLanes = 1 << 20;
+// candidate tasks from which a build lists the live ones first (below, the list costs a
+// launch and saves little: one water has 900 candidates, 16 waters 50 000)
+constexpr long long kListFrom = 8192;
 
 // log2 of the lanes that share a ket of kprim primitives against a bra of bprim, in a launch of
 // `quartets` shell quartets: doubled while the launch would leave the chip idle otherwise, or
@@ -137,7 +140,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                 };
                 std::vector<Cand> cs;
                 double total = 0.0;
-                FockLaunch L{cx, cy, g, 0, 1, 0, 0, 0};
+                FockLaunch L{cx, cy, g, 0, 1, 0, 0, 0, {0, 0}};
                 for (size_t m = 0; m < mols.size(); ++m) {
                     if (mols[m].group != g) continue;
                     for (size_t X = 0; X < runs[m].size(); ++X)
@@ -195,7 +198,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                         return UNO_EINVAL;
                     }
                 }
-                L.nblocks = (int)nb;
+                L.ncand = (int)nb;
                 std::vector<int> blk;
                 int k = 0;
                 for (long long b = 0; b <= nb + 63; b += 64) {
@@ -206,6 +209,31 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                 L.blk = put(blk.data(), blk.size() * sizeof(int));
                 launches.push_back(L);
             }
+    // the task lists' sources: counter and list of launch k and precision p (2 k + p in a mixed
+    // build, k otherwise)
+    long long total = 0;
+    for (FockLaunch& l : launches)
+        for (int p = 0; p < 2; ++p) {
+            l.list[p] = (int)std::min<long long>(total, INT32_MAX);
+            total += l.ncand;
+        }
+    listed = total > 2 * kListFrom && total <= (long long)INT32_MAX;
+    std::vector<FockTaskSource> hsrc[2];
+    if (listed) {
+        for (int m = 0; m < 2; ++m) {
+            int nb = 0;
+            for (const FockLaunch& l : launches)
+                for (int p = 0; p <= m; ++p) {
+                    hsrc[m].push_back(FockTaskSource{(long long)l.sp, (long long)l.blk, nb, l.ncand, l.list[p], p});
+                    nb += (l.ncand + kTaskThreads - 1) / kTaskThreads;
+                }
+            nsrc[m] = (int)hsrc[m].size();
+            src_blocks[m] = nb;
+            UNO_HIP(src[m].upload(hsrc[m].data(), hsrc[m].size(), st));
+        }
+        UNO_HIP(lists.alloc((size_t)total));
+    }
+    UNO_HIP(ctr.alloc(2 * launches.size()));
     DBuf<PairRun> dr;
     DBuf<int> dcm;
     UNO_HIP(dr.upload(pr.data(), pr.size(), st));
@@ -230,10 +258,15 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
     return UNO_OK;
 }
 
-FockArgs FockStore::args(const FockLaunch& l, const PairHdr* d_pairs, const PrimPair* d_prims, const double* pairQ) const {
+FockArgs FockStore::args(int k, int prec, bool mixed, const PairHdr* d_pairs, const PrimPair* d_prims,
+                         const double* pairQ) const {
+    const FockLaunch& l = launches[k];
     FockArgs a{};
     a.sp = reinterpret_cast<const FockSpace*>(tables.p + l.sp);
     a.blk = reinterpret_cast<const int*>(tables.p + l.blk);
+    a.list = listed ? lists.p + l.list[prec] : nullptr;
+    a.ctr = ctr.p + (mixed ? 2 * k + prec : k);
+    a.ncand = l.ncand;
     a.pairs = d_pairs;
     a.prims = d_prims;
     a.bprim = bprim.p;
@@ -250,6 +283,12 @@ FockArgs FockStore::args(const FockLaunch& l, const PairHdr* d_pairs, const Prim
     a.dp = dp.p;
     a.dmax = dmax.p;
     return a;
+}
+
+int FockStore::list_tasks(bool mixed, const FockArgs& a, hipStream_t st) const {
+    const int m = mixed ? 1 : 0;
+    if (listed) UNO_HIP(fock_tasks(nsrc[m], src[m].p, src_blocks[m], tables.p, a, ctr.p, lists.p, st));
+    return UNO_OK;
 }
 
 // tuned configurations, shared by every context of the same layout (basis size, shells, pairs
@@ -290,6 +329,7 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
     cl.add(fs.jp.p, fs.njp);
     cl.add(fs.nquart.p, 2 * kQuartSlots);
     cl.add(fs.dmax.p, 1);
+    cl.add(fs.ctr.p, 2 * (long long)fs.launches.size());
     UNO_HIP(fock_clear(cl, st));
     // shell-block density maxima for the screen, the largest of them, and the densities in the
     // pairs' order
@@ -297,15 +337,22 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
                         uhf ? c->D2.p : nullptr, c->Dsh.p, fs.dmax.p, st));
     UNO_HIP(pair_density(fs.npair, fs.kidx.p, fs.kjo.p, c->D0.p, c->Dsh.p, c->n, c->nsh, nullptr, nullptr, fs.dp.p,
                          fs.dpair.p, st));
+    if (!fs.launches.empty()) {
+        FockArgs a = fs.args(0, 0, mixed, c->d_pairs.p, c->d_prims.p, c->d_pairQ.p);
+        a.tau = c->tau;
+        a.fp32_thr = mixed ? c->fp32_thr : 0.0;
+        if (int rc = fs.list_tasks(mixed, a, st)) return rc;
+    }
     const int mode = uhf ? kDigestUHF : kDigestRHF;
     // (the tuner times each launch on the context's stream)
     const int nls = c->tuning ? 1 : std::max(1, std::min(kMaxLaunchStreams, c->launch_streams));
     if (int rc = c->ls.prepare(nls)) return rc;
     if (int rc = c->ls.begin(nls, st)) return rc;
     int nlaunch = 0;
-    for (const FockLaunch& l : fs.launches)
+    for (int k = 0; k < (int)fs.launches.size(); ++k)
         for (int prec = 0; prec < (mixed ? 2 : 1); ++prec) {
-            FockArgs a = fs.args(l, c->d_pairs.p, c->d_prims.p, c->d_pairQ.p);
+            const FockLaunch& l = fs.launches[k];
+            FockArgs a = fs.args(k, prec, mixed, c->d_pairs.p, c->d_prims.p, c->d_pairQ.p);
             a.tau = c->tau;
             a.primcut = c->primcut;
             a.fp32_thr = mixed ? c->fp32_thr : 0.0;
@@ -335,7 +382,7 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
             }
             const int ci = prec * kNumPairClasses * kNumPairClasses + l.cx * kNumPairClasses + l.cy;
             auto launch = [&](const FockConfig& g, hipStream_t s) {
-                return fock_launch(mode, prec == 1, l.cx, l.cy, a, l.nblocks, g, l.ncols, s);
+                return fock_launch(mode, prec == 1, l.cx, l.cy, a, g, l.ncols, s);
             };
             if (c->tuning && rows && !wave) {
                 // time every candidate (each one run three times, the fastest counts)
@@ -344,15 +391,17 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
                 hipEvent_t t0, t1;
                 UNO_HIP(hipEventCreate(&t0));
                 UNO_HIP(hipEventCreate(&t1));
-                for (int k = 0; k < 16; ++k) {
+                for (int v = 0; v < 16; ++v) {
                     FockConfig g;
-                    g.variant = k & 3;
-                    g.dlds = (k >> 2) & 1;
-                    g.mlds = (k >> 3) & 1;
+                    g.variant = v & 3;
+                    g.dlds = (v >> 2) & 1;
+                    g.mlds = (v >> 3) & 1;
                     if (g.dlds && (!g.variant || c->row_dens == 0)) continue;
                     if (!fock_config_fits(l.cx, l.cy, g, mode, l.ncols, c->nsh, prec == 1)) continue;
                     float ms_min = 1e30f;
                     for (int rep = 0; rep < 3; ++rep) {
+                        // the tasks from the first one again
+                        UNO_HIP(hipMemsetAsync(&a.ctr->head, 0, sizeof(int), st));
                         UNO_HIP(hipEventRecord(t0, st));
                         UNO_HIP(launch(g, st));
                         UNO_HIP(hipEventRecord(t1, st));
@@ -378,16 +427,16 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
             hipEvent_t e1 = nullptr;
             if (prof) {
                 a.counter = c->d_counter.p + 2 * kCounterSlots * slot;
-                const size_t k = c->prof_pending++;
-                while (c->prof_ev.size() < 2 * (k + 1)) {
+                const size_t pe = c->prof_pending++;
+                while (c->prof_ev.size() < 2 * (pe + 1)) {
                     hipEvent_t e = nullptr;
                     UNO_HIP(hipEventCreate(&e));
                     c->prof_ev.push_back(e);
                 }
-                if (c->prof_evslot.size() < k + 1) c->prof_evslot.resize(k + 1);
-                c->prof_evslot[k] = slot;
-                e1 = c->prof_ev[2 * k + 1];
-                UNO_HIP(hipEventRecord(c->prof_ev[2 * k], ls));
+                if (c->prof_evslot.size() < pe + 1) c->prof_evslot.resize(pe + 1);
+                c->prof_evslot[pe] = slot;
+                e1 = c->prof_ev[2 * pe + 1];
+                UNO_HIP(hipEventRecord(c->prof_ev[2 * pe], ls));
             }
             UNO_HIP(launch(f, ls));
             if (prof) UNO_HIP(hipEventRecord(e1, ls));
