@@ -207,7 +207,7 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const Bat
     const bool vl = jacobi_v_fits(n);
     double* V = vl ? lds + n * ld : M.V;   // V[p ldv + i] = component i of vector p
     const int ldv = vl ? ld : n;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     double f2 = 0.0;
     for (int e = tid; e < n * n; e += kJacobiThreads) {
         const int i = e / n, j = e - i * n;
@@ -261,32 +261,41 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const Bat
                 sn[tid] = s;
             }
             __syncthreads();
-            for (int x = tid; x < mk * mk; x += kJacobiThreads) {
-                const int k = x / mk, l = x - k * mk;
-                const double ck = cs[k], sk = sn[k], cl = cs[l], sl = sn[l];
-                if (sk == 0.0 && sl == 0.0) continue;
+            // a wave takes whole rows of blocks (pair k, its rotation uniform), its lanes the pairs
+            // l; then whole rotations of the eigenvectors, its lanes the components
+            for (int l0 = 0; l0 < mk; l0 += 64) {
+                const int l = l0 + lane;
+                const bool on = l < mk;
+                const double cl = on ? cs[l] : 1.0, sl = on ? sn[l] : 0.0;
+                const int pl = on ? pp[l] : 0, ql = on ? qq[l] : n;
                 // (the dummy index of an odd n only meets rotations with s = 0: its row and
                 // column are left out)
-                const int pk = pp[k], qk = qq[k], pl = pp[l], ql = qq[l];
-                const bool vk = qk < n, vq = ql < n;
-                const double a00 = A[pk * ld + pl], a01 = vq ? A[pk * ld + ql] : 0.0;
-                const double a10 = vk ? A[qk * ld + pl] : 0.0, a11 = vk && vq ? A[qk * ld + ql] : 0.0;
-                const double r00 = ck * a00 - sk * a10, r01 = ck * a01 - sk * a11;
-                const double r10 = sk * a00 + ck * a10, r11 = sk * a01 + ck * a11;
-                A[pk * ld + pl] = cl * r00 - sl * r01;
-                if (vq) A[pk * ld + ql] = sl * r00 + cl * r01;
-                if (vk) A[qk * ld + pl] = cl * r10 - sl * r11;
-                if (vk && vq) A[qk * ld + ql] = sl * r10 + cl * r11;
+                const bool vq = ql < n;
+                for (int k = wave; k < mk; k += kJacobiThreads / 64) {
+                    const double ck = cs[k], sk = sn[k];
+                    if (!on || (sk == 0.0 && sl == 0.0)) continue;
+                    const int pk = pp[k], qk = qq[k];
+                    const bool vk = qk < n;
+                    const double a00 = A[pk * ld + pl], a01 = vq ? A[pk * ld + ql] : 0.0;
+                    const double a10 = vk ? A[qk * ld + pl] : 0.0, a11 = vk && vq ? A[qk * ld + ql] : 0.0;
+                    const double r00 = ck * a00 - sk * a10, r01 = ck * a01 - sk * a11;
+                    const double r10 = sk * a00 + ck * a10, r11 = sk * a01 + ck * a11;
+                    A[pk * ld + pl] = cl * r00 - sl * r01;
+                    if (vq) A[pk * ld + ql] = sl * r00 + cl * r01;
+                    if (vk) A[qk * ld + pl] = cl * r10 - sl * r11;
+                    if (vk && vq) A[qk * ld + ql] = sl * r10 + cl * r11;
+                }
             }
-            for (int e = tid; e < mk * n; e += kJacobiThreads) {
-                const int k = e / n, i = e - k * n;
-                const double s = sn[k];
+            for (int k = wave; k < mk; k += kJacobiThreads / 64) {
+                const double c = cs[k], s = sn[k];
                 if (s == 0.0) continue;
-                const double c = cs[k];
-                const int p = pp[k] * ldv + i, q = qq[k] * ldv + i;
-                const double vp = V[p], vq = V[q];
-                V[p] = c * vp - s * vq;
-                V[q] = s * vp + c * vq;
+                double* vp = V + pp[k] * ldv;
+                double* vq = V + qq[k] * ldv;
+                for (int i = lane; i < n; i += 64) {
+                    const double x = vp[i], y = vq[i];
+                    vp[i] = c * x - s * y;
+                    vq[i] = s * x + c * y;
+                }
             }
             __syncthreads();
         }

@@ -44,24 +44,26 @@ LaunchStreams::~LaunchStreams() {
     if (fork) (void)hipEventDestroy(fork);
 }
 
-// lanes that fill the chip several times over (1024 SIMDs x 8 waves x 64): below it a launch's
-// kets get several lanes each
-constexpr double kFillLanes = 1 << 20;
 // candidate tasks from which a build lists the live ones first (below, the list costs a
 // launch and saves little: one water has 900 candidates, 16 waters 50 000)
 constexpr long long kListFrom = 8192;
 
+// lanes the chip holds at two waves per SIMD
+constexpr double kChipLanes = 2 * 1024 * 64;
+
 // log2 of the lanes that share a ket of kprim primitives against a bra of bprim, in a launch of
-// `quartets` shell quartets: doubled while the launch would leave the chip idle otherwise, or
-// while the split costs next to nothing (the rounds over the ket's primitives stay nearly full, and
-// each lane keeps primitive quartets enough that adding up the group's blocks does not show)
-static int lanes_per_ket(int bprim, int kprim, double quartets) {
+// about `prims` primitive quartets: doubled while the split costs next to nothing (the rounds over
+// the ket's primitives stay nearly full, and each lane keeps primitive quartets enough that
+// adding up the group's blocks does not show), or while one lane's loop over a quartet's
+// primitives is longer than the launch could take with its work spread over the chip.  (A third
+// of the candidates are taken to survive the screens.)
+static int lanes_per_ket(int bprim, int kprim, double prims) {
+    const double share = std::max(8.0, 0.3 * prims / kChipLanes);
     int lg = 0;
     while ((1 << lg) < kprim && lg < 6) {
-        const int g = 2 << lg, rounds = (kprim + g - 1) / g;
-        const bool fill = quartets * g <= kFillLanes;
+        const int g = 2 << lg, rounds = (kprim + g - 1) / g, now = (kprim + (1 << lg) - 1) >> lg;
         const bool cheap = kprim >= 0.85 * rounds * g && bprim * rounds >= 16;
-        if (!fill && !cheap) break;
+        if (!cheap && bprim * now <= share) break;
         ++lg;
     }
     return lg;
@@ -139,7 +141,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                     int bprim, kprim;
                 };
                 std::vector<Cand> cs;
-                double total = 0.0;
+                double total = 0.0, prims = 0.0;
                 FockLaunch L{cx, cy, g, 0, 1, 0, 0, 0, {0, 0}};
                 for (size_t m = 0; m < mols.size(); ++m) {
                     if (mols[m].group != g) continue;
@@ -161,7 +163,9 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                             s.kp0 = k.kp0;
                             s.jo0 = k.jo0;
                             cs.push_back(Cand{s, b.maxprim, k.maxprim});
-                            total += (s.same ? 0.5 : 1.0) * s.nbra * (double)s.nket;
+                            const double nq = (s.same ? 0.5 : 1.0) * s.nbra * (double)s.nket;
+                            total += nq;
+                            prims += nq * b.maxprim * k.maxprim;
                             L.ncols = std::max(L.ncols, s.ncols);
                             L.nket = std::max(L.nket, s.nket);
                         }
@@ -183,7 +187,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                         if (fock_is_wave(cx, cy)) {
                             s.seg = longer * (int)std::max(1.0, std::min<double>(kWaveSeg, total / 4096.0));
                         } else {
-                            s.lg = lanes_per_ket(c.bprim, c.kprim, total);
+                            s.lg = lanes_per_ket(c.bprim, c.kprim, prims);
                             const int pass = kLaneBlock >> s.lg;
                             s.seg = longer * pass * (int)std::max(1.0, std::min(32.0, total / (pass * 8192.0)));
                         }
