@@ -123,13 +123,14 @@ struct EigWork {
     double* V;      // n x n reflector vectors (row k = v_k, zero outside its support)
     double* tau;    // n
     double* p;      // n
-    double* d;      // n  diagonal of T
-    double* e;      // n  off-diagonal of T
+    double* d;      // n, and zeros up to a multiple of 16: diagonal of T
+    double* e;      // the same: off-diagonal of T
     double* scal;   // 4 scalars
     double* evals;  // n  eigenvalues of T (ascending)
     double* Y;      // n x n eigenvectors of T, one per column (Yt)
-    double* wk;     // 5 n^2 inverse-iteration work
+    double* wk;     // work space of at least eig_work_doubles(n), at most 5 n^2
 };
+size_t eig_work_doubles(int n);
 hipError_t householder_tridiag(int n, EigWork& w, hipStream_t st);
 // Z <- Q Z with Q = H_0 ... H_{n-3} from the reflectors in w.V / w.tau (uses w.wk)
 hipError_t apply_q(int n, EigWork& w, double* Z, hipStream_t st);

@@ -622,7 +622,7 @@ hipError_t sp2_state_read(const void* states, int k, int* cur, int* done, int* s
 //   p = tau A22 v, K = tau/2 p.v, w = p - K v, A22 -= v w^T + w v^T
 // d[k] = A[k][k], e[k] = alpha.  Reflector k is stored in row k of V (absolute column
 // indices).  One launch per column k: every block first finishes step k-1 for itself
-// (K and w of step k-1 from the previous launch's p and partial sums, row k updated on the
+// (K and w of step k-1 from the previous launch's p and its terms of p.v, row k updated on the
 // fly, reflector k from it: the same arithmetic in the same order in every block, so every
 // block holds the same reflector; block 0 stores it), then applies the rank-2 update of
 // step k-1 to its trailing rows and forms their p of step k.  The trailing matrix stays
@@ -636,94 +636,154 @@ __device__ __forceinline__ void hh_reflector(double nx2, double x0, double& alph
     t = (nx2 == 0.0 || vn2 == 0.0) ? 0.0 : 2.0 / vn2;
 }
 
-// launch of column k (four trailing rows per block, one wave per row).  Pp/partp: p and
-// partial sums of step k-1 (read), Pc/partc: those of step k (written).  Dynamic LDS: 3 n
-// doubles (v of step k, v and w of step k-1).
-__global__ __launch_bounds__(256) void k_hh_col(int n, int k, double* A, double* V, double* tau, double* d, double* e,
-                                                const double* Pp, const double* partp, int npartp, double* Pc,
-                                                double* partc) {
+// rows of the tridiagonal's chains, in chunks whose operands are read together; d and e carry zeros
+// up to the next whole chunk
+constexpr int kEigChunk = 16;
+__host__ __device__ constexpr int eig_pad(int n) { return (n + kEigChunk - 1) / kEigChunk * kEigChunk; }
+
+// sum over the wave in every lane, by DPP moves inside the vector unit (six LDS-crossbar shuffles
+// cost four times their latency): quads, halves and rows of 16 by swaps, then rows 0 -> 1 and
+// 2 -> 3 and halves 0 -> 1 by broadcasts, which leaves the total in lane 63
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+    return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// sum over the 16 lanes of a row, in every lane of it
+__device__ __forceinline__ double row_total(double v) {
+    v = dpp_add<0xb1, 0xf>(v);    // quad_perm 1,0,3,2
+    v = dpp_add<0x4e, 0xf>(v);    // quad_perm 2,3,0,1
+    v = dpp_add<0x141, 0xf>(v);   // row_half_mirror
+    return dpp_add<0x140, 0xf>(v);   // row_mirror
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {   // lane: the same in the whole wave
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_total(double v) {
+    v = row_total(v);
+    v = dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+    return lane_value(v, 63);
+}
+
+// launch of column k (four rows per block, one wave per row; b0: the first block of the launch, a
+// multiple of the XCD count, so that a row stays on one XCD and in its L2 from launch to launch).  Pp/partp: p and the rows'
+// terms of p.v of step k-1 (read), Pc/partc: those of step k (written).  Dynamic LDS: 3 n
+// doubles (v of step k, v and w of step k-1).  What a launch costs is its chain of latencies, not
+// the matrix (9.7 MB at n = 1216, cache-resident): every global load that does not depend on
+// another is issued first, and the two sums the reflector needs are shuffles and one barrier
+// each (with tree reductions over the block, the partial sums read in a loop and rows that changed
+// their XCD from column to column: 9.8 us a column at n = 1216; now 6.4).
+constexpr int kHhVec = 6, kHhRow = 20;   // prefetched per thread: vector entries, row entries
+__global__ __launch_bounds__(256) void k_hh_col(int n, int k, int b0, double* A, double* V, double* tau, double* d, double* e,
+                                                const double* Pp, const double* partp, double* Pc, double* partc) {
     extern __shared__ double lds[];
-    double* sv = lds;            // v_k (absolute indices k+1..n-1)
+    double* sv = lds;            // x of step k (absolute indices k+1..n-1)
     double* svp = lds + n;       // v_{k-1} (k..n-1)
     double* swp = lds + 2 * n;   // w_{k-1} (k..n-1)
-    __shared__ double sh[256];
-    __shared__ double pv[4];
-    double K = 0.0;
+    __shared__ double sh[8];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int m = n - k - 1;
+    const int r = (blockIdx.x + b0) * 4 + wave, row = r - k - 1;
+    const bool on = row >= 0 && row < m;
+    const double* vp = V + (long)(k - 1) * n;
+    const double* ak = A + (long)k * n;
+    double* a = A + (long)r * n;
+    double pa[kHhRow], pv[kHhVec], pw[kHhVec], px[kHhVec], ps[kHhVec];
+#pragma unroll
+    for (int c = 0; c < kHhVec; ++c) {
+        const int j = k + 1 + tid + 256 * c;
+        pv[c] = (k > 0 && j < n) ? vp[j] : 0.0;
+        pw[c] = (k > 0 && j < n) ? Pp[j] : 0.0;
+        px[c] = j < n ? ak[j] : 0.0;
+        ps[c] = (k > 0 && j <= n) ? partp[j - k - 1] : 0.0;   // step k-1 had n - k rows
+    }
+#pragma unroll
+    for (int c = 0; c < kHhRow; ++c) {
+        const int j = k + 1 + lane + 64 * c;
+        pa[c] = (on && j < n) ? a[j] : 0.0;
+    }
+    double K = 0.0, vk = 0.0, wk = 0.0;
     if (k > 0) {
         double s = 0.0;
-        for (int b = threadIdx.x; b < npartp; b += 256) s += partp[b];
-        K = 0.5 * tau[k - 1] * block_sum(s, sh);
-        const double* vp = V + (long)(k - 1) * n;
-        for (int j = k + threadIdx.x; j < n; j += 256) {
-            const double vj = vp[j];
-            svp[j] = vj;
-            swp[j] = Pp[j] - K * vj;
-        }
+#pragma unroll
+        for (int c = 0; c < kHhVec; ++c) s += ps[c];
+        for (int j = tid + 256 * kHhVec; j <= m; j += 256) s += partp[j];
+        vk = vp[k];
+        wk = Pp[k];
+        s = wave_total(s);
+        if (lane == 0) sh[wave] = s;
         __syncthreads();
+        K = 0.5 * tau[k - 1] * ((sh[0] + sh[1]) + (sh[2] + sh[3]));
+        wk -= K * vk;
     }
     // row k of the matrix after step k-1, and reflector k from it
-    const double* ak = A + (long)k * n;
-    const double vk = k > 0 ? svp[k] : 0.0, wk = k > 0 ? swp[k] : 0.0;
     double s2 = 0.0;
-    for (int j = k + 1 + threadIdx.x; j < n; j += 256) {
-        const double x = k > 0 ? ak[j] - (vk * swp[j] + wk * svp[j]) : ak[j];
+    auto entry = [&](int j, double v, double p, double x) {
+        const double w = p - K * v;
+        x = k > 0 ? x - (vk * w + wk * v) : x;
+        svp[j] = v;
+        swp[j] = w;
         sv[j] = x;
         s2 = fma(x, x, s2);
+    };
+#pragma unroll
+    for (int c = 0; c < kHhVec; ++c) {
+        const int j = k + 1 + tid + 256 * c;
+        if (j < n) entry(j, pv[c], pw[c], px[c]);
     }
-    const double nx2 = block_sum(s2, sh);   // also orders the sv writes before the reads below
+    for (int j = k + 1 + tid + 256 * kHhVec; j < n; j += 256) entry(j, k > 0 ? vp[j] : 0.0, k > 0 ? Pp[j] : 0.0, ak[j]);
+    s2 = wave_total(s2);
+    if (lane == 0) sh[4 + wave] = s2;
+    __syncthreads();
     const double x0 = sv[k + 1];
     double alpha, v0, t;
-    hh_reflector(nx2, x0, alpha, v0, t);
-    __syncthreads();   // every thread has read sv[k + 1]
-    if (threadIdx.x == 0) sv[k + 1] = v0;
-    __syncthreads();
+    hh_reflector((sh[4] + sh[5]) + (sh[6] + sh[7]), x0, alpha, v0, t);
     if (blockIdx.x == 0) {
         double* vrow = V + (long)k * n;
-        for (int j = k + 1 + threadIdx.x; j < n; j += 256) vrow[j] = sv[j];
-        if (threadIdx.x == 0) {
+        for (int j = k + 1 + tid; j < n; j += 256) vrow[j] = j == k + 1 ? v0 : sv[j];
+        if (tid == 0) {
             tau[k] = t;
             d[k] = k > 0 ? ak[k] - (vk * wk + wk * vk) : ak[k];
             e[k] = t == 0.0 ? x0 : alpha;
         }
     }
     // the block's trailing rows: update of step k-1, then p of step k
-    const int m = n - k - 1;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + wave;
-    double pr = 0.0;
-    if (row < m) {
-        const int r = k + 1 + row;
-        double* a = A + (long)r * n;
-        double acc = 0.0;
+    if (!on) return;   // whole wave
+    double acc = 0.0;
+    const double vr = svp[r], wr = swp[r];
+    auto step = [&](int j, double x) {
         if (k > 0) {
-            const double vr = svp[r], wr = swp[r];
-            for (int j = k + 1 + lane; j < n; j += 64) {
-                const double x = a[j] - (vr * swp[j] + wr * svp[j]);
-                a[j] = x;
-                acc = fma(x, sv[j], acc);
-            }
-        } else {
-            for (int j = k + 1 + lane; j < n; j += 64) acc = fma(a[j], sv[j], acc);
+            x -= vr * swp[j] + wr * svp[j];
+            a[j] = x;
         }
-        for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-        pr = t * acc;
-        if (lane == 0) Pc[r] = pr;
+        acc = fma(x, j == k + 1 ? v0 : sv[j], acc);
+    };
+#pragma unroll
+    for (int c = 0; c < kHhRow; ++c) {
+        const int j = k + 1 + lane + 64 * c;
+        if (j < n) step(j, pa[c]);
     }
-    if (lane == 0) pv[wave] = row < m ? pr * sv[k + 1 + row] : 0.0;
-    __syncthreads();
-    if (threadIdx.x == 0) partc[blockIdx.x] = (pv[0] + pv[1]) + (pv[2] + pv[3]);
+    for (int j = k + 1 + lane + 64 * kHhRow; j < n; j += 64) step(j, a[j]);
+    acc = wave_total(acc);
+    if (lane == 0) {
+        const double pr = t * acc;
+        Pc[r] = pr;
+        partc[row] = pr * (row == 0 ? v0 : sv[r]);
+    }
 }
 
 // after the last reflector (step n-3): its w on the trailing 2 x 2 block, the update
 // there, and that block's d, e
-__global__ __launch_bounds__(256) void k_hh_tail(int n, const double* A, const double* V, const double* tau,
-                                                 const double* P, const double* part, int nparts, double* d, double* e) {
-    __shared__ double sh[256];
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nparts; b += 256) s += part[b];
+__global__ void k_hh_tail(int n, const double* A, const double* V, const double* tau, const double* P, const double* part,
+                          double* d, double* e) {
     const int k = n - 3, r0 = n - 2, r1 = n - 1;
-    const double K = 0.5 * tau[k] * block_sum(s, sh);
     if (threadIdx.x == 0) {
+        const double K = 0.5 * tau[k] * (part[0] + part[1]);
         const double* v = V + (long)k * n;
         const double w0 = P[r0] - K * v[r0], w1 = P[r1] - K * v[r1];
         d[r0] = A[(long)r0 * n + r0] - (v[r0] * w0 + w0 * v[r0]);
@@ -731,34 +791,138 @@ __global__ __launch_bounds__(256) void k_hh_tail(int n, const double* A, const d
         d[r1] = A[(long)r1 * n + r1] - (v[r1] * w1 + w1 * v[r1]);
         e[r1] = 0.0;
     }
+    for (int j = n + threadIdx.x; j < eig_pad(n); j += 64) d[j] = e[j] = 0.0;
+}
+
+// The whole reduction in one block for n <= kHhOneN, the matrix in the registers of its 8 waves: a
+// column takes two barriers and two vectors through LDS instead of a launch, and every wave does
+// the vector work (reflector, K, w) for itself.  Row r lies in slot r / 32 of the 16 lanes
+// (r / 4 % 8, r % 4) = (wave, row of lanes), column j in lane j % 16 of them: a sum over the columns
+// is four DPP moves for four rows at once.  n = 133: 313 us (one row per wave, six moves each: 408 us;
+// a launch per column: 0.77 ms).
+constexpr int kHhOneN = 192, kHhSlots = kHhOneN / 32, kHhCols = kHhOneN / 16;
+__global__ __launch_bounds__(512) void k_hh_one(int n, const double* __restrict__ A0, double* V, double* tau, double* d,
+                                                double* e) {
+    __shared__ double sx[kHhOneN], sp[kHhOneN];
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15;
+    const int row0 = __builtin_amdgcn_readfirstlane(tid >> 6) * 4, row = row0 + (lane >> 4);
+    double a[kHhSlots][kHhCols];
+#pragma unroll
+    for (int s = 0; s < kHhSlots; ++s)
+#pragma unroll
+        for (int c = 0; c < kHhCols; ++c) {
+            const int r = 32 * s + row, j = col + 16 * c;
+            a[s][c] = (r < n && j < n) ? A0[(long)r * n + j] : 0.0;
+        }
+    for (int j = tid; j < kHhOneN; j += 512) sp[j] = 0.0;
+    for (int k = 0; k + 2 < n; ++k) {
+#pragma unroll
+        for (int s = 0; s < kHhSlots; ++s)
+            if (32 * s + row == k) {
+#pragma unroll
+                for (int c = 0; c < kHhCols; ++c) sx[col + 16 * c] = a[s][c];
+            }
+        __syncthreads();
+        // the entries up to k of v are zero: those columns and rows keep what they have
+        double v[kHhCols], w[kHhCols], s2 = 0.0;
+#pragma unroll
+        for (int c = 0; c < kHhCols; ++c) {
+            v[c] = col + 16 * c > k ? sx[col + 16 * c] : 0.0;
+            s2 = fma(v[c], v[c], s2);
+        }
+        const double x0 = sx[k + 1], dk = sx[k];
+        double alpha, v0, t;
+        hh_reflector(row_total(s2), x0, alpha, v0, t);
+#pragma unroll
+        for (int c = 0; c < kHhCols; ++c)
+            if (col + 16 * c == k + 1) v[c] = v0;
+        if (tid < 16) {
+#pragma unroll
+            for (int c = 0; c < kHhCols; ++c)
+                if (col + 16 * c > k && col + 16 * c < n) V[(long)k * n + col + 16 * c] = v[c];
+            if (tid == 0) {
+                tau[k] = t;
+                d[k] = dk;
+                e[k] = t == 0.0 ? x0 : alpha;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < kHhSlots; ++s) {
+            if (32 * s + row0 + 3 > k && 32 * s + row0 < n) {   // the same in the wave
+                double acc = 0.0;
+#pragma unroll
+                for (int c = 0; c < kHhCols; ++c) acc = fma(a[s][c], v[c], acc);
+                acc = t * row_total(acc);
+                if (col == 0) sp[32 * s + row] = acc;
+            }
+        }
+        double vr[kHhSlots];
+#pragma unroll
+        for (int s = 0; s < kHhSlots; ++s) {
+            const int r = 32 * s + row;
+            vr[s] = r == k + 1 ? v0 : r > k ? sx[r] : 0.0;
+        }
+        __syncthreads();
+        double pv = 0.0;
+#pragma unroll
+        for (int c = 0; c < kHhCols; ++c) {
+            w[c] = col + 16 * c > k ? sp[col + 16 * c] : 0.0;
+            pv = fma(w[c], v[c], pv);
+        }
+        const double K = 0.5 * t * row_total(pv);
+#pragma unroll
+        for (int c = 0; c < kHhCols; ++c) w[c] -= K * v[c];
+#pragma unroll
+        for (int s = 0; s < kHhSlots; ++s)
+            if (32 * s + row0 + 3 > k && 32 * s + row0 < n) {
+                const int r = 32 * s + row;
+                const double wr = r > k ? sp[r] - K * vr[s] : 0.0;
+#pragma unroll
+                for (int c = 0; c < kHhCols; ++c) a[s][c] -= vr[s] * w[c] + wr * v[c];
+            }
+    }
+#pragma unroll
+    for (int s = 0; s < kHhSlots; ++s) {
+        const int r = 32 * s + row;
+#pragma unroll
+        for (int c = 0; c < kHhCols; ++c) {
+            const int j = col + 16 * c;
+            if (r < n && r == j && r >= n - 2) d[r] = a[s][c];
+            if (r == n - 1 && j == n - 2) e[j] = a[s][c];
+        }
+    }
+    if (tid == 0) e[n - 1] = 0.0;
+    for (int j = n + tid; j < eig_pad(n); j += 512) d[j] = e[j] = 0.0;
+}
+
+// dynamic LDS above 64 KB has to be allowed; always the same `top`, so that threads with different
+// sizes do not lower it for each other
+static hipError_t lds_limit(const void* kernel, size_t bytes, size_t top) {
+    if (bytes <= 64 * 1024) return hipSuccess;
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)std::max(bytes, top));
 }
 
 hipError_t householder_tridiag(int n, EigWork& w, hipStream_t st) {
     if (n < 3) return hipErrorInvalidValue;   // the callers solve n <= 2 in closed form
     // reflector rows must be zero outside their support for the blocked back-transform
     UNO_LAUNCH_FILL((long)n * n, w.V, st);
+    if (n <= kHhOneN) {
+        hipLaunchKernelGGL(k_hh_one, dim3(1), dim3(512), 0, st, n, (const double*)w.A, w.V, w.tau, w.d, w.e);
+        return hipGetLastError();
+    }
     // the inverse-iteration work space is unused until the tridiagonal is done: p and the
-    // partial sums of the steps of even and odd k live there
+    // rows' terms of p.v of the steps of even and odd k live there
     double* P[2] = {w.wk, w.wk + n};
     double* part[2] = {w.wk + 2L * n, w.wk + 3L * n};
     const size_t lds = 3 * (size_t)n * sizeof(double);
-    static size_t attr = 0;
-    if (lds > attr) {
-        hipError_t er = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_hh_col),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (er != hipSuccess) return er;
-        attr = lds;
-    }
-    int nbp = 0;
+    if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_hh_col), lds, 150 * 1024)) return er;
     for (int k = 0; k + 2 < n; ++k) {
-        const int m = n - k - 1;
-        const int nb = (m + 3) / 4;
-        hipLaunchKernelGGL(k_hh_col, dim3((unsigned)nb), dim3(256), lds, st, n, k, w.A, w.V, w.tau, w.d, w.e,
-                           P[(k + 1) & 1], part[(k + 1) & 1], nbp, P[k & 1], part[k & 1]);
-        nbp = nb;
+        const int b0 = (k + 1) / 32 * 8;
+        hipLaunchKernelGGL(k_hh_col, dim3((unsigned)((n + 3) / 4 - b0)), dim3(256), lds, st, n, k, b0, w.A, w.V, w.tau, w.d, w.e,
+                           P[(k + 1) & 1], part[(k + 1) & 1], P[k & 1], part[k & 1]);
     }
-    hipLaunchKernelGGL(k_hh_tail, dim3(1), dim3(256), 0, st, n, w.A, w.V, w.tau, P[(n - 3) & 1], part[(n - 3) & 1], nbp,
-                       w.d, w.e);
+    hipLaunchKernelGGL(k_hh_tail, dim3(1), dim3(64), 0, st, n, w.A, w.V, w.tau, P[(n - 3) & 1], part[(n - 3) & 1], w.d,
+                       w.e);
     return hipGetLastError();
 }
 
@@ -827,12 +991,51 @@ __global__ __launch_bounds__(256) void k_wy_m(int n, int nref, const double* __r
     }
 }
 
+// The reflectors applied one by one, a wave per column of Z with the column in registers and the
+// next reflectors' rows read ahead: for n <= kHhOneN the whole back-transform is one launch of
+// n - 2 steps of a few hundred cycles.  n = 133: 33 us (57 us for the blocks' T and 11 us for each of
+// their ten GEMMs before).
+__global__ __launch_bounds__(64) void k_apply_q_one(int n, const double* __restrict__ V, const double* __restrict__ tau,
+                                                    double* __restrict__ Z) {
+    constexpr int C = kHhOneN / 64, kAhead = 4;
+    const int i = blockIdx.x, lane = threadIdx.x;
+    double z[C], v[kAhead][C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) z[c] = lane + 64 * c < n ? Z[(long)(lane + 64 * c) * n + i] : 0.0;
+    auto read = [&](int k, double* r) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) r[c] = (k >= 0 && lane + 64 * c < n) ? V[(long)k * n + lane + 64 * c] : 0.0;
+    };
+    const int k1 = n - 3;
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) read(k1 - q, v[q]);
+    for (int k = k1; k >= 0; k -= kAhead) {
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) {
+            double s = 0.0;
+#pragma unroll
+            for (int c = 0; c < C; ++c) s = fma(v[q][c], z[c], s);
+            s = wave_total(s) * (k >= q ? tau[max(k - q, 0)] : 0.0);
+#pragma unroll
+            for (int c = 0; c < C; ++c) z[c] = fma(-s, v[q][c], z[c]);
+            read(k - q - kAhead, v[q]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        if (lane + 64 * c < n) Z[(long)(lane + 64 * c) * n + i] = z[c];
+}
+
 hipError_t apply_q(int n, EigWork& w, double* Z, hipStream_t st) {
     const int nref = n - 2;
     if (nref <= 0) return hipSuccess;
+    if (n <= kHhOneN) {
+        hipLaunchKernelGGL(k_apply_q_one, dim3((unsigned)n), dim3(64), 0, st, n, (const double*)w.V, (const double*)w.tau, Z);
+        return hipGetLastError();
+    }
     const int nblk = (nref + kWy - 1) / kWy;
-    double* M = w.wk;              // nblk * kWy rows of n (within the 5 n^2 work space)
-    double* wy = w.wk + 2L * n * n;  // kWy x n
+    double* M = w.wk;                      // nref x n
+    double* wy = w.wk + (long)nref * n;    // at most kWy x n
     hipLaunchKernelGGL(k_wy_m, dim3((unsigned)nblk), dim3(256), 0, st, n, nref, w.V, w.tau, M);
     for (int b = nblk - 1; b >= 0; --b) {
         const int k0 = b * kWy, nb = std::min(kWy, nref - k0);
@@ -851,13 +1054,23 @@ hipError_t apply_q(int n, EigWork& w, double* Z, hipStream_t st) {
 // the search starts from the Gershgorin interval and stops at the same width as plain
 // bisection would (2 eps max|end| + 4 pivmin).
 // ---------------------------------------------------------------------------
+// 1/a to rounding from the hardware estimate and two Newton steps; 1e-300 <= |a|, finite (0 where 1/a is subnormal)
+__device__ __forceinline__ double recip(double a) {
+    double r = __builtin_amdgcn_rcp(a);
+    r = fma(fma(-a, r, 1.0), r, r);
+    return fma(fma(-a, r, 1.0), r, r);
+}
+
+// (the loop is one chain of dependent operations: the quotient is a reciprocal and a product, half
+// the length of a divide: 0.83 ms instead of 1.19 at n = 1216.  |q| stays between pivmin >= 1e-300 and 1 / 2.2e-308, which recip takes)
 __device__ __forceinline__ int sturm_count(int n, const double* d, const double* e2, double x, double pivmin) {
     int c = 0;
     double q = d[0] - x;
     if (fabs(q) < pivmin) q = -pivmin;
     if (q < 0.0) ++c;
+#pragma unroll 8
     for (int k = 1; k < n; ++k) {
-        q = d[k] - x - e2[k - 1] / q;
+        q = fma(-e2[k - 1], recip(q), d[k] - x);
         if (fabs(q) < pivmin) q = -pivmin;
         if (q < 0.0) ++c;
     }
@@ -1049,6 +1262,149 @@ __global__ __launch_bounds__(64) void k_inviter(int n, const double* __restrict_
     }
 }
 
+// The same solves with every work array in LDS, `lanes` eigenvectors per one-wave block: the factors'
+// reciprocal pivots and multipliers and the vector itself.  A row interchange is one bit; the
+// superdiagonals of U follow from d, e, the bits and the multipliers.  The solves are chains of
+// dependent operations, so rows go in
+// chunks of 16, padded with rows that do nothing (d and e are padded with zeros), whose operands
+// are read ahead of the chain, without branches; the scaling of one solve is done by the next
+// one's loads.  T - lam is scaled by a power of two to norm 1, which keeps every pivot
+// within the range of recip.  n = 1216: 0.63 ms, n = 133: 79 us (with the arrays in global memory and
+// divides: 2.07 ms and 237 us).
+constexpr size_t kInvLds = 156 * 1024;
+static size_t inviter_bytes(int n) {   // LDS of one eigenvector
+    const size_t np = eig_pad(n);
+    return (3 * np + 1) * sizeof(double) + (np / kEigChunk + 1) / 2 * sizeof(double);
+}
+__global__ __launch_bounds__(64) void k_inviter_lds(int n, int lanes, const double* __restrict__ d,
+                                                    const double* __restrict__ e, const double* __restrict__ evals,
+                                                    double* __restrict__ Yt) {
+    extern __shared__ double lds[];
+    constexpr int kCh = kEigChunk;
+    const int S = lanes, t = threadIdx.x, i = blockIdx.x * lanes + t, np = eig_pad(n);
+    double tnorm = 0.0;
+    for (int k = t; k < n; k += 64)
+        tnorm = fmax(tnorm, fabs(d[k]) + (k + 1 < n ? fabs(e[k]) : 0.0) + (k > 0 ? fabs(e[k - 1]) : 0.0));
+    tnorm = wave_max(tnorm);
+    if (t >= lanes || i >= n) return;
+    double* U1 = lds + t;                      // [k S]: reciprocal of the diagonal of U
+    double* L = U1 + (long)np * S;             // multipliers
+    double* x = L + (long)np * S;              // np + 1 entries
+    unsigned* piv = reinterpret_cast<unsigned*>(lds + (3L * np + 1) * S) + t;   // [chunk S]
+    const double sc = tnorm > 0.0 ? ldexp(1.0, -max(ilogb(tnorm), -1000)) : 1.0;
+    const double lam = evals[i] * sc;
+    const double tiny = tnorm > 0.0 ? 2.2204460492503131e-16 * (tnorm * sc) : 2.2204460492503131e-16;
+    // factor T - lam I = P L U, row by row
+    double a = d[0] * sc - lam, b = e[0] * sc;
+    for (int k0 = 0; k0 < np; k0 += kCh) {
+        double ds[kCh], es[kCh + 1];
+        const bool last = k0 + kCh >= np;
+#pragma unroll
+        for (int c = 0; c < kCh; ++c) es[c] = e[k0 + c] * sc;
+#pragma unroll
+        for (int c = 0; c + 1 < kCh; ++c) ds[c] = d[k0 + c + 1] * sc - lam;
+        es[kCh] = last ? 0.0 : e[last ? 0 : k0 + kCh] * sc;
+        ds[kCh - 1] = last ? 0.0 : d[last ? 0 : k0 + kCh] * sc - lam;
+        unsigned bits = 0;
+        double u1[kCh], ls[kCh];
+#pragma unroll
+        for (int c = 0; c < kCh; ++c) {
+            const double sub = es[c];
+            const bool swap = !(fabs(a) >= fabs(sub));
+            const double num = swap ? a : sub, u = swap ? sub : a;
+            const double p = fabs(u) < tiny ? copysign(tiny, u) : u;
+            const double rp = recip(p);
+            double l = num * rp;
+            l = fma(fma(-l, p, num), rp, l);
+            const double up = swap ? ds[c] : b, dn = swap ? b : ds[c], en = es[c + 1];
+            a = dn - l * up;
+            b = swap ? -l * en : en;
+            u1[c] = rp;
+            ls[c] = l;
+            bits |= swap ? 1u << c : 0u;
+        }
+        if (last) {   // the rows from n on do nothing, and row n - 1 has no successor
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) {
+                if (k0 + c >= n) u1[c] = 0.0;
+                if (k0 + c >= n - 1) ls[c] = 0.0;
+            }
+            bits &= (1u << (n - 1 - k0)) - 1;
+        }
+#pragma unroll
+        for (int c = 0; c < kCh; ++c) {
+            U1[(k0 + c) * S] = u1[c];
+            L[(k0 + c) * S] = ls[c];
+        }
+        piv[k0 / kCh * S] = bits;
+    }
+    // start vector
+    unsigned int h = 2654435761u * (unsigned)(i + 1);
+    for (int k = 0; k < n; ++k) {
+        h ^= h << 13; h ^= h >> 17; h ^= h << 5;
+        x[k * S] = ((double)(h & 0xffffff) / 16777216.0) - 0.5 + 1e-3;
+    }
+    for (int k = n; k <= np; ++k) x[k * S] = 0.0;
+    double nrm = 1.0;
+    for (int it = 0; it < 3; ++it) {
+        // forward: apply the row interchanges and multipliers
+        double xk = x[0] * nrm;
+        for (int k0 = 0; k0 < np; k0 += kCh) {
+            double xs[kCh], ls[kCh];
+            const unsigned bits = piv[k0 / kCh * S];
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) {
+                xs[c] = x[(k0 + c + 1) * S] * nrm;
+                ls[c] = L[(k0 + c) * S];
+            }
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) {
+                const bool swap = bits >> c & 1;
+                const double xn = xs[c], hi = swap ? xk : xn, lo = swap ? xn : xk;
+                xs[c] = lo;
+                xk = hi - ls[c] * lo;
+            }
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) x[(k0 + c) * S] = xs[c];
+        }
+        // back substitution with the banded U, then the norm
+        double x1 = 0.0, x2 = 0.0, s2 = 0.0;
+        for (int k0 = np - kCh; k0 >= 0; k0 -= kCh) {
+            double xs[kCh], u1[kCh], u2[kCh], u3[kCh];
+            // bit c + 1: row k0 + c was interchanged; bit 0: the row before the chunk
+            const int before = k0 ? 1 : 0;
+            const unsigned bits = piv[k0 / kCh * S] << 1 | before * (piv[(k0 / kCh - before) * S] >> (kCh - 1));
+            double lp = L[(k0 - before) * S];
+            const bool last = k0 + kCh >= np;
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) {
+                xs[c] = x[(k0 + c) * S];
+                u1[c] = U1[(k0 + c) * S];
+                const int k1 = last && c + 1 == kCh ? 0 : k0 + c + 1;   // past the end: not used
+                const double dn = d[k1] * sc - lam, ec = e[k0 + c] * sc, en = last && c + 1 == kCh ? 0.0 : e[k1] * sc;
+                const double ub = (bits >> c & 1) ? -lp * ec : ec;
+                const bool swap = bits >> (c + 1) & 1;
+                u2[c] = swap ? dn : ub;
+                u3[c] = swap ? en : 0.0;
+                lp = L[(k0 + c) * S];
+            }
+#pragma unroll
+            for (int c = kCh - 1; c >= 0; --c) {
+                const double v = ((xs[c] - u2[c] * x1) - u3[c] * x2) * u1[c];
+                xs[c] = v;
+                s2 = fma(v, v, s2);
+                x2 = x1;
+                x1 = v;
+            }
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) x[(k0 + c) * S] = xs[c];
+        }
+        nrm = 1.0 / sqrt(s2);
+    }
+#pragma unroll 8
+    for (int k = 0; k < n; ++k) Yt[(long)k * n + i] = x[k * S] * nrm;
+}
+
 // modified Gram-Schmidt (two passes) inside each cluster of close eigenvalues (columns
 // of Yt): clusters[2c], clusters[2c+1] = first and one-past-last index; one block per
 // cluster
@@ -1089,13 +1445,32 @@ __global__ __launch_bounds__(256) void k_cluster_mgs(int n, const int* __restric
     }
 }
 
+// doubles of EigWork::wk that a solve of this size uses: p and p.v of the column launches, the
+// blocked back-transform's rows, and the factors of the inverse iteration where LDS does not
+// hold one vector's (at most 5 n^2 for every n >= 3)
+size_t eig_work_doubles(int n) {
+    const size_t sq = (size_t)n * n, wy = sq + (size_t)std::min(kWy, n) * n;
+    return inviter_bytes(n) <= kInvLds ? std::max(wy, 4 * (size_t)n) : 5 * sq;
+}
+
 hipError_t tridiag_eigen(int n, EigWork& w, int nclusters, const int* clusters, hipStream_t st) {
     if (nclusters < 0) {
         const size_t lds = 2 * (size_t)n * sizeof(double);
         hipLaunchKernelGGL(k_bisect, dim3((unsigned)((n + 3) / 4)), dim3(256), lds, st, n, w.d, w.e, w.evals);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_inviter, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, n, w.d, w.e, w.evals, w.Y, w.wk);
+    // as many eigenvectors per block as LDS holds, but no fewer blocks than compute units; sizes
+    // whose one vector does not fit use the work space in global memory
+    const int fit = (int)std::min<size_t>(64, kInvLds / inviter_bytes(n));
+    if (fit >= 1) {
+        const int lanes = std::max(1, std::min(fit, (n + 255) / 256));
+        const size_t lds = (size_t)lanes * inviter_bytes(n);
+        if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_inviter_lds), lds, kInvLds)) return er;
+        hipLaunchKernelGGL(k_inviter_lds, dim3((unsigned)((n + lanes - 1) / lanes)), dim3(64), lds, st, n, lanes,
+                           (const double*)w.d, (const double*)w.e, (const double*)w.evals, w.Y);
+    } else {
+        hipLaunchKernelGGL(k_inviter, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, n, w.d, w.e, w.evals, w.Y, w.wk);
+    }
     if (nclusters > 0) hipLaunchKernelGGL(k_cluster_mgs, dim3((unsigned)nclusters), dim3(256), 0, st, n, clusters, w.Y);
     return hipGetLastError();
 }

@@ -1,14 +1,14 @@
 // Dense symmetric eigensolver for device-resident matrices (contract of the
 // reference's SymmPack::rsp, SymmPack.cpp:272-288: eigenvalues ascending, eigenvectors
 // in the columns of a row-major Z).  All steps run on the GPU:
-//   1. Householder tridiagonalisation A = Q T Q^T (one reflector per column, one launch
+//   1. Householder tridiagonalisation A = Q T Q^T (one block up to n = 192, above it one launch
 //      per column: the previous rank-2 update fused with the next matrix-vector product);
 //   2. eigenvalues of T by multisection on Sturm counts, one eigenvalue per wave;
 //   3. eigenvectors of T by inverse iteration, one per thread (the vectors stored as the
 //      columns of Yt, so a wave's accesses coalesce), then two-pass modified Gram-Schmidt
 //      inside clusters of close eigenvalues (exact degeneracies included);
-//   4. Z = Q Yt: the reflectors applied to Yt in compact-WY blocks of 32 (every block's
-//      T Vb formed in one launch, then two MFMA GEMMs per block).
+//   4. Z = Q Yt: the reflectors applied to Yt one by one up to n = 192, above it in compact-WY
+//      blocks of 32 (every block's T Vb formed in one launch, then two MFMA GEMMs per block).
 // The reference reduces with Householder and diagonalises T with implicit QL
 // (SymmPack.cpp:67-269); the contract (not the steps) is what the callers rely on.
 #include <algorithm>
@@ -24,23 +24,40 @@ struct EigBufs {
     int* clusters;
 };
 
+// the buffers of an n x n solve with `work` doubles of work space, each 256-byte aligned, from `ws`;
+// returns the doubles they take
+static size_t eig_layout(int n, size_t work, double* ws, EigBufs& b) {
+    const size_t sq = (size_t)n * n;
+    size_t off = 0;
+    auto take = [&](size_t count) {
+        double* p = ws ? ws + off : nullptr;
+        off += (count + 31) / 32 * 32;
+        return p;
+    };
+    b.V = take(sq);
+    b.Y = take(sq);
+    b.wk = take(work);
+    b.tau = take(n);
+    b.p = take(n);
+    b.d = take(n);
+    b.e = take(n);
+    b.evals = take(n);
+    b.scal = take(4);
+    b.clusters = reinterpret_cast<int*>(take(n / 2 + 1));
+    return off;
+}
+
+// one allocation, of what the solver's kernels for this size use
 struct EigenWS {
     int n = 0;
-    DBuf<double> V, tau, p, d, e, scal, evals, Y, wk;
-    DBuf<int> clusters;
+    DBuf<double> buf;
     std::vector<double> hev;
     std::vector<int> hcl;
     hipError_t ensure(int nn) {
-        if (nn <= n && V.p) return hipSuccess;
+        if (nn <= n && buf.p) return hipSuccess;
         n = nn;
-        const size_t sq = (size_t)nn * nn;
-        hipError_t r;
-        if ((r = V.alloc(sq)) || (r = tau.alloc(nn)) || (r = p.alloc(nn)) ||
-            (r = d.alloc(nn)) ||
-            (r = e.alloc(nn)) || (r = scal.alloc(4)) || (r = evals.alloc(nn)) || (r = Y.alloc(sq)) ||
-            (r = wk.alloc(5 * sq)) || (r = clusters.alloc(2 * (size_t)nn)))
-            return r;
-        return hipSuccess;
+        EigBufs b;
+        return buf.alloc(eig_layout(nn, eig_work_doubles(nn), nullptr, b));
     }
 };
 
@@ -106,7 +123,8 @@ static int eigh_impl(EigenWS& w, int n, double* dA, double* dZ, double* h_evals,
     UNO_HIP(w.ensure(n));
     w.hev.resize(std::max(n, 1));
     w.hcl.resize(std::max(n, 2));
-    const EigBufs b{w.V.p, w.tau.p, w.p.p, w.d.p, w.e.p, w.scal.p, w.evals.p, w.Y.p, w.wk.p, w.clusters.p};
+    EigBufs b;
+    eig_layout(n, eig_work_doubles(n), w.buf.p, b);
     return eigh_core(n, dA, dZ, h_evals, b, w.hev.data(), w.hcl.data(), st);
 }
 
@@ -123,24 +141,8 @@ size_t eigh_ws_doubles(int n) {
 
 int eigh_in_workspace(int n, double* dA, double* dZ, double* h_evals, double* ws, double* hev, int* hcl,
                       hipStream_t st) {
-    const size_t sq = (size_t)n * n;
-    size_t off = 0;
-    auto take = [&](size_t count) {
-        double* p = ws + off;
-        off += (count + 31) / 32 * 32;
-        return p;
-    };
     EigBufs b;
-    b.V = take(sq);
-    b.Y = take(sq);
-    b.wk = take(5 * sq);
-    b.tau = take(n);
-    b.p = take(n);
-    b.d = take(n);
-    b.e = take(n);
-    b.evals = take(n);
-    b.scal = take(4);
-    b.clusters = reinterpret_cast<int*>(take(n / 2 + 1));
+    const size_t off = eig_layout(n, 5 * (size_t)n * n, ws, b);
     if (off > eigh_ws_doubles(n)) {
         set_error("eigensolver work space layout exceeds its size");
         return UNO_EINVAL;
