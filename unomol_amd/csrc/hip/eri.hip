@@ -77,34 +77,86 @@ __device__ __forceinline__ void eri_block(const EriArgs& a, const PairHdr& P1, c
 // ---------------------------------------------------------------------------
 // one lane per shell quartet of an explicit list (block / Schwarz modes)
 // ---------------------------------------------------------------------------
-template <int LA, int LB, int LC, int LD, int MODE, typename T>
+template <int LA, int LB, int LC, int LD, typename T>
 __global__ __launch_bounds__(256) void k_eri_lane(const EriArgs a) {
-    using CI = ClassInfo<LA, LB, LC, LD>;
-    constexpr int NA = CI::NA, NB = CI::NB, NC = CI::NC, ND = CI::ND, NCOMP = CI::NCOMP;
+    constexpr int NCOMP = ClassInfo<LA, LB, LC, LD>::NCOMP;
     const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    static_assert(MODE == kDigestBlock || MODE == kDigestSchwarz, "Fock builds have kernels of their own");
     if (g >= a.nquart) return;
-    const int pab = a.explicit_q[g].x, pcd = a.explicit_q[g].y;
-    const PairHdr P1 = a.pairs[pab];
-    const PairHdr P2 = a.pairs[pcd];
+    const PairHdr P1 = a.pairs[a.explicit_q[g].x];
+    const PairHdr P2 = a.pairs[a.explicit_q[g].y];
     T e[NCOMP];
-    eri_block<LA, LB, LC, LD, T>(a, P1, P2, e, rys_table_of<CI::NR, T>(a.rys2_exact));
+    eri_block<LA, LB, LC, LD, T>(a, P1, P2, e, rys_table_of<ClassInfo<LA, LB, LC, LD>::NR, T>(a.rys2_exact));
     normalise_block<LA, LB, LC, LD, T>(e, (T)1);
-    if constexpr (MODE == kDigestBlock) {
 #pragma unroll
-        for (int c = 0; c < NCOMP; ++c) a.out[g * NCOMP + c] = (double)e[c];
-    } else if constexpr (MODE == kDigestSchwarz) {
-        double m = 0.0;
-#pragma unroll
-        for (int i = 0; i < NA; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                if constexpr (LA == LC && LB == LD) m = fmax(m, fabs((double)e[((i * NB + j) * NC + i) * ND + j]));
-            }
-        a.out[pab] = sqrt(m);
-    }
+    for (int c = 0; c < NCOMP; ++c) a.out[g * NCOMP + c] = (double)e[c];
 }
 
+// Schwarz bound of a pair: only the diagonal components (ij|ij), and each unordered pair of its
+// primitives once (a product pair and its exchange give the same diagonal).  Bound by its longest
+// chain, the 36 x 36 primitives of two first-row core shells, so kSchwarzLanes lanes share a pair's
+// primitive quartets: 32 waters (ss|ss) 15 us, (ps|ps) 14 us (a pair per lane, whole blocks:
+// 246 and 451 us).
+constexpr int kSchwarzLanes = 16;
+template <int LA, int LB>
+__global__ __launch_bounds__(256) void k_schwarz(const EriArgs a) {
+    using CI = ClassInfo<LA, LB, LA, LB>;
+    constexpr int NA = CI::NA, NB = CI::NB, NR = CI::NR;
+    const long long gt = (long long)blockIdx.x * 256 + threadIdx.x;
+    const long long g = gt / kSchwarzLanes;
+    const int sub = (int)(gt % kSchwarzLanes);
+    if (g >= a.nquart) return;   // the group's lanes together
+    const int pair = a.explicit_q[g].x;
+    const PairHdr P = a.pairs[pair];
+    const double* tab = rys_table_of<NR, double>(a.rys2_exact);
+    double e[NA * NB];
+#pragma unroll
+    for (int c = 0; c < NA * NB; ++c) e[c] = 0.0;
+    // row i, column j <= i of the primitive triangle, kSchwarzLanes entries at a time
+    int i = 0, j = sub;
+    for (;;) {
+        while (i < P.nprim && j > i) j -= ++i;
+        if (i >= P.nprim) break;
+        const PrimPair pp = a.prims[P.prim0 + i], qq = a.prims[P.prim0 + j];
+        const double p = pp.p, q = qq.p;
+        const double rt = rsqrt_nr(p + q), it = rt * rt;
+        const double pref = kTwoPi25 * pp.K * qq.K * pp.ip * qq.ip * rt * (i == j ? 1.0 : 2.0);
+        const double PQ[3] = {pp.P[0] - qq.P[0], pp.P[1] - qq.P[1], pp.P[2] - qq.P[2]};
+        const double x = p * q * it * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]);
+        double u[NR], w[NR];
+        rys_roots<NR, double>(x, u, w, tab);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const double fff = u[r] * it;
+            const double B00 = 0.5 * fff, B1 = (0.5 - B00 * q) * pp.ip, B1p = (0.5 - B00 * p) * qq.ip;
+            double I[3][CI::TBL];
+#pragma unroll
+            for (int ax = 0; ax < 3; ++ax)
+                axis_table<LA, LB, LA, LB, double>(pp.P[ax] - P.A[ax] - q * PQ[ax] * fff, qq.P[ax] - P.A[ax] + p * PQ[ax] * fff,
+                                                   B00, B1, B1p, P.AB[ax], P.AB[ax], I[ax]);
+            const double wr = w[r] * pref;
+#pragma unroll
+            for (int ca = 0; ca < NA; ++ca)
+#pragma unroll
+                for (int cb = 0; cb < NB; ++cb)
+                    e[ca * NB + cb] = fma(wr * I[0][CI::tix(ca, cb, ca, cb, 0)],
+                                          I[1][CI::tix(ca, cb, ca, cb, 1)] * I[2][CI::tix(ca, cb, ca, cb, 2)], e[ca * NB + cb]);
+        }
+        j += kSchwarzLanes;
+    }
+    double m = 0.0;
+#pragma unroll
+    for (int ca = 0; ca < NA; ++ca)
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) {
+            double v = e[ca * NB + cb];
+#pragma unroll
+            for (int o = 1; o < kSchwarzLanes; o <<= 1) v += __shfl_xor(v, o, kSchwarzLanes);
+            // each function's normalisation stands twice in (ij|ij)
+            const double nrm = cart_nrm(LA, ca) * cart_nrm(LB, cb);
+            m = fmax(m, fabs(v * (nrm * nrm)));
+        }
+    if (sub == 0) a.out[pair] = sqrt(m);
+}
 
 // one quartet of an explicit list per wave (classes of more than kLaneMaxComp components)
 template <int LA, int LB, int LC, int LD, int MODE, typename T>
@@ -120,11 +172,13 @@ __global__ __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>())) void k_eri_
         wave_eri<LA, LB, LC, LD, T>(P1, P2, a.prims, a.primcut, a.rys2_exact, (T)1, sE);
         if constexpr (MODE == kDigestBlock) {
             for (int c = lane; c < NCOMP; c += 64) a.out[g * NCOMP + c] = (double)sE[c];
-        } else if (lane == 0) {
-            double m = 0.0;
-            for (int i = 0; i < NA; ++i)
-                for (int j = 0; j < NB; ++j) m = fmax(m, fabs((double)sE[((i * NB + j) * NC + i) * ND + j]));
-            a.out[q.x] = sqrt(m);
+        } else {
+            static_assert(NA * NB <= 64, "one diagonal component per lane");
+            const int i = lane / NB, j = lane - i * NB;
+            double m = lane < NA * NB ? fabs((double)sE[((i * NB + j) * NC + i) * ND + j]) : 0.0;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) m = fmax(m, __shfl_xor(m, o, 64));
+            if (lane == 0) a.out[q.x] = sqrt(m);
         }
         __syncthreads();
     }
@@ -133,43 +187,50 @@ __global__ __launch_bounds__(64, (wave_min_waves<LA, LB, LC, LD>())) void k_eri_
 // ---------------------------------------------------------------------------
 // launchers of the explicit lists: dispatch on the class and mode
 // ---------------------------------------------------------------------------
-// quartets per block: one per lane, or for the wave kernel 8
-static constexpr int quartets_per_block(int ncomp) { return ncomp <= kLaneMaxComp ? 256 : 8; }
-
-template <int LA, int LB, int LC, int LD, int MODE, typename T = double>
-static hipError_t launch_cls(const EriArgs& a, hipStream_t st) {
-    using CI = ClassInfo<LA, LB, LC, LD>;
+// blocks: a quartet per lane; per wave 8 quartets in turn, or one where only a bound is wanted (a list
+// of pairs, not of quartets)
+template <int LA, int LB, int LC, int LD>
+static hipError_t launch_block(const EriArgs& a, hipStream_t st) {
     if (a.nquart <= 0) return hipSuccess;
     EriArgs b = a;
-    b.qpb = quartets_per_block(CI::NCOMP);
-    const long long nb = (a.nquart + b.qpb - 1) / b.qpb;
-    if constexpr (CI::NCOMP <= kLaneMaxComp)
-        hipLaunchKernelGGL((k_eri_lane<LA, LB, LC, LD, MODE, T>), dim3((unsigned)nb), dim3(256), 0, st, b);
-    else
-        hipLaunchKernelGGL((k_eri_wave<LA, LB, LC, LD, MODE, T>), dim3((unsigned)nb), dim3(64), 0, st, b);
+    constexpr bool lane = ClassInfo<LA, LB, LC, LD>::NCOMP <= kLaneMaxComp;
+    b.qpb = lane ? 256 : 8;
+    const unsigned nb = (unsigned)((a.nquart + b.qpb - 1) / b.qpb);
+    if constexpr (lane) hipLaunchKernelGGL((k_eri_lane<LA, LB, LC, LD, double>), dim3(nb), dim3(256), 0, st, b);
+    else hipLaunchKernelGGL((k_eri_wave<LA, LB, LC, LD, kDigestBlock, double>), dim3(nb), dim3(64), 0, st, b);
     return hipGetLastError();
 }
 
-template <int MODE, typename T>
-static hipError_t launch_mode(int cb, int ck, const EriArgs& a, hipStream_t st) {
-#define UNO_Q(X, Y, LA, LB, LC, LD) \
-    if (cb == X && ck == Y) return launch_cls<LA, LB, LC, LD, MODE, T>(a, st);
-    UNO_QUARTET_CLASSES(UNO_Q)
-#undef UNO_Q
-    return hipErrorInvalidValue;
+template <int LA, int LB>
+static hipError_t launch_schwarz(const EriArgs& a, hipStream_t st) {
+    if (a.nquart <= 0) return hipSuccess;
+    EriArgs b = a;
+    b.qpb = 1;
+    if constexpr (ClassInfo<LA, LB, LA, LB>::NCOMP <= kLaneMaxComp) {
+        const unsigned nb = (unsigned)((a.nquart * kSchwarzLanes + 255) / 256);
+        hipLaunchKernelGGL((k_schwarz<LA, LB>), dim3(nb), dim3(256), 0, st, b);
+    } else {
+        hipLaunchKernelGGL((k_eri_wave<LA, LB, LA, LB, kDigestSchwarz, double>), dim3((unsigned)a.nquart), dim3(64), 0, st, b);
+    }
+    return hipGetLastError();
 }
 
 hipError_t eri_launch(int mode, int cb, int ck, const EriArgs& a, hipStream_t st) {
-    if (mode == kDigestBlock) return launch_mode<kDigestBlock, double>(cb, ck, a, st);
+    if (mode == kDigestBlock) {
+#define UNO_Q(X, Y, LA, LB, LC, LD) \
+    if (cb == X && ck == Y) return launch_block<LA, LB, LC, LD>(a, st);
+        UNO_QUARTET_CLASSES(UNO_Q)
+#undef UNO_Q
+    }
     // Schwarz: diagonal classes only
     if (mode != kDigestSchwarz || cb != ck) return hipErrorInvalidValue;
     switch (cb) {
-        case 0: return launch_cls<0, 0, 0, 0, kDigestSchwarz>(a, st);
-        case 1: return launch_cls<1, 0, 1, 0, kDigestSchwarz>(a, st);
-        case 2: return launch_cls<1, 1, 1, 1, kDigestSchwarz>(a, st);
-        case 3: return launch_cls<2, 0, 2, 0, kDigestSchwarz>(a, st);
-        case 4: return launch_cls<2, 1, 2, 1, kDigestSchwarz>(a, st);
-        case 5: return launch_cls<2, 2, 2, 2, kDigestSchwarz>(a, st);
+        case 0: return launch_schwarz<0, 0>(a, st);
+        case 1: return launch_schwarz<1, 0>(a, st);
+        case 2: return launch_schwarz<1, 1>(a, st);
+        case 3: return launch_schwarz<2, 0>(a, st);
+        case 4: return launch_schwarz<2, 1>(a, st);
+        case 5: return launch_schwarz<2, 2>(a, st);
     }
     return hipErrorInvalidValue;
 }

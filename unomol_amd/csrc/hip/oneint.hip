@@ -1,5 +1,5 @@
 // One-electron matrices on the GPU: overlap S, kinetic T and core Hamiltonian H = T + V,
-// one lane per shell pair, specialised per (la, lb) with la >= lb.
+// one wave per shell pair, specialised per (la, lb) with la >= lb.
 //
 // Same method and arithmetic as the host code (McMurchie-Davidson Hermite expansion,
 // the reference's OneElectronInts.cpp:6-124 and MD_Dfunction.hpp:39-72): per primitive
@@ -32,22 +32,36 @@ __host__ __device__ constexpr double cnorm(int l, int k) {
     return (cpow(l, k, 0) == 2 || cpow(l, k, 1) == 2 || cpow(l, k, 2) == 2) ? 0.57735026918962576451 : 1.0;
 }
 
-__device__ void boys_ref(double* f, double t, int m) {
+// 1 / (m + 1/2 + i), i = 1 .. 200: the series' divides, which were most of its time
+template <int M>
+struct BoysRecip {
+    double r[200];
+    constexpr BoysRecip() : r{} {
+        for (int i = 0; i < 200; ++i) r[i] = 1.0 / (M + 1.5 + i);
+    }
+};
+template <int M>
+__device__ const BoysRecip<M> kBoysRecip{};
+
+template <int M>
+__device__ void boys_ref(double* f, double t) {
     if (t > 20.0) {
+        const double rt = 1.0 / t;
         f[0] = 0.88622692545275801365 / sqrt(t);
-        for (int i = 1; i <= m; ++i) f[i] = f[i - 1] * (i - 0.5) / t;
+#pragma unroll
+        for (int i = 1; i <= M; ++i) f[i] = f[i - 1] * (i - 0.5) * rt;
         return;
     }
-    const double mh = m + 0.5;
-    double term = 0.5 / mh, s = term;
-    for (int i = 1; i <= 200; ++i) {
-        term *= t / (mh + i);
+    double term = 0.5 / (M + 0.5), s = term;
+    for (int i = 0; i < 200; ++i) {
+        term *= t * kBoysRecip<M>.r[i];
         s += term;
         if (term < 1e-12) break;
     }
     const double et = exp(-t);
-    f[m] = s * et;
-    for (int i = m - 1; i >= 0; --i) f[i] = (2.0 * t * f[i + 1] + et) / (2.0 * i + 1.0);
+    f[M] = s * et;
+#pragma unroll
+    for (int i = M - 1; i >= 0; --i) f[i] = (2.0 * t * f[i + 1] + et) * (1.0 / (2.0 * i + 1.0));
 }
 
 // E^{ij}_t, i <= I, j <= J, t <= i + j
@@ -79,18 +93,20 @@ struct Herm {
     }
 };
 
-// lanes per shell pair: each sums the nuclear attraction over every kOiSplit-th centre,
-// the partial sums then reduced over the group in a fixed order (the centre loop is the
-// kernel's work; one lane per pair left most of the GPU idle)
-constexpr int kOiSplit = 8;
+// A wave per shell pair, its lanes sharing the pair's work, primitive pairs times nuclei: `np` (a
+// power of two) lanes step over the primitive pairs and 64 / np over the nuclei, whichever np
+// makes the lanes' longest share shortest; the partial sums are then reduced over the wave in
+// a fixed order.  Bound by the Boys series (14 million of them at 32 waters, (s|s) 184 us;
+// 8 lanes per pair over the nuclei only, one division per term of the series: 394 us, and with
+// 8 lanes sharing both: 296 us, the chain of two core shells' 36 primitive pairs).
+// kOiHerm: what a primitive pair's Hermite coefficients cost, in nuclei.
+constexpr int kOiHerm = 3;
 
 template <int LA, int LB>
 __global__ __launch_bounds__(128) void k_oneint(int npair, const int2* __restrict__ pairs, OneIntArgs a) {
-    constexpr int NA = nc1(LA), NB = nc1(LB), L = LA + LB;
-    const long gt = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    // groups of kOiSplit consecutive lanes: a group is wholly in or out of range
-    const int g = (int)(gt / kOiSplit), sub = (int)(gt % kOiSplit);
-    if (g >= npair) return;
+    constexpr int NA = nc1(LA), NB = nc1(LB), L = LA + LB, G = 64;
+    const int g = blockIdx.x * 2 + (threadIdx.x >> 6), sub = threadIdx.x & 63;
+    if (g >= npair) return;   // whole wave
     const int sa = pairs[g].x, sb = pairs[g].y;
     const OneIntShell A = a.shells[sa], B = a.shells[sb];
     const double* ra = a.xyz + 3 * A.cen;
@@ -100,100 +116,115 @@ __global__ __launch_bounds__(128) void k_oneint(int npair, const int2* __restric
     double s[NA * NB], t[NA * NB], v[NA * NB];
 #pragma unroll
     for (int o = 0; o < NA * NB; ++o) s[o] = t[o] = v[o] = 0.0;
-    for (int i = 0; i < A.npr; ++i)
-        for (int j = 0; j < B.npr; ++j) {
-            const double ea = a.alpha[A.poff + i], eb = a.alpha[B.poff + j];
-            const double p = ea + eb, ip = 1.0 / p;
-            const double K = exp(-ea * eb * ip * ab2);
-            double P[3];
+    const int nprim = A.npr * B.npr;
+    int lg = 0, best = 1 << 30;
 #pragma unroll
-            for (int x = 0; x < 3; ++x) P[x] = (ea * ra[x] + eb * rb[x]) * ip;
-            Herm<LA + 1, LB + 1> hx, hy, hz;
-            hx.build(0.5 * ip, P[0] - ra[0], P[0] - rb[0]);
-            hy.build(0.5 * ip, P[1] - ra[1], P[1] - rb[1]);
-            hz.build(0.5 * ip, P[2] - ra[2], P[2] - rb[2]);
-            const double s00 = pow(M_PI * ip, 1.5) * K;
-            const double cc = a.coef[A.poff + i] * a.coef[B.poff + j];
-            // V_tuv = -sum_c Z_c R_tuv(P - C), t + u + v <= L
-            double V[L + 1][L + 1][L + 1];
+    for (int k = 0; (1 << k) <= G; ++k) {
+        const int cost = ((nprim + (1 << k) - 1) >> k) * (kOiHerm + (a.ncen + (G >> k) - 1) / (G >> k));
+        if (cost < best) best = cost, lg = k;
+    }
+    const int c0 = sub >> lg, cstep = G >> lg;
+    for (int ij = sub & ((1 << lg) - 1); ij < nprim; ij += 1 << lg) {
+        const int i = ij / B.npr, j = ij - i * B.npr;
+        const double ea = a.alpha[A.poff + i], eb = a.alpha[B.poff + j];
+        const double p = ea + eb, ip = 1.0 / p;
+        const double K = exp(-ea * eb * ip * ab2);
+        double P[3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) P[x] = (ea * ra[x] + eb * rb[x]) * ip;
+        Herm<LA + 1, LB + 1> hx, hy, hz;
+        hx.build(0.5 * ip, P[0] - ra[0], P[0] - rb[0]);
+        hy.build(0.5 * ip, P[1] - ra[1], P[1] - rb[1]);
+        hz.build(0.5 * ip, P[2] - ra[2], P[2] - rb[2]);
+        const double s00 = M_PI * ip * sqrt(M_PI * ip) * K;
+        const double cc = a.coef[A.poff + i] * a.coef[B.poff + j];
+        // V_tuv = -sum_c Z_c R_tuv(P - C), t + u + v <= L
+        double V[L + 1][L + 1][L + 1];
+#pragma unroll
+        for (int x = 0; x <= L; ++x)
+#pragma unroll
+            for (int y = 0; y <= L; ++y)
+#pragma unroll
+                for (int z = 0; z <= L; ++z) V[x][y][z] = 0.0;
+        const double pref = 2.0 * M_PI * ip * K;
+        for (int c = c0; c < a.ncen; c += cstep) {
+            if (c == a.skip) continue;   // OneElectronInts.cpp:43
+            const double pc[3] = {P[0] - a.xyz[3 * c], P[1] - a.xyz[3 * c + 1], P[2] - a.xyz[3 * c + 2]};
+            double f[L + 1];
+            boys_ref<L>(f, p * (pc[0] * pc[0] + pc[1] * pc[1] + pc[2] * pc[2]));
+            double w[L + 1][L + 1][L + 1][L + 1];   // [n][t][u][v]
+            double mp = 1.0;
+#pragma unroll
+            for (int n = 0; n <= L; ++n) {
+                w[n][0][0][0] = pref * mp * f[n];
+                mp *= -2.0 * p;
+            }
+#pragma unroll
+            for (int n = L - 1; n >= 0; --n) {
+#pragma unroll
+                for (int tt = 0; tt <= L - n; ++tt)
+#pragma unroll
+                    for (int u = 0; u <= L - n - tt; ++u)
+#pragma unroll
+                        for (int vv = 0; vv <= L - n - tt - u; ++vv) {
+                            if (tt + u + vv == 0) continue;
+                            double r;
+                            if (tt) r = pc[0] * w[n + 1][tt - 1][u][vv] + (tt > 1 ? (tt - 1) * w[n + 1][tt - 2][u][vv] : 0.0);
+                            else if (u) r = pc[1] * w[n + 1][tt][u - 1][vv] + (u > 1 ? (u - 1) * w[n + 1][tt][u - 2][vv] : 0.0);
+                            else r = pc[2] * w[n + 1][tt][u][vv - 1] + (vv > 1 ? (vv - 1) * w[n + 1][tt][u][vv - 2] : 0.0);
+                            w[n][tt][u][vv] = r;
+                        }
+            }
+            const double zc = a.charge[c];
 #pragma unroll
             for (int x = 0; x <= L; ++x)
 #pragma unroll
-                for (int y = 0; y <= L; ++y)
+                for (int y = 0; y <= L - x; ++y)
 #pragma unroll
-                    for (int z = 0; z <= L; ++z) V[x][y][z] = 0.0;
-            const double pref = 2.0 * M_PI * ip * K;
-            for (int c = sub; c < a.ncen; c += kOiSplit) {
-                if (c == a.skip) continue;   // OneElectronInts.cpp:43
-                const double pc[3] = {P[0] - a.xyz[3 * c], P[1] - a.xyz[3 * c + 1], P[2] - a.xyz[3 * c + 2]};
-                double f[L + 1];
-                boys_ref(f, p * (pc[0] * pc[0] + pc[1] * pc[1] + pc[2] * pc[2]), L);
-                double w[L + 1][L + 1][L + 1][L + 1];   // [n][t][u][v]
-                double mp = 1.0;
-#pragma unroll
-                for (int n = 0; n <= L; ++n) {
-                    w[n][0][0][0] = pref * mp * f[n];
-                    mp *= -2.0 * p;
-                }
-#pragma unroll
-                for (int n = L - 1; n >= 0; --n) {
-#pragma unroll
-                    for (int tt = 0; tt <= L - n; ++tt)
-#pragma unroll
-                        for (int u = 0; u <= L - n - tt; ++u)
-#pragma unroll
-                            for (int vv = 0; vv <= L - n - tt - u; ++vv) {
-                                if (tt + u + vv == 0) continue;
-                                double r;
-                                if (tt) r = pc[0] * w[n + 1][tt - 1][u][vv] + (tt > 1 ? (tt - 1) * w[n + 1][tt - 2][u][vv] : 0.0);
-                                else if (u) r = pc[1] * w[n + 1][tt][u - 1][vv] + (u > 1 ? (u - 1) * w[n + 1][tt][u - 2][vv] : 0.0);
-                                else r = pc[2] * w[n + 1][tt][u][vv - 1] + (vv > 1 ? (vv - 1) * w[n + 1][tt][u][vv - 2] : 0.0);
-                                w[n][tt][u][vv] = r;
-                            }
-                }
-                const double zc = a.charge[c];
-#pragma unroll
-                for (int x = 0; x <= L; ++x)
-#pragma unroll
-                    for (int y = 0; y <= L - x; ++y)
-#pragma unroll
-                        for (int z = 0; z <= L - x - y; ++z) V[x][y][z] -= zc * w[0][x][y][z];
-            }
-#pragma unroll
-            for (int ia = 0; ia < NA; ++ia)
-#pragma unroll
-                for (int ib = 0; ib < NB; ++ib) {
-                    const int l1 = cpow(LA, ia, 0), m1 = cpow(LA, ia, 1), n1 = cpow(LA, ia, 2);
-                    const int l2 = cpow(LB, ib, 0), m2 = cpow(LB, ib, 1), n2 = cpow(LB, ib, 2);
-                    const double nf = cnorm(LA, ia) * cnorm(LB, ib) * cc;
-                    const double ex = hx.e[l1][l2][0], ey = hy.e[m1][m2][0], ez = hz.e[n1][n2][0];
-                    const int o = ia * NB + ib;
-                    s[o] += nf * s00 * ex * ey * ez;
-                    auto kin = [&](const Herm<LA + 1, LB + 1>& h, int k1, int k2) {
-                        double r = 2.0 * ea * eb * h.e[k1 + 1][k2 + 1][0];
-                        if (k1) r -= k1 * eb * h.e[k1 - 1][k2 + 1][0];
-                        if (k2) r -= k2 * ea * h.e[k1 + 1][k2 - 1][0];
-                        if (k1 && k2) r += 0.5 * k1 * k2 * h.e[k1 - 1][k2 - 1][0];
-                        return r;
-                    };
-                    t[o] += nf * s00 * (kin(hx, l1, l2) * ey * ez + kin(hy, m1, m2) * ex * ez + kin(hz, n1, n2) * ex * ey);
-                    double vs = 0.0;
-#pragma unroll
-                    for (int x = 0; x <= l1 + l2; ++x)
-#pragma unroll
-                        for (int y = 0; y <= m1 + m2; ++y) {
-                            const double exy = hx.e[l1][l2][x] * hy.e[m1][m2][y];
-#pragma unroll
-                            for (int z = 0; z <= n1 + n2; ++z) vs += exy * hz.e[n1][n2][z] * V[x][y][z];
-                        }
-                    v[o] += nf * vs;
-                }
+                    for (int z = 0; z <= L - x - y; ++z) V[x][y][z] -= zc * w[0][x][y][z];
         }
-    // the group's partial nuclear sums (every lane of the group holds the total after)
 #pragma unroll
-    for (int o = 0; o < NA * NB; ++o)
+        for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
-        for (int m = 1; m < kOiSplit; m <<= 1) v[o] += __shfl_xor(v[o], m, kOiSplit);
+            for (int ib = 0; ib < NB; ++ib) {
+                const int l1 = cpow(LA, ia, 0), m1 = cpow(LA, ia, 1), n1 = cpow(LA, ia, 2);
+                const int l2 = cpow(LB, ib, 0), m2 = cpow(LB, ib, 1), n2 = cpow(LB, ib, 2);
+                const double nf = cnorm(LA, ia) * cnorm(LB, ib) * cc;
+                const double ex = hx.e[l1][l2][0], ey = hy.e[m1][m2][0], ez = hz.e[n1][n2][0];
+                const int o = ia * NB + ib;
+                s[o] += nf * s00 * ex * ey * ez;
+                auto kin = [&](const Herm<LA + 1, LB + 1>& h, int k1, int k2) {
+                    double r = 2.0 * ea * eb * h.e[k1 + 1][k2 + 1][0];
+                    if (k1) r -= k1 * eb * h.e[k1 - 1][k2 + 1][0];
+                    if (k2) r -= k2 * ea * h.e[k1 + 1][k2 - 1][0];
+                    if (k1 && k2) r += 0.5 * k1 * k2 * h.e[k1 - 1][k2 - 1][0];
+                    return r;
+                };
+                t[o] += nf * s00 * (kin(hx, l1, l2) * ey * ez + kin(hy, m1, m2) * ex * ez + kin(hz, n1, n2) * ex * ey);
+                double vs = 0.0;
+#pragma unroll
+                for (int x = 0; x <= l1 + l2; ++x)
+#pragma unroll
+                    for (int y = 0; y <= m1 + m2; ++y) {
+                        const double exy = hx.e[l1][l2][x] * hy.e[m1][m2][y];
+#pragma unroll
+                        for (int z = 0; z <= n1 + n2; ++z) vs += exy * hz.e[n1][n2][z] * V[x][y][z];
+                    }
+                v[o] += nf * vs;
+            }
+    }
+    // the wave's partial sums (every lane holds the totals after); the lanes of one
+    // primitive pair have the same overlap and kinetic terms, which count once
+#pragma unroll
+    for (int o = 0; o < NA * NB; ++o) {
+        if (c0) s[o] = t[o] = 0.0;
+#pragma unroll
+        for (int m = 1; m < G; m <<= 1) {
+            s[o] += __shfl_xor(s[o], m, G);
+            t[o] += __shfl_xor(t[o], m, G);
+            v[o] += __shfl_xor(v[o], m, G);
+        }
+    }
     if (sub) return;
     const int n = a.n;
 #pragma unroll
@@ -215,7 +246,7 @@ __global__ __launch_bounds__(128) void k_oneint(int npair, const int2* __restric
 
 hipError_t oneint_launch(int la, int lb, int npair, const int2* pairs, const OneIntArgs& a, hipStream_t st) {
     if (npair <= 0) return hipSuccess;
-    const dim3 grid((unsigned)(((long)npair * kOiSplit + 127) / 128)), block(128);
+    const dim3 grid((unsigned)((npair + 1) / 2)), block(128);
 #define UNO_O(LA_, LB_)                                                                          \
     if (la == LA_ && lb == LB_) {                                                                \
         hipLaunchKernelGGL((k_oneint<LA_, LB_>), grid, block, 0, st, npair, pairs, a);           \

@@ -158,23 +158,28 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     UNO_HIP(dq.alloc(np));
     std::vector<int> pcls(np);
     for (int p = 0; p < np; ++p) pcls[p] = pair_class(B.sh[c->pairs[p].sh1].l, B.sh[c->pairs[p].sh2].l);
+    // the pairs class by class, one list and one launch per class
+    std::vector<int2> ql((size_t)np);
+    int q0[kNumPairClasses + 1] = {};
+    for (int p = 0; p < np; ++p) ++q0[pcls[p] + 1];
+    for (int X = 0; X < kNumPairClasses; ++X) q0[X + 1] += q0[X];
+    {
+        int at[kNumPairClasses];
+        std::copy(q0, q0 + kNumPairClasses, at);
+        for (int p = 0; p < np; ++p) ql[(size_t)at[pcls[p]]++] = make_int2(p, p);
+    }
+    DBuf<int2> dql;
+    UNO_HIP(dql.upload(ql.data(), ql.size(), st));
     for (int X = 0; X < kNumPairClasses; ++X) {
-        std::vector<int2> ql;
-        for (int p = 0; p < np; ++p)
-            if (pcls[p] == X) ql.push_back(make_int2(p, p));
-        if (ql.empty()) continue;
-        DBuf<int2> dql;
-        UNO_HIP(dql.upload(ql.data(), ql.size(), st));
         EriArgs a = base_args(c);
-        a.explicit_q = dql.p;
-        a.nquart = (long long)ql.size();
+        a.explicit_q = dql.p + q0[X];
+        a.nquart = q0[X + 1] - q0[X];
         a.out = dq.p;
         // bounds from the uncut integrals: with the primitive cut a pair of distant
         // tight primitives can lose its whole diagonal quartet while its quartets with
         // diffuse partners survive the cut, so a cut diagonal would under-bound them
         a.primcut = 0.0;
         UNO_HIP(eri_launch(kDigestSchwarz, X, X, a, st));
-        UNO_HIP(hipStreamSynchronize(st));
     }
     UNO_HIP(hipMemcpyAsync(c->pairQ.data(), dq.p, np * sizeof(double), hipMemcpyDeviceToHost, st));
     UNO_HIP(hipStreamSynchronize(st));
