@@ -1,5 +1,5 @@
 """GPU tests of the kernels that run once per geometry: Schwarz bounds whose lanes share a pair's
-primitives, and one-electron integrals whose wave shares primitives and nuclei."""
+primitives, and one-electron integrals whose lanes share primitives and nuclei."""
 import numpy as np
 import pytest
 
@@ -37,8 +37,8 @@ def test_schwarz_is_the_largest_diagonal(tmp_path, waters, basis):
     assert np.abs(q * q - ref).max() < 1e-11
 
 
-# fewer nuclei than lanes, more, and a ragged share
-@pytest.mark.parametrize("waters", [1, 5, 23])
+# fewer nuclei than lanes; one and several primitive pairs at a time
+@pytest.mark.parametrize("waters", [1, 7, 8, 23])
 def test_oneint_lane_shares(tmp_path, waters):
     """Against the host's integrals, with the bounds of the device integrals' other test scaled by
     the number of nuclei, whose terms are what is summed in another order."""

@@ -22,7 +22,9 @@ struct OneIntArgs {
 };
 
 // pairs (shell of angular momentum la, shell of lb), la >= lb <= 2; every element of the
-// three matrices belongs to exactly one pair's block or its transpose
-hipError_t oneint_launch(int la, int lb, int npair, const int2* pairs, const OneIntArgs& a, hipStream_t st);
+// three matrices belongs to exactly one pair's block or its transpose.  The first nmany pairs
+// are those of at least kOiMany primitive pairs
+constexpr int kOiMany = 4;
+hipError_t oneint_launch(int la, int lb, int npair, int nmany, const int2* pairs, const OneIntArgs& a, hipStream_t st);
 
 }  // namespace uno

@@ -39,6 +39,40 @@ EriArgs base_args(uno_ctx* c) {
     return a;
 }
 
+// order: the pairs by run key ascending, then bound descending, ties in their own order.  A
+// counting sort into the runs, then pieces of a run sorted by the threads and merged (64 waters,
+// 60 305 pairs: 0.6 ms; one stable sort of the indices through the two arrays: 4.2 ms).
+static void sort_runs(const std::vector<int>& runkey, const std::vector<double>& q, std::vector<int>& order) {
+    constexpr int kKeys = kNumPairClasses * kNumBuckets, kPiece = 2048;
+    const int np = (int)runkey.size();
+    std::vector<std::pair<double, int>> v(np);
+    int off[kKeys + 1] = {}, at[kKeys];
+    for (int p = 0; p < np; ++p) ++off[runkey[p] + 1];
+    for (int r = 0; r < kKeys; ++r) off[r + 1] += off[r];
+    std::copy(off, off + kKeys, at);
+    for (int p = 0; p < np; ++p) v[at[runkey[p]]++] = {-q[p], p};
+    std::vector<std::pair<int, int>> piece;
+    for (int r = 0; r < kKeys; ++r)
+        for (int lo = off[r]; lo < off[r + 1]; lo += kPiece) piece.emplace_back(lo, std::min(lo + kPiece, off[r + 1]));
+#pragma omp parallel for schedule(dynamic)
+    for (size_t k = 0; k < piece.size(); ++k) std::sort(v.begin() + piece[k].first, v.begin() + piece[k].second);
+    struct Merge {
+        int lo, mid, hi;
+    };
+    std::vector<Merge> merge;
+    for (long len = kPiece; len < np; len *= 2) {
+        merge.clear();
+        for (int r = 0; r < kKeys; ++r)
+            for (long lo = off[r]; lo + len < off[r + 1]; lo += 2 * len)
+                merge.push_back({(int)lo, (int)(lo + len), (int)std::min<long>(lo + 2 * len, off[r + 1])});
+#pragma omp parallel for schedule(dynamic)
+        for (size_t k = 0; k < merge.size(); ++k)
+            std::inplace_merge(v.begin() + merge[k].lo, v.begin() + merge[k].mid, v.begin() + merge[k].hi);
+    }
+#pragma omp parallel for schedule(static)
+    for (int p = 0; p < np; ++p) order[p] = v[p].second;
+}
+
 int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     using bclk = std::chrono::steady_clock;
     auto since = [](bclk::time_point t) { return std::chrono::duration<double, std::milli>(bclk::now() - t).count(); };
@@ -192,11 +226,7 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     std::vector<int> runkey(np);
     for (int p = 0; p < np; ++p) runkey[p] = pcls[p] * kNumBuckets + prim_bucket(c->pairs[p].nprim);
     std::vector<int> order(np);
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        if (runkey[x] != runkey[y]) return runkey[x] < runkey[y];
-        return c->pairQ[x] > c->pairQ[y];
-    });
+    sort_runs(runkey, c->pairQ, order);
     // new primitive offsets, in run order
     std::vector<int> nprim0(np);
     for (int k = 0, tp = 0; k < np; ++k) {
@@ -300,6 +330,19 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
         UNO_HIP(c->oi_charge.upload(B.q.data(), B.q.size(), st));
         for (int k = 0; k < kNumPairClasses; ++k) {
             c->oi_npair[k] = (int)pl[k].size();
+            // longest primitive loops first (a counting sort): a wave's pairs are alike, and the
+            // long ones start early
+            auto nprim = [&](const int2& p) { return B.sh[p.x].npr * B.sh[p.y].npr; };
+            std::vector<int> at;
+            for (const int2& p : pl[k]) {
+                if ((int)at.size() < nprim(p) + 2) at.resize(nprim(p) + 2);
+                ++at[nprim(p)];
+            }
+            for (int q = (int)at.size() - 2; q >= 0; --q) at[q] += at[q + 1];   // pairs of at least q
+            c->oi_many[k] = (int)at.size() > kOiMany ? at[kOiMany] : 0;
+            std::vector<int2> sorted(pl[k].size());
+            for (const int2& p : pl[k]) sorted[at[nprim(p) + 1]++] = p;
+            pl[k].swap(sorted);
             UNO_HIP(c->oi_pairs[k].upload(pl[k].data(), pl[k].size(), st));
         }
     }
@@ -333,7 +376,7 @@ int oneint_device(uno_ctx* c, double* S, double* T, double* H) {
     a.H = H;
     static const int kl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
     for (int k = 0; k < kNumPairClasses; ++k)
-        UNO_HIP(oneint_launch(kl[k][0], kl[k][1], c->oi_npair[k], c->oi_pairs[k].p, a, c->st));
+        UNO_HIP(oneint_launch(kl[k][0], kl[k][1], c->oi_npair[k], c->oi_many[k], c->oi_pairs[k].p, a, c->st));
     return UNO_OK;
 }
 

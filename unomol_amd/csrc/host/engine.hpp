@@ -222,7 +222,7 @@ struct uno_ctx {
     uno::DBuf<uno::OneIntShell> oi_shells;
     uno::DBuf<double> oi_alpha, oi_coef, oi_xyz, oi_charge;
     uno::DBuf<int2> oi_pairs[uno::kNumPairClasses];
-    int oi_npair[uno::kNumPairClasses] = {};
+    int oi_npair[uno::kNumPairClasses] = {}, oi_many[uno::kNumPairClasses] = {};
     ~uno_ctx();
 };
 
