@@ -1,9 +1,11 @@
 // Dense kernels of the batched SCF: many small molecules (N <= 256 functions each) whose
 // matrices live back to back in one store, row-major N_m x N_m at offset off[m].
 //
-//  * grouped GEMM: C_m = alpha op(A_m) op(B_m) + beta C_m for every molecule, one 32 x 32
-//    output tile per 256-thread block (2 x 2 outputs per thread, K through LDS in steps
-//    of 32); the host lists the (molecule, tile) pairs;
+// A launch takes the slots (molecule, spin) of both spins: everything an iteration launches is
+// described by one list of slots and one of their tiles, which change when a molecule stops.
+//
+//  * grouped GEMM: C_m = op(A_m) op(B_m) for every slot, one 32 x 32 output tile per
+//    256-thread block (2 x 2 outputs per thread, K through LDS in steps of 32);
 //  * batched Jacobi eigensolver: one block per molecule, cyclic sweeps in parallel
 //    (round-robin) order, each round applying N/2 disjoint rotations to rows, then
 //    columns, then the eigenvector columns; eigenvalues ascending with their vectors;
@@ -17,27 +19,31 @@ namespace uno {
 // ---------------------------------------------------------------------------
 // grouped GEMM
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_grouped_gemm(const GemmTile* __restrict__ tiles, const GemmGroup* __restrict__ groups,
-                                                      double alpha, double beta) {
+__global__ __launch_bounds__(256) void k_grouped_gemm(const GemmTile* __restrict__ tiles, const MatSlot* __restrict__ slots,
+                                                      int ta, int tb, int occ, Store As, Store Bs, Store Cs) {
     __shared__ double sA[32][33];
     __shared__ double sB[32][33];
     const GemmTile t = tiles[blockIdx.x];
-    const GemmGroup g = groups[t.group];
+    const MatSlot m = slots[t.slot];
+    const int n = m.n, kn = occ ? m.nocc : n;
+    const double* A = As.s[m.spin] + m.off;
+    const double* B = Bs.s[m.spin] + m.off;
+    double* C = Cs.s[m.spin] + m.off;
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;   // 16 x 16 threads, 2 x 2 outputs each
     const int i0 = t.ti * 32, j0 = t.tj * 32;
     double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-    for (int k0 = 0; k0 < g.k; k0 += 32) {
+    for (int k0 = 0; k0 < kn; k0 += 32) {
         for (int e = threadIdx.x; e < 32 * 32; e += 256) {
             const int r = e >> 5, c = e & 31;
             // op(A)[i][k], i = i0 + r, k = k0 + c
             const int i = i0 + r, k = k0 + c;
             double av = 0.0;
-            if (i < g.m && k < g.k) av = g.ta ? g.A[(long)k * g.lda + i] : g.A[(long)i * g.lda + k];
+            if (i < n && k < kn) av = ta ? A[k * n + i] : A[i * n + k];
             sA[r][c] = av;
             // op(B)[k][j], k = k0 + r, j = j0 + c
             const int kk = k0 + r, j = j0 + c;
             double bv = 0.0;
-            if (kk < g.k && j < g.n) bv = g.tb ? g.B[(long)j * g.ldb + kk] : g.B[(long)kk * g.ldb + j];
+            if (kk < kn && j < n) bv = tb ? B[j * n + kk] : B[kk * n + j];
             sB[r][c] = bv;
         }
         __syncthreads();
@@ -57,17 +63,14 @@ __global__ __launch_bounds__(256) void k_grouped_gemm(const GemmTile* __restrict
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             const int i = i0 + ty * 2 + a, j = j0 + tx * 2 + b;
-            if (i < g.m && j < g.n) {
-                double* c = g.C + (long)i * g.ldc + j;
-                *c = alpha * acc[a][b] + (beta != 0.0 ? beta * *c : 0.0);
-            }
+            if (i < n && j < n) C[i * n + j] = acc[a][b];
         }
 }
 
-hipError_t grouped_gemm(int ntiles, const GemmTile* tiles, const GemmGroup* groups, double alpha, double beta,
-                        hipStream_t st) {
+hipError_t grouped_gemm(int ntiles, const GemmTile* tiles, const MatSlot* slots, bool ta, bool tb, bool occ, Store A, Store B,
+                        Store C, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_grouped_gemm, dim3(ntiles), dim3(256), 0, st, tiles, groups, alpha, beta);
+    hipLaunchKernelGGL(k_grouped_gemm, dim3(ntiles), dim3(256), 0, st, tiles, slots, ta ? 1 : 0, tb ? 1 : 0, occ ? 1 : 0, A, B, C);
     return hipGetLastError();
 }
 
@@ -82,18 +85,24 @@ hipError_t grouped_gemm(int ntiles, const GemmTile* tiles, const GemmGroup* grou
 // relative test alone never settles next to zero diagonal entries, where rounding keeps
 // a_pq above it); sweeps stop when none is applied.
 constexpr int kJacobiThreads = 1024;
+// a rotation of (x, y); the roundings are spelled out because the vectors inside an exactly
+// degenerate level follow them, and both kernels have to pick the same
+__device__ __forceinline__ double turn_p(double c, double s, double x, double y) { return fma(c, x, -(s * y)); }
+__device__ __forceinline__ double turn_q(double c, double s, double x, double y) { return fma(s, x, c * y); }
 constexpr int kJacobiLdsN = 140;   // largest matrix of the LDS kernel below
-__global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMat* __restrict__ mats, int max_sweeps,
-                                                                   int* __restrict__ sweeps_out) {
+__global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const MatSlot* __restrict__ slots, Store As, Store Vs,
+                                                                   Store evals, Store Zs, int max_sweeps) {
     __shared__ double cs[128], sn[128];
     __shared__ int pp[128], qq[128];
     __shared__ int nrot;
     __shared__ double red[kJacobiThreads / 64];
-    const BatchMat M = mats[blockIdx.x];
+    const MatSlot M = slots[blockIdx.x];
     const int n = M.n;
     if (n <= kJacobiLdsN) return;   // the LDS kernel's
-    double* A = M.A;
-    double* V = M.V;
+    double* A = As.s[M.spin] + M.off;
+    double* V = Vs.s[M.spin] + M.off;
+    double* ev = evals.s[M.spin] + M.off;
+    double* Z = Zs.s[M.spin] + M.off;
     const int tid = threadIdx.x;
     double f2 = 0.0;
     for (long e = tid; e < (long)n * n; e += blockDim.x) {
@@ -145,8 +154,8 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMa
                 if (q >= n || sn[k] == 0.0) continue;
                 const double c = cs[k], s = sn[k];
                 const double ap = A[(long)p * n + j], aq = A[(long)q * n + j];
-                A[(long)p * n + j] = c * ap - s * aq;
-                A[(long)q * n + j] = s * ap + c * aq;
+                A[(long)p * n + j] = turn_p(c, s, ap, aq);
+                A[(long)q * n + j] = turn_q(c, s, ap, aq);
             }
             __syncthreads();
             // columns p, q of A and of V: A <- A J, V <- V J
@@ -156,11 +165,11 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMa
                 if (q >= n || sn[k] == 0.0) continue;
                 const double c = cs[k], s = sn[k];
                 const double ap = A[(long)i * n + p], aq = A[(long)i * n + q];
-                A[(long)i * n + p] = c * ap - s * aq;
-                A[(long)i * n + q] = s * ap + c * aq;
+                A[(long)i * n + p] = turn_p(c, s, ap, aq);
+                A[(long)i * n + q] = turn_q(c, s, ap, aq);
                 const double vp = V[(long)i * n + p], vq = V[(long)i * n + q];
-                V[(long)i * n + p] = c * vp - s * vq;
-                V[(long)i * n + q] = s * vp + c * vq;
+                V[(long)i * n + p] = turn_p(c, s, vp, vq);
+                V[(long)i * n + q] = turn_q(c, s, vp, vq);
             }
             __syncthreads();
         }
@@ -177,135 +186,215 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi(const BatchMa
             const double dj = A[(long)j * n + j];
             if (dj < di || (dj == di && j < i)) ++rank;
         }
-        M.evals[rank] = di;
-        for (int r = 0; r < n; ++r) M.Z[(long)r * n + rank] = V[(long)r * n + i];
+        ev[rank] = di;
+        for (int r = 0; r < n; ++r) Z[(long)r * n + rank] = V[(long)r * n + i];
     }
-    if (tid == 0 && sweeps_out) sweeps_out[blockIdx.x] = sweep;
 }
 
-// The same rotations in the same order with the matrix in LDS, for n <= kJacobiLdsN (157 KB of the
-// 160 at 140 functions): a round is two phases, the rotations and one pass that applies them
-// to both sides of every 2 x 2 block of the pairs (k, l), rows first, and to the eigenvectors: the
-// other kernel's arithmetic, so that the vectors it picks inside an exactly degenerate level (a
-// linear molecule's pi pairs) are the same.  The eigenvectors are kept transposed (the two vectors of a rotation are
-// rows), in LDS as well while both fit, else in V.  With the matrix in global memory every round
-// made three passes over it at L2 latency: 5.7 ms a launch for 32 molecules of up to 95 functions (mean
-// of an SCF, most of them warm), 1.0 ms here.
-__host__ __device__ constexpr int jacobi_ld(int n) { return n | 1; }   // odd: columns fall on different banks
-__host__ __device__ constexpr bool jacobi_v_fits(int n) { return 2 * n * jacobi_ld(n) <= kJacobiLdsN * jacobi_ld(kJacobiLdsN); }
-__global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const BatchMat* __restrict__ mats, int max_sweeps,
-                                                                       int* __restrict__ sweeps_out) {
+// The same rotations in the same order with the matrix in LDS, for n <= kJacobiLdsN (158 KB of the
+// 160 at 140 functions), in the other kernel's arithmetic, so that the vectors it picks inside an
+// exactly degenerate level (a linear molecule's pi pairs) are the same.  A round is one pass over
+// the matrix, which applies the rotations to both sides of every 2 x 2 block of the pairs (k, l),
+// rows first, and one phase in which two waves compute the next round's rotations (a chain of
+// divides and square roots) while the others turn the eigenvectors.  These are kept
+// transposed (the two vectors of a rotation are rows), in LDS as well while both fit, else in V.
+// Bound by latency: a wave reads what all its blocks need before it uses any of it, and a round
+// without rotations costs the test alone.  32 molecules of up to 114 functions, mean launch of an SCF
+// (most of them warm): 5.7 ms with the matrix in global memory, 1.35 here.
+// LDS of a matrix: padded to an even size with zeros (the dummy index of an odd n then needs no
+// exceptions), odd row strides so that columns fall on different banks
+__host__ __device__ constexpr int jacobi_a(int n) { return (n + (n & 1)) * (n + (n & 1) + 1); }
+__host__ __device__ constexpr int jacobi_v(int n) { return n * (n | 1); }
+constexpr int kJacobiLds = 19904;   // doubles a block may take (99 functions with their vectors: 19901)
+static_assert(jacobi_a(kJacobiLdsN) <= kJacobiLds, "the largest matrix fits");
+__host__ __device__ constexpr bool jacobi_v_fits(int n) { return jacobi_a(n) + jacobi_v(n) <= kJacobiLds; }
+__global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const MatSlot* __restrict__ slots, Store As, Store Vs,
+                                                                       Store evals, Store Zs, int max_sweeps) {
+    constexpr int kPairs = kJacobiLdsN / 2, kWaves = kJacobiThreads / 64;
+    constexpr int kRotWaves = (kPairs + 63) / 64;                             // waves of the rotations
+    constexpr int kPer = 3;                                                   // rows of blocks in flight
+    constexpr int kVPer = 5;                                                  // pairs of vectors in flight
     extern __shared__ double lds[];
-    __shared__ double cs[kJacobiLdsN / 2], sn[kJacobiLdsN / 2];
-    __shared__ int pp[kJacobiLdsN / 2], qq[kJacobiLdsN / 2];
-    __shared__ int nrot;
-    __shared__ double red[kJacobiThreads / 64];
-    const BatchMat M = mats[blockIdx.x];
-    const int n = M.n, ld = jacobi_ld(n);
+    // rotations of this round and the next: (c, s), the pair, and how many there are
+    __shared__ double2 rot[2][kPairs];
+    __shared__ int2 pq[2][kPairs];
+    __shared__ int nrot[2];
+    __shared__ double red[kWaves];
+    const MatSlot M = slots[blockIdx.x];
+    const int n = M.n;
     if (n > kJacobiLdsN) return;   // the other kernel's
+    const int m = n + (n & 1), mk = m / 2, ld = m + 1, lv = n | 1;
+    const double* A0 = As.s[M.spin] + M.off;
+    double* ev = evals.s[M.spin] + M.off;
+    double* Z = Zs.s[M.spin] + M.off;
     double* A = lds;
+    // component i of vector p in V[p ldv + i], in one of two address spaces: the accesses name theirs
     const bool vl = jacobi_v_fits(n);
-    double* V = vl ? lds + n * ld : M.V;   // V[p ldv + i] = component i of vector p
-    const int ldv = vl ? ld : n;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    typedef __attribute__((address_space(1))) double Global;
+    double* const VL = lds + jacobi_a(n);
+    Global* const VG = (Global*)(Vs.s[M.spin] + M.off);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double f2 = 0.0;
+    if (n & 1)
+        for (int e = tid; e < m; e += kJacobiThreads) A[e * ld + n] = A[n * ld + e] = 0.0;
     for (int e = tid; e < n * n; e += kJacobiThreads) {
         const int i = e / n, j = e - i * n;
-        const double v = M.A[e];
+        const double v = A0[e];
         A[i * ld + j] = v;
-        V[i * ldv + j] = i == j ? 1.0 : 0.0;
+        if (vl) VL[i * lv + j] = i == j ? 1.0 : 0.0;
+        else VG[e] = i == j ? 1.0 : 0.0;
         f2 = fma(v, v, f2);
     }
     for (int o = 32; o >= 1; o >>= 1) f2 += __shfl_xor(f2, o, 64);
     if ((tid & 63) == 0) red[tid >> 6] = f2;
+    if (tid < 2) nrot[tid] = 0;
     __syncthreads();
     double fro2 = 0.0;
-    for (int w = 0; w < kJacobiThreads / 64; ++w) fro2 += red[w];
+    for (int w = 0; w < kWaves; ++w) fro2 += red[w];
     const double abs_tol = 1e-15 * sqrt(fro2);
-    const int m = n + (n & 1), mk = m / 2;
-    int sweep = 0;
-    while (sweep < max_sweeps && n > 1) {
-        ++sweep;
-        if (tid == 0) nrot = 0;
-        __syncthreads();
-        for (int r = 0; r < m - 1; ++r) {
-            if (tid < mk) {
-                int a, b;
-                if (tid == 0) {
-                    a = m - 1;
-                    b = r;
-                } else {
-                    a = r + tid;
-                    if (a >= m - 1) a -= m - 1;
-                    b = r - tid;
-                    if (b < 0) b += m - 1;
+    // the rotations of round r into buffer d
+    auto rotations = [&](int r, int d) {
+        double c = 1.0, s = 0.0;
+        if (tid < mk) {
+            int a, b;
+            if (tid == 0) {
+                a = m - 1;
+                b = r;
+            } else {
+                a = r + tid;
+                if (a >= m - 1) a -= m - 1;
+                b = r - tid;
+                if (b < 0) b += m - 1;
+            }
+            const int p = a < b ? a : b, q = a < b ? b : a;
+            if (q < n) {
+                const double apq = A[p * ld + q];
+                const double app = A[p * ld + p], aqq = A[q * ld + q];
+                if (fabs(apq) > fmax(1.1102230246251565e-16 * sqrt(fabs(app * aqq)), abs_tol)) {
+                    const double theta = (aqq - app) / (2.0 * apq);
+                    const double t = fabs(theta) < 1e150
+                                         ? (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0))
+                                         : 0.5 / theta;
+                    c = 1.0 / sqrt(t * t + 1.0);
+                    s = t * c;
                 }
-                const int p = a < b ? a : b, q = a < b ? b : a;
-                double c = 1.0, s = 0.0;
-                if (q < n) {
-                    const double apq = A[p * ld + q];
-                    const double app = A[p * ld + p], aqq = A[q * ld + q];
-                    if (fabs(apq) > fmax(1.1102230246251565e-16 * sqrt(fabs(app * aqq)), abs_tol)) {
-                        const double theta = (aqq - app) / (2.0 * apq);
-                        const double t = fabs(theta) < 1e150
-                                             ? (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0))
-                                             : 0.5 / theta;
-                        c = 1.0 / sqrt(t * t + 1.0);
-                        s = t * c;
-                        atomicAdd(&nrot, 1);
+            }
+            rot[d][tid] = make_double2(c, s);
+            pq[d][tid] = make_int2(p, q);
+        }
+        const unsigned long long any = __ballot(s != 0.0);
+        if (lane == 0 && any) atomicAdd(&nrot[d], 1);
+    };
+    // the rotations of buffer d applied to the eigenvectors by the other waves, kVPer of them in flight
+    auto turn = [&](auto* V, int ldv, int d) {
+        constexpr int kC = (kJacobiLdsN + 63) / 64;
+        for (int k0 = wave - kRotWaves; k0 < mk; k0 += (kWaves - kRotWaves) * kVPer) {
+            double2 rv[kVPer];
+            int2 pv[kVPer];
+            double x[kVPer][kC], y[kVPer][kC];
+#pragma unroll
+            for (int u = 0; u < kVPer; ++u) {
+                const int k = k0 + (kWaves - kRotWaves) * u;
+                rv[u] = rot[d][min(k, mk - 1)];
+                pv[u] = pq[d][min(k, mk - 1)];
+                if (k >= mk) rv[u].y = 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < kVPer; ++u)
+                if (rv[u].y != 0.0) {
+                    const int vp = __builtin_amdgcn_readfirstlane(pv[u].x) * ldv, vq = __builtin_amdgcn_readfirstlane(pv[u].y) * ldv;
+#pragma unroll
+                    for (int c = 0; c < kC; ++c)
+                        if (lane + 64 * c < n) {
+                            x[u][c] = V[vp + lane + 64 * c];
+                            y[u][c] = V[vq + lane + 64 * c];
+                        }
+                }
+#pragma unroll
+            for (int u = 0; u < kVPer; ++u)
+                if (rv[u].y != 0.0) {
+                    const int vp = __builtin_amdgcn_readfirstlane(pv[u].x) * ldv, vq = __builtin_amdgcn_readfirstlane(pv[u].y) * ldv;
+                    const double c0 = rv[u].x, s0 = rv[u].y;
+#pragma unroll
+                    for (int c = 0; c < kC; ++c)
+                        if (lane + 64 * c < n) {
+                            V[vp + lane + 64 * c] = turn_p(c0, s0, x[u][c], y[u][c]);
+                            V[vq + lane + 64 * c] = turn_q(c0, s0, x[u][c], y[u][c]);
+                        }
+                }
+        }
+    };
+    if (n > 1 && wave < kRotWaves) rotations(0, 0);
+    __syncthreads();
+    int d = 0;
+    for (int sweep = 0; sweep < max_sweeps && n > 1; ++sweep) {
+        bool turned = false;   // some rotation in this sweep
+        for (int r = 0; r < m - 1; ++r, d ^= 1) {
+            const bool some = nrot[d] != 0;
+            turned = turned || some;
+            if (some) {
+                // a wave takes whole rows of blocks (pair k, its rotation uniform), kPer at a time, its
+                // lanes the pairs l
+                for (int l0 = 0; l0 < mk; l0 += 64) {
+                    const int l = min(l0 + lane, mk - 1);
+                    const bool on = l0 + lane < mk;
+                    const double2 rl = rot[d][l];
+                    const int2 pl = pq[d][l];
+                    const double cl = rl.x, sl = rl.y;
+                    double* cp = A + pl.x;
+                    double* cq = A + pl.y;
+                    for (int k0 = wave; k0 < mk; k0 += kWaves * kPer) {
+                        double2 rk[kPer];
+                        int2 pk[kPer];
+                        double a[kPer][4];
+#pragma unroll
+                        for (int u = 0; u < kPer; ++u) {
+                            const int k = min(k0 + kWaves * u, mk - 1);
+                            rk[u] = rot[d][k];
+                            pk[u] = pq[d][k];
+                        }
+#pragma unroll
+                        for (int u = 0; u < kPer; ++u) {
+                            const int rp = __builtin_amdgcn_readfirstlane(pk[u].x) * ld;
+                            const int rq = __builtin_amdgcn_readfirstlane(pk[u].y) * ld;
+                            a[u][0] = cp[rp];
+                            a[u][1] = cq[rp];
+                            a[u][2] = cp[rq];
+                            a[u][3] = cq[rq];
+                        }
+#pragma unroll
+                        for (int u = 0; u < kPer; ++u) {
+                            const double ck = rk[u].x, sk = rk[u].y;
+                            const double r00 = turn_p(ck, sk, a[u][0], a[u][2]), r01 = turn_p(ck, sk, a[u][1], a[u][3]);
+                            const double r10 = turn_q(ck, sk, a[u][0], a[u][2]), r11 = turn_q(ck, sk, a[u][1], a[u][3]);
+                            if (k0 + kWaves * u < mk && on && (sk != 0.0 || sl != 0.0)) {
+                                const int rp = __builtin_amdgcn_readfirstlane(pk[u].x) * ld;
+                                const int rq = __builtin_amdgcn_readfirstlane(pk[u].y) * ld;
+                                cp[rp] = turn_p(cl, sl, r00, r01);
+                                cq[rp] = turn_q(cl, sl, r00, r01);
+                                cp[rq] = turn_p(cl, sl, r10, r11);
+                                cq[rq] = turn_q(cl, sl, r10, r11);
+                            }
+                        }
                     }
                 }
-                pp[tid] = p;
-                qq[tid] = q;
-                cs[tid] = c;
-                sn[tid] = s;
+                __syncthreads();
             }
-            __syncthreads();
-            // a wave takes whole rows of blocks (pair k, its rotation uniform), its lanes the pairs
-            // l; then whole rotations of the eigenvectors, its lanes the components
-            for (int l0 = 0; l0 < mk; l0 += 64) {
-                const int l = l0 + lane;
-                const bool on = l < mk;
-                const double cl = on ? cs[l] : 1.0, sl = on ? sn[l] : 0.0;
-                const int pl = on ? pp[l] : 0, ql = on ? qq[l] : n;
-                // (the dummy index of an odd n only meets rotations with s = 0: its row and
-                // column are left out)
-                const bool vq = ql < n;
-                for (int k = wave; k < mk; k += kJacobiThreads / 64) {
-                    const double ck = cs[k], sk = sn[k];
-                    if (!on || (sk == 0.0 && sl == 0.0)) continue;
-                    const int pk = pp[k], qk = qq[k];
-                    const bool vk = qk < n;
-                    const double a00 = A[pk * ld + pl], a01 = vq ? A[pk * ld + ql] : 0.0;
-                    const double a10 = vk ? A[qk * ld + pl] : 0.0, a11 = vk && vq ? A[qk * ld + ql] : 0.0;
-                    const double r00 = ck * a00 - sk * a10, r01 = ck * a01 - sk * a11;
-                    const double r10 = sk * a00 + ck * a10, r11 = sk * a01 + ck * a11;
-                    A[pk * ld + pl] = cl * r00 - sl * r01;
-                    if (vq) A[pk * ld + ql] = sl * r00 + cl * r01;
-                    if (vk) A[qk * ld + pl] = cl * r10 - sl * r11;
-                    if (vk && vq) A[qk * ld + ql] = sl * r10 + cl * r11;
-                }
+            // the next round's rotations (the next sweep's first after the last), and the vectors
+            if (wave < kRotWaves) {
+                rotations(r + 1 < m - 1 ? r + 1 : 0, d ^ 1);
+            } else if (some) {
+                if (vl) turn(VL, lv, d);
+                else turn(VG, n, d);
             }
-            for (int k = wave; k < mk; k += kJacobiThreads / 64) {
-                const double c = cs[k], s = sn[k];
-                if (s == 0.0) continue;
-                double* vp = V + pp[k] * ldv;
-                double* vq = V + qq[k] * ldv;
-                for (int i = lane; i < n; i += 64) {
-                    const double x = vp[i], y = vq[i];
-                    vp[i] = c * x - s * y;
-                    vq[i] = s * x + c * y;
-                }
-            }
+            if (tid == 0 && some) nrot[d] = 0;   // read by all before the pass, written again after this barrier
             __syncthreads();
         }
-        const int done = nrot == 0;
-        __syncthreads();
-        if (done) break;
+        if (!turned) break;
     }
     __syncthreads();
     // eigenvalues ascending (ties by index) with their vectors as columns of Z
-    int* rank = reinterpret_cast<int*>(cs);   // n <= 140 ints in 70 doubles
+    int* rank = reinterpret_cast<int*>(&rot[0][0]);   // n ints in n / 2 (c, s)
     for (int i = tid; i < n; i += kJacobiThreads) {
         const double di = A[i * ld + i];
         int r = 0;
@@ -313,33 +402,29 @@ __global__ __launch_bounds__(kJacobiThreads) void k_batched_jacobi_lds(const Bat
             const double dj = A[j * ld + j];
             if (dj < di || (dj == di && j < i)) ++r;
         }
-        M.evals[r] = di;
+        ev[r] = di;
         rank[i] = r;
     }
     __syncthreads();
     for (int e = tid; e < n * n; e += kJacobiThreads) {
         const int i = e / n, r = e - i * n;
-        M.Z[(long)r * n + rank[i]] = V[i * ldv + r];
+        Z[(long)r * n + rank[i]] = vl ? VL[i * lv + r] : VG[e];
     }
-    if (tid == 0 && sweeps_out) sweeps_out[blockIdx.x] = sweep;
 }
 
-hipError_t batched_jacobi(int nmat, const BatchMat* mats, int maxn, int max_sweeps, int* sweeps, hipStream_t st) {
-    if (nmat <= 0) return hipSuccess;
-    const int nl = std::min(maxn, kJacobiLdsN);
-    const size_t lds = sizeof(double) * (size_t)(jacobi_v_fits(nl) ? 2 : 1) * nl * jacobi_ld(nl);
+hipError_t batched_jacobi(int nslot, const MatSlot* slots, Store A, Store V, Store evals, Store Z, int maxn, int max_sweeps,
+                          hipStream_t st) {
+    if (nslot <= 0) return hipSuccess;
     // (a smaller matrix of the launch may keep its vectors in LDS where the largest does not)
-    const size_t need = jacobi_v_fits(nl) ? lds : sizeof(double) * (size_t)kJacobiLdsN * jacobi_ld(kJacobiLdsN);
-    static size_t attr = 0;
-    if (need > attr) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_batched_jacobi_lds),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)need);
-        if (e != hipSuccess) return e;
-        attr = need;
-    }
-    hipLaunchKernelGGL(k_batched_jacobi_lds, dim3(nmat), dim3(kJacobiThreads), need, st, mats, max_sweeps, sweeps);
+    const int nl = std::min(maxn, kJacobiLdsN);
+    const size_t need = sizeof(double) * (size_t)(jacobi_v_fits(nl) ? jacobi_a(nl) + jacobi_v(nl) : kJacobiLds);
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_batched_jacobi_lds),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kJacobiLds * sizeof(double))))
+        return e;
+    hipLaunchKernelGGL(k_batched_jacobi_lds, dim3(nslot), dim3(kJacobiThreads), need, st, slots, A, V, evals, Z,
+                       max_sweeps);
     if (maxn > kJacobiLdsN)
-        hipLaunchKernelGGL(k_batched_jacobi, dim3(nmat), dim3(kJacobiThreads), 0, st, mats, max_sweeps, sweeps);
+        hipLaunchKernelGGL(k_batched_jacobi, dim3(nslot), dim3(kJacobiThreads), 0, st, slots, A, V, evals, Z, max_sweeps);
     return hipGetLastError();
 }
 
@@ -356,40 +441,67 @@ __device__ __forceinline__ double block_reduce_sum(double v, double* red) {
     return s;
 }
 
-// out[k] (+)= sum_ij A_k,ij B_k,ij over slot k's n x n matrices
-__global__ __launch_bounds__(256) void k_batch_dot(const MatSlot* __restrict__ slots, const double* __restrict__ A,
-                                                   const double* __restrict__ B, double* __restrict__ out, int acc) {
+// out[q nslot + k] = sum_ij A_q,ij B_q,ij over slot k's n x n matrices
+__global__ __launch_bounds__(256) void k_batch_dots(const MatSlot* __restrict__ slots, DotPairs q, double* __restrict__ out) {
     __shared__ double red[4];
     const MatSlot m = slots[blockIdx.x];
+    const double* A = q.a[blockIdx.y][m.spin];
+    const double* B = q.b[blockIdx.y][m.spin];
+    if (!A || !B) return;
     double s = 0.0;
-    for (long e = threadIdx.x; e < (long)m.n * m.n; e += blockDim.x) s += A[m.off + e] * B[m.off + e];
+    for (int e = threadIdx.x; e < m.n * m.n; e += 256) s += A[m.off + e] * B[m.off + e];
     s = block_reduce_sum(s, red);
-    if (threadIdx.x == 0) out[blockIdx.x] = acc ? out[blockIdx.x] + s : s;
+    if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
 // out[k] = sqrt(sum (A - B)^2) / n over slot k
-__global__ __launch_bounds__(256) void k_batch_diffnorm(const MatSlot* __restrict__ slots, const double* __restrict__ A,
-                                                        const double* __restrict__ B, double* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_batch_diffnorm(const MatSlot* __restrict__ slots, Store A, Store B,
+                                                        double* __restrict__ out) {
     __shared__ double red[4];
     const MatSlot m = slots[blockIdx.x];
+    const double* a = A.s[m.spin] + m.off;
+    const double* b = B.s[m.spin] + m.off;
     double s = 0.0;
-    for (long e = threadIdx.x; e < (long)m.n * m.n; e += blockDim.x) {
-        const double d = A[m.off + e] - B[m.off + e];
+    for (int e = threadIdx.x; e < m.n * m.n; e += 256) {
+        const double d = a[e] - b[e];
         s += d * d;
     }
     s = block_reduce_sum(s, red);
     if (threadIdx.x == 0) out[blockIdx.x] = sqrt(s) / m.n;
 }
 
-// G = W + W^T (or G += ...) per slot
-__global__ __launch_bounds__(256) void k_batch_sym(const MatSlot* __restrict__ slots, const double* __restrict__ W,
-                                                   double* __restrict__ G, int acc) {
+// element-wise kernels: kSlotBlocks blocks share a slot's matrix
+constexpr int kSlotBlocks = 8;
+
+// G = W + W^T, or W - W^T as 2 W - (W + W^T)
+template <bool ANTI>
+__global__ __launch_bounds__(256) void k_batch_sym(const MatSlot* __restrict__ slots, Store W, Store G) {
     const MatSlot m = slots[blockIdx.x];
-    for (long e = threadIdx.x; e < (long)m.n * m.n; e += blockDim.x) {
-        const int i = (int)(e / m.n), j = (int)(e % m.n);
-        const double v = W[m.off + e] + W[m.off + (long)j * m.n + i];
-        G[m.off + e] = acc ? G[m.off + e] + v : v;
+    const double* w = W.s[m.spin] + m.off;
+    double* g = G.s[m.spin] + m.off;
+    for (int e = blockIdx.y * 256 + threadIdx.x; e < m.n * m.n; e += 256 * kSlotBlocks) {
+        const int i = e / m.n, j = e - i * m.n;
+        const double x = w[e], v = x + w[j * m.n + i];
+        g[e] = ANTI ? fma(2.0, x, -v) : v;
     }
+}
+
+__global__ __launch_bounds__(256) void k_batch_add(const MatSlot* __restrict__ slots, const double* __restrict__ H, Store G,
+                                                   Store F) {
+    const MatSlot m = slots[blockIdx.x];
+    const double* h = H + m.off;
+    const double* g = G.s[m.spin] + m.off;
+    double* f = F.s[m.spin] + m.off;
+    for (int e = blockIdx.y * 256 + threadIdx.x; e < m.n * m.n; e += 256 * kSlotBlocks) f[e] = h[e] + g[e];
+}
+
+__global__ __launch_bounds__(256) void k_batch_densities(long long len, Store P, double* __restrict__ D0, Store Pold) {
+    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= len) return;
+    const double a = P.s[0][e], b = P.s[1][e];
+    D0[e] = a + b;
+    Pold.s[0][e] = a;
+    Pold.s[1][e] = b;
 }
 
 // Dsh_m[s][t] = max |D| over the function block of shells s, t of every active molecule m (D1,
@@ -424,36 +536,49 @@ __global__ __launch_bounds__(256) void k_batch_shell_max(const MolDesc* __restri
     if ((threadIdx.x & 63) == 0 && big > 0.0) atomicMax(dmax + mol, (unsigned long long)__double_as_longlong(big));
 }
 
-// F_k = sum_j c[k * ncoef + j] H_j,k: a linear combination of ncoef stores per slot
-__global__ __launch_bounds__(256) void k_batch_lincomb(const MatSlot* __restrict__ slots, int ncoef,
-                                                       const double* __restrict__ coef, const double* const* __restrict__ src,
-                                                       double* __restrict__ F) {
+// F_k = sum_j c[k kMaxLin + j] H_j,k: a linear combination of stores per slot
+__global__ __launch_bounds__(256) void k_batch_lincomb(const MatSlot* __restrict__ slots, const double* __restrict__ coef,
+                                                       LinSources src, Store F) {
     const MatSlot m = slots[blockIdx.x];
-    for (long e = threadIdx.x; e < (long)m.n * m.n; e += blockDim.x) {
+    double* f = F.s[m.spin] + m.off;
+    for (int e = blockIdx.y * 256 + threadIdx.x; e < m.n * m.n; e += 256 * kSlotBlocks) {
         double v = 0.0;
-        for (int j = 0; j < ncoef; ++j) {
-            const double cj = coef[(long)blockIdx.x * ncoef + j];
-            if (cj != 0.0) v = fma(cj, src[j][m.off + e], v);
+#pragma unroll
+        for (int j = 0; j < kMaxLin; ++j) {
+            const double cj = coef[blockIdx.x * kMaxLin + j];
+            if (cj != 0.0) v = fma(cj, src.s[j][m.spin][m.off + e], v);
         }
-        F[m.off + e] = v;
+        f[e] = v;
     }
 }
 
-hipError_t batch_dot(int nslot, const MatSlot* slots, const double* A, const double* B, double* out, bool acc,
-                     hipStream_t st) {
-    if (nslot <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_batch_dot, dim3(nslot), dim3(256), 0, st, slots, A, B, out, acc ? 1 : 0);
+hipError_t batch_dots(int nslot, const MatSlot* slots, const DotPairs& q, double* out, hipStream_t st) {
+    if (nslot <= 0 || q.n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_batch_dots, dim3(nslot, q.n), dim3(256), 0, st, slots, q, out);
     return hipGetLastError();
 }
-hipError_t batch_diffnorm(int nslot, const MatSlot* slots, const double* A, const double* B, double* out,
-                          hipStream_t st) {
+hipError_t batch_diffnorm(int nslot, const MatSlot* slots, Store A, Store B, double* out, hipStream_t st) {
     if (nslot <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_batch_diffnorm, dim3(nslot), dim3(256), 0, st, slots, A, B, out);
     return hipGetLastError();
 }
-hipError_t batch_sym(int nslot, const MatSlot* slots, const double* W, double* G, bool acc, hipStream_t st) {
+hipError_t batch_sym(int nslot, const MatSlot* slots, Store W, Store G, hipStream_t st) {
     if (nslot <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_batch_sym, dim3(nslot), dim3(256), 0, st, slots, W, G, acc ? 1 : 0);
+    hipLaunchKernelGGL((k_batch_sym<false>), dim3(nslot, kSlotBlocks), dim3(256), 0, st, slots, W, G);
+    return hipGetLastError();
+}
+hipError_t batch_antisym(int nslot, const MatSlot* slots, Store W, Store out, hipStream_t st) {
+    if (nslot <= 0) return hipSuccess;
+    hipLaunchKernelGGL((k_batch_sym<true>), dim3(nslot, kSlotBlocks), dim3(256), 0, st, slots, W, out);
+    return hipGetLastError();
+}
+hipError_t batch_add(int nslot, const MatSlot* slots, const double* H, Store G, Store F, hipStream_t st) {
+    if (nslot <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_batch_add, dim3(nslot, kSlotBlocks), dim3(256), 0, st, slots, H, G, F);
+    return hipGetLastError();
+}
+hipError_t batch_densities(long long len, Store P, double* D0, Store Pold, hipStream_t st) {
+    hipLaunchKernelGGL(k_batch_densities, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, st, len, P, D0, Pold);
     return hipGetLastError();
 }
 hipError_t batch_shell_max(int nmol, int maxsh, const MolDesc* mols, const int* shoff, const int* active,
@@ -464,10 +589,10 @@ hipError_t batch_shell_max(int nmol, int maxsh, const MolDesc* mols, const int* 
                        sh_off, sh_n, D, D1, D2, Dsh, reinterpret_cast<unsigned long long*>(dmax));
     return hipGetLastError();
 }
-hipError_t batch_lincomb(int nslot, const MatSlot* slots, int ncoef, const double* coef, const double* const* src,
-                         double* F, hipStream_t st) {
+hipError_t batch_lincomb(int nslot, const MatSlot* slots, const double* coef, const LinSources& src, Store F,
+                         hipStream_t st) {
     if (nslot <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_batch_lincomb, dim3(nslot), dim3(256), 0, st, slots, ncoef, coef, src, F);
+    hipLaunchKernelGGL(k_batch_lincomb, dim3(nslot, kSlotBlocks), dim3(256), 0, st, slots, coef, src, F);
     return hipGetLastError();
 }
 

@@ -42,23 +42,15 @@ using clk = std::chrono::steady_clock;
 double secs(clk::time_point a, clk::time_point b) { return std::chrono::duration<double>(b - a).count(); }
 
 
-// Device copies of the small per-iteration arrays (GEMM groups and tiles, matrix lists,
-// quartet entries, DIIS coefficients): the k-th upload of an iteration reuses slot k,
-// grown when needed, so the steady state allocates nothing.  Every iteration ends with a
-// stream synchronisation before reset() hands the slots out again.
-struct Scratch {
-    std::vector<DBuf<char>> slot;
-    size_t next = 0;
-    void reset() { next = 0; }
-    template <class T>
-    hipError_t upload(const T* h, size_t n, hipStream_t st, T** out) {
-        if (next == slot.size()) slot.emplace_back();
-        DBuf<char>& s = slot[next++];
-        hipError_t e = s.alloc(std::max<size_t>(n, 1) * sizeof(T));
-        if (e != hipSuccess) return e;
-        *out = reinterpret_cast<T*>(s.p);
-        return n ? hipMemcpyAsync(s.p, h, n * sizeof(T), hipMemcpyHostToDevice, st) : hipSuccess;
-    }
+// pinned host memory, so that the small copies of an iteration are asynchronous
+struct Pinned {
+    char* p = nullptr;
+    size_t n = 0;
+    Pinned() = default;
+    Pinned(const Pinned&) = delete;
+    Pinned& operator=(const Pinned&) = delete;
+    hipError_t alloc(size_t bytes) { return n = bytes, hipHostMalloc((void**)&p, bytes, hipHostMallocDefault); }
+    ~Pinned() { if (p) (void)hipHostFree(p); }
 };
 
 }  // namespace
@@ -74,14 +66,26 @@ struct uno_batch {
     DBuf<MolDesc> mdesc;
     DBuf<int> mshoff;           // per molecule: its first shell in the shell tables
     // stores (each sum_m N_m^2 doubles); index 0 alpha / closed shell, 1 beta
-    DBuf<double> H, S, X, P[2], Pold[2], F[2], G[2], C[2], Fp, Tm, Tm2, V, Z, D0, D1, D2, W0, W1, Dsh, ev[2];
+    DBuf<double> H, S, X, D0, P[2], Pold[2], F[2], G[2], C[2], Fp[2], Tm[2], Tm2[2], V[2], Z[2], W[2], Dsh, ev[2];
     // per spin: the last eigenvectors of X^T F X (orthogonal basis), the next eigensolve's
-    // starting basis once warm[spin] is set
-    DBuf<double> Wp[2];
+    // starting basis once warm[spin] is set, and the buffer the next ones go to
+    DBuf<double> Wp[2], Wn[2];
     bool warm[2] = {false, false};
     DBuf<double> dF[kBatchDiis][2], dE[kBatchDiis][2];
-    DBuf<double> red;
-    Scratch scratch;
+    DBuf<double> red, coef;
+    // the active slots, those of spin 0 first (nslot[s] of spin s, of molecules who[k]), and their
+    // GEMM tiles in the same order; rewritten when a molecule stops
+    DBuf<MatSlot> slots;
+    DBuf<GemmTile> tiles;
+    int nslot[2] = {0, 0}, ntile[2] = {0, 0};
+    std::vector<int> who;
+    // host sides of the copies, a place each: written or read only while the stream is idle
+    Pinned host;
+    int* h_active = nullptr;
+    MatSlot* h_slots = nullptr;
+    GemmTile* h_tiles = nullptr;
+    double *h_coef = nullptr, *h_dots = nullptr, *h_pdiff = nullptr;
+    hipEvent_t ev_fock[2] = {}, ev_diag[2] = {};
     // the Fock kernels' pair data and launches over all molecules, every pair's molecule, the
     // per-molecule active flags, and the build captured as a HIP graph (replayed every
     // iteration of a run)
@@ -108,62 +112,55 @@ struct uno_batch {
         for (BatchMol& m : mol)
             if (m.ctx) uno_ctx_destroy(m.ctx);
         if (st) (void)hipStreamSynchronize(st);
+        for (hipEvent_t e : {ev_fock[0], ev_fock[1], ev_diag[0], ev_diag[1]})
+            if (e) (void)hipEventDestroy(e);
         if (st) (void)hipStreamDestroy(st);
     }
 };
 
 namespace {
 
-// slots: per (molecule, spin) matrix; spin 1 only for UHF molecules
-void make_slots(const uno_batch* b, bool only_active, int spin, std::vector<MatSlot>& out, std::vector<int>& who) {
-    out.clear();
-    who.clear();
-    for (int m = 0; m < (int)b->mol.size(); ++m) {
-        const BatchMol& x = b->mol[m];
-        if (only_active && !x.active) continue;
-        if (spin == 1 && !x.uhf) continue;
-        out.push_back(MatSlot{x.moff, x.n});
-        who.push_back(m);
+Store both(DBuf<double>* x) { return Store{{x[0].p, x[1].p}}; }
+Store same(const DBuf<double>& x) { return Store{{x.p, x.p}}; }
+
+// the slots and tiles of the active molecules (spin 1 only for UHF molecules), and the active flags
+int refresh_slots(uno_batch* b) {
+    b->who.clear();
+    int nt = 0;
+    for (int s = 0; s < 2; ++s) {
+        const int k0 = (int)b->who.size(), t0 = nt;
+        for (int m = 0; m < (int)b->mol.size(); ++m) {
+            const BatchMol& x = b->mol[m];
+            b->h_active[m] = x.active ? 1 : 0;
+            if (!x.active || (s == 1 && !x.uhf)) continue;
+            const int k = (int)b->who.size();
+            b->who.push_back(m);
+            b->h_slots[k] = MatSlot{x.moff, x.n, x.nocc[s], s};
+            const int nb = (x.n + 31) / 32;
+            for (int i = 0; i < nb; ++i)
+                for (int j = 0; j < nb; ++j) b->h_tiles[nt++] = GemmTile{k, i, j};
+        }
+        b->nslot[s] = (int)b->who.size() - k0;
+        b->ntile[s] = nt - t0;
     }
+    hipStream_t st = b->st;
+    UNO_HIP(hipMemcpyAsync(b->active_d.p, b->h_active, b->mol.size() * sizeof(int), hipMemcpyHostToDevice, st));
+    UNO_HIP(hipMemcpyAsync(b->slots.p, b->h_slots, b->who.size() * sizeof(MatSlot), hipMemcpyHostToDevice, st));
+    UNO_HIP(hipMemcpyAsync(b->tiles.p, b->h_tiles, nt * sizeof(GemmTile), hipMemcpyHostToDevice, st));
+    return UNO_OK;
 }
 
-struct GemmBatch {
-    std::vector<GemmGroup> g;
-    std::vector<GemmTile> t;
-    Scratch* sc;
-    explicit GemmBatch(Scratch& s) : sc(&s) {}
-    void add(int m, int n, int k, bool ta, bool tb, const double* A, const double* B, double* C, int lda, int ldb,
-             int ldc) {
-        if (m <= 0 || n <= 0 || k <= 0) return;
-        const int gi = (int)g.size();
-        g.push_back(GemmGroup{m, n, k, ta ? 1 : 0, tb ? 1 : 0, A, B, C, lda, ldb, ldc});
-        for (int i = 0; i < (m + 31) / 32; ++i)
-            for (int j = 0; j < (n + 31) / 32; ++j) t.push_back(GemmTile{gi, i, j});
-    }
-    int run(double alpha, double beta, hipStream_t st) {
-        if (t.empty()) return UNO_OK;
-        GemmGroup* dg = nullptr;
-        GemmTile* dt = nullptr;
-        UNO_HIP(sc->upload(g.data(), g.size(), st, &dg));
-        UNO_HIP(sc->upload(t.data(), t.size(), st, &dt));
-        UNO_HIP(grouped_gemm((int)t.size(), dt, dg, alpha, beta, st));
-        // the group / tile arrays are pageable host memory: keep them alive until done
-        UNO_HIP(hipStreamSynchronize(st));
-        return UNO_OK;
-    }
-};
-
-// Z, evals of every slot's symmetric matrix A (destroyed), A given per slot
-int batch_eigh(uno_batch* b, const std::vector<MatSlot>& sl, double* A, double* evals_base,
-               const std::vector<long long>& evoff) {
-    std::vector<BatchMat> bm(sl.size());
-    for (size_t k = 0; k < sl.size(); ++k)
-        bm[k] = BatchMat{sl[k].n, A + sl[k].off, b->V.p + sl[k].off, evals_base + evoff[k], b->Z.p + sl[k].off};
-    BatchMat* d = nullptr;
-    UNO_HIP(b->scratch.upload(bm.data(), bm.size(), b->st, &d));
-    UNO_HIP(batched_jacobi((int)bm.size(), d, b->maxn, 50, nullptr, b->st));
-    UNO_HIP(hipStreamSynchronize(b->st));
+// C = op(A) op(B) over the active slots of spins [s0, s1)
+int gemm(uno_batch* b, int s0, int s1, bool ta, bool tb, bool occ, Store A, Store B, Store C) {
+    const int lo = s0 ? b->ntile[0] : 0, hi = s1 > 1 ? b->ntile[0] + b->ntile[1] : b->ntile[0];
+    UNO_HIP(grouped_gemm(hi - lo, b->tiles.p + lo, b->slots.p, ta, tb, occ, A, B, C, b->st));
     return UNO_OK;
+}
+
+double elapsed(hipEvent_t* e) {
+    float ms = 0.f;
+    (void)hipEventElapsedTime(&ms, e[0], e[1]);
+    return 1e-3 * ms;
 }
 
 }  // namespace
@@ -178,13 +175,13 @@ static int enqueue_fock(uno_batch* b) {
     FockStore& fs = b->fs;
     const int np = fs.npair, nm = (int)b->mol.size();
     ClearList cl;
-    cl.add(b->W0.p, b->store);
-    cl.add(b->W1.p, b->store);
+    cl.add(b->W[0].p, b->store);
+    cl.add(b->W[1].p, b->store);
     cl.add(fs.jp.p, fs.njp);
     cl.add(fs.dmax.p, nm);
     cl.add(fs.ctr.p, 2 * (long long)fs.launches.size());
     UNO_HIP(fock_clear(cl, st));
-    UNO_HIP(batch_shell_max(nm, b->maxsh, b->mdesc.p, b->mshoff.p, b->active_d.p, b->sh_off.p, b->sh_n.p, b->D0.p, b->D1.p, b->D2.p,
+    UNO_HIP(batch_shell_max(nm, b->maxsh, b->mdesc.p, b->mshoff.p, b->active_d.p, b->sh_off.p, b->sh_n.p, b->D0.p, b->P[0].p, b->P[1].p,
                             b->Dsh.p, fs.dmax.p, st));
     UNO_HIP(pair_density(np, fs.kidx.p, fs.kjo.p, b->D0.p, b->Dsh.p, 0, 0, b->mdesc.p, b->pmol.p, fs.dp.p, fs.dpair.p, st));
     const uno_ctx* c0 = b->mol[0].ctx;
@@ -210,11 +207,11 @@ static int enqueue_fock(uno_batch* b) {
         a.jp = fs.jp.p;
         a.nquart = fs.nquart.p;
         a.D0 = b->D0.p;
-        a.W0 = b->W0.p;
+        a.W0 = b->W[0].p;
         if (uhf) {
-            a.D1 = b->D1.p;
-            a.D2 = b->D2.p;
-            a.W1 = b->W1.p;
+            a.D1 = b->P[0].p;
+            a.D2 = b->P[1].p;
+            a.W1 = b->W[1].p;
         }
         a.mols = b->mdesc.p;
         a.mol_active = b->active_d.p;
@@ -223,17 +220,13 @@ static int enqueue_fock(uno_batch* b) {
         UNO_HIP(fock_launch(mode, false, l.cx, l.cy, a, f, l.ncols, b->ls.of((int)(k % (size_t)nls), st)));
     }
     if (int rc = b->ls.end(nls, st)) return rc;
-    UNO_HIP(jp_scatter(np, fs.kidx.p, fs.kjo.p, fs.jp.p, b->W0.p, b->W1.p, 0, b->mdesc.p, b->pmol.p, st));
+    UNO_HIP(jp_scatter(np, fs.kidx.p, fs.kjo.p, fs.jp.p, b->W[0].p, b->W[1].p, 0, b->mdesc.p, b->pmol.p, st));
     return UNO_OK;
 }
 
-// batched Fock build on the densities in D0 (D1, D2): W0 (W1) accumulators
+// batched Fock build on the densities in P, D0 their sum: W accumulators
 static int batch_fock(uno_batch* b) {
     hipStream_t st = b->st;
-    const int nm = (int)b->mol.size();
-    std::vector<int> act(nm);
-    for (int m = 0; m < nm; ++m) act[m] = b->mol[m].active ? 1 : 0;
-    UNO_HIP(hipMemcpyAsync(b->active_d.p, act.data(), nm * sizeof(int), hipMemcpyHostToDevice, st));
     if (int rc = b->ls.prepare(std::max(1, std::min(kMaxLaunchStreams, b->launch_streams)))) return rc;
     if (b->use_graph) {
         if (!b->gexec) {
@@ -255,7 +248,6 @@ static int batch_fock(uno_batch* b) {
     } else {
         if (int rc = enqueue_fock(b)) return rc;
     }
-    UNO_HIP(hipStreamSynchronize(st));
     return UNO_OK;
 }
 
@@ -345,8 +337,9 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
     }
     const size_t S = (size_t)b->store;
     DBuf<double>* stores[] = {&b->H, &b->S, &b->X, &b->P[0], &b->P[1], &b->Pold[0], &b->Pold[1], &b->F[0], &b->F[1],
-                              &b->G[0], &b->G[1], &b->C[0], &b->C[1], &b->Fp, &b->Tm, &b->Tm2, &b->V, &b->Z,
-                              &b->D0, &b->D1, &b->D2, &b->W0, &b->W1, &b->Wp[0], &b->Wp[1]};
+                              &b->G[0], &b->G[1], &b->C[0], &b->C[1], &b->Fp[0], &b->Fp[1], &b->Tm[0], &b->Tm[1],
+                              &b->Tm2[0], &b->Tm2[1], &b->V[0], &b->V[1], &b->Z[0], &b->Z[1], &b->D0, &b->W[0],
+                              &b->W[1], &b->Wp[0], &b->Wp[1], &b->Wn[0], &b->Wn[1]};
     for (DBuf<double>* p : stores)
         if (p->alloc(S) != hipSuccess) { set_error("batched SCF: device allocation failed"); delete b; return UNO_ENOMEM; }
     for (int k = 0; k < kBatchDiis; ++k)
@@ -357,11 +350,40 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
                 return UNO_ENOMEM;
             }
     if (b->Dsh.alloc(std::max<long long>(1, b->dsh_total)) != hipSuccess || b->ev[0].alloc(S) != hipSuccess ||
-        b->ev[1].alloc(S) != hipSuccess || b->red.alloc(8 * (size_t)nmol * (kBatchDiis + 4)) != hipSuccess) {
+        b->ev[1].alloc(S) != hipSuccess) {
         set_error("batched SCF: device allocation failed");
         delete b;
         return UNO_ENOMEM;
     }
+    // the iteration's small arrays, sized for every slot active
+    size_t ns = 0, nt = 0;
+    for (const BatchMol& x : b->mol) {
+        const size_t nb = (x.n + 31) / 32, k = x.uhf ? 2 : 1;
+        ns += k;
+        nt += k * nb * nb;
+    }
+    const size_t sz[6] = {nmol * sizeof(int), ns * sizeof(MatSlot), nt * sizeof(GemmTile), ns * kMaxLin * sizeof(double),
+                          ns * kMaxDots * sizeof(double), ns * sizeof(double)};
+    size_t at[7] = {};
+    for (int k = 0; k < 6; ++k) at[k + 1] = at[k] + (sz[k] + 63) / 64 * 64;
+    if (b->slots.alloc(ns) != hipSuccess || b->tiles.alloc(nt) != hipSuccess || b->coef.alloc(ns * kMaxLin) != hipSuccess ||
+        b->red.alloc(ns * kMaxDots) != hipSuccess || b->host.alloc(at[6]) != hipSuccess) {
+        set_error("batched SCF: allocation failed");
+        delete b;
+        return UNO_ENOMEM;
+    }
+    b->h_active = reinterpret_cast<int*>(b->host.p + at[0]);
+    b->h_slots = reinterpret_cast<MatSlot*>(b->host.p + at[1]);
+    b->h_tiles = reinterpret_cast<GemmTile*>(b->host.p + at[2]);
+    b->h_coef = reinterpret_cast<double*>(b->host.p + at[3]);
+    b->h_dots = reinterpret_cast<double*>(b->host.p + at[4]);
+    b->h_pdiff = reinterpret_cast<double*>(b->host.p + at[5]);
+    for (hipEvent_t* ep : {&b->ev_fock[0], &b->ev_fock[1], &b->ev_diag[0], &b->ev_diag[1]})
+        if (hipEventCreate(ep) != hipSuccess) {
+            set_error("HIP event creation failed");
+            delete b;
+            return UNO_EDEVICE;
+        }
     *out = b;
     return UNO_OK;
 }
@@ -422,7 +444,6 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
     }
     const auto t0 = clk::now();
     hipStream_t st = b->st;
-    b->scratch.reset();
     b->warm[0] = b->warm[1] = false;
     // the captured build belongs to one run
     b->drop_graph();
@@ -435,43 +456,29 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
     }
     const int nm = (int)b->mol.size();
     const long long S = b->store;
-    // per-molecule eigenvalue offsets into ev stores: reuse the matrix offsets (n <= n^2)
+    // (the eigenvalues of a slot are at its matrix offset: n <= n^2)
     // one-electron matrices of every molecule
     for (BatchMol& x : b->mol) {
         x.active = true;
         x.converged = false;
         x.iterations = 0;
         x.eold = x.energy = x.ediff = x.pdiff = 0.0;
-        if (int rc = oneint_device(x.ctx, b->S.p + x.moff, b->Tm.p + x.moff, b->H.p + x.moff)) return rc;
-        UNO_HIP(hipStreamSynchronize(x.ctx->st));
+        if (int rc = oneint_device(x.ctx, b->S.p + x.moff, b->Tm[0].p + x.moff, b->H.p + x.moff)) return rc;
     }
+    for (BatchMol& x : b->mol) UNO_HIP(hipStreamSynchronize(x.ctx->st));
     for (int s = 0; s < 2; ++s) {
         UNO_HIP(k_fill(S, 0.0, b->P[s].p, st));
         UNO_HIP(k_fill(S, 0.0, b->G[s].p, st));
     }
-    std::vector<MatSlot> sl[2];
-    std::vector<int> who[2];
-    std::vector<DBuf<MatSlot>> dsl(2);
-    auto refresh_slots = [&]() -> int {
-        for (int s = 0; s < 2; ++s) {
-            make_slots(b, true, s, sl[s], who[s]);
-            if (!sl[s].empty()) UNO_HIP(dsl[s].upload(sl[s].data(), sl[s].size(), st));
-        }
-        return UNO_OK;
-    };
-    if (int rc = refresh_slots()) return rc;
-    auto evoff = [&](int s) {
-        std::vector<long long> o;
-        for (const MatSlot& m : sl[s]) o.push_back(m.off);
-        return o;
-    };
+    if (int rc = refresh_slots(b)) return rc;
     // X = U s^-1/2 (RHF.hpp:214-233): Jacobi of S, column scaling on the host read-back
     {
-        UNO_HIP(hipMemcpyAsync(b->Tm.p, b->S.p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
-        if (int rc = batch_eigh(b, sl[0], b->Tm.p, b->ev[0].p, evoff(0))) return rc;
+        UNO_HIP(hipMemcpyAsync(b->Tm[0].p, b->S.p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
+        UNO_HIP(batched_jacobi(b->nslot[0], b->slots.p, same(b->Tm[0]), same(b->V[0]), same(b->ev[0]), same(b->Z[0]), b->maxn,
+                               50, st));
         std::vector<double> ev(S), Z(S);
         UNO_HIP(hipMemcpyAsync(ev.data(), b->ev[0].p, S * sizeof(double), hipMemcpyDeviceToHost, st));
-        UNO_HIP(hipMemcpyAsync(Z.data(), b->Z.p, S * sizeof(double), hipMemcpyDeviceToHost, st));
+        UNO_HIP(hipMemcpyAsync(Z.data(), b->Z[0].p, S * sizeof(double), hipMemcpyDeviceToHost, st));
         UNO_HIP(hipStreamSynchronize(st));
         for (const BatchMol& x : b->mol) {
             for (int j = 0; j < x.n; ++j) {
@@ -483,207 +490,132 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
             }
         }
         UNO_HIP(b->X.upload(Z.data(), S, st));
+        UNO_HIP(hipStreamSynchronize(st));   // Z is pageable
     }
-    // F (store, per spin) -> P per spin slot: X^T F X, Jacobi, C = X W, P = C_occ C_occ^T
-    double diag_s = 0.0;
-    auto diag_to_P = [&](int s, const double* Fs) -> int {
-        if (sl[s].empty()) return UNO_OK;
-        const auto td = clk::now();
-        struct Acc { double& t; clk::time_point t0; ~Acc() { t += secs(t0, clk::now()); } } acc{diag_s, td};
-        GemmBatch g1(b->scratch), g2(b->scratch);
-        for (const MatSlot& m : sl[s]) g1.add(m.n, m.n, m.n, false, false, Fs + m.off, b->X.p + m.off, b->Tm.p + m.off, m.n, m.n, m.n);
-        if (int rc = g1.run(1.0, 0.0, st)) return rc;
-        for (const MatSlot& m : sl[s]) g2.add(m.n, m.n, m.n, true, false, b->X.p + m.off, b->Tm.p + m.off, b->Fp.p + m.off, m.n, m.n, m.n);
-        if (int rc = g2.run(1.0, 0.0, st)) return rc;
+    const Store X = same(b->X), Fp = both(b->Fp), Tm = both(b->Tm), Tm2 = both(b->Tm2), Z = both(b->Z), P = both(b->P),
+                C = both(b->C);
+    // F -> P over the slots of spins [0, ns): X^T F X, Jacobi, C = X W, P = C_occ C_occ^T.  Nothing here
+    // waits for the device: the slots, the tiles and the stores are all the launches need.
+    auto diag_to_P = [&](int ns, Store F) -> int {
+        UNO_HIP(hipEventRecord(b->ev_diag[0], st));
+        if (int rc = gemm(b, 0, ns, false, false, false, F, X, Tm)) return rc;
+        if (int rc = gemm(b, 0, ns, true, false, false, X, Tm, Fp)) return rc;
         // after their first eigensolve the molecules start from their last eigenvectors Wp:
         // in that basis the matrix is nearly diagonal and the Jacobi sweeps settle in a few
-        // rounds (W = Wp Z after)
-        std::vector<char> warm(sl[s].size(), 0);
-        GemmBatch w1(b->scratch), w2(b->scratch), w3(b->scratch);
-        for (size_t k = 0; k < sl[s].size(); ++k) {
-            const MatSlot& m = sl[s][k];
-            warm[k] = b->warm[s];
-            if (warm[k]) {
-                w1.add(m.n, m.n, m.n, false, false, b->Fp.p + m.off, b->Wp[s].p + m.off, b->Tm.p + m.off, m.n, m.n, m.n);
-                w2.add(m.n, m.n, m.n, true, false, b->Wp[s].p + m.off, b->Tm.p + m.off, b->Tm2.p + m.off, m.n, m.n, m.n);
-                w3.add(m.n, m.n, m.n, false, false, b->Wp[s].p + m.off, b->Z.p + m.off, b->Tm.p + m.off, m.n, m.n, m.n);
-            }
+        // rounds (W = Wp Z after; the first one's Z is W).  Spin 0 is warm when spin 1 is.
+        const int nw = b->warm[1] ? ns : b->warm[0] ? 1 : 0;
+        const Store Wp = both(b->Wp), Wn = both(b->Wn);
+        if (nw) {
+            if (int rc = gemm(b, 0, nw, false, false, false, Fp, Wp, Tm)) return rc;
+            if (int rc = gemm(b, 0, nw, true, false, false, Wp, Tm, Tm2)) return rc;
         }
-        if (int rc = w1.run(1.0, 0.0, st)) return rc;
-        if (int rc = w2.run(1.0, 0.0, st)) return rc;
-        {
-            std::vector<BatchMat> bm(sl[s].size());
-            for (size_t k = 0; k < sl[s].size(); ++k) {
-                const MatSlot& m = sl[s][k];
-                bm[k] = BatchMat{m.n, (warm[k] ? b->Tm2.p : b->Fp.p) + m.off, b->V.p + m.off, b->ev[s].p + m.off,
-                                 b->Z.p + m.off};
-            }
-            BatchMat* d = nullptr;
-            UNO_HIP(b->scratch.upload(bm.data(), bm.size(), st, &d));
-            UNO_HIP(batched_jacobi((int)bm.size(), d, b->maxn, 50, nullptr, st));
-            // bm is pageable host memory: its upload must be done before it goes
-            UNO_HIP(hipStreamSynchronize(st));
+        Store A, E;
+        for (int s = 0; s < 2; ++s) {
+            A.s[s] = s < nw ? Tm2.s[s] : Fp.s[s];
+            E.s[s] = s < nw ? Z.s[s] : Wn.s[s];
         }
-        if (int rc = w3.run(1.0, 0.0, st)) return rc;
-        // the new starting bases in one launch: Wp Z (warm, in Tm) or Z (cold)
-        {
-            std::vector<double> coef(2 * sl[s].size());
-            for (size_t k = 0; k < sl[s].size(); ++k) {
-                coef[2 * k] = warm[k] ? 1.0 : 0.0;
-                coef[2 * k + 1] = warm[k] ? 0.0 : 1.0;
-            }
-            const double* src[2] = {b->Tm.p, b->Z.p};
-            double* dcoef = nullptr;
-            const double** dsrc = nullptr;
-            UNO_HIP(b->scratch.upload(coef.data(), coef.size(), st, &dcoef));
-            UNO_HIP(b->scratch.upload(src, 2, st, &dsrc));
-            UNO_HIP(batch_lincomb((int)sl[s].size(), dsl[s].p, 2, dcoef, dsrc, b->Wp[s].p, st));
-            UNO_HIP(hipStreamSynchronize(st));
+        UNO_HIP(batched_jacobi(b->nslot[0] + (ns > 1 ? b->nslot[1] : 0), b->slots.p, A, both(b->V), both(b->ev), E, b->maxn, 50,
+                               st));
+        if (nw)
+            if (int rc = gemm(b, 0, nw, false, false, false, Wp, Z, Wn)) return rc;
+        for (int s = 0; s < ns; ++s) {
+            std::swap(b->Wp[s], b->Wn[s]);
+            b->warm[s] = true;
         }
-        b->warm[s] = true;
-        GemmBatch g3(b->scratch), g4(b->scratch);
-        for (const MatSlot& m : sl[s]) g3.add(m.n, m.n, m.n, false, false, b->X.p + m.off, b->Wp[s].p + m.off, b->C[s].p + m.off, m.n, m.n, m.n);
-        if (int rc = g3.run(1.0, 0.0, st)) return rc;
-        for (size_t k = 0; k < sl[s].size(); ++k) {
-            const MatSlot& m = sl[s][k];
-            g4.add(m.n, m.n, b->mol[who[s][k]].nocc[s], false, true, b->C[s].p + m.off, b->C[s].p + m.off,
-                   b->P[s].p + m.off, m.n, m.n, m.n);
-        }
-        return g4.run(1.0, 0.0, st);
+        if (int rc = gemm(b, 0, ns, false, false, false, X, Wn, C)) return rc;
+        if (int rc = gemm(b, 0, ns, false, true, true, C, C, P)) return rc;
+        UNO_HIP(hipEventRecord(b->ev_diag[1], st));
+        return UNO_OK;
     };
     // core-Hamiltonian guess (UHF beta reuses the alpha orbitals, UHF.hpp:206-215)
-    if (int rc = diag_to_P(0, b->H.p)) return rc;
-    if (!sl[1].empty()) {
-        GemmBatch g(b->scratch);
-        for (size_t k = 0; k < sl[1].size(); ++k) {
-            const MatSlot& m = sl[1][k];
-            g.add(m.n, m.n, b->mol[who[1][k]].nocc[1], false, true, b->C[0].p + m.off, b->C[0].p + m.off,
-                  b->P[1].p + m.off, m.n, m.n, m.n);
-        }
-        if (int rc = g.run(1.0, 0.0, st)) return rc;
-    }
+    if (int rc = diag_to_P(1, same(b->H))) return rc;
+    if (int rc = gemm(b, 1, 2, false, true, true, same(b->C[0]), same(b->C[0]), P)) return rc;
+    UNO_HIP(hipStreamSynchronize(st));
+    double diag_s = elapsed(b->ev_diag);
     double eps = o.eps;
-    std::vector<double> hs(4 * (size_t)nm + 8);
     int ndiis = 0, slot_next = 0;
     std::vector<double> Bm((size_t)nm * kBatchDiis * kBatchDiis, 0.0);
+    static_assert(kBatchDiis <= kMaxLin && kBatchDiis + 4 <= kMaxDots, "one launch per combination and per row");
+    LinSources hist;
+    for (int j = 0; j < kBatchDiis; ++j)
+        for (int s = 0; s < 2; ++s) hist.s[j][s] = b->dF[j][s].p;
     int iteration = 0;
     double fock_s = 0.0;
     int nstopped = 0;
     double wall99 = -1.0;
+    // Two waits an iteration: for the energies and the DIIS row, whose coefficients the host solves
+    // for, and for the density changes, which decide who stops.
     while (true) {
-        b->scratch.reset();   // the previous iteration ended synchronised
-        // densities of the build: D1 = Pa, D2 = Pb (zero for closed shells), D0 = D1 + D2
-        const auto tf = clk::now();
-        UNO_HIP(hipMemcpyAsync(b->D1.p, b->P[0].p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
-        UNO_HIP(hipMemcpyAsync(b->D2.p, b->P[1].p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
-        UNO_HIP(k_axpby(S, 1.0, b->D1.p, 1.0, b->D2.p, b->D0.p, st));
+        const int n0 = b->nslot[0], n = n0 + b->nslot[1];
+        UNO_HIP(hipEventRecord(b->ev_fock[0], st));
+        UNO_HIP(batch_densities(S, P, b->D0.p, both(b->Pold), st));
         if (int rc = batch_fock(b)) return rc;
-        UNO_HIP(batch_sym((int)sl[0].size(), dsl[0].p, b->W0.p, b->G[0].p, false, st));
-        if (!sl[1].empty()) UNO_HIP(batch_sym((int)sl[1].size(), dsl[1].p, b->W1.p, b->G[1].p, false, st));
-        fock_s += secs(tf, clk::now());
-        // energies: e1 = tr(Pa H) + tr(Pb H), e2 = tr(Pa Ga) + tr(Pb Gb)
-        double* r = b->red.p;
-        const int n0 = (int)sl[0].size();
-        UNO_HIP(batch_dot(n0, dsl[0].p, b->P[0].p, b->H.p, r, false, st));
-        UNO_HIP(batch_dot(n0, dsl[0].p, b->P[1].p, b->H.p, r, true, st));
-        UNO_HIP(batch_dot(n0, dsl[0].p, b->P[0].p, b->G[0].p, r + nm, false, st));
-        UNO_HIP(batch_dot(n0, dsl[0].p, b->P[1].p, b->G[1].p, r + nm, true, st));
-        UNO_HIP(hipMemcpyAsync(hs.data(), r, 2 * (size_t)nm * sizeof(double), hipMemcpyDeviceToHost, st));
+        UNO_HIP(batch_sym(n, b->slots.p, both(b->W), both(b->G), st));
+        UNO_HIP(hipEventRecord(b->ev_fock[1], st));
+        // F = H + G and its DIIS error X^T (FPS - SPF) X, FPS - SPF = FPS - (FPS)^T, on every active
+        // slot (one shared history position per iteration)
+        const int slot = slot_next;
+        slot_next = (slot_next + 1) % kBatchDiis;
+        if (ndiis < kBatchDiis) ++ndiis;
+        const Store F = both(b->dF[slot]), E = both(b->dE[slot]);
+        UNO_HIP(batch_add(n, b->slots.p, b->H.p, both(b->G), F, st));
+        if (int rc = gemm(b, 0, 2, false, false, false, F, P, Tm)) return rc;
+        if (int rc = gemm(b, 0, 2, false, false, false, Tm, same(b->S), Fp)) return rc;
+        UNO_HIP(batch_antisym(n, b->slots.p, Fp, Tm2, st));
+        if (int rc = gemm(b, 0, 2, false, false, false, Tm2, X, Tm)) return rc;
+        if (int rc = gemm(b, 0, 2, true, false, false, X, Tm, E)) return rc;
+        // energies: e1 = tr(Pa H) + tr(Pb H), e2 = tr(Pa Ga) + tr(Pb Gb), from the slots of spin 0; and
+        // the B-matrix row of the new error: sum over spins of <E_new, E_j>
+        DotPairs q{};
+        q.add(P.s[0], nullptr, b->H.p, nullptr);
+        q.add(P.s[1], nullptr, b->H.p, nullptr);
+        q.add(P.s[0], nullptr, b->G[0].p, nullptr);
+        q.add(P.s[1], nullptr, b->G[1].p, nullptr);
+        for (int j = 0; j < ndiis; ++j) q.add(E.s[0], E.s[1], b->dE[j][0].p, b->dE[j][1].p);
+        UNO_HIP(batch_dots(n, b->slots.p, q, b->red.p, st));
+        UNO_HIP(hipMemcpyAsync(b->h_dots, b->red.p, (size_t)q.n * n * sizeof(double), hipMemcpyDeviceToHost, st));
         UNO_HIP(hipStreamSynchronize(st));
+        fock_s += elapsed(b->ev_fock);
+        auto dot = [&](int pair, int k) { return b->h_dots[(size_t)pair * n + k]; };
+        std::vector<double> row((size_t)nm * kBatchDiis, 0.0);
+        for (int k = 0; k < n; ++k)
+            for (int j = 0; j < ndiis; ++j) row[(size_t)b->who[k] * kBatchDiis + j] += dot(4 + j, k);
+        std::vector<int> first(nm, -1);   // a molecule's spin-0 slot
         for (int k = 0; k < n0; ++k) {
-            BatchMol& x = b->mol[who[0][k]];
-            const double e1 = hs[k], e2 = hs[nm + k];
+            const int m = b->who[k];
+            BatchMol& x = b->mol[m];
+            const double e1 = dot(0, k) + dot(1, k), e2 = dot(2, k) + dot(3, k);
             x.energy = x.uhf ? e1 + 0.5 * e2 : 2.0 * e1 + e2;
             x.ediff = x.energy - x.eold;
             x.eold = x.energy;
             if (iteration == 0) x.init_energy = x.energy + x.nuc;
-        }
-        // F = H + G; DIIS on every active slot (one shared history position per iteration)
-        for (int s = 0; s < 2; ++s) UNO_HIP(k_axpby(S, 1.0, b->H.p, 1.0, b->G[s].p, b->F[s].p, st));
-        const int slot = slot_next;
-        slot_next = (slot_next + 1) % kBatchDiis;
-        if (ndiis < kBatchDiis) ++ndiis;
-        for (int s = 0; s < 2; ++s) {
-            if (sl[s].empty()) continue;
-            UNO_HIP(hipMemcpyAsync(b->dF[slot][s].p, b->F[s].p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
-            GemmBatch g1(b->scratch), g2(b->scratch), g3(b->scratch), g4(b->scratch);
-            for (const MatSlot& m : sl[s]) g1.add(m.n, m.n, m.n, false, false, b->F[s].p + m.off, b->P[s].p + m.off, b->Tm.p + m.off, m.n, m.n, m.n);
-            if (int rc = g1.run(1.0, 0.0, st)) return rc;
-            for (const MatSlot& m : sl[s]) g2.add(m.n, m.n, m.n, false, false, b->Tm.p + m.off, b->S.p + m.off, b->Fp.p + m.off, m.n, m.n, m.n);
-            if (int rc = g2.run(1.0, 0.0, st)) return rc;
-            // FPS - SPF = FPS - (FPS)^T
-            UNO_HIP(batch_sym((int)sl[s].size(), dsl[s].p, b->Fp.p, b->Tm2.p, false, st));
-            UNO_HIP(k_axpby(S, 2.0, b->Fp.p, -1.0, b->Tm2.p, b->Tm2.p, st));
-            for (const MatSlot& m : sl[s]) g3.add(m.n, m.n, m.n, false, false, b->Tm2.p + m.off, b->X.p + m.off, b->Tm.p + m.off, m.n, m.n, m.n);
-            if (int rc = g3.run(1.0, 0.0, st)) return rc;
-            for (const MatSlot& m : sl[s]) g4.add(m.n, m.n, m.n, true, false, b->X.p + m.off, b->Tm.p + m.off, b->dE[slot][s].p + m.off, m.n, m.n, m.n);
-            if (int rc = g4.run(1.0, 0.0, st)) return rc;
-        }
-        // B-matrix row of the new vector: sum over spins of <E_new, E_j>
-        std::vector<double> row((size_t)kBatchDiis * nm, 0.0);
-        for (int j = 0; j < ndiis; ++j) {
-            UNO_HIP(batch_dot(n0, dsl[0].p, b->dE[slot][0].p, b->dE[j][0].p, r, false, st));
-            std::vector<double> t0v(n0);
-            UNO_HIP(hipMemcpyAsync(t0v.data(), r, n0 * sizeof(double), hipMemcpyDeviceToHost, st));
-            std::vector<double> t1v(sl[1].size());
-            if (!sl[1].empty()) {
-                UNO_HIP(batch_dot((int)sl[1].size(), dsl[1].p, b->dE[slot][1].p, b->dE[j][1].p, r + nm, false, st));
-                UNO_HIP(hipMemcpyAsync(t1v.data(), r + nm, t1v.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-            }
-            UNO_HIP(hipStreamSynchronize(st));
-            for (int k = 0; k < n0; ++k) row[(size_t)who[0][k] * kBatchDiis + j] = t0v[k];
-            for (size_t k = 0; k < t1v.size(); ++k) row[(size_t)who[1][k] * kBatchDiis + j] += t1v[k];
-        }
-        std::vector<double> coef((size_t)n0 * kBatchDiis, 0.0);
-        bool any = false;
-        for (int k = 0; k < n0; ++k) {
-            const int m = who[0][k];
             double* Bmm = &Bm[(size_t)m * kBatchDiis * kBatchDiis];
             for (int j = 0; j < ndiis; ++j) Bmm[slot * kBatchDiis + j] = Bmm[j * kBatchDiis + slot] = row[(size_t)m * kBatchDiis + j];
-            coef[(size_t)k * kBatchDiis + slot] = 1.0;
-            if (ndiis >= 2 && diis_coefficients(Bmm, kBatchDiis, ndiis, slot, &coef[(size_t)k * kBatchDiis]) >= 2)
-                any = true;
+            double* ck = b->h_coef + (size_t)k * kMaxLin;
+            std::fill(ck, ck + kMaxLin, 0.0);
+            ck[slot] = 1.0;
+            if (ndiis >= 2) diis_coefficients(Bmm, kBatchDiis, ndiis, slot, ck);
+            first[m] = k;
         }
-        if (any) {
-            for (int s = 0; s < 2; ++s) {
-                if (sl[s].empty()) continue;
-                std::vector<const double*> src(kBatchDiis);
-                for (int j = 0; j < kBatchDiis; ++j) src[j] = b->dF[j][s].p;
-                const double** dsrc = nullptr;
-                UNO_HIP(b->scratch.upload(src.data(), src.size(), st, &dsrc));
-                // coefficients of slot k of spin s: the molecule's row (spin 1 slots are a subset)
-                std::vector<double> cs((size_t)sl[s].size() * kBatchDiis);
-                for (size_t k = 0; k < sl[s].size(); ++k) {
-                    const int m = who[s][k];
-                    const size_t k0 = std::find(who[0].begin(), who[0].end(), m) - who[0].begin();
-                    std::copy(&coef[k0 * kBatchDiis], &coef[k0 * kBatchDiis] + kBatchDiis, &cs[k * kBatchDiis]);
-                }
-                double* dcs = nullptr;
-                UNO_HIP(b->scratch.upload(cs.data(), cs.size(), st, &dcs));
-                UNO_HIP(batch_lincomb((int)sl[s].size(), dsl[s].p, kBatchDiis, dcs, dsrc, b->F[s].p, st));
-                UNO_HIP(hipStreamSynchronize(st));
-            }
-        }
+        for (int k = n0; k < n; ++k)
+            std::copy_n(b->h_coef + (size_t)first[b->who[k]] * kMaxLin, kMaxLin, b->h_coef + (size_t)k * kMaxLin);
+        UNO_HIP(hipMemcpyAsync(b->coef.p, b->h_coef, (size_t)n * kMaxLin * sizeof(double), hipMemcpyHostToDevice, st));
+        UNO_HIP(batch_lincomb(n, b->slots.p, b->coef.p, hist, both(b->F), st));
         // new densities
-        for (int s = 0; s < 2; ++s)
-            UNO_HIP(hipMemcpyAsync(b->Pold[s].p, b->P[s].p, S * sizeof(double), hipMemcpyDeviceToDevice, st));
-        for (int s = 0; s < 2; ++s)
-            if (int rc = diag_to_P(s, b->F[s].p)) return rc;
-        UNO_HIP(batch_diffnorm(n0, dsl[0].p, b->P[0].p, b->Pold[0].p, r, st));
-        if (!sl[1].empty()) UNO_HIP(batch_diffnorm((int)sl[1].size(), dsl[1].p, b->P[1].p, b->Pold[1].p, r + nm, st));
-        std::vector<double> pd(2 * (size_t)nm, 0.0);
-        UNO_HIP(hipMemcpyAsync(pd.data(), r, 2 * (size_t)nm * sizeof(double), hipMemcpyDeviceToHost, st));
+        if (int rc = diag_to_P(2, both(b->F))) return rc;
+        UNO_HIP(batch_diffnorm(n, b->slots.p, P, both(b->Pold), b->red.p, st));
+        UNO_HIP(hipMemcpyAsync(b->h_pdiff, b->red.p, n * sizeof(double), hipMemcpyDeviceToHost, st));
         UNO_HIP(hipStreamSynchronize(st));
+        diag_s += elapsed(b->ev_diag);
         ++iteration;
         bool changed = false;
-        for (int k = 0; k < n0; ++k) {
-            BatchMol& x = b->mol[who[0][k]];
-            x.pdiff = pd[k];
+        for (int k = 0; k < n; ++k) {
+            BatchMol& x = b->mol[b->who[k]];
+            x.pdiff = k < n0 ? b->h_pdiff[k] : x.pdiff + b->h_pdiff[k];
             x.iterations = iteration;
         }
-        for (size_t k = 0; k < sl[1].size(); ++k) b->mol[who[1][k]].pdiff += pd[nm + k];
         for (int k = 0; k < n0; ++k) {
-            BatchMol& x = b->mol[who[0][k]];
+            BatchMol& x = b->mol[b->who[k]];
             bool conv = false;
             if (iteration >= 2) {
                 if (o.cflag == 0) conv = x.ediff < eps;
@@ -707,7 +639,7 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
         for (const BatchMol& x : b->mol) any_active = any_active || x.active;
         if (!any_active) break;
         if (changed) {
-            if (int rc = refresh_slots()) return rc;
+            if (int rc = refresh_slots(b)) return rc;
         }
     }
     const double wall = secs(t0, clk::now());
