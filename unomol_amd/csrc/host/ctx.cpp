@@ -39,38 +39,37 @@ EriArgs base_args(uno_ctx* c) {
     return a;
 }
 
-// order: the pairs by run key ascending, then bound descending, ties in their own order.  A
-// counting sort into the runs, then pieces of a run sorted by the threads and merged (64 waters,
-// 60 305 pairs: 0.6 ms; one stable sort of the indices through the two arrays: 4.2 ms).
+// order: the pairs by run key ascending, then bound descending, ties in their own order: a radix sort of
+// the bounds' bits (positive numbers order like their bits), 11 at a time, and a last pass by
+// run key.  On one thread: a parallel region that finds its threads asleep costs milliseconds (a
+// parallel merge sort: 19 ms in a new program's context of 16 waters, 0.6 warm).  The stage around it,
+// 32 waters: 1.05 ms, with one stable sort of the indices through the two arrays 2.1.
 static void sort_runs(const std::vector<int>& runkey, const std::vector<double>& q, std::vector<int>& order) {
-    constexpr int kKeys = kNumPairClasses * kNumBuckets, kPiece = 2048;
-    const int np = (int)runkey.size();
-    std::vector<std::pair<double, int>> v(np);
-    int off[kKeys + 1] = {}, at[kKeys];
-    for (int p = 0; p < np; ++p) ++off[runkey[p] + 1];
-    for (int r = 0; r < kKeys; ++r) off[r + 1] += off[r];
-    std::copy(off, off + kKeys, at);
-    for (int p = 0; p < np; ++p) v[at[runkey[p]]++] = {-q[p], p};
-    std::vector<std::pair<int, int>> piece;
-    for (int r = 0; r < kKeys; ++r)
-        for (int lo = off[r]; lo < off[r + 1]; lo += kPiece) piece.emplace_back(lo, std::min(lo + kPiece, off[r + 1]));
-#pragma omp parallel for schedule(dynamic)
-    for (size_t k = 0; k < piece.size(); ++k) std::sort(v.begin() + piece[k].first, v.begin() + piece[k].second);
-    struct Merge {
-        int lo, mid, hi;
+    struct Rec {
+        std::uint64_t key;
+        int pair;
     };
-    std::vector<Merge> merge;
-    for (long len = kPiece; len < np; len *= 2) {
-        merge.clear();
-        for (int r = 0; r < kKeys; ++r)
-            for (long lo = off[r]; lo + len < off[r + 1]; lo += 2 * len)
-                merge.push_back({(int)lo, (int)(lo + len), (int)std::min<long>(lo + 2 * len, off[r + 1])});
-#pragma omp parallel for schedule(dynamic)
-        for (size_t k = 0; k < merge.size(); ++k)
-            std::inplace_merge(v.begin() + merge[k].lo, v.begin() + merge[k].mid, v.begin() + merge[k].hi);
+    const int np = (int)runkey.size();
+    constexpr int kBits = 11, kDigits = 1 << kBits;
+    static_assert(kNumPairClasses * kNumBuckets <= kDigits, "run keys are one digit");
+    std::vector<Rec> v(np), w(np);
+    for (int p = 0; p < np; ++p) {
+        std::uint64_t b;
+        std::memcpy(&b, &q[p], sizeof b);
+        v[p] = Rec{~b, p};
     }
-#pragma omp parallel for schedule(static)
-    for (int p = 0; p < np; ++p) order[p] = v[p].second;
+    std::vector<int> at(kDigits + 1);
+    auto pass = [&](auto digit) {
+        std::fill(at.begin(), at.end(), 0);
+        for (const Rec& r : v) ++at[digit(r) + 1];
+        if (np && at[digit(v[0]) + 1] == np) return;   // all alike
+        for (int k = 0; k < kDigits; ++k) at[k + 1] += at[k];
+        for (const Rec& r : v) w[at[digit(r)]++] = r;
+        v.swap(w);
+    };
+    for (int s = 0; s < 64; s += kBits) pass([s](const Rec& r) { return (int)(r.key >> s & (kDigits - 1)); });
+    pass([&](const Rec& r) { return runkey[r.pair]; });
+    for (int p = 0; p < np; ++p) order[p] = v[p].pair;
 }
 
 int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
@@ -237,7 +236,7 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     std::vector<PrimPair> prims2(c->prims.size());
     std::vector<double> q2(np);
     std::vector<int> newidx(np);
-#pragma omp parallel for schedule(static)
+#pragma omp parallel for schedule(static) if (np >= 16384)   // below, one thread is done before the others wake
     for (int k = 0; k < np; ++k) {
         PairHdr h = c->pairs[order[k]];
         const int p0 = h.prim0;
