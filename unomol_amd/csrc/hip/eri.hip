@@ -297,7 +297,11 @@ FockConfig fock_default(int cb, int ck, int mode, int ncols, int nsh, bool fp32,
     }
     f.mlds = 1;
     if (!ok(f)) f.mlds = 0;
-    if (f.variant && dens != 0) {
+    // (the exchange density rows in LDS cost a class the blocks they displace: only (ss|ss), which
+    // keeps its five blocks per compute unit with them, is faster, 3.63 -> 3.48 ms at 64 waters; of
+    // the others (ds|ss) goes 4.56 -> 3.96 ms without, the whole build 56.0 -> 54.8, the FP32 build
+    // of 37 waters 17.8 -> 16.7)
+    if (f.variant && (dens > 0 || (dens < 0 && cb == 0))) {
         f.dlds = 1;
         if (!ok(f)) f.dlds = 0;
     }

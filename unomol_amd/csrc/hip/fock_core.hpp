@@ -25,9 +25,6 @@ namespace uno {
 // classes up to kLaneMaxComp components run one ket per lane (the component block in registers);
 // larger ones one quartet per wave
 constexpr int kLaneMaxComp = 162;
-#ifndef UNO_NT_COMP
-#define UNO_NT_COMP 0
-#endif
 // Rys tables of up to this many roots are staged in LDS by the kernels without LDS rows
 constexpr int kLdsTabMaxRoots = 3;
 // every quartet class: pair classes (0 ss, 1 ps, 2 pp, 3 ds, 4 dp, 5 dd) and shells
@@ -269,11 +266,15 @@ __host__ __device__ constexpr int dens_row_count() {
     return (ncart_c(LA) + ncart_c(LB)) * (MODE == kDigestUHF ? 2 : 1);
 }
 
-// threads of a block: the waves of a block share its LDS rows, so the classes whose registers
-// allow four waves per SIMD run eight waves a block
+// four waves a block share its LDS rows (eight: (ds|ss) of 64 waters 6.4 -> 4.9 ms, most other
+// classes and 16 waters slower)
+constexpr int kRowThreads = 256, kRowWaves = kRowThreads / 64;
+// waves per SIMD asked of the registers: the classes that miss two by little, 257 registers of (ds|ds)
+// and 312 of (ds|pp), gain from holding to it (64 waters 1.49 -> 1.12 and 2.17 -> 1.76 ms); the ones
+// that would spill more, from 350 on, lose (dd|ss 1.14 -> 1.76 ms)
 template <int LA, int LB, int LC, int LD>
-constexpr int row_threads() {
-    return ClassInfo<LA, LB, LC, LD>::NCOMP <= UNO_NT_COMP ? 512 : 256;
+constexpr int row_min_waves() {
+    return LA == 2 && LB == 0 && LC + LD == 2 ? 2 : 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -288,8 +289,7 @@ constexpr int row_threads() {
 // TL the Rys table.
 // ---------------------------------------------------------------------------
 template <int LA, int LB, int LC, int LD, int MODE, typename T, int ROWS, bool TL>
-__global__ __launch_bounds__((row_threads<LA, LB, LC, LD>())) void k_fock(const FockArgs a) {
-    constexpr int kRowThreads = row_threads<LA, LB, LC, LD>(), kRowWaves = kRowThreads / 64;
+__global__ __launch_bounds__(kRowThreads, (row_min_waves<LA, LB, LC, LD>())) void k_fock(const FockArgs a) {
     using CI = ClassInfo<LA, LB, LC, LD>;
     constexpr int NA = CI::NA, NB = CI::NB, NC = CI::NC, ND = CI::ND, NCOMP = CI::NCOMP, NR = CI::NR;
     constexpr bool FB = ROWS == kRowsAll, RW = ROWS != kRowsNone, F32 = sizeof(T) == 4;

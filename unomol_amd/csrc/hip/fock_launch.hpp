@@ -30,8 +30,8 @@ static hipError_t fock_launch_v(const FockArgs& a, size_t dyn, hipStream_t st) {
         attr = dyn;
     }
     unsigned grid = 1;
-    if (hipError_t e = fock_grid(kernel, row_threads<LA, LB, LC, LD>(), dyn, a.ncand, grid)) return e;
-    hipLaunchKernelGGL((k_fock<LA, LB, LC, LD, MODE, T, ROWS, TL>), dim3(grid), dim3((row_threads<LA, LB, LC, LD>())), dyn, st,
+    if (hipError_t e = fock_grid(kernel, kRowThreads, dyn, a.ncand, grid)) return e;
+    hipLaunchKernelGGL((k_fock<LA, LB, LC, LD, MODE, T, ROWS, TL>), dim3(grid), dim3(kRowThreads), dyn, st,
                        a);
     return hipGetLastError();
 }

@@ -21,7 +21,7 @@ constexpr int kLaneBlock = 256;   // lanes of a block of the lane kernels
 constexpr int kWaveSeg = 8;       // kets of a block of the wave kernels
 bool fock_is_wave(int bra_class, int ket_class);
 // the first of (force, 1, 2, 3) that fits the LDS budget at ncols columns (rows false: 0), with
-// what else fits; dens 0: no density rows
+// what else fits; density rows: dens 0 none, 1 where they fit, -1 where they pay
 FockConfig fock_default(int bra_class, int ket_class, int mode, int ncols, int nsh, bool fp32, bool rows, int force,
                         int dens);
 bool fock_config_fits(int bra_class, int ket_class, const FockConfig& f, int mode, int ncols, int nsh, bool fp32);

@@ -197,7 +197,7 @@ struct uno_ctx {
     // last steps: the small launches then run side by side
     int launch_streams = 3;
     uno::LaunchStreams ls;
-    int row_dens = -1;       // exchange density rows in LDS: -1 when they fit, 0 never, 1 forced where they fit
+    int row_dens = -1;       // exchange density rows in LDS: -1 where they pay, 0 never, 1 where they fit
     // autotuned configuration per launch (class pair, precision, UHF, mixed build); tuning = 1
     // while uno_autotune times the candidates
     std::map<std::tuple<int, int, int, int>, uno::FockConfig> tune;
