@@ -233,9 +233,10 @@ int uno_mlp_set_params(uno_mlp* m, const float* p) {
 int uno_mlp_forward(uno_mlp* m, long n, const float* X, float* Y) {
     if (!m || !X || !Y || n <= 0) { set_error("bad argument"); return UNO_EINVAL; }
     const int in = m->dims[0], out = m->dims.back();
-    const int chunk = 4096;
-    if (int rc = ensure_batch(m, chunk)) return rc;
     const size_t rows = (size_t)((n + 63) / 64) * 64;
+    // rows of a pass: as many as there are, to 16384 (a pass ends waiting for its copy)
+    const int chunk = (int)std::min<size_t>(std::max<size_t>(rows, 4096), 16384);
+    if (int rc = ensure_batch(m, chunk)) return rc;
     UNO_HIP(m->xin.alloc(rows * in));
     UNO_HIP(hipMemcpyAsync(m->xin.p, X, (size_t)n * in * sizeof(float), hipMemcpyHostToDevice, m->st));
     if (rows > (size_t)n) UNO_HIP(hipMemsetAsync(m->xin.p + (size_t)n * in, 0, (rows - n) * in * sizeof(float), m->st));
