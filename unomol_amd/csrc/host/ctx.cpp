@@ -236,7 +236,7 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     std::vector<PrimPair> prims2(c->prims.size());
     std::vector<double> q2(np);
     std::vector<int> newidx(np);
-#pragma omp parallel for schedule(static) if (np >= 16384)   // below, one thread is done before the others wake
+#pragma omp parallel for schedule(static) if (np >= 65536)   // below, one thread is done before the others wake
     for (int k = 0; k < np; ++k) {
         PairHdr h = c->pairs[order[k]];
         const int p0 = h.prim0;
