@@ -391,8 +391,8 @@ class Batch:
         return e, list(res)
 
     def set(self, key, value):
-        """Fock-build option: "graph" (capture and replay the build) or "queue" (work-queue
-        launches), 1 or 0."""
+        """Fock-build option: "graph" (capture and replay the build), 1 or 0, or "launch_streams";
+        "queue" is accepted and has no effect (every launch takes its tasks from a counter)."""
         N.check(N.lib().uno_batch_set(self.h, key.encode(), C.c_double(value)))
 
     def get(self, key):

@@ -906,6 +906,8 @@ hipError_t householder_tridiag(int n, EigWork& w, hipStream_t st) {
     if (n < 3) return hipErrorInvalidValue;   // the callers solve n <= 2 in closed form
     // reflector rows must be zero outside their support for the blocked back-transform
     UNO_LAUNCH_FILL((long)n * n, w.V, st);
+    // (one block while the registers of eight waves hold the matrix: a whole solve of 192 takes 0.92 ms,
+    // of 193 by column launches and blocked back-transform 1.54)
     if (n <= kHhOneN) {
         hipLaunchKernelGGL(k_hh_one, dim3(1), dim3(512), 0, st, n, (const double*)w.A, w.V, w.tau, w.d, w.e);
         return hipGetLastError();

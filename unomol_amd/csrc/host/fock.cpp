@@ -44,8 +44,8 @@ LaunchStreams::~LaunchStreams() {
     if (fork) (void)hipEventDestroy(fork);
 }
 
-// candidate tasks from which a build lists the live ones first (below, the list costs a
-// launch and saves little: one water has 900 candidates, 16 waters 50 000)
+// candidate tasks from which a build lists the live ones first (below, the list costs a launch and
+// the blocks would find few dead ones)
 constexpr long long kListFrom = 8192;
 
 // lanes the chip holds at two waves per SIMD
