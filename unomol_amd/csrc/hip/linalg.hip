@@ -777,34 +777,19 @@ __global__ __launch_bounds__(256) void k_hh_col(int n, int k, int b0, double* A,
     }
 }
 
-// after the last reflector (step n-3): its w on the trailing 2 x 2 block, the update
-// there, and that block's d, e
-__global__ void k_hh_tail(int n, const double* A, const double* V, const double* tau, const double* P, const double* part,
-                          double* d, double* e) {
-    const int k = n - 3, r0 = n - 2, r1 = n - 1;
-    if (threadIdx.x == 0) {
-        const double K = 0.5 * tau[k] * (part[0] + part[1]);
-        const double* v = V + (long)k * n;
-        const double w0 = P[r0] - K * v[r0], w1 = P[r1] - K * v[r1];
-        d[r0] = A[(long)r0 * n + r0] - (v[r0] * w0 + w0 * v[r0]);
-        e[r0] = A[(long)r1 * n + r0] - (v[r1] * w0 + w1 * v[r0]);
-        d[r1] = A[(long)r1 * n + r1] - (v[r1] * w1 + w1 * v[r1]);
-        e[r1] = 0.0;
-    }
-    for (int j = n + threadIdx.x; j < eig_pad(n); j += 64) d[j] = e[j] = 0.0;
-}
-
-// The whole reduction in one block for n <= kHhOneN, the matrix in the registers of its 8 waves: a
-// column takes two barriers and two vectors through LDS instead of a launch, and every wave does
-// the vector work (reflector, K, w) for itself.  Row r lies in slot r / 32 of the 16 lanes
-// (r / 4 % 8, r % 4) = (wave, row of lanes), column j in lane j % 16 of them: a sum over the columns
-// is four DPP moves for four rows at once.  n = 133: 313 us (one row per wave, six moves each: 408 us;
-// a launch per column: 0.77 ms).
+// The reduction of the trailing m = n - k0 <= kHhOneN rows (all of a small matrix) in one block, the
+// matrix in the registers of its 8 waves: a column takes two barriers and two vectors through LDS
+// instead of a launch, and every wave does the vector work (reflector, K, w) for itself.  After
+// k0 > 0 column launches the update of step k0-1 is still to be applied (Pp, partp: its p and
+// terms of p.v).  Row r lies in slot r / 32 of the 16 lanes (r / 4 % 8, r % 4) = (wave, row of
+// lanes), column j in lane j % 16 of them: a sum over the columns is four DPP moves for four
+// rows at once.  n = 133: 313 us (one row per wave, six moves each: 408 us; a launch per
+// column: 0.77 ms).
 constexpr int kHhOneN = 192, kHhSlots = kHhOneN / 32, kHhCols = kHhOneN / 16;
-__global__ __launch_bounds__(512) void k_hh_one(int n, const double* __restrict__ A0, double* V, double* tau, double* d,
-                                                double* e) {
+__global__ __launch_bounds__(512) void k_hh_one(int n, int k0, const double* __restrict__ A0, double* V, double* tau, double* d,
+                                                double* e, const double* __restrict__ Pp, const double* __restrict__ partp) {
     __shared__ double sx[kHhOneN], sp[kHhOneN];
-    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15;
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, m = n - k0;
     const int row0 = __builtin_amdgcn_readfirstlane(tid >> 6) * 4, row = row0 + (lane >> 4);
     double a[kHhSlots][kHhCols];
 #pragma unroll
@@ -812,10 +797,32 @@ __global__ __launch_bounds__(512) void k_hh_one(int n, const double* __restrict_
 #pragma unroll
         for (int c = 0; c < kHhCols; ++c) {
             const int r = 32 * s + row, j = col + 16 * c;
-            a[s][c] = (r < n && j < n) ? A0[(long)r * n + j] : 0.0;
+            a[s][c] = (r < m && j < m) ? A0[(long)(k0 + r) * n + k0 + j] : 0.0;
         }
+    if (k0 > 0) {   // the update of step k0 - 1: its v into sx, its w into sp
+        double t = 0.0;
+        for (int j = lane; j < m; j += 64) t += partp[j];
+        const double K = 0.5 * tau[k0 - 1] * wave_total(t);
+        for (int j = tid; j < kHhOneN; j += 512) {
+            const double v = j < m ? V[(long)(k0 - 1) * n + k0 + j] : 0.0;
+            sx[j] = v;
+            sp[j] = j < m ? Pp[k0 + j] - K * v : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < kHhSlots; ++s) {
+            const double vr = sx[32 * s + row], wr = sp[32 * s + row];
+#pragma unroll
+            for (int c = 0; c < kHhCols; ++c) a[s][c] -= vr * sp[col + 16 * c] + wr * sx[col + 16 * c];
+        }
+        __syncthreads();
+    }
     for (int j = tid; j < kHhOneN; j += 512) sp[j] = 0.0;
-    for (int k = 0; k + 2 < n; ++k) {
+    V += (long)k0 * n + k0;
+    tau += k0;
+    d += k0;
+    e += k0;
+    for (int k = 0; k + 2 < m; ++k) {
 #pragma unroll
         for (int s = 0; s < kHhSlots; ++s)
             if (32 * s + row == k) {
@@ -839,7 +846,7 @@ __global__ __launch_bounds__(512) void k_hh_one(int n, const double* __restrict_
         if (tid < 16) {
 #pragma unroll
             for (int c = 0; c < kHhCols; ++c)
-                if (col + 16 * c > k && col + 16 * c < n) V[(long)k * n + col + 16 * c] = v[c];
+                if (col + 16 * c > k && col + 16 * c < m) V[(long)k * n + col + 16 * c] = v[c];
             if (tid == 0) {
                 tau[k] = t;
                 d[k] = dk;
@@ -848,7 +855,7 @@ __global__ __launch_bounds__(512) void k_hh_one(int n, const double* __restrict_
         }
 #pragma unroll
         for (int s = 0; s < kHhSlots; ++s) {
-            if (32 * s + row0 + 3 > k && 32 * s + row0 < n) {   // the same in the wave
+            if (32 * s + row0 + 3 > k && 32 * s + row0 < m) {   // the same in the wave
                 double acc = 0.0;
 #pragma unroll
                 for (int c = 0; c < kHhCols; ++c) acc = fma(a[s][c], v[c], acc);
@@ -874,7 +881,7 @@ __global__ __launch_bounds__(512) void k_hh_one(int n, const double* __restrict_
         for (int c = 0; c < kHhCols; ++c) w[c] -= K * v[c];
 #pragma unroll
         for (int s = 0; s < kHhSlots; ++s)
-            if (32 * s + row0 + 3 > k && 32 * s + row0 < n) {
+            if (32 * s + row0 + 3 > k && 32 * s + row0 < m) {
                 const int r = 32 * s + row;
                 const double wr = r > k ? sp[r] - K * vr[s] : 0.0;
 #pragma unroll
@@ -887,12 +894,12 @@ __global__ __launch_bounds__(512) void k_hh_one(int n, const double* __restrict_
 #pragma unroll
         for (int c = 0; c < kHhCols; ++c) {
             const int j = col + 16 * c;
-            if (r < n && r == j && r >= n - 2) d[r] = a[s][c];
-            if (r == n - 1 && j == n - 2) e[j] = a[s][c];
+            if (r < m && r == j && r >= m - 2) d[r] = a[s][c];
+            if (r == m - 1 && j == m - 2) e[j] = a[s][c];
         }
     }
-    if (tid == 0) e[n - 1] = 0.0;
-    for (int j = n + tid; j < eig_pad(n); j += 512) d[j] = e[j] = 0.0;
+    if (tid == 0) e[m - 1] = 0.0;
+    for (int j = n + tid; j < eig_pad(n); j += 512) d[j - k0] = e[j - k0] = 0.0;
 }
 
 // dynamic LDS above 64 KB has to be allowed; always the same `top`, so that threads with different
@@ -906,25 +913,23 @@ hipError_t householder_tridiag(int n, EigWork& w, hipStream_t st) {
     if (n < 3) return hipErrorInvalidValue;   // the callers solve n <= 2 in closed form
     // reflector rows must be zero outside their support for the blocked back-transform
     UNO_LAUNCH_FILL((long)n * n, w.V, st);
-    // (one block while the registers of eight waves hold the matrix: a whole solve of 192 takes 0.92 ms,
-    // of 193 by column launches and blocked back-transform 1.54)
-    if (n <= kHhOneN) {
-        hipLaunchKernelGGL(k_hh_one, dim3(1), dim3(512), 0, st, n, (const double*)w.A, w.V, w.tau, w.d, w.e);
-        return hipGetLastError();
-    }
+    // column launches down to the size that one block's registers hold: a whole solve of 192 takes
+    // 0.90 ms; of 193, 1.12, and 1.54 by column launches to the end
+    const int k1 = std::max(0, n - kHhOneN);
     // the inverse-iteration work space is unused until the tridiagonal is done: p and the
     // rows' terms of p.v of the steps of even and odd k live there
     double* P[2] = {w.wk, w.wk + n};
     double* part[2] = {w.wk + 2L * n, w.wk + 3L * n};
     const size_t lds = 3 * (size_t)n * sizeof(double);
-    if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_hh_col), lds, 150 * 1024)) return er;
-    for (int k = 0; k + 2 < n; ++k) {
+    if (k1 > 0)
+        if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_hh_col), lds, 150 * 1024)) return er;
+    for (int k = 0; k < k1; ++k) {
         const int b0 = (k + 1) / 32 * 8;
         hipLaunchKernelGGL(k_hh_col, dim3((unsigned)((n + 3) / 4 - b0)), dim3(256), lds, st, n, k, b0, w.A, w.V, w.tau, w.d, w.e,
                            P[(k + 1) & 1], part[(k + 1) & 1], P[k & 1], part[k & 1]);
     }
-    hipLaunchKernelGGL(k_hh_tail, dim3(1), dim3(64), 0, st, n, w.A, w.V, w.tau, P[(n - 3) & 1], part[(n - 3) & 1], w.d,
-                       w.e);
+    hipLaunchKernelGGL(k_hh_one, dim3(1), dim3(512), 0, st, n, k1, (const double*)w.A, w.V, w.tau, w.d, w.e,
+                       (const double*)P[(k1 + 1) & 1], (const double*)part[(k1 + 1) & 1]);
     return hipGetLastError();
 }
 

@@ -1,8 +1,8 @@
 // Dense symmetric eigensolver for device-resident matrices (contract of the
 // reference's SymmPack::rsp, SymmPack.cpp:272-288: eigenvalues ascending, eigenvectors
 // in the columns of a row-major Z).  All steps run on the GPU:
-//   1. Householder tridiagonalisation A = Q T Q^T (one block up to n = 192, above it one launch
-//      per column: the previous rank-2 update fused with the next matrix-vector product);
+//   1. Householder tridiagonalisation A = Q T Q^T (one block for the last 192 rows, before them one
+//      launch per column: the previous rank-2 update fused with the next matrix-vector product);
 //   2. eigenvalues of T by multisection on Sturm counts, one eigenvalue per wave;
 //   3. eigenvectors of T by inverse iteration, one per thread (the vectors stored as the
 //      columns of Yt, so a wave's accesses coalesce), then two-pass modified Gram-Schmidt
