@@ -99,6 +99,8 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     for (const Shell& s : B.sh)
         for (double a : s.a) amin = std::min(amin, a);
     const double qmin = 2.0 * amin;
+    std::vector<double> low(nsh);   // a shell's most diffuse exponent
+    for (int a = 0; a < nsh; ++a) low[a] = *std::min_element(B.sh[a].a.begin(), B.sh[a].a.end());
     c->pairs.clear();
     c->prims.clear();
     c->pair_of.assign((size_t)nsh * nsh, -1);
@@ -125,6 +127,12 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
                 h.AB[x] = A[x] - Bc[x];
                 ab2 += h.AB[x] * h.AB[x];
             }
+            // no primitive pair of distant shells passes the bound below where the largest overlap
+            // and the smallest exponent sum together do not (1e-6 for the roundings)
+            const double plow = low[a] + low[bsh];
+            if (kTwoPi25 * std::exp(-low[a] * low[bsh] / plow * ab2) / (plow * qmin * std::sqrt(plow + qmin)) <
+                c->primcut * (1.0 - 1e-6))
+                continue;
             h.f1 = B.off[s1];
             h.f2 = B.off[s2];
             h.prim0 = (int)pv.size();   // within this shell's list; made global below
@@ -236,7 +244,7 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     std::vector<PrimPair> prims2(c->prims.size());
     std::vector<double> q2(np);
     std::vector<int> newidx(np);
-#pragma omp parallel for schedule(static) if (np >= 65536)   // below, one thread is done before the others wake
+#pragma omp parallel for schedule(static) if (np >= 32768)   // below, one thread is done before the others wake
     for (int k = 0; k < np; ++k) {
         PairHdr h = c->pairs[order[k]];
         const int p0 = h.prim0;
