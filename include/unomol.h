@@ -315,7 +315,9 @@ int uno_shell_rotation(int l, const double* Q, double* M);
  * builds from the core-Hamiltonian guess; opts->cflag / eps / maxits as for uno_scf_run.
  * The Fock build's launches (one per class pair and shell kind over all molecules) skip
  * converged molecules by a device flag, and the whole build is captured once per run as a
- * HIP graph and replayed every iteration. */
+ * HIP graph and replayed every iteration.  Orbitals whose levels coincide (within 1e-10 Eh)
+ * across the Fermi level of a Fock matrix are filled in the order they had in the iteration before, so
+ * that a half-filled exactly degenerate level does not depend on rounding. */
 typedef struct uno_batch uno_batch;
 int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_batch** out);
 int uno_batch_destroy(uno_batch* batch);

@@ -429,6 +429,72 @@ hipError_t batched_jacobi(int nslot, const MatSlot* slots, Store A, Store V, Sto
 }
 
 // ---------------------------------------------------------------------------
+// Occupation of coinciding levels.  Where the highest occupied and the lowest empty level lie
+// within kTieLevel of each other (a pi pair of a linear molecule that the first builds leave half
+// filled: exactly degenerate, 2e-16 apart), rounding decides which of their orbitals Jacobi lists
+// first, and with it the order in which the Fock atomics arrived: an HF molecule converged to
+// |dE| < 1e-8 then has one of two mirror-image densities, 2.4e-7 apart, and from run to run not the
+// same.  Such orbitals keep the order that they had in the iteration before.  Z holds the eigenvectors
+// over that iteration's orbitals, so the first of the level becomes the projection into it of the
+// first orbital whose projection is at least half as long as the longest, the next the same among
+// what is orthogonal to it.  (Exactly equal levels come out in that order anyway, ties by index.)  kTieLevel is
+// far above the rounding of the levels (1e-14) and far below what a distortion splits them by.
+// One block per slot; without such levels (nearly always) it reads two numbers and ends.
+// ---------------------------------------------------------------------------
+constexpr double kTieLevel = 1e-10;
+__global__ __launch_bounds__(256) void k_batch_ties(const MatSlot* __restrict__ slots, Store evals, Store Zs) {
+    __shared__ double red[4], w[256];
+    __shared__ int first;
+    const MatSlot m = slots[blockIdx.x];
+    const int n = m.n;
+    if (m.nocc <= 0 || m.nocc >= n) return;
+    const double* ev = evals.s[m.spin] + m.off;
+    if (!(ev[m.nocc] - ev[m.nocc - 1] <= kTieLevel)) return;
+    double* Z = Zs.s[m.spin] + m.off;
+    int lo = m.nocc - 1, hi = m.nocc + 1;
+    while (lo > 0 && ev[lo] - ev[lo - 1] <= kTieLevel) --lo;
+    while (hi < n && ev[hi] - ev[hi - 1] <= kTieLevel) ++hi;
+    const int r = threadIdx.x, lane = r & 63;
+    double* row = Z + (long)r * n;   // n <= 256: a row per thread
+    for (int c0 = lo; c0 < m.nocc; ++c0) {
+        double s = 0.0;
+        if (r < n)
+            for (int c = c0; c < hi; ++c) s = fma(row[c], row[c], s);
+        double big = s;
+        for (int o = 32; o >= 1; o >>= 1) big = fmax(big, __shfl_xor(big, o, 64));
+        if (lane == 0) red[r >> 6] = big;
+        if (r == 0) first = n;
+        __syncthreads();
+        big = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+        if (r < n && s >= 0.25 * big) atomicMin(&first, r);
+        __syncthreads();
+        const int f = first;
+        if (f >= n) return;   // not a number
+        // the reflection of the level's orbitals that takes row f to (|row|, 0, ..): v = row - |row| e
+        if (r < hi - c0) w[r] = Z[(long)f * n + c0 + r];
+        __syncthreads();
+        double tail = 0.0;
+        for (int c = 1; c < hi - c0; ++c) tail = fma(w[c], w[c], tail);
+        const double x = w[0], len = sqrt(fma(x, x, tail));
+        const double v0 = x > 0.0 ? -tail / (x + len) : x - len, v2 = fma(v0, v0, tail);
+        if (v2 > 0.0 && r < n) {
+            double t = v0 * row[c0];
+            for (int c = 1; c < hi - c0; ++c) t = fma(w[c], row[c0 + c], t);
+            t *= 2.0 / v2;
+            row[c0] = fma(-t, v0, row[c0]);
+            for (int c = 1; c < hi - c0; ++c) row[c0 + c] = fma(-t, w[c], row[c0 + c]);
+        }
+        __syncthreads();
+    }
+}
+
+hipError_t batch_ties(int nslot, const MatSlot* slots, Store evals, Store Z, hipStream_t st) {
+    if (nslot <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_batch_ties, dim3(nslot), dim3(256), 0, st, slots, evals, Z);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // per-molecule helpers: one 256-thread block per slot
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double block_reduce_sum(double v, double* red) {

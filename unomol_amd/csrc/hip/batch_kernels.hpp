@@ -27,6 +27,10 @@ hipError_t grouped_gemm(int ntiles, const GemmTile* tiles, const MatSlot* slots,
 hipError_t batched_jacobi(int nslot, const MatSlot* slots, Store A, Store V, Store evals, Store Z, int maxn, int max_sweeps,
                           hipStream_t st);
 
+// the eigenvectors (columns of Z, n <= 256) of levels that coincide across a slot's Fermi level, in the
+// order of Z's rows, which rounding does not decide
+hipError_t batch_ties(int nslot, const MatSlot* slots, Store evals, Store Z, hipStream_t st);
+
 // out[q nslot + k] = sum_ij A_q,ij B_q,ij over slot k, for the pairs q that name stores of its spin
 constexpr int kMaxDots = 12;
 struct DotPairs {

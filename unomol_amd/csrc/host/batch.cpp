@@ -516,8 +516,11 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
         }
         UNO_HIP(batched_jacobi(b->nslot[0] + (ns > 1 ? b->nslot[1] : 0), b->slots.p, A, both(b->V), both(b->ev), E, b->maxn, 50,
                                st));
-        if (nw)
+        if (nw) {
+            // (not for the core Hamiltonian, whose levels come out the same in every run)
+            UNO_HIP(batch_ties(b->nslot[0] + (ns > 1 ? b->nslot[1] : 0), b->slots.p, both(b->ev), E, st));
             if (int rc = gemm(b, 0, nw, false, false, false, Wp, Z, Wn)) return rc;
+        }
         for (int s = 0; s < ns; ++s) {
             std::swap(b->Wp[s], b->Wn[s]);
             b->warm[s] = true;
