@@ -117,7 +117,8 @@ struct GemmDetScope {
     GemmDetScope& operator=(const GemmDetScope&) = delete;
 };
 
-// eigensolver pieces (linalg.hip)
+// eigensolver pieces (linalg.hip), 3 <= n <= kEigMaxN
+constexpr int kEigMaxN = 6752;   // where a block's LDS ends (linalg.hip)
 struct EigWork {
     double* A;      // n x n working copy (destroyed)
     double* V;      // n x n reflector vectors (row k = v_k, zero outside its support)

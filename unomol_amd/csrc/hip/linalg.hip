@@ -904,13 +904,16 @@ __global__ __launch_bounds__(512) void k_hh_one(int n, int k0, const double* __r
 
 // dynamic LDS above 64 KB has to be allowed; always the same `top`, so that threads with different
 // sizes do not lower it for each other
+constexpr size_t kLdsMax = 160 * 1024;   // of a block
 static hipError_t lds_limit(const void* kernel, size_t bytes, size_t top) {
     if (bytes <= 64 * 1024) return hipSuccess;
     return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)std::max(bytes, top));
 }
 
+static constexpr size_t hh_col_bytes(int n) { return 3 * (size_t)n * sizeof(double); }
+
 hipError_t householder_tridiag(int n, EigWork& w, hipStream_t st) {
-    if (n < 3) return hipErrorInvalidValue;   // the callers solve n <= 2 in closed form
+    if (n < 3 || n > kEigMaxN) return hipErrorInvalidValue;   // the callers solve n <= 2 in closed form
     // reflector rows must be zero outside their support for the blocked back-transform
     UNO_LAUNCH_FILL((long)n * n, w.V, st);
     // column launches down to the size that one block's registers hold: a whole solve of 192 takes
@@ -920,9 +923,9 @@ hipError_t householder_tridiag(int n, EigWork& w, hipStream_t st) {
     // rows' terms of p.v of the steps of even and odd k live there
     double* P[2] = {w.wk, w.wk + n};
     double* part[2] = {w.wk + 2L * n, w.wk + 3L * n};
-    const size_t lds = 3 * (size_t)n * sizeof(double);
+    const size_t lds = hh_col_bytes(n);
     if (k1 > 0)
-        if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_hh_col), lds, 150 * 1024)) return er;
+        if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_hh_col), lds, hh_col_bytes(kEigMaxN))) return er;
     for (int k = 0; k < k1; ++k) {
         const int b0 = (k + 1) / 32 * 8;
         hipLaunchKernelGGL(k_hh_col, dim3((unsigned)((n + 3) / 4 - b0)), dim3(256), lds, st, n, k, b0, w.A, w.V, w.tau, w.d, w.e,
@@ -1141,135 +1144,10 @@ __global__ __launch_bounds__(256) void k_bisect(int n, const double* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Inverse iteration: thread i solves (T - lambda_i I) x = b three times with a
-// partially pivoted LU of the tridiagonal (tiny pivots replaced by eps*|T|), from a
-// pseudo-random start vector seeded by i.  Work arrays and the vectors are interleaved
-// [k][thread] so the lanes of a wave touch consecutive addresses: the output Yt holds
-// eigenvector i in column i (Yt[k n + i]).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_inviter(int n, const double* __restrict__ d, const double* __restrict__ e,
-                                               const double* __restrict__ evals, double* __restrict__ Yt,
-                                               double* __restrict__ wk) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const long S = n;   // stride between k entries of one thread
-    double* U1 = wk;                  // reciprocal of the diagonal of U
-    double* U2 = wk + (long)n * S;    // first superdiagonal of U
-    double* U3 = wk + 2L * n * S;     // second superdiagonal (from pivoting)
-    double* L = wk + 3L * n * S;      // multipliers
-    double* x = Yt + i;               // x[k S]
-    double tnorm = 0.0;
-    for (int k = 0; k < n; ++k) tnorm = fmax(tnorm, fabs(d[k]) + (k + 1 < n ? fabs(e[k]) : 0.0) + (k > 0 ? fabs(e[k - 1]) : 0.0));
-    const double lam = evals[i];
-    const double tiny = 2.2204460492503131e-16 * fmax(tnorm, 1e-300);
-    int* piv = (int*)(wk + 4L * n * S);   // n*S ints fit in the space of n*S doubles
-    // factor T - lam I = P L U, row by row
-    double a = d[0] - lam, b = (n > 1) ? e[0] : 0.0;
-    auto pivot = [&](double u) {
-        if (fabs(u) < tiny) u = copysign(tiny, u == 0.0 ? 1.0 : u);
-        return 1.0 / u;
-    };
-    for (int k = 0; k < n - 1; ++k) {
-        const double sub = e[k], dn = d[k + 1] - lam, en = (k + 2 < n) ? e[k + 1] : 0.0;
-        if (fabs(a) >= fabs(sub)) {
-            const double aa = (a == 0.0) ? tiny : a;
-            const double l = sub / aa;
-            U1[(long)k * S + i] = pivot(aa); U2[(long)k * S + i] = b; U3[(long)k * S + i] = 0.0;
-            L[(long)k * S + i] = l; piv[(long)k * S + i] = 0;
-            a = dn - l * b;
-            b = en;
-        } else {
-            const double l = a / sub;
-            U1[(long)k * S + i] = pivot(sub); U2[(long)k * S + i] = dn; U3[(long)k * S + i] = en;
-            L[(long)k * S + i] = l; piv[(long)k * S + i] = 1;
-            a = b - l * dn;
-            b = -l * en;
-        }
-    }
-    U1[(long)(n - 1) * S + i] = pivot((a == 0.0) ? tiny : (fabs(a) < tiny ? copysign(tiny, a) : a));
-    // the last row's superdiagonals do not exist: stored as zeros, since the solves below
-    // multiply them (by zero) without a branch and the work space is not cleared
-    U2[(long)(n - 1) * S + i] = 0.0;
-    U3[(long)(n - 1) * S + i] = 0.0;
-    // start vector
-    unsigned int h = 2654435761u * (unsigned)(i + 1);
-    for (int k = 0; k < n; ++k) {
-        h ^= h << 13; h ^= h >> 17; h ^= h << 5;
-        x[k * S] = ((double)(h & 0xffffff) / 16777216.0) - 0.5 + 1e-3;
-    }
-    // the solves walk the vector in chunks of kCh entries: a chunk's loads are issued
-    // together ahead of its dependent chain (one memory latency per chunk, not per entry)
-    constexpr int kCh = 16;
-    for (int it = 0; it < 3; ++it) {
-        // forward: apply the row interchanges and multipliers
-        double xk = x[0];
-        for (int k0 = 0; k0 < n - 1; k0 += kCh) {
-            double xs[kCh], ls[kCh];
-            int ps[kCh];
-#pragma unroll
-            for (int c = 0; c < kCh; ++c) {
-                const int k = k0 + c;
-                if (k < n - 1) {
-                    xs[c] = x[(long)(k + 1) * S];
-                    ls[c] = L[(long)k * S + i];
-                    ps[c] = piv[(long)k * S + i];
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < kCh; ++c) {
-                if (k0 + c < n - 1) {
-                    const double xn = xs[c];
-                    if (ps[c]) {
-                        xs[c] = xn;
-                        xk = xk - ls[c] * xn;
-                    } else {
-                        xs[c] = xk;
-                        xk = xn - ls[c] * xk;
-                    }
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < kCh; ++c)
-                if (k0 + c < n - 1) x[(long)(k0 + c) * S] = xs[c];
-        }
-        x[(long)(n - 1) * S] = xk;
-        // back substitution with the banded U, then the norm
-        double x1 = 0.0, x2 = 0.0, nrm = 0.0;
-        for (int k1 = n - 1; k1 >= 0; k1 -= kCh) {
-            double xs[kCh], u1[kCh], u2[kCh], u3[kCh];
-#pragma unroll
-            for (int c = 0; c < kCh; ++c) {
-                const int k = k1 - c;
-                if (k >= 0) {
-                    xs[c] = x[(long)k * S];
-                    u1[c] = U1[(long)k * S + i];
-                    u2[c] = U2[(long)k * S + i];
-                    u3[c] = U3[(long)k * S + i];
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < kCh; ++c) {
-                if (k1 - c >= 0) {
-                    double v = xs[c];
-                    v -= u2[c] * x1;
-                    v -= u3[c] * x2;
-                    v *= u1[c];
-                    xs[c] = v;
-                    nrm = fma(v, v, nrm);
-                    x2 = x1;
-                    x1 = v;
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < kCh; ++c)
-                if (k1 - c >= 0) x[(long)(k1 - c) * S] = xs[c];
-        }
-        nrm = 1.0 / sqrt(nrm);
-        for (int k = 0; k < n; ++k) x[(long)k * S] *= nrm;
-    }
-}
-
-// The same solves with every work array in LDS, `lanes` eigenvectors per one-wave block: the factors'
+// Inverse iteration: a thread solves (T - lambda_i I) x = b three times with a partially pivoted
+// LU of the tridiagonal (tiny pivots replaced by eps*|T|), from a pseudo-random start vector
+// seeded by i; the output Yt holds eigenvector i in column i (Yt[k n + i]).  Every work array is in
+// LDS, `lanes` eigenvectors per one-wave block: the factors'
 // reciprocal pivots and multipliers and the vector itself.  A row interchange is one bit; the
 // superdiagonals of U follow from d, e, the bits and the multipliers.  The solves are chains of
 // dependent operations, so rows go in
@@ -1279,7 +1157,7 @@ __global__ __launch_bounds__(64) void k_inviter(int n, const double* __restrict_
 // within the range of recip.  n = 1216: 0.63 ms, n = 133: 79 us (with the arrays in global memory and
 // divides: 2.07 ms and 237 us).
 constexpr size_t kInvLds = 156 * 1024;
-static size_t inviter_bytes(int n) {   // LDS of one eigenvector
+static constexpr size_t inviter_bytes(int n) {   // LDS of one eigenvector
     const size_t np = eig_pad(n);
     return (3 * np + 1) * sizeof(double) + (np / kEigChunk + 1) / 2 * sizeof(double);
 }
@@ -1452,32 +1330,31 @@ __global__ __launch_bounds__(256) void k_cluster_mgs(int n, const int* __restric
     }
 }
 
-// doubles of EigWork::wk that a solve of this size uses: p and p.v of the column launches, the
-// blocked back-transform's rows, and the factors of the inverse iteration where LDS does not
-// hold one vector's (at most 5 n^2 for every n >= 3)
+// the largest matrix: one eigenvector's solves, and the column launches' three vectors, in a block's LDS
+static_assert(inviter_bytes(kEigMaxN) <= kLdsMax && inviter_bytes(kEigMaxN + 1) > kLdsMax, "one eigenvector per block");
+static_assert(kEigMaxN == eig_pad(kEigMaxN) && hh_col_bytes(kEigMaxN) + 64 <= kLdsMax, "a column launch's vectors");
+
+// doubles of EigWork::wk that a solve of this size uses: p and p.v of the column launches, and the
+// blocked back-transform's rows (at most 5 n^2 for every n >= 3)
 size_t eig_work_doubles(int n) {
-    const size_t sq = (size_t)n * n, wy = sq + (size_t)std::min(kWy, n) * n;
-    return inviter_bytes(n) <= kInvLds ? std::max(wy, 4 * (size_t)n) : 5 * sq;
+    return std::max((size_t)n * n + (size_t)std::min(kWy, n) * n, 4 * (size_t)n);
 }
 
 hipError_t tridiag_eigen(int n, EigWork& w, int nclusters, const int* clusters, hipStream_t st) {
+    if (n > kEigMaxN) return hipErrorInvalidValue;
     if (nclusters < 0) {
         const size_t lds = 2 * (size_t)n * sizeof(double);
+        if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_bisect), lds, 2 * kEigMaxN * sizeof(double))) return er;
         hipLaunchKernelGGL(k_bisect, dim3((unsigned)((n + 3) / 4)), dim3(256), lds, st, n, w.d, w.e, w.evals);
         return hipGetLastError();
     }
-    // as many eigenvectors per block as LDS holds, but no fewer blocks than compute units; sizes
-    // whose one vector does not fit use the work space in global memory
-    const int fit = (int)std::min<size_t>(64, kInvLds / inviter_bytes(n));
-    if (fit >= 1) {
-        const int lanes = std::max(1, std::min(fit, (n + 255) / 256));
-        const size_t lds = (size_t)lanes * inviter_bytes(n);
-        if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_inviter_lds), lds, kInvLds)) return er;
-        hipLaunchKernelGGL(k_inviter_lds, dim3((unsigned)((n + lanes - 1) / lanes)), dim3(64), lds, st, n, lanes,
-                           (const double*)w.d, (const double*)w.e, (const double*)w.evals, w.Y);
-    } else {
-        hipLaunchKernelGGL(k_inviter, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, n, w.d, w.e, w.evals, w.Y, w.wk);
-    }
+    // as many eigenvectors per block as LDS holds, but no fewer blocks than compute units
+    const int fit = (int)std::min<size_t>(64, std::max<size_t>(1, kInvLds / inviter_bytes(n)));
+    const int lanes = std::max(1, std::min(fit, (n + 255) / 256));
+    const size_t lds = (size_t)lanes * inviter_bytes(n);
+    if (hipError_t er = lds_limit(reinterpret_cast<const void*>(&k_inviter_lds), lds, kLdsMax)) return er;
+    hipLaunchKernelGGL(k_inviter_lds, dim3((unsigned)((n + lanes - 1) / lanes)), dim3(64), lds, st, n, lanes,
+                       (const double*)w.d, (const double*)w.e, (const double*)w.evals, w.Y);
     if (nclusters > 0) hipLaunchKernelGGL(k_cluster_mgs, dim3((unsigned)nclusters), dim3(256), 0, st, n, clusters, w.Y);
     return hipGetLastError();
 }

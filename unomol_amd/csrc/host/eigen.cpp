@@ -4,9 +4,9 @@
 //   1. Householder tridiagonalisation A = Q T Q^T (one block for the last 192 rows, before them one
 //      launch per column: the previous rank-2 update fused with the next matrix-vector product);
 //   2. eigenvalues of T by multisection on Sturm counts, one eigenvalue per wave;
-//   3. eigenvectors of T by inverse iteration, one per thread (the vectors stored as the
-//      columns of Yt, so a wave's accesses coalesce), then two-pass modified Gram-Schmidt
-//      inside clusters of close eigenvalues (exact degeneracies included);
+//   3. eigenvectors of T by inverse iteration in LDS, one per thread and a few per block (stored
+//      as the columns of Yt), then two-pass modified Gram-Schmidt inside clusters of close
+//      eigenvalues (exact degeneracies included);
 //   4. Z = Q Yt: the reflectors applied to Yt one by one up to n = 192, above it in compact-WY
 //      blocks of 32 (every block's T Vb formed in one launch, then two MFMA GEMMs per block).
 // The reference reduces with Householder and diagonalises T with implicit QL
@@ -120,6 +120,10 @@ static int eigh_core(int n, double* dA, double* dZ, double* h_evals, const EigBu
 }
 
 static int eigh_impl(EigenWS& w, int n, double* dA, double* dZ, double* h_evals, hipStream_t st) {
+    if (n > kEigMaxN) {
+        set_error("eigensolver: n = " + std::to_string(n) + " is above its largest size, " + std::to_string(kEigMaxN));
+        return UNO_EINVAL;
+    }
     UNO_HIP(w.ensure(n));
     w.hev.resize(std::max(n, 1));
     w.hcl.resize(std::max(n, 2));
