@@ -101,8 +101,8 @@ int uno_ctx_set(uno_ctx* ctx, const char* key, double value);
 /* Reads the knobs above and, read-only: "last_quartets" (shell quartets evaluated by the
  * last Fock build), "last_quartets32" (of which in FP32), "pairs" (significant shell
  * pairs), "pair_runs" (runs of the pair array: one per angular pair class and
- * primitive-count bucket, at most 36), "quartet_launches" (quartet spaces of a Fock build, the
- * pairs of those runs; one launch per class pair and precision walks them),
+ * primitive-count bucket, at most 36), "quartet_launches" (quartet spaces in the launches'
+ * tables, one for every two runs; one launch per class pair and precision walks its own),
  * and the context build's host milliseconds: "ctx_ms_pairs" (pair and primitive records
  * and their upload), "ctx_ms_schwarz" (Schwarz bounds on the device), "ctx_ms_runs"
  * (sorted runs, applied on the device) and "ctx_ms_rest". */
@@ -326,8 +326,8 @@ int uno_batch_nmol(const uno_batch* batch);
  * "queue" (0-2: kept for callers that set it; the launches no longer take work from a queue),
  * "launch_streams" (1-4: streams the launches are spread over, forked and joined
  * inside the build, parallel branches of the captured graph; default 3).  uno_batch_get
- * also reads the last run's "space_builds", "graph_builds", "graph_replays" and
- * "launches_per_build". */
+ * also reads "space_builds" (how often the launches' quartet spaces were built: with the
+ * batch), the last run's "graph_builds" and "graph_replays", and "launches_per_build". */
 int uno_batch_set(uno_batch* batch, const char* key, double value);
 int uno_batch_get(const uno_batch* batch, const char* key, double* value);
 /* The final density of molecule m after uno_batch_run, dense row-major N x N: the RHF half

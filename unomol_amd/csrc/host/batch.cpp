@@ -334,6 +334,7 @@ int uno_batch_create(int nmol, const uno_basis* bases, const int* nelec, uno_bat
             delete b;
             return rc;
         }
+        ++b->space_builds;
     }
     const size_t S = (size_t)b->store;
     DBuf<double>* stores[] = {&b->H, &b->S, &b->X, &b->P[0], &b->P[1], &b->Pold[0], &b->Pold[1], &b->F[0], &b->F[1],
@@ -447,7 +448,6 @@ int uno_batch_run(uno_batch* b, const uno_scf_opts* opts, uno_scf_result* res, d
     b->warm[0] = b->warm[1] = false;
     // the captured build belongs to one run
     b->drop_graph();
-    b->space_builds = 1;
     b->graph_builds = b->graph_replays = 0;
     {
         ClearList cl;

@@ -346,7 +346,7 @@ int uno_ctx_get(uno_ctx* c, const char* key, double* v) {
         *v = k == "last_quartets" ? c->last_quartets : c->last_quartets32;
     }
     else if (k == "pair_runs") *v = (double)c->cls.size();
-    else if (k == "quartet_launches") *v = (double)(c->cls.size() * (c->cls.size() + 1) / 2);
+    else if (k == "quartet_launches") *v = (double)c->fs.nspaces;
     else if (k == "pairs") *v = (double)c->pairs.size();
     else { set_error("unknown option " + k); return UNO_EINVAL; }
     return UNO_OK;

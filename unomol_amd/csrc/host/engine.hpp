@@ -104,6 +104,7 @@ struct FockLaunch {
 struct FockStore {
     int npair = 0;
     long long njp = 0, kps = 0;
+    int nspaces = 0;                       // in the tables, over all launches
     std::vector<FockLaunch> launches;
     DBuf<char> tables;
     // task lists (builds of more than a few thousand candidates): the launches as sources, FP64

@@ -126,6 +126,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
     // the launches: per launch group and class pair the spaces of every molecule, the ones with
     // the longest primitive loops first
     launches.clear();
+    nspaces = 0;
     std::vector<char> host;
     auto put = [&](const void* p, size_t bytes) {
         const size_t off = (host.size() + 15) / 16 * 16;
@@ -210,6 +211,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
                     blk.push_back(k);
                 }
                 L.sp = put(sp.data(), sp.size() * sizeof(FockSpace));
+                nspaces += (int)sp.size();
                 L.blk = put(blk.data(), blk.size() * sizeof(int));
                 launches.push_back(L);
             }
