@@ -119,7 +119,7 @@ struct FockStore {
     DBuf<int4> kidx, kjo;
     DBuf<int> knp, colinv;
     DBuf<int2> kcol;
-    DBuf<unsigned long long> nquart;       // FP64 launches' counters, then FP32's
+    DBuf<unsigned long long> nquart;       // FP64 launches' counters, then FP32's, then the tuner's
     int build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, const PrimPair* d_prims, int np, long long nprims,
               hipStream_t st);
     // arguments of launch k's FP64 (prec 0) or FP32 half, but for the densities and thresholds

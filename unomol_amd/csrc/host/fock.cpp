@@ -257,7 +257,7 @@ int FockStore::build(const std::vector<FockMol>& mols, const PairHdr* d_pairs, c
     UNO_HIP(dp.alloc((size_t)std::max(njp, 1LL)));
     UNO_HIP(jp.alloc((size_t)std::max(njp, 1LL)));
     UNO_HIP(dmax.alloc(mols.size()));
-    UNO_HIP(nquart.alloc(2 * kQuartSlots));
+    UNO_HIP(nquart.alloc(3 * kQuartSlots));
     UNO_HIP(pair_store(np, (int)pr.size(), dr.p, d_pairs, d_prims, dcm.p, bprim.p, kprim.p, kps, kgeo.p, kidx.p, kjo.p,
                        knp.p, kcol.p, st));
     UNO_HIP(hipStreamSynchronize(st));   // the host tables and the scratch buffers go
@@ -397,6 +397,8 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
                 hipEvent_t t0, t1;
                 UNO_HIP(hipEventCreate(&t0));
                 UNO_HIP(hipEventCreate(&t1));
+                unsigned long long* const counted = a.nquart;
+                a.nquart = fs.nquart.p + 2 * kQuartSlots;   // the candidates' counts go nowhere
                 for (int v = 0; v < 16; ++v) {
                     FockConfig g;
                     g.variant = v & 3;
@@ -423,6 +425,10 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
                 }
                 (void)hipEventDestroy(t0);
                 (void)hipEventDestroy(t1);
+                // once more with the chosen one, which counts
+                a.nquart = counted;
+                UNO_HIP(hipMemsetAsync(&a.ctr->head, 0, sizeof(int), st));
+                UNO_HIP(launch(best, st));
                 c->tune[key] = best;
                 c->tune_ms += best_ms;
                 continue;
