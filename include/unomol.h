@@ -100,7 +100,7 @@ int uno_ctx_destroy(uno_ctx* ctx);
 int uno_ctx_set(uno_ctx* ctx, const char* key, double value);
 /* Reads the knobs above and, read-only: "last_quartets" (shell quartets evaluated by the
  * last Fock build), "last_quartets32" (of which in FP32), "pairs" (significant shell
- * pairs), "pair_runs" (runs of the pair array: one per angular pair class and
+ * pairs), "tuned_launches" (the autotuner's configurations that this context holds), "pair_runs" (runs of the pair array: one per angular pair class and
  * primitive-count bucket, at most 36), "quartet_launches" (quartet spaces in the launches'
  * tables, one for every two runs; one launch per class pair and precision walks its own),
  * and the context build's host milliseconds: "ctx_ms_pairs" (pair and primitive records
@@ -208,7 +208,8 @@ int uno_schwarz(uno_ctx* ctx, double* q);
  * none, with and without the density rows and shell maxima in LDS) of every ERI launch
  * of one Fock build on the given density (PB null: RHF P; else UHF Pa, Pb; packed, as
  * uno_fock_rhf/uhf) and keeps the fastest per launch, for this context and for every later
- * context of the same basis layout in this process.  mixed = 1 tunes the mixed-precision
+ * context of the same basis layout in this process (functions, shells, pairs, and the classes and
+ * primitive buckets of their runs).  mixed = 1 tunes the mixed-precision
  * build's launches.  best_ms (optional) receives the tuned launches' summed kernel time.
  * G is not produced; the next Fock build starts from scratch. */
 int uno_autotune(uno_ctx* ctx, const double* P, const double* PB, int mixed, double* best_ms);

@@ -29,3 +29,30 @@ def test_quartet_counts_survive_tuning(tmp_path, mixed):
     assert counts[0] > 0 and (counts[1] > 0) == mixed
     assert t.autotune(P, mixed=mixed) > 0.0
     assert (t.get("last_quartets"), t.get("last_quartets32")) == counts
+
+
+def _deck_text(prims):
+    """Twelve close atoms (no shell pair is cut) with three s shells each, the first of them a contraction
+    of `prims`."""
+    first = [(38.36, 0.0238), (5.77, 0.1549), (1.24, 0.4699)][-prims:]
+    shells = [(c, s) for c in range(12) for s in (first, [(0.85, 1.0)], [(0.298, 1.0)])]
+    text = ["%6d %6d %6d %3d" % (36, 36, 12, 0), "%6d %6d" % (24, 60), " 1e-10", " 0 0", " 2 0 0", " 0 0 0"]
+    text += ["2.0 %.6f %.6f %.6f" % (1.0 * (c % 3), 1.05 * (c // 3), 0.02 * c) for c in range(12)]
+    for c, s in shells:
+        text.append("%3d 0 %d" % (len(s), c))
+        text += ["%.10f %.10f" % p for p in s]
+    return "\n".join(text) + "\n"
+
+
+def test_tuning_is_recalled_for_the_same_contraction_only():
+    """Two bases of equal functions, shells and pairs whose runs differ in their primitive buckets."""
+    print("[gpu-test] tuning recalled by layout", flush=True)
+    one, three = unomol_amd.Basis(text=_deck_text(1)), unomol_amd.Basis(text=_deck_text(3))
+    t = unomol_amd.TwoElectronInts(three)
+    t.set("row_min_kets", 1)
+    other = unomol_amd.TwoElectronInts(one)
+    assert t.get("pairs") == other.get("pairs") and t.get("pair_runs") != other.get("pair_runs")
+    P = np.ascontiguousarray(np.eye(36)[np.tril_indices(36)])
+    assert t.autotune(P) > 0.0 and t.get("tuned_launches") == 1
+    assert unomol_amd.TwoElectronInts(three).get("tuned_launches") == 1
+    assert unomol_amd.TwoElectronInts(one).get("tuned_launches") == 0

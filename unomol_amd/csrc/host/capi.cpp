@@ -347,6 +347,7 @@ int uno_ctx_get(uno_ctx* c, const char* key, double* v) {
     }
     else if (k == "pair_runs") *v = (double)c->cls.size();
     else if (k == "quartet_launches") *v = (double)c->fs.nspaces;
+    else if (k == "tuned_launches") *v = (double)c->tune.size();
     else if (k == "pairs") *v = (double)c->pairs.size();
     else { set_error("unknown option " + k); return UNO_EINVAL; }
     return UNO_OK;

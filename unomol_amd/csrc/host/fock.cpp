@@ -7,6 +7,7 @@
 #include <climits>
 #include <cstdint>
 #include <cmath>
+#include <mutex>
 #include "engine.hpp"
 
 namespace uno {
@@ -297,20 +298,26 @@ int FockStore::list_tasks(bool mixed, const FockArgs& a, hipStream_t st) const {
     return UNO_OK;
 }
 
-// tuned configurations, shared by every context of the same layout (basis size, shells, pairs
-// and launches) in this process
-static std::map<std::tuple<int, int, int, int>, std::map<std::tuple<int, int, int, int>, FockConfig>> g_tuning;
+// tuned configurations, shared by every context of the same layout in this process: basis size,
+// shells, pairs and the runs' classes and primitive buckets (two contractions of the same shells
+// differ in those alone)
+static std::map<std::vector<int>, std::map<std::tuple<int, int, int, int>, FockConfig>> g_tuning;
+static std::mutex g_tuning_mutex;
 
-static std::tuple<int, int, int, int> tuning_key(const uno_ctx* c) {
-    return std::make_tuple(c->n, c->nsh, (int)c->pairs.size(), (int)c->fs.launches.size());
+static std::vector<int> tuning_key(const uno_ctx* c) {
+    std::vector<int> key{c->n, c->nsh, (int)c->pairs.size()};
+    for (const PairClassList& L : c->cls) key.push_back(L.lcls * kNumBuckets + L.bucket);
+    return key;
 }
 
 void remember_tuning(uno_ctx* c) {
+    const std::lock_guard<std::mutex> lock(g_tuning_mutex);
     auto& m = g_tuning[tuning_key(c)];
     for (const auto& kv : c->tune) m[kv.first] = kv.second;
 }
 
 void recall_tuning(uno_ctx* c) {
+    const std::lock_guard<std::mutex> lock(g_tuning_mutex);
     auto it = g_tuning.find(tuning_key(c));
     c->tune.clear();
     if (it != g_tuning.end()) c->tune = it->second;
