@@ -88,8 +88,8 @@ int uno_ctx_destroy(uno_ctx* ctx);
  * bra row and the Rys table, 2 every bra row, 3 the first bra shell's rows; 0, the
  * default, takes the first that fits the LDS budget; another value, or a layout that does not
  * fit, falls back to that choice), "row_density_lds" (the bra's exchange density rows staged
- * in LDS beside the merged rows: -1, the default, wherever they fit the budget and the
- * autotuner does not prefer otherwise; 0 never; 1 wherever they fit), "rys2_exact" (0, the
+ * in LDS beside the merged rows: -1, the default, for (ss|ss) where they fit the budget, or as
+ * the autotuner found best; 0 never; 1 wherever they fit), "rys2_exact" (0, the
  * default: the two-root classes use the reference's own two-root quadrature,
  * Rys.cpp:413-631, which for 15 < x <= 33 departs from the exact quadrature by up to
  * 3.5e-4 relative, so that ERIs match the reference to 1e-12; 1: the exact quadrature),
@@ -209,7 +209,8 @@ int uno_schwarz(uno_ctx* ctx, double* q);
  * of one Fock build on the given density (PB null: RHF P; else UHF Pa, Pb; packed, as
  * uno_fock_rhf/uhf) and keeps the fastest per launch, for this context and for every later
  * context of the same basis layout in this process (functions, shells, pairs, and the classes and
- * primitive buckets of their runs).  mixed = 1 tunes the mixed-precision
+ * primitive buckets of their runs).  A row_variant or row_density_lds that the caller sets goes
+ * before what was found.  mixed = 1 tunes the mixed-precision
  * build's launches.  best_ms (optional) receives the tuned launches' summed kernel time.
  * G is not produced; the next Fock build starts from scratch. */
 int uno_autotune(uno_ctx* ctx, const double* P, const double* PB, int mixed, double* best_ms);

@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 import unomol_amd
+from unomol_amd import _native as N
 
 pytestmark = pytest.mark.gpu
 
@@ -29,6 +30,32 @@ def test_quartet_counts_survive_tuning(tmp_path, mixed):
     assert counts[0] > 0 and (counts[1] > 0) == mixed
     assert t.autotune(P, mixed=mixed) > 0.0
     assert (t.get("last_quartets"), t.get("last_quartets32")) == counts
+
+
+def _launches_by_kind(t, P):
+    slots = [np.zeros(432) for _ in range(4)]
+    N.check(N.lib().uno_profile(t.ctx, 1, None, None, None, None))
+    t.formGmatrix(P, np.zeros_like(P))
+    N.check(N.lib().uno_profile(t.ctx, -1, *[N.ptr(s) for s in slots]))
+    N.check(N.lib().uno_profile(t.ctx, 0, None, None, None, None))
+    return slots[1].reshape(6, 2, 6, 6)[:, 0].sum(axis=(1, 2))
+
+
+@pytest.mark.parametrize("variant", [1, 2, 3])
+def test_forced_layout_goes_before_the_tuned_one(tmp_path, variant):
+    """Every launch of the lane kernels (products of up to 162 components) in the forced layout, and
+    all of them again as tuned when the knob is back at its default."""
+    print("[gpu-test] forced layout %d after tuning" % variant, flush=True)
+    b, t, P = _context(tmp_path)
+    t.set("row_min_kets", 1)
+    assert t.autotune(P) > 0.0
+    tuned = _launches_by_kind(t, P)
+    t.set("row_variant", variant)
+    comps = np.array([1, 3, 9, 6, 18, 36])
+    lane = int(((np.multiply.outer(comps, comps) <= 162) & np.tril(np.ones((6, 6), bool))).sum())
+    assert _launches_by_kind(t, P)[variant] == lane
+    t.set("row_variant", 0)
+    assert np.array_equal(_launches_by_kind(t, P), tuned)
 
 
 def _deck_text(prims):

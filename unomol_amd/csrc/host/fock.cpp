@@ -387,11 +387,17 @@ int fock_build(uno_ctx* c, bool uhf, bool mixed) {
             const bool rows = rows_on && l.nket >= c->row_min_kets;
             FockConfig f = fock_default(l.cx, l.cy, mode, l.ncols, c->nsh, prec == 1, rows, c->row_variant, c->row_dens);
             const auto key = std::make_tuple(kNumPairClasses * l.cx + l.cy, prec, uhf ? 1 : 0, mixed ? 1 : 0);
-            if (rows && !c->tuning) {
+            // (a layout that the caller forces, and that fits, goes before the tuned one)
+            if (rows && !c->tuning && !(c->row_variant && f.variant == c->row_variant)) {
                 auto it = c->tune.find(key);
-                if (it != c->tune.end() &&
-                    fock_config_fits(l.cx, l.cy, it->second, mode, l.ncols, c->nsh, prec == 1))
-                    f = it->second;
+                if (it != c->tune.end()) {
+                    auto fits = [&](const FockConfig& g) { return fock_config_fits(l.cx, l.cy, g, mode, l.ncols, c->nsh, prec == 1); };
+                    FockConfig g = it->second;
+                    if (c->row_dens == 0) g.dlds = 0;
+                    if (fits(g)) f = g;
+                    g.dlds = 1;
+                    if (c->row_dens > 0 && g.variant && fits(g)) f = g;
+                }
             }
             const int ci = prec * kNumPairClasses * kNumPairClasses + l.cx * kNumPairClasses + l.cy;
             auto launch = [&](const FockConfig& g, hipStream_t s) {
