@@ -74,8 +74,18 @@ int upload_params(uno_mlp* m, const float* hp) {
     return UNO_OK;
 }
 
+// rows of the buffers for batches of B: up to 65536 the next power of two, so that a row count that
+// creeps up from call to call does not free and allocate them each time
+int row_capacity(int B) {
+    int cap = 64;
+    while (cap < B && cap < 65536) cap *= 2;
+    return std::max(cap, B);
+}
+
 int ensure_batch(uno_mlp* m, int B) {
     if (B <= m->bcap) return UNO_OK;
+    B = row_capacity(B);
+    m->bcap = 0;   // until every buffer is there
     const int L = nlayers(m);
     int wmax = 0;
     for (int d : m->dims) wmax = std::max(wmax, d);
@@ -235,9 +245,10 @@ int uno_mlp_forward(uno_mlp* m, long n, const float* X, float* Y) {
     const int in = m->dims[0], out = m->dims.back();
     const size_t rows = (size_t)((n + 63) / 64) * 64;
     // rows of a pass: as many as there are, to 16384 (a pass ends waiting for its copy)
-    const int chunk = (int)std::min<size_t>(std::max<size_t>(rows, 4096), 16384);
+    constexpr size_t kMaxPass = 16384;
+    const int chunk = (int)std::min(std::max<size_t>(rows, 4096), kMaxPass);
     if (int rc = ensure_batch(m, chunk)) return rc;
-    UNO_HIP(m->xin.alloc(rows * in));
+    UNO_HIP(m->xin.alloc(rows <= kMaxPass ? (size_t)m->bcap * in : (rows + kMaxPass - 1) / kMaxPass * kMaxPass * in));
     UNO_HIP(hipMemcpyAsync(m->xin.p, X, (size_t)n * in * sizeof(float), hipMemcpyHostToDevice, m->st));
     if (rows > (size_t)n) UNO_HIP(hipMemsetAsync(m->xin.p + (size_t)n * in, 0, (rows - n) * in * sizeof(float), m->st));
     for (long r0 = 0; r0 < n; r0 += chunk) {
