@@ -244,7 +244,11 @@ int ctx_build(uno_ctx* c, const uno_basis* b, int start_shell) {
     std::vector<PrimPair> prims2(c->prims.size());
     std::vector<double> q2(np);
     std::vector<int> newidx(np);
-#pragma omp parallel for schedule(static) if (np >= 32768)   // below, one thread is done before the others wake
+    // all threads from 32768 pairs on; below, one is done before the others wake.  The stage on one
+    // thread and on all, ms: 22849 pairs 0.8 and 1.4 when contexts follow each other, 1.6-1.9 and 1.5 for
+    // one after a pause; 31839 pairs 1.1 and 1.8, 2.3-3.4 and 2.1; 52064 pairs 2.9-3.5 and 2.8-3.1, 4.7
+    // and 3.4
+#pragma omp parallel for schedule(static) if (np >= 32768)
     for (int k = 0; k < np; ++k) {
         PairHdr h = c->pairs[order[k]];
         const int p0 = h.prim0;
