@@ -472,6 +472,7 @@ int scf_run(uno_ctx* c, int nelec, const uno_scf_opts& o, uno_scf_result& r, dou
             c->tau = tau0;
             if (rc) return rc;
         }
+        const double enqueue_s = secs(t0, clk::now());
         for (int s = 0; s < ns; ++s) {
             UNO_HIP(k_sym_w(n, s == 0 ? c->W0.p : c->W1.p, b.G[s].p, st, !full));
             if (o.incremental)
@@ -492,9 +493,9 @@ int scf_run(uno_ctx* c, int nelec, const uno_scf_opts& o, uno_scf_result& r, dou
         r.quartets32 += c->last_quartets32;
         if (o.verbose > 1)
             std::fprintf(stderr,
-                         "[scf] build %d: %s %s, %.2f ms, %.3e shell quartets (%.3e FP32)\n", r.nfock + 1,
-                         full ? "full" : "incremental", mixed ? "mixed" : "FP64", 1e3 * build_s, c->last_quartets,
-                         c->last_quartets32);
+                         "[scf] build %d: %s %s, %.2f ms (host: enqueue %.2f), %.3e shell quartets (%.3e FP32)\n",
+                         r.nfock + 1, full ? "full" : "incremental", mixed ? "mixed" : "FP64", 1e3 * build_s,
+                         1e3 * enqueue_s, c->last_quartets, c->last_quartets32);
         r.quartets += c->last_quartets;
         ++r.nfock;
         energy = uhf ? hs[0] + 0.5 * hs[1] : 2.0 * hs[0] + hs[1];
