@@ -411,7 +411,7 @@ def main():
         return t, hf, e, dt
 
     step_opts = fp64_opts if args.fp64_only else fast_opts
-    # autotuner (outside the timed region, once per basis layout): every quartet space's
+    # autotuner (outside the timed region, once per basis layout): every ERI launch's
     # row-merge configuration timed on a two-iteration density, for the mixed and the FP64
     # builds; later contexts of this deck pick the choices up
     tune = None
@@ -449,7 +449,7 @@ def main():
         ablation["mixed+learned, no FP32 quartets"] = {"scf_s": round(dta, 4), "iterations": hfa.result.iterations,
                                                        "energy_diff_vs_fp64": ea - e64}
         log("ablation no FP32 quartets: E=%.10f in %.2f s, %d iterations" % (ea, dta, hfa.result.iterations))
-        # deterministic Fock builds (fixed-point J/K accumulation, wave tasks only) beside the
+        # deterministic Fock builds (fixed-point J/K accumulation, without LDS rows) beside the
         # default FP64 build on the FP64 run's converged density: wall time per build (packed P
         # up, packed G down included), bitwise repeat, largest difference from the default
         def timed_build(ctx):

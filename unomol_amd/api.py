@@ -73,7 +73,7 @@ class TwoElectronInts:
         return v.value
 
     def autotune(self, P, PB=None, mixed=False):
-        """Times the row-merge configurations of every quartet space on density P (packed;
+        """Times the row-merge configurations of every ERI launch on density P (packed;
         PB for UHF) and keeps the fastest; returns the tuned build's kernel milliseconds."""
         P = np.ascontiguousarray(P, dtype=np.float64)
         pb = None if PB is None else np.ascontiguousarray(PB, dtype=np.float64)
@@ -396,8 +396,8 @@ class Batch:
         N.check(N.lib().uno_batch_set(self.h, key.encode(), C.c_double(value)))
 
     def get(self, key):
-        """An option, or a counter of the last run: space_builds, graph_builds, graph_replays,
-        launches_per_build."""
+        """An option, or a counter: of the last run graph_builds and graph_replays, of the batch
+        space_builds and launches_per_build."""
         v = C.c_double()
         N.check(N.lib().uno_batch_get(self.h, key.encode(), C.byref(v)))
         return v.value
