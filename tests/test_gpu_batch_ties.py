@@ -1,5 +1,5 @@
-"""GPU tests of the batched SCF where an exactly degenerate level is half filled on the way: HF in
-6-31G, whose pi pair the first Fock builds leave with one of its two orbitals occupied."""
+"""GPU tests of the batched SCF where an exactly degenerate level is half filled on the way: HF, whose
+pi pair the first Fock builds leave with one of its two orbitals occupied."""
 import numpy as np
 import pytest
 
@@ -11,9 +11,9 @@ SEEDS = range(101, 125)
 AXES = {"z": (0, 0, 1), "x": (1, 0, 0), "skew": (0.36, -0.48, 0.8)}
 
 
-def _deck(tmp_path, seed, axis):
+def _deck(tmp_path, seed, axis, basis="6-31G"):
     path = str(tmp_path / "hf.dat")
-    unomol_amd.generate_deck(path, "molecule", 1, seed, "6-31G", 0, 1e-8, 200)
+    unomol_amd.generate_deck(path, "molecule", 1, seed, basis, 0, 1e-8, 200)
     with open(path) as f:
         deck = parse_deck(f.read())
     assert list(deck["charge"]) == [9.0, 1.0]
@@ -32,13 +32,14 @@ def _densities(decks):
     return out
 
 
+@pytest.mark.parametrize("basis", ["6-31G", "6-31G*"])
 @pytest.mark.parametrize("axis", sorted(AXES))
-def test_half_filled_pair_repeats(tmp_path, axis):
+def test_half_filled_pair_repeats(tmp_path, axis, basis):
     """The densities of 24 HF molecules from two runs of one batch, and from batches of a few with a
     water for company (other launches, another order of the Fock sums), agree to 1e-9; the other
     choice of the pair is 2e-7 away.  (Rounding alone leaves less than 1e-11.)"""
-    print("[gpu-test] batch, half-filled pi pairs along %s" % axis, flush=True)
-    decks = [_deck(tmp_path, s, axis) for s in SEEDS]
+    print("[gpu-test] batch, half-filled pi pairs along %s, %s" % (axis, basis), flush=True)
+    decks = [_deck(tmp_path, s, axis, basis) for s in SEEDS]
     water = str(tmp_path / "water.dat")
     unomol_amd.generate_deck(water, "water_cluster", 4, 5, "6-31G*", 0, 1e-8, 200)
     runs = _densities(decks)
