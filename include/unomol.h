@@ -116,7 +116,8 @@ int uno_fock_rhf(uno_ctx* ctx, const double* P, double* G);
  * Gs += J[PA+PB] - K[Ps]. */
 int uno_fock_uhf(uno_ctx* ctx, const double* PA, const double* PB, double* GA, double* GB);
 
-/* Replaces SymmPack::rsp(n, a, z, evals, tmp) (SymmPack.cpp:272-288). */
+/* Replaces SymmPack::rsp(n, a, z, evals, tmp) (SymmPack.cpp:272-288).  n up to 6752, where the
+ * solver's vectors fill a block's shared memory; larger n returns UNO_EINVAL. */
 int uno_eigh_packed(int n, double* a, double* z, double* evals);
 /* No counterpart in the reference: uno_eigh_packed for callers that cannot allocate device
  * memory (code under stream capture, tight serving loops, harnesses that forbid hipMalloc).
